@@ -24,6 +24,7 @@ struct GridDev {
     float bminx, bminy, bminz, bmaxx, bmaxy, bmaxz;
     float h1x, h1y, h1z;   // Level1 half extents
     float h2x, h2y, h2z;   // Level2 half extents
+    float s2x, s2y, s2z, d2x, d2y, d2z;   // Level2 SAT rows: scale and table deviation per axis (SatScale)
     const float* c1x; const float* c1y; const float* c1z;   // [n]    Level1 SAT centers
     const float* r1x; const float* r1y; const float* r1z;   // [n]    Level1 ray origins
     const float* c2x; const float* c2y; const float* c2z;   // [n*n2] Level2 SAT centers
@@ -44,7 +45,7 @@ struct MeshOff {
     uint32_t b0;
     uint32_t ptask0;   // first Level1 parity task (16 layers x 64 columns of one row)
     uint32_t pw0;      // first Level2 parity wave (set on the host once boundary counts are known)
-    uint32_t pad;
+    uint32_t sg0;      // first Level2 SAT group (set on the host likewise)
 };
 
 // Per-mesh results accumulated on the device.
@@ -101,7 +102,7 @@ void launch_fill_u64(uint64_t* p, uint64_t v, int64_t n, hipStream_t s);
 void launch_mesh_ids(const MeshOff* off, int nm, int64_t T, uint32_t* tri_mesh, hipStream_t s);
 // part 1 (and 3) also raise *bad_input for a coordinate outside the domain
 void launch_tri_setup(const float* tris, int64_t T, const GridDev& g0, const Meshes& M, int4* box0, int4* box1,
-                      uint32_t* sat_items, int4* ray_rng, uint32_t* ray_items, double4* slab1, float4* slab2, int part,
+                      uint32_t* sat_items, int4* ray_rng, uint32_t* ray_items, double4* slab1, int part,
                       unsigned long long* bad_input, hipStream_t s);
 
 // exclusive scan of n u32 into out[0..n] (out[n] = total); tmp sized by
@@ -136,17 +137,16 @@ struct TileSortTmp {
 };
 size_t ts_tiles(uint64_t nkeys);
 
-// Level2 SAT voxel groups (k_l2_sat_grp): at most kL2GroupMax voxels, their
-// Level2 words within one wave's 64 and their 3 * n2 centers each within
-// kL2GroupCenters floats of LDS
+// Level2 SAT voxel groups (k_l2_sat): consecutive boundary voxels of a mesh
+// that share a wave, at most `most` and kL2GroupMax of them, their layer bits
+// (a byte per sub-column, two above n2 = 8) within kL2GroupBytes of LDS
 constexpr int kL2GroupMax = 16;
-constexpr int kL2GroupCenters = 192;
-__host__ __device__ inline int l2_group_voxels(int w2, int n2)
+constexpr int kL2GroupBytes = 1024;
+__host__ __device__ inline int l2_group_voxels(int n2, int most)
 {
-    int c = w2 > 0 ? 64 / w2 : 64;
+    int c = n2 > 0 ? kL2GroupBytes / (n2 * n2 * (n2 > 8 ? 2 : 1)) : kL2GroupMax;
     if (c > kL2GroupMax) c = kL2GroupMax;
-    if (n2 > 0 && c > kL2GroupCenters / (3 * n2)) c = kL2GroupCenters / (3 * n2);
-    return c;
+    return c < most ? c : most;
 }
 // column entries (key = column << 32 | triangle) -> CSR by column with the MT
 // records; ncol <= 2^27
@@ -190,14 +190,10 @@ void launch_bin_pairs(uint64_t* bits, bool ranked, const uint32_t* tri, uint64_t
 // per-mesh bin totals and largest bin (multi-mesh runs)
 void launch_mesh_bins(const uint32_t* boff, int64_t B, const Meshes& M, hipStream_t s);
 
-// Level2 SAT work groups of consecutive boundary voxels: flag[B], gidx[B+1]
-// (gidx[B] = group count), gstart[B+1]
-void launch_l2_groups(const uint32_t* boff, int64_t B, const GridDev& g0, const Meshes& M, uint32_t* flag,
-                      uint32_t* gidx, uint32_t* scan_tmp, uint32_t* gstart, hipStream_t s);
-// gmax: an upper bound of the group count (grouped form); waves: per block (1, 2, 4)
-void launch_l2_sat(const float* tris, const int32_t* bidx, int64_t B, const uint32_t* boff, const uint32_t* list,
-                   const uint64_t* pmask, const float4* slab2, const uint32_t* gstart, const uint32_t* ngroups,
-                   int64_t gmax, int waves, const GridDev& g0, const Meshes& M, uint64_t* sat2, hipStream_t s);
+// ngroups waves of at most gmost voxels each (l2_group_voxels); waves: per block (1, 2, 4)
+void launch_l2_sat(const float* tris, const int32_t* bidx, int64_t B, int64_t ngroups, int gmost, const uint32_t* boff,
+                   const uint32_t* list, const uint64_t* pmask, int waves, const GridDev& g0, const Meshes& M,
+                   uint64_t* sat2, hipStream_t s);
 // det/u/v pass bits per (column entry, sub-column): stride words per entry
 void launch_col_pass(const float4* rec, const GridDev& g0, const Meshes& M, uint64_t nent, int stride, int waves,
                      uint64_t* cpass, hipStream_t s);

@@ -16,6 +16,7 @@
 // with integer OR / ballot only, so results are deterministic.
 #include "gpv_device.hpp"
 #include "gpv_internal.hpp"
+#include "gpv_satrow.hpp"
 #include "gpv_slab.hpp"
 
 namespace gpv {
@@ -301,7 +302,6 @@ __global__ __launch_bounds__(256) void k_tri_setup(const float* __restrict__ tri
                                                    int4* __restrict__ ray_rng,
                                                    uint32_t* __restrict__ ray_items,
                                                    double4* __restrict__ slab1,
-                                                   float4* __restrict__ slab2,
                                                    unsigned long long* __restrict__ bad_input)
 {
     uint64_t tests = 0;
@@ -348,16 +348,6 @@ __global__ __launch_bounds__(256) void k_tri_setup(const float* __restrict__ tri
                 const PlaneSlab sl = plane_slab(tv, g.h1x, g.h1y, g.h1z, clo, chi);
                 slab1[t] = make_double4(sl.nx, sl.ny, sl.nz, sl.lim);
             }
-            if (any && g.n2 > 0) {
-                // over every Level2 center of the index AABB's Level1 voxels (the
-                // tables are monotone, so the extreme entries bound them)
-                const int n2 = g.n2;
-                const double clo[3] = {g.c2x[(int64_t)lo[0] * n2], g.c2y[(int64_t)lo[1] * n2], g.c2z[(int64_t)lo[2] * n2]};
-                const double chi[3] = {g.c2x[(int64_t)(lo[0] + dd[0]) * n2 - 1], g.c2y[(int64_t)(lo[1] + dd[1]) * n2 - 1],
-                                       g.c2z[(int64_t)(lo[2] + dd[2]) * n2 - 1]};
-                const FloatSlab f = float_slab(plane_slab(tv, g.h2x, g.h2y, g.h2z, clo, chi), tv, clo, chi);
-                slab2[t] = make_float4(f.nx, f.ny, f.nz, f.lim);
-            }
         }
         if constexpr ((kPart & 2) == 0) continue;
         uint32_t rit = 0;
@@ -395,30 +385,30 @@ __global__ __launch_bounds__(256) void k_tri_setup(const float* __restrict__ tri
 
 template <int kPart>
 static void tri_setup_part(const float* tris, int64_t T, const GridDev& g0, const Meshes& M, int4* box0, int4* box1,
-                           uint32_t* sat_items, int4* ray_rng, uint32_t* ray_items, double4* slab1, float4* slab2,
+                           uint32_t* sat_items, int4* ray_rng, uint32_t* ray_items, double4* slab1,
                            unsigned long long* bad_input, hipStream_t s)
 {
     if (M.nm > 1)
         k_tri_setup<true, kPart><<<grid_for(T, 256, 1 << 30), 256, 0, s>>>(tris, T, g0, M, box0, box1, sat_items,
-                                                                            ray_rng, ray_items, slab1, slab2,
+                                                                            ray_rng, ray_items, slab1,
                                                                             bad_input);
     else
         k_tri_setup<false, kPart><<<grid_for(T, 256, 1024), 256, 0, s>>>(tris, T, g0, M, box0, box1, sat_items,
-                                                                          ray_rng, ray_items, slab1, slab2,
+                                                                          ray_rng, ray_items, slab1,
                                                                           bad_input);
 }
 
 void launch_tri_setup(const float* tris, int64_t T, const GridDev& g0, const Meshes& M, int4* box0, int4* box1,
-                      uint32_t* sat_items, int4* ray_rng, uint32_t* ray_items, double4* slab1, float4* slab2,
+                      uint32_t* sat_items, int4* ray_rng, uint32_t* ray_items, double4* slab1,
                       int part, unsigned long long* bad_input, hipStream_t s)
 {
     if (T <= 0) return;
     if (part == 1)
-        tri_setup_part<1>(tris, T, g0, M, box0, box1, sat_items, ray_rng, ray_items, slab1, slab2, bad_input, s);
+        tri_setup_part<1>(tris, T, g0, M, box0, box1, sat_items, ray_rng, ray_items, slab1, bad_input, s);
     else if (part == 2)
-        tri_setup_part<2>(tris, T, g0, M, box0, box1, sat_items, ray_rng, ray_items, slab1, slab2, bad_input, s);
+        tri_setup_part<2>(tris, T, g0, M, box0, box1, sat_items, ray_rng, ray_items, slab1, bad_input, s);
     else
-        tri_setup_part<3>(tris, T, g0, M, box0, box1, sat_items, ray_rng, ray_items, slab1, slab2, bad_input, s);
+        tri_setup_part<3>(tris, T, g0, M, box0, box1, sat_items, ray_rng, ray_items, slab1, bad_input, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -1733,30 +1723,29 @@ void launch_mesh_bins(const uint32_t* boff, int64_t B, const Meshes& M, hipStrea
 }
 
 // ---------------------------------------------------------------------------
-// Level2 SAT (src/Object.cpp:2344-2424).  Two forms: one wave per boundary
-// voxel (k_l2_sat_voxel), and one wave per group of consecutive boundary
-// voxels (k_l2_sat_grp: same mesh, first bin entries in one 64-entry chunk,
-// at most L2_GMAX voxels and 64 Level2 words), so voxels with few bin entries
-// share the wave's rounds and SAT batches.  Each bin entry carries its box-axis masks
-// (the SAT's own box-axis predicate per sub-index, computed with the bins)
-// and its triangle a plane slab (gpv_slab.hpp) valid over every Level2
-// center of its index AABB.  The lanes take the (entry, sub-column) items its
-// x/y masks allow, drop sub-columns whose e x z edge predicates separate, and
-// keep the sub-voxels r whose float |N.(c - t0)| the slab admits (the bound
-// is grown by that evaluation's error, so the SAT rejects every other one);
-// those queue for the full float SAT in 64-lane batches.  Sub-voxels already
-// set are skipped (the result is an OR).
+// Level2 SAT (src/Object.cpp:2344-2424).  One wave per group of consecutive
+// boundary voxels of a mesh (l2_group_voxels).  Up to 32 bin entries at a time
+// are staged, two lanes each: what the rows of the entry share
+// (gpv_satrow.hpp) goes to LDS.  The lanes then take the (entry, row of
+// sub-voxels) items and walk each row's columns, which gives per column the
+// layers the SAT accepts for certain and those it has to be run on: the
+// first go straight into the wave's accumulator, the others (0.05 per entry
+// on the torus knot, 9 on a lattice-snapped mesh at 512/16) queue for the
+// reference's float SAT in 64-lane batches.
+//
+// What bounds it: VALU issue (0.58-0.65 of the measured rate at 4.5 waves per
+// SIMD; 85 registers and 7 KB of LDS allow five).  Running the float SAT on
+// every box a plane slab kept took 3.0e8 more instructions on the torus knot:
+// 0.556 -> 0.277 ms alone at 256/8; lattice-snapped mesh at 512/16, 5.25 ->
+// 3.6 ms.  Two staging lanes per entry and 32 entries per staging, because the
+// 40 floats an entry's rows share would otherwise fill LDS (64 entries: three
+// waves per SIMD), and recomputing them in every row costs 330 instructions a
+// round (torus knot 0.36 ms).
 // ---------------------------------------------------------------------------
 // ring of queued (triangle, sub-voxel) entries per wave: a round pushes at
 // most 64 entries onto fewer than 64 already queued, so it holds 128
 constexpr int L2_QCAP = 128;
-constexpr int L2_GMAX = kL2GroupMax;   // voxels per group
-constexpr int L2_CMAX = kL2GroupCenters;   // center floats per group: 3 * voxels * n2
-
-// 1/d for the sub-box widths d = 1..16 (float quotients, as 1.0f / d)
-__constant__ float kInvSmall[17] = {0.0f,        1.0f,        0.5f,        1.0f / 3.0f, 0.25f,       0.2f,
-                                    1.0f / 6.0f, 1.0f / 7.0f, 0.125f,      1.0f / 9.0f, 0.1f,        1.0f / 11.0f,
-                                    1.0f / 12.0f, 1.0f / 13.0f, 1.0f / 14.0f, 1.0f / 15.0f, 0.0625f};
+constexpr int L2_STAGE = 32;   // entries staged at once
 
 // value of a float register in lane `l` (l uniform across the wave)
 __device__ __forceinline__ float lane_f(float v, int l)
@@ -1764,513 +1753,289 @@ __device__ __forceinline__ float lane_f(float v, int l)
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
 
-// voxels of a group: the capacity for a mesh's resolution
-__device__ __forceinline__ uint32_t l2_group_cap(int w2, int n2)
+// Lane l holds row l of a 64x64 bit matrix (bit j = entry (l, j)); returns
+// column l (bit j = entry (j, l)).  Six block swaps of halving size.
+__device__ __forceinline__ uint64_t wave_transpose64(uint64_t v)
 {
-    return (uint32_t)l2_group_voxels(w2, n2);
-}
-
-// Group starts: flag[b] = 1 where a new group begins (mesh start, a new
-// 64-entry chunk of first bin entries, or a full group).
-template <bool kM>
-__global__ void k_l2_group_flags(const uint32_t* __restrict__ boff, int64_t B, GridDev g0, Meshes M,
-                                 uint32_t* __restrict__ flag)
-{
-    for (int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; b < B; b += (int64_t)gridDim.x * blockDim.x) {
-        const int mesh = kM ? (int)M.bmesh[b] : 0;
-        const GridDev& g = grid_of<kM>(g0, M, mesh);
-        const int64_t lb = b - (int64_t)(kM ? M.off[mesh].b0 : 0u);
-        const bool st =
-            lb == 0 || lb % (int64_t)l2_group_cap(g.w2, g.n2) == 0 || (boff[b] >> 6) != (boff[b - 1] >> 6);
-        flag[b] = st ? 1u : 0u;
+    const int lane = __lane_id();
+    const uint64_t masks[6] = {0x00000000FFFFFFFFull, 0x0000FFFF0000FFFFull, 0x00FF00FF00FF00FFull,
+                               0x0F0F0F0F0F0F0F0Full, 0x3333333333333333ull, 0x5555555555555555ull};
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+        const int s = 32 >> k;
+        const uint64_t m = masks[k];
+        const uint64_t x = shfl64(v, lane ^ s);
+        // branch-free select: the upper lane of each pair keeps the ~m half
+        const uint64_t sel = (uint64_t)0 - (uint64_t)((lane >> (5 - k)) & 1);
+        const uint64_t lo = (v & m) | ((x & m) << s);
+        const uint64_t hi = (v & ~m) | ((x & ~m) >> s);
+        v = (lo & ~sel) | (hi & sel);
     }
-}
-
-__global__ void k_l2_group_starts(const uint32_t* __restrict__ flag, const uint32_t* __restrict__ gidx, int64_t B,
-                                  uint32_t* __restrict__ gstart)
-{
-    for (int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; b < B; b += (int64_t)gridDim.x * blockDim.x) {
-        if (flag[b]) gstart[gidx[b]] = (uint32_t)b;
-        if (b == B - 1) gstart[gidx[B]] = (uint32_t)B;
-    }
-}
-
-void launch_l2_groups(const uint32_t* boff, int64_t B, const GridDev& g0, const Meshes& M, uint32_t* flag,
-                      uint32_t* gidx, uint32_t* scan_tmp, uint32_t* gstart, hipStream_t s)
-{
-    if (B <= 0) return;
-    const int blocks = grid_for(B, 256, 16384);
-    if (M.nm > 1)
-        k_l2_group_flags<true><<<blocks, 256, 0, s>>>(boff, B, g0, M, flag);
-    else
-        k_l2_group_flags<false><<<blocks, 256, 0, s>>>(boff, B, g0, M, flag);
-    launch_scan_u32_u32(flag, gidx, B, scan_tmp, nullptr, s);
-    k_l2_group_starts<<<blocks, 256, 0, s>>>(flag, gidx, B, gstart);
+    return v;
 }
 
 // LDS of one wave of the Level2 SAT
 struct L2Lds {
-    unsigned long long acc[64];   // Level2 boundary words of the group's voxels
-    float tv[64 * 9];             // staged triangles
+    union {
+        float4 e[L2_STAGE][kSatEntry4];                  // staged entries
+        unsigned long long words[kL2GroupBytes / 8];     // output words, once the bins are done
+    };
+    // per sub-column (v * n2^2 + q * n2 + p) its layer bits, in bytes up to
+    // n2 = 8 and in 16 bits above
+    uint32_t acc[kL2GroupBytes / 4];
     uint32_t q[L2_QCAP];          // ring of queued SAT entries
-    uint32_t dec[64];             // staged entry: sub-box origin/extent and box bit
-    unsigned long long mk[64];    // staged entry: box-axis masks
-    float4 sl[64];                // staged entry: Level2 slab
-    uint32_t off[64];             // staged entry: first item in the chunk's item space
-    uint8_t ev[64];               // staged entry: its voxel in the group
+    uint32_t dec[L2_STAGE];       // staged entry: first column, row and layer, last layer, columns, voxel, loose
+    uint32_t vb[kL2GroupMax + 1]; // group voxel v: first bin entry
+    int ci[kL2GroupMax][3];       // its sub-center 0 in the tables
     uint8_t win[64];              // per round: staged entry starting at each item position
-    uint32_t vb[L2_GMAX + 1];     // group voxel v: first bin entry
-    float c[L2_CMAX];             // centers: x [v*n2+p], y [nv*n2 + ...], z [2*nv*n2 + ...]
 };
 
-// Full float SAT for queued entries (one per lane); entry = p | q<<4 | r<<8 |
-// j<<12 | box<<18 where j is the staged triangle (its voxel is ev[j]) and box
-// says the box-axis predicates are already known to hold.
-__device__ __forceinline__ void l2_sat_run(uint32_t ent, bool valid, const L2Lds& L, unsigned long long* acc, int n2,
-                                           int nvn2, int w2, float h2x, float h2y, float h2z)
+// where the layer bits of sub-column `col` lie: word index and first bit
+__device__ __forceinline__ uint32_t l2_col_word(uint32_t col, int n2, uint32_t& bit)
 {
-    const int p = ent & 15, q = (ent >> 4) & 15, r = (ent >> 8) & 15, j = (ent >> 12) & 63;
-    const bool box = (ent >> 18) & 1;
-    const int v = valid ? (int)L.ev[j] : 0;
-    const int s = (r * n2 + q) * n2 + p;
-    const int wi = v * w2 + (s >> 6);
-    if (!valid || ((acc[wi] >> (s & 63)) & 1ull)) return;
-    const float ccx = L.c[v * n2 + p], ccy = L.c[nvn2 + v * n2 + q], ccz = L.c[2 * nvn2 + v * n2 + r];
+    const int sh = n2 > 8 ? 1 : 2;
+    bit = (col & ((1u << sh) - 1u)) << (5 - sh);
+    return col >> sh;
+}
+
+// Full float SAT for queued entries (one per lane); entry = p | q<<4 | r<<8 |
+// v<<12 | j<<16 where v is the voxel in the group and j the bin entry from base.
+__device__ __forceinline__ void l2_sat_run(uint32_t ent, bool valid, L2Lds& L, const GridDev& g,
+                                           const float* __restrict__ tris, const uint32_t* __restrict__ list,
+                                           uint32_t base)
+{
+    if (!valid) return;
+    const int n2 = g.n2;
+    const int p = ent & 15, q = (ent >> 4) & 15, r = (ent >> 8) & 15, v = (ent >> 12) & 15;
+    uint32_t bit;
+    const uint32_t w = l2_col_word((uint32_t)((v * n2 + q) * n2 + p), n2, bit);
+    if ((L.acc[w] >> (bit + r)) & 1u) return;
+    const uint64_t t = list[base + (ent >> 16)];
     float tv[9];
 #pragma unroll
-    for (int c = 0; c < 9; ++c) tv[c] = L.tv[j * 9 + c];
-    // every queued entry's column passed xy_edges_ok
-    const bool hit = box ? tri_box_overlap<false, false>(ccx, ccy, ccz, h2x, h2y, h2z, tv)
-                         : tri_box_overlap<true, false>(ccx, ccy, ccz, h2x, h2y, h2z, tv);
-    if (hit) atomicOr(&acc[wi], 1ull << (s & 63));
+    for (int c = 0; c < 9; ++c) tv[c] = tris[t * 9 + c];
+    if (tri_box_overlap(g.c2x[L.ci[v][0] + p], g.c2y[L.ci[v][1] + q], g.c2z[L.ci[v][2] + r], g.h2x, g.h2y, g.h2z, tv))
+        atomicOr(&L.acc[w], 1u << (bit + r));
 }
 
 template <bool kM, int W>
-__global__ __launch_bounds__(64 * W) void k_l2_sat_grp(const float* __restrict__ tris,
-                                                          const int32_t* __restrict__ bidx,
-                                                          const uint32_t* __restrict__ boff,
-                                                          const uint32_t* __restrict__ list,
-                                                          const uint64_t* __restrict__ pmask,
-                                                          const float4* __restrict__ slab2,
-                                                          const uint32_t* __restrict__ gstart,
-                                                          const uint32_t* __restrict__ ngroups, GridDev g0,
-                                                          Meshes M, uint64_t* __restrict__ sat2)
+__global__ __launch_bounds__(64 * W) void k_l2_sat(const float* __restrict__ tris, const int32_t* __restrict__ bidx,
+                                                   int64_t B, int64_t ngroups, int gmost,
+                                                   const uint32_t* __restrict__ boff,
+                                                   const uint32_t* __restrict__ list,
+                                                   const uint64_t* __restrict__ pmask, GridDev g0, Meshes M,
+                                                   uint64_t* __restrict__ sat2)
 {
     __shared__ L2Lds s_l[W];
     const int wv = threadIdx.x >> 6;
     const int lane = __lane_id();
     L2Lds& L = s_l[wv];
-    unsigned long long* acc = L.acc;
-    const uint32_t G = *ngroups;
-    for (uint32_t grp = blockIdx.x * W + wv; grp < G; grp += gridDim.x * W) {
-        const uint32_t vb0 = gstart[grp];
-        const int nv = (int)(gstart[grp + 1] - vb0);
-        const int mesh = kM ? uniform_i((int)M.bmesh[vb0]) : 0;
-        const GridDev& g = grid_of<kM>(g0, M, mesh);
-        const int n2 = g.n2, w2 = g.w2, gnx = g.nx, gny = g.ny;
-        const float h2x = g.h2x, h2y = g.h2y, h2z = g.h2z;
-        if (kM && n2 == 0) continue;
-        const int nvn2 = nv * n2;
-        uint64_t* out =
-            sat2 + (kM ? M.off[mesh].l2w0 + (uint64_t)(vb0 - M.off[mesh].b0) * w2 : (uint64_t)vb0 * w2);
-        for (int i = lane; i < nv * w2; i += 64) acc[i] = 0ull;
-        if (lane <= nv) L.vb[lane] = boff[vb0 + lane];
-        // the group's Level2 centers: x, y, z tables of each voxel
-        for (int i = lane; i < nvn2; i += 64) {
-            const int v = i / n2, pp = i - v * n2;
-            const int vox = bidx[vb0 + v];
-            const int nxy = gnx * gny;
-            const int k1 = vox / nxy;
-            const int ij = vox - k1 * nxy;
-            const int j1 = ij / gnx;
-            const int i1 = ij - j1 * gnx;
-            L.c[i] = g.c2x[(int64_t)i1 * n2 + pp];
-            L.c[nvn2 + i] = g.c2y[(int64_t)j1 * n2 + pp];
-            L.c[2 * nvn2 + i] = g.c2z[(int64_t)k1 * n2 + pp];
-        }
-        __builtin_amdgcn_wave_barrier();
-        uint32_t qh = 0, qt = 0;   // ring head/tail (uniform)
-        const uint32_t e0 = L.vb[0], e1 = L.vb[nv];
-        for (uint32_t base = e0; base < e1; base += 64) {
-            // the queue refers to staged triangles by slot: drain it before restaging
-            while (qt != qh) {
-                const uint32_t n = qt - qh < 64 ? qt - qh : 64;
-                const bool valid = (uint32_t)lane < n;
-                const uint32_t ent = valid ? L.q[(qh + lane) % L2_QCAP] : 0u;
-                l2_sat_run(ent, valid, L, acc, n2, nvn2, w2, h2x, h2y, h2z);
-                qh += n;
-            }
-            __builtin_amdgcn_wave_barrier();
-            // staging: lane j owns bin entry base + j -- vertices, masks, slab,
-            // sub-box decode and its voxel go to LDS
-            const uint32_t i = base + lane;
-            uint32_t P = 0;
-            if (i < e1) {
-                const uint64_t t = list[i];
-#pragma unroll
-                for (int c = 0; c < 9; ++c) L.tv[lane * 9 + c] = tris[t * 9 + c];
-                int lo = 0, hi = nv;   // the voxel whose entries hold i: vb[lo] <= i < vb[lo + 1]
-                while (hi - lo > 1) {
-                    const int mid = (lo + hi) >> 1;
-                    if (L.vb[mid] <= i) lo = mid;
-                    else hi = mid;
-                }
-                L.ev[lane] = (uint8_t)lo;
-                const uint64_t mk = pmask[i];
-                const uint32_t mx = (uint32_t)(mk & 0xffffu), my = (uint32_t)((mk >> 16) & 0xffffu),
-                               mz = (uint32_t)((mk >> 32) & 0xffffu);
-                if (mx && my && mz) {
-                    const int pa = __ffs(mx) - 1, pb = 31 - __clz(mx);
-                    const int qa = __ffs(my) - 1, qb = 31 - __clz(my);
-                    const int ra = __ffs(mz) - 1, rb = 31 - __clz(mz);
-                    const int dp = pb - pa + 1, dq = qb - qa + 1, dr = rb - ra + 1;
-                    // contiguous passing sets (centers are monotone in the index) mean
-                    // the box-axis predicates hold on the whole sub-box
-                    const uint32_t boxbit =
-                        (__popc(mx) == dp && __popc(my) == dq && __popc(mz) == dr) ? 1u : 0u;
-                    L.dec[lane] = (uint32_t)pa | ((uint32_t)qa << 4) | ((uint32_t)ra << 8) | ((uint32_t)rb << 12) |
-                                  ((uint32_t)dp << 16) | (boxbit << 24);
-                    L.mk[lane] = mk;
-                    L.sl[lane] = slab2[t];
-                    P = (uint32_t)(dp * dq);
-                }
-            }
-            const uint32_t incl = wave_incl_scan<uint32_t>(P);
-            const uint32_t so = incl - P;   // this lane's entry: items [so, so + P)
-            L.off[lane] = so;
-            const uint32_t S = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
-            __builtin_amdgcn_wave_barrier();
-            // the chunk's (entry, sub-column) items, 64 per round
-            for (uint32_t l0 = 0; l0 < S; l0 += 64) {
-                // each item's entry, as in k_l2_sat_voxel: entries mark their
-                // first position in the window, an item takes the highest mark
-                // at or below it
-                L.win[lane] = 0xff;
-                __builtin_amdgcn_wave_barrier();
-                if (P && so < l0 + 64u && so + P > l0) L.win[so > l0 ? so - l0 : 0u] = (uint8_t)lane;
-                __builtin_amdgcn_wave_barrier();
-                const uint32_t wj = L.win[lane];
-                const uint64_t marks = __ballot(wj != 0xffu) & ((2ull << lane) - 1ull);
-                const int top = marks ? 63 - __clzll((long long)marks) : 0;
-                const int jw = __shfl((int)wj, top);
-                __builtin_amdgcn_wave_barrier();
-                const uint32_t l = l0 + (uint32_t)lane;
-                uint32_t keep = 0;
-                int p = 0, q = 0, j = 0, v = 0, ra = 0, rb = -1;
-                uint32_t boxbit = 0, mz = 0;
-                if (l < S) {
-                    j = jw;
-                    v = (int)L.ev[j];
-                    const uint32_t d = L.dec[j];
-                    const int pa = d & 15, qa = (d >> 4) & 15;
-                    ra = (d >> 8) & 15;
-                    rb = (d >> 12) & 15;
-                    const int dp = (d >> 16) & 255;
-                    boxbit = (d >> 24) & 1u;
-                    const int lj = (int)(l - L.off[j]);
-                    // exact small-integer division: (lj + 0.5)/dp is >= 1/32 from an integer
-                    const int rem = (int)(((float)lj + 0.5f) * kInvSmall[dp]);
-                    p = pa + lj - rem * dp;
-                    q = qa + rem;
-                    const uint64_t mk = L.mk[j];
-                    const uint32_t mx = (uint32_t)(mk & 0xffffu), my = (uint32_t)((mk >> 16) & 0xffffu);
-                    mz = (uint32_t)((mk >> 32) & 0xffffu);
-                    if ((mx >> p) & (my >> q) & 1u) {
-                        const float ccx = L.c[v * n2 + p], ccy = L.c[nvn2 + v * n2 + q];
-                        // the e x z edge predicates hold or fail for the whole sub-column
-                        if (xy_edges_ok(ccx, ccy, h2x, h2y, L.tv + j * 9)) {
-                            const float4 sl = L.sl[j];
-                            const float t0x = L.tv[j * 9 + 0], t0y = L.tv[j * 9 + 1], t0z = L.tv[j * 9 + 2];
-                            // float_slab_keeps, with the (x, y) part shared by the sub-column
-                            const float A = sl.x * (ccx - t0x) + sl.y * (ccy - t0y);
-                            const float* cz = L.c + 2 * nvn2 + v * n2;
-                            for (int r = ra; r <= rb; ++r) {
-                                const float sd = A + sl.z * (cz[r] - t0z);
-                                keep |= (uint32_t)(fabsf(sd) <= sl.w && ((mz >> r) & 1u)) << r;
-                            }
-                        }
-                    }
-                }
-                // queue the kept sub-voxels not yet set, one r per lane per round
-                while (__ballot(keep != 0)) {
-                    const int r = keep ? __ffs(keep) - 1 : 0;
-                    const bool has = keep != 0;
-                    keep &= keep - 1;
-                    const int sv = (r * n2 + q) * n2 + p;
-                    const bool push = has && !((acc[(v * w2 + (sv >> 6)) & 63] >> (sv & 63)) & 1ull);
-                    const uint64_t m = __ballot(push);
-                    if (push) {
-                        const uint32_t at = qt + (uint32_t)__popcll(m & lanes_below_mask());
-                        L.q[at % L2_QCAP] = (uint32_t)p | ((uint32_t)q << 4) | ((uint32_t)r << 8) |
-                                            ((uint32_t)j << 12) | (boxbit << 18);
-                    }
-                    qt += (uint32_t)__popcll(m);
-                    __builtin_amdgcn_wave_barrier();
-                    if (qt - qh >= 64) {   // a full wave of work
-                        const uint32_t ent = L.q[(qh + lane) % L2_QCAP];
-                        l2_sat_run(ent, true, L, acc, n2, nvn2, w2, h2x, h2y, h2z);
-                        qh += 64;
-                        __builtin_amdgcn_wave_barrier();
-                    }
-                }
-            }
-        }
-        while (qt != qh) {
-            const uint32_t n = qt - qh < 64 ? qt - qh : 64;
-            const bool valid = (uint32_t)lane < n;
-            const uint32_t ent = valid ? L.q[(qh + lane) % L2_QCAP] : 0u;
-            l2_sat_run(ent, valid, L, acc, n2, nvn2, w2, h2x, h2y, h2z);
-            qh += n;
-        }
-        __builtin_amdgcn_wave_barrier();
-        for (int i = lane; i < nv * w2; i += 64) out[i] = acc[i];
-        __builtin_amdgcn_wave_barrier();
-    }
-}
-
-// One wave per boundary voxel: the form for voxels with many bin entries
-// (the parent's sub-centers stay in lane registers, entry p in lane p).
-// Full float SAT for queued entries (one per lane); entry = p | q<<4 | r<<8 |
-// j<<12 | box<<18 where j is the staged triangle and box says the box-axis
-// predicates are already known to hold.
-__device__ __forceinline__ void l2_sat_run_v(uint32_t ent, bool valid, const float* stv, float cxl, float cyl,
-                                           float czl, int n2, float h2x, float h2y, float h2z,
-                                           unsigned long long* acc)
-{
-    const int p = ent & 15, q = (ent >> 4) & 15, r = (ent >> 8) & 15, j = (ent >> 12) & 63;
-    const bool box = (ent >> 18) & 1;
-    const float ccx = __shfl(cxl, p), ccy = __shfl(cyl, q), ccz = __shfl(czl, r);
-    const int s = (r * n2 + q) * n2 + p;
-    if (!valid || ((acc[s >> 6] >> (s & 63)) & 1ull)) return;
-    float tv[9];
-#pragma unroll
-    for (int c = 0; c < 9; ++c) tv[c] = stv[j * 9 + c];
-    // every queued entry's column passed xy_edges_ok
-    const bool hit = box ? tri_box_overlap<false, false>(ccx, ccy, ccz, h2x, h2y, h2z, tv)
-                         : tri_box_overlap<true, false>(ccx, ccy, ccz, h2x, h2y, h2z, tv);
-    if (hit) atomicOr(&acc[s >> 6], 1ull << (s & 63));
-}
-
-// Eight waves per SIMD: at most 64 VGPRs and 4.7 KB of LDS per wave (the
-// staged entries' masks and item offsets stay in their lanes' registers and
-// are read across lanes).
-template <bool kM, int W>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(8))) void k_l2_sat_voxel(
-    const float* __restrict__ tris, const int32_t* __restrict__ bidx, int64_t B, const uint32_t* __restrict__ boff,
-    const uint32_t* __restrict__ list, const uint64_t* __restrict__ pmask, const float4* __restrict__ slab2,
-    GridDev g0, Meshes M, uint64_t* __restrict__ sat2)
-{
-    __shared__ unsigned long long s_acc[W][64];
-    __shared__ float s_tv[W][64 * 9];
-    __shared__ uint32_t s_q[W][L2_QCAP];
-    // per staged triangle: sub-box origin and extents, and its slab (its
-    // masks and the start of its sub-columns in the chunk's flattened
-    // (triangle, sub-column) item space stay in the staging lane)
-    __shared__ uint32_t s_dec[W][64];
-    __shared__ float4 s_sl[W][64];
-    __shared__ float s_cz[W][16];
-    __shared__ uint8_t s_win[W][64];   // per round: staged entry starting at each item position
-    const int wv = threadIdx.x >> 6;
-    const int lane = __lane_id();
-    const int64_t b = (int64_t)blockIdx.x * W + wv;
-    if (b >= B) return;
-    const int mesh = kM ? uniform_i((int)M.bmesh[b]) : 0;
+    const int64_t grp = (int64_t)blockIdx.x * W + wv;
+    if (grp >= ngroups) return;
+    int mesh = 0;
+    if constexpr (kM)
+        mesh = wave_mesh_search(M.off, M.nm, (uint64_t)grp, [](const MeshOff& o) { return (uint64_t)o.sg0; });
     const GridDev& g = grid_of<kM>(g0, M, mesh);
-    const int n2 = g.n2, w2 = g.w2, gnx = g.nx, gny = g.ny;
-    const float h2x = g.h2x, h2y = g.h2y, h2z = g.h2z;
+    const int n2 = g.n2, w2 = g.w2, nsc = n2 * n2;
     if (kM && n2 == 0) return;
-    uint64_t* out = sat2 + (kM ? M.off[mesh].l2w0 + (uint64_t)(b - M.off[mesh].b0) * w2 : (uint64_t)b * w2);
-    unsigned long long* acc = s_acc[wv];
-    for (int i = lane; i < w2; i += 64) acc[i] = 0ull;
-    const int v = bidx[b];
-    const int nxy = gnx * gny;
-    const int k1 = v / nxy;
-    const int ij = v - k1 * nxy;
-    const int j1 = ij / gnx;
-    const int i1 = ij - j1 * gnx;
-    // the parent's n2 sub-centers per axis in registers, entry p in lane p;
-    // z also in LDS for per-lane layer lookups
-    const float cxl = lane < n2 ? g.c2x[(int64_t)i1 * n2 + lane] : 0.0f;
-    const float cyl = lane < n2 ? g.c2y[(int64_t)j1 * n2 + lane] : 0.0f;
-    const float czl = lane < n2 ? g.c2z[(int64_t)k1 * n2 + lane] : 0.0f;
-    float* cz = s_cz[wv];
-    if (lane < n2) cz[lane] = czl;
-    float* stv = s_tv[wv];
-    uint32_t* sq = s_q[wv];
-    uint32_t* dec = s_dec[wv];
-    float4* ssl = s_sl[wv];
-    uint8_t* win = s_win[wv];
+    const int64_t mb0 = kM ? (int64_t)M.off[mesh].b0 : 0, mb1 = kM ? (int64_t)M.off[mesh + 1].b0 : B;
+    const int G = l2_group_voxels(n2, gmost);
+    const int64_t vb0 = mb0 + (grp - (kM ? (int64_t)M.off[mesh].sg0 : 0)) * G;
+    if (vb0 >= mb1) return;
+    const int nv = (int)(mb1 - vb0 < G ? mb1 - vb0 : G);
+    uint64_t* out = sat2 + (kM ? M.off[mesh].l2w0 : 0) + (uint64_t)(vb0 - mb0) * w2;
+    for (int i = lane; i < (nv * nsc * (n2 > 8 ? 2 : 1) + 3) / 4; i += 64) L.acc[i] = 0u;
+    if (lane <= nv) L.vb[lane] = boff[vb0 + lane];
+    if (lane < nv) {
+        const int vox = bidx[vb0 + lane];
+        const int nxy = g.nx * g.ny;
+        const int k1 = vox / nxy;
+        const int ij = vox - k1 * nxy;
+        const int j1 = ij / g.nx;
+        const int i1 = ij - j1 * g.nx;
+        L.ci[lane][0] = i1 * n2;
+        L.ci[lane][1] = j1 * n2;
+        L.ci[lane][2] = k1 * n2;
+    }
     __builtin_amdgcn_wave_barrier();
+    const SatScale sc{g.s2x, g.s2y, g.s2z, g.d2x, g.d2y, g.d2z};
     uint32_t qh = 0, qt = 0;   // ring head/tail (uniform)
-    const uint32_t e0 = boff[b], e1 = boff[b + 1];
-    for (uint32_t base = e0; base < e1; base += 64) {
-        // the queue refers to staged triangles by slot: drain it before restaging
-        while (qt != qh) {
-            const uint32_t n = qt - qh < 64 ? qt - qh : 64;
-            const bool valid = (uint32_t)lane < n;
-            const uint32_t ent = valid ? sq[(qh + lane) % L2_QCAP] : 0u;
-            l2_sat_run_v(ent, valid, stv, cxl, cyl, czl, n2, h2x, h2y, h2z, acc);
-            qh += n;
+    const uint32_t e0 = (uint32_t)uniform_i((int)L.vb[0]), e1 = (uint32_t)uniform_i((int)L.vb[nv]);
+    uint32_t qbase = e0;       // the bin entry that queued entries count from
+    for (uint32_t base = e0; base < e1; base += L2_STAGE) {
+        if (base - qbase > 0xffffu - L2_STAGE) {   // their 16 bits would not do
+            const bool valid = (uint32_t)lane < qt - qh;
+            l2_sat_run(valid ? L.q[(qh + lane) % L2_QCAP] : 0u, valid, L, g, tris, list, qbase);
+            qh = qt;
+            qbase = base;
+            __builtin_amdgcn_wave_barrier();
         }
-        __builtin_amdgcn_wave_barrier();
-        // staging: lane j owns bin entry base + j -- vertices, masks, slab and
-        // its sub-box decode go to LDS
-        const uint32_t i = base + lane;
-        uint32_t P = 0;
-        uint64_t mk_reg = 0;
+        // staging: lanes j and j + 32 make bin entry base + j
+        const int js = lane & (L2_STAGE - 1), h = lane >> 5;
+        const uint32_t i = base + (uint32_t)js;
+        uint32_t P = 0;   // rows of the entry (lanes below 32)
         if (i < e1) {
             const uint64_t t = list[i];
-#pragma unroll
-            for (int c = 0; c < 9; ++c) stv[lane * 9 + c] = tris[t * 9 + c];
             const uint64_t mk = pmask[i];
+            float tv[9];
+#pragma unroll
+            for (int c = 0; c < 9; ++c) tv[c] = tris[t * 9 + c];
+            int v = 0, hi = nv;   // the voxel whose entries hold i: vb[v] <= i < vb[v + 1]
+            while (hi - v > 1) {
+                const int mid = (v + hi) >> 1;
+                if (L.vb[mid] <= i) v = mid;
+                else hi = mid;
+            }
+            const bool loose = sat_entry_part(h, tv, g.c2x[L.ci[v][0]], g.c2y[L.ci[v][1]], g.c2z[L.ci[v][2]], sc, L.e[js]);
             const uint32_t mx = (uint32_t)(mk & 0xffffu), my = (uint32_t)((mk >> 16) & 0xffffu),
                            mz = (uint32_t)((mk >> 32) & 0xffffu);
-            if (mx && my && mz) {
-                const int pa = __ffs(mx) - 1, pb = 31 - __clz(mx);
-                const int qa = __ffs(my) - 1, qb = 31 - __clz(my);
-                const int ra = __ffs(mz) - 1, rb = 31 - __clz(mz);
-                const int dp = pb - pa + 1, dq = qb - qa + 1, dr = rb - ra + 1;
-                // contiguous passing sets (centers are monotone in the index) mean
-                // the box-axis predicates hold on the whole sub-box
-                const uint32_t boxbit =
-                    (__popc(mx) == dp && __popc(my) == dq && __popc(mz) == dr) ? 1u : 0u;
-                dec[lane] = (uint32_t)pa | ((uint32_t)qa << 4) | ((uint32_t)ra << 8) | ((uint32_t)rb << 12) |
-                            ((uint32_t)dp << 16) | (boxbit << 24);
-                mk_reg = mk;
-                ssl[lane] = slab2[t];
-                P = (uint32_t)(dp * dq);
+            const bool any = mx && my && mz;
+            const int pa = __ffs(mx) - 1, pb = 31 - __clz(mx);
+            const int qa = __ffs(my) - 1, qb = 31 - __clz(my);
+            const int ra = __ffs(mz) - 1, rb = 31 - __clz(mz);
+            // the boxes that pass the box-axis predicates are one run per axis
+            // (the tables are monotone); were they not, the rows would be
+            // undecided and the float SAT settle them
+            const bool runs = __popc(mx) == pb - pa + 1 && __popc(my) == qb - qa + 1 && __popc(mz) == rb - ra + 1;
+            const uint64_t bad = __ballot(loose || !runs);
+            if (h == 0 && any) {
+                L.dec[js] = (uint32_t)pa | ((uint32_t)qa << 4) | ((uint32_t)ra << 8) | ((uint32_t)rb << 12) |
+                            ((uint32_t)(pb - pa) << 16) | ((uint32_t)v << 20) |
+                            (((bad >> js) | (bad >> (js + 32))) & 1ull ? 0x80000000u : 0u);
+                P = (uint32_t)(qb - qa + 1);
             }
         }
         const uint32_t incl = wave_incl_scan<uint32_t>(P);
         const uint32_t so = incl - P;   // this lane's entry: items [so, so + P)
         const uint32_t S = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
         __builtin_amdgcn_wave_barrier();
-        // the chunk's (triangle, sub-column) items, 64 per round
+        // the chunk's (entry, row) items, 64 per round
         for (uint32_t l0 = 0; l0 < S; l0 += 64) {
             // each item's entry: every entry with items in [l0, l0 + 64) marks
             // its first position there (the one running into the window marks
             // 0; starts are distinct), and item l takes the mark at the highest
             // marked position <= l
-            win[lane] = 0xff;
+            L.win[lane] = 0xff;
             __builtin_amdgcn_wave_barrier();
-            if (P && so < l0 + 64u && so + P > l0) win[so > l0 ? so - l0 : 0u] = (uint8_t)lane;
+            if (P && so < l0 + 64u && so + P > l0) L.win[so > l0 ? so - l0 : 0u] = (uint8_t)lane;
             __builtin_amdgcn_wave_barrier();
-            const uint32_t wj = win[lane];
+            const uint32_t wj = L.win[lane];
             const uint64_t marks = __ballot(wj != 0xffu) & ((2ull << lane) - 1ull);
             const int top = marks ? 63 - __clzll((long long)marks) : 0;
-            const int jw = __shfl((int)wj, top);
-            // the item's entry fields, read across lanes by every lane
-            const uint32_t so_j = (uint32_t)__shfl((int)so, jw);
-            const uint32_t mklo_j = (uint32_t)__shfl((int)(uint32_t)mk_reg, jw);
-            const uint32_t mkhi_j = (uint32_t)__shfl((int)(uint32_t)(mk_reg >> 32), jw);
+            const int j = __shfl((int)wj, top) & (L2_STAGE - 1);
+            const uint32_t so_j = (uint32_t)__shfl((int)so, j);
             __builtin_amdgcn_wave_barrier();
             const uint32_t l = l0 + (uint32_t)lane;
-            uint32_t keep = 0;
-            int p = 0, q = 0, j = 0, ra = 0, rb = -1;
-            uint32_t boxbit = 0, mz = 0;
-            bool in = false;
-            if (l < S) {
-                j = jw;
-                const uint32_t d = dec[j];
-                const int pa = d & 15, qa = (d >> 4) & 15;
-                ra = (d >> 8) & 15;
-                rb = (d >> 12) & 15;
-                const int dp = (d >> 16) & 255;
-                boxbit = (d >> 24) & 1u;
-                const int lj = (int)(l - so_j);
-                // exact small-integer division: (lj + 0.5)/dp is >= 1/32 from an integer
-                const int rem = (int)(((float)lj + 0.5f) * kInvSmall[dp]);
-                p = pa + lj - rem * dp;
-                q = qa + rem;
-                const uint32_t mx = mklo_j & 0xffffu, my = mklo_j >> 16;
-                mz = mkhi_j & 0xffffu;
-                in = ((mx >> p) & (my >> q) & 1u) != 0;
-            }
-            // every lane takes part in the cross-lane reads
-            const float ccx = __shfl(cxl, p), ccy = __shfl(cyl, q);
-            // the e x z edge predicates hold or fail for the whole sub-column
-            if (in) in = xy_edges_ok(ccx, ccy, h2x, h2y, stv + j * 9);
-            if (in) {
-                const float4 sl = ssl[j];
-                const float t0x = stv[j * 9 + 0], t0y = stv[j * 9 + 1], t0z = stv[j * 9 + 2];
-                // float_slab_keeps, with the (x, y) part shared by the sub-column
-                const float A = sl.x * (ccx - t0x) + sl.y * (ccy - t0y);
-                for (int r = ra; r <= rb; ++r) {
-                    const float sd = A + sl.z * (cz[r] - t0z);
-                    keep |= (uint32_t)(fabsf(sd) <= sl.w && ((mz >> r) & 1u)) << r;
+            // lanes past the last item repeat one with no columns to do
+            const uint32_t d = L.dec[j];
+            const int q = ((d >> 4) & 15) + (int)(l - so_j), ra = (d >> 8) & 15, rb = (d >> 12) & 15;
+            const int v = (int)((d >> 20) & 15u);
+            const bool loose = d >> 31 != 0;
+            int p = d & 15, left = (int)((d >> 16) & 15) + 1;   // columns of the row
+            SatRow row = sat_row(L.e[j], q, ra, rb, loose, p, left);
+            left = l < S ? left : 0;
+            const uint32_t all = ((2u << rb) - 1u) & ~((1u << ra) - 1u);
+            uint32_t col = (uint32_t)((v * n2 + q) * n2 + p);
+            const uint32_t ent = (uint32_t)p | ((uint32_t)q << 4) | ((uint32_t)v << 12) | ((base - qbase + (uint32_t)j) << 16);
+            const bool any_loose = __ballot(loose && left > 0) != 0;
+            for (int k = 0; __ballot(k < left); ++k, ++col) {
+                uint32_t in, may;
+                sat_row_column(row, in, may);
+                if (any_loose) {
+                    in = loose ? 0u : in;
+                    may = loose ? all : may;
                 }
-            }
-            // queue the kept sub-voxels not yet set, one r per lane per round
-            while (__ballot(keep != 0)) {
-                const int r = keep ? __ffs(keep) - 1 : 0;
-                const bool has = keep != 0;
-                keep &= keep - 1;
-                const int sv = (r * n2 + q) * n2 + p;
-                const bool push = has && !((acc[(sv & 4095) >> 6] >> (sv & 63)) & 1ull);
-                const uint64_t m = __ballot(push);
-                if (push) {
-                    const uint32_t at = qt + (uint32_t)__popcll(m & lanes_below_mask());
-                    sq[at % L2_QCAP] = (uint32_t)p | ((uint32_t)q << 4) | ((uint32_t)r << 8) |
-                                       ((uint32_t)j << 12) | (boxbit << 18);
+                const bool on = k < left;
+                in = on ? in : 0u;
+                uint32_t unk = on ? may & ~in : 0u;
+                if (in) {
+                    uint32_t bit;
+                    const uint32_t w = l2_col_word(col, n2, bit);
+                    atomicOr(&L.acc[w], in << bit);
                 }
-                qt += (uint32_t)__popcll(m);
-                __builtin_amdgcn_wave_barrier();
-                if (qt - qh >= 64) {   // a full wave of work
-                    const uint32_t ent = sq[(qh + lane) % L2_QCAP];
-                    l2_sat_run_v(ent, true, stv, cxl, cyl, czl, n2, h2x, h2y, h2z, acc);
-                    qh += 64;
+                // the undecided boxes, one layer per lane per pass
+                for (uint64_t m; (m = __ballot(unk != 0)) != 0;) {
+                    if (unk) {
+                        const uint32_t r = (uint32_t)__ffs(unk) - 1u;
+                        L.q[(qt + (uint32_t)__popcll(m & lanes_below_mask())) % L2_QCAP] = (ent + (uint32_t)k) | (r << 8);
+                        unk &= unk - 1;
+                    }
+                    qt += (uint32_t)__popcll(m);
                     __builtin_amdgcn_wave_barrier();
+                    if (qt - qh >= 64) {   // a full wave of work
+                        l2_sat_run(L.q[(qh + lane) % L2_QCAP], true, L, g, tris, list, qbase);
+                        qh += 64;
+                        __builtin_amdgcn_wave_barrier();
+                    }
                 }
             }
         }
     }
-    while (qt != qh) {
-        const uint32_t n = qt - qh < 64 ? qt - qh : 64;
-        const bool valid = (uint32_t)lane < n;
-        const uint32_t ent = valid ? sq[(qh + lane) % L2_QCAP] : 0u;
-        l2_sat_run_v(ent, valid, stv, cxl, cyl, czl, n2, h2x, h2y, h2z, acc);
-        qh += n;
+    if (qt != qh) {
+        const bool valid = (uint32_t)lane < qt - qh;
+        l2_sat_run(valid ? L.q[(qh + lane) % L2_QCAP] : 0u, valid, L, g, tris, list, qbase);
     }
     __builtin_amdgcn_wave_barrier();
-    for (int i = lane; i < w2; i += 64) out[i] = acc[i];
+    // layer bits per sub-column -> words of sub-voxels: bit s of word m is
+    // sub-voxel 64 m + s = layer * n2^2 + sub-column
+    const uint8_t* a8 = reinterpret_cast<const uint8_t*>(L.acc);
+    const uint16_t* a16 = reinterpret_cast<const uint16_t*>(L.acc);
+    if (n2 == 8) {
+        // bit 8v + r of lane c: layer r of sub-column c of voxel v; transposed,
+        // lane 8v + r holds word r of voxel v
+        for (int v0 = 0; v0 < nv; v0 += 8) {
+            uint64_t b = 0;
+            for (int v = 0; v < 8 && v0 + v < nv; ++v) b |= (uint64_t)a8[(v0 + v) * 64 + lane] << (8 * v);
+            b = wave_transpose64(b);
+            if (v0 * 8 + lane < nv * 8) out[v0 * 8 + lane] = b;
+        }
+        return;
+    }
+    if (n2 == 16) {
+        // bit 16k + r of lane c: layer r of sub-column 64k + c; transposed, lane
+        // 16k + r holds word 4r + k
+        for (int v = 0; v < nv; ++v) {
+            uint64_t b = 0;
+            for (int k = 0; k < 4; ++k) b |= (uint64_t)a16[v * 256 + k * 64 + lane] << (16 * k);
+            out[v * 64 + 4 * (lane & 15) + (lane >> 4)] = wave_transpose64(b);
+        }
+        return;
+    }
+    const float inv = 1.0f / (float)nsc;
+    for (int m = 0; m < w2; ++m) {
+        const int s = 64 * m + lane;
+        const int r = (int)(((float)s + 0.5f) * inv);   // exact: s + 1/2 is at least 1/512 of n2^2 from a multiple
+        const int sub = s - r * nsc;
+        for (int v = 0; v < nv; ++v) {
+            const uint32_t bits = n2 > 8 ? (uint32_t)a16[v * nsc + sub] : (uint32_t)a8[v * nsc + sub];
+            const uint64_t wd = __ballot(r < n2 && ((bits >> r) & 1u));
+            if (lane == 0) L.words[v * w2 + m] = wd;
+        }
+    }
+    __builtin_amdgcn_wave_barrier();
+    for (int i = lane; i < nv * w2; i += 64) out[i] = L.words[i];
 }
 
 template <int W>
-static void launch_l2_sat_w(const float* tris, const int32_t* bidx, int64_t B, const uint32_t* boff,
-                            const uint32_t* list, const uint64_t* pmask, const float4* slab2, const uint32_t* gstart,
-                            const uint32_t* ngroups, int64_t gmax, const GridDev& g0, const Meshes& M,
-                            uint64_t* sat2, hipStream_t s)
+static void launch_l2_sat_w(const float* tris, const int32_t* bidx, int64_t B, int64_t ngroups, int gmost,
+                            const uint32_t* boff, const uint32_t* list, const uint64_t* pmask, const GridDev& g0,
+                            const Meshes& M, uint64_t* sat2, hipStream_t s)
 {
-    const dim3 bs(64 * W);
-    if (gstart) {
-        // one wave per group, for an upper bound gmax on the group count
-        const unsigned blocks = (unsigned)std::max<int64_t>(1, (gmax + W - 1) / W);
-        if (M.nm > 1)
-            k_l2_sat_grp<true, W><<<blocks, bs, 0, s>>>(tris, bidx, boff, list, pmask, slab2, gstart, ngroups, g0, M,
-                                                        sat2);
-        else
-            k_l2_sat_grp<false, W><<<blocks, bs, 0, s>>>(tris, bidx, boff, list, pmask, slab2, gstart, ngroups, g0, M,
-                                                         sat2);
-        return;
-    }
-    const unsigned vblocks = (unsigned)((B + W - 1) / W);
+    const unsigned blocks = (unsigned)((ngroups + W - 1) / W);
     if (M.nm > 1)
-        k_l2_sat_voxel<true, W><<<vblocks, bs, 0, s>>>(tris, bidx, B, boff, list, pmask, slab2, g0, M, sat2);
+        k_l2_sat<true, W><<<blocks, 64 * W, 0, s>>>(tris, bidx, B, ngroups, gmost, boff, list, pmask, g0, M, sat2);
     else
-        k_l2_sat_voxel<false, W><<<vblocks, bs, 0, s>>>(tris, bidx, B, boff, list, pmask, slab2, g0, M, sat2);
+        k_l2_sat<false, W><<<blocks, 64 * W, 0, s>>>(tris, bidx, B, ngroups, gmost, boff, list, pmask, g0, M, sat2);
 }
 
-void launch_l2_sat(const float* tris, const int32_t* bidx, int64_t B, const uint32_t* boff, const uint32_t* list,
-                   const uint64_t* pmask, const float4* slab2, const uint32_t* gstart, const uint32_t* ngroups,
-                   int64_t gmax, int waves, const GridDev& g0, const Meshes& M, uint64_t* sat2, hipStream_t s)
+void launch_l2_sat(const float* tris, const int32_t* bidx, int64_t B, int64_t ngroups, int gmost, const uint32_t* boff,
+                   const uint32_t* list, const uint64_t* pmask, int waves, const GridDev& g0, const Meshes& M,
+                   uint64_t* sat2, hipStream_t s)
 {
-    if (B <= 0) return;
-    if (waves <= 1)
-        launch_l2_sat_w<1>(tris, bidx, B, boff, list, pmask, slab2, gstart, ngroups, gmax, g0, M, sat2, s);
-    else if (waves == 2)
-        launch_l2_sat_w<2>(tris, bidx, B, boff, list, pmask, slab2, gstart, ngroups, gmax, g0, M, sat2, s);
-    else
-        launch_l2_sat_w<4>(tris, bidx, B, boff, list, pmask, slab2, gstart, ngroups, gmax, g0, M, sat2, s);
+    if (B <= 0 || ngroups <= 0) return;
+    if (waves <= 1) launch_l2_sat_w<1>(tris, bidx, B, ngroups, gmost, boff, list, pmask, g0, M, sat2, s);
+    else if (waves == 2) launch_l2_sat_w<2>(tris, bidx, B, ngroups, gmost, boff, list, pmask, g0, M, sat2, s);
+    else launch_l2_sat_w<4>(tris, bidx, B, ngroups, gmost, boff, list, pmask, g0, M, sat2, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -2306,27 +2071,6 @@ __device__ __forceinline__ bool colrec_xy(const ColRec& r, float ox, float oy, f
     m.e2x = r.e2x; m.e2y = r.e2y; m.e2z = r.e2z;
     m.inv_det = r.inv;
     return mt_column(m, r.v1x, r.v1y, ox, oy, tx, ty);
-}
-
-// Lane l holds row l of a 64x64 bit matrix (bit j = entry (l, j)); returns
-// column l (bit j = entry (j, l)).  Six block swaps of halving size.
-__device__ __forceinline__ uint64_t wave_transpose64(uint64_t v)
-{
-    const int lane = __lane_id();
-    const uint64_t masks[6] = {0x00000000FFFFFFFFull, 0x0000FFFF0000FFFFull, 0x00FF00FF00FF00FFull,
-                               0x0F0F0F0F0F0F0F0Full, 0x3333333333333333ull, 0x5555555555555555ull};
-#pragma unroll
-    for (int k = 0; k < 6; ++k) {
-        const int s = 32 >> k;
-        const uint64_t m = masks[k];
-        const uint64_t x = shfl64(v, lane ^ s);
-        // branch-free select: the upper lane of each pair keeps the ~m half
-        const uint64_t sel = (uint64_t)0 - (uint64_t)((lane >> (5 - k)) & 1);
-        const uint64_t lo = (v & m) | ((x & m) << s);
-        const uint64_t hi = (v & ~m) | ((x & ~m) >> s);
-        v = (lo & ~sel) | (hi & sel);
-    }
-    return v;
 }
 
 // The z-independent half of the MT test (det/u/v, src/TriRayIntersection.cpp:

@@ -6,6 +6,7 @@
 // citations per function) and this file is compiled with -ffp-contract=off.
 #include "gpv.h"
 #include "gpv_internal.hpp"
+#include "gpv_satrow.hpp"
 #include "gpv_serve.h"
 
 #include <hip/hip_runtime.h>
@@ -225,7 +226,7 @@ struct gpv_ctx {
     float* tab_buf = nullptr;   // pinned staging of a job's center tables
     size_t tab_cap = 0;
     int num_cu = 256;
-    gpv_tune tune{16, 8, 2048, 1, 1, 2, 128};
+    gpv_tune tune{16, 56, 2048, 1, 1, 2, 128};
     std::vector<hipEvent_t> events;   // recycled stage events of finished jobs
     hipEvent_t na_ev[16] = {};        // stage events of gpv_voxelize_noalloc (created with the context)
 };
@@ -264,7 +265,6 @@ struct Job {
     // per triangle
     int4 *box0 = nullptr, *box1 = nullptr, *rng = nullptr;
     double4* slab1 = nullptr;   // plane slab of triangles spanning several layers
-    float4* slab2 = nullptr;    // plane slab over the Level2 centers of the index AABB (float form)
     uint32_t *sat_items = nullptr, *ray_items = nullptr;
     uint64_t *sat_off = nullptr, *ray_off = nullptr, *scan64 = nullptr;
     uint64_t* scan_ray = nullptr;   // scan temporary of the ray half of the set-up (side stream)
@@ -300,8 +300,8 @@ struct Job {
     uint32_t* cs_cnt = nullptr;
     uint4* cs_bucket = nullptr;
     uint64_t* cpass = nullptr;   // det/u/v pass bits per column entry and sub-column
-    uint32_t *gflag = nullptr, *gidx = nullptr, *gstart = nullptr;   // Level2 SAT voxel groups
-    int64_t l2p_waves = 0;   // Level2 parity waves (l2_parity_plan)
+    int64_t l2p_waves = 0, l2s_groups = 0;   // Level2 parity waves, SAT groups (l2_plan)
+    int l2s_most = 1;                        // most voxels of a SAT group
     uint32_t *hcnt = nullptr, *hoff = nullptr;
     float4* hrec = nullptr;
     // GL-stencil-equivalent Level1 fill (meshes with params.l1_stencil):
@@ -667,6 +667,10 @@ int job_create(gpv_ctx* c, const gpv_mesh_desc* d, int nm, int on_device, Job** 
         g = grid_dev(J->info[m]);
         g.normals = d[m].params.normals ? 1 : 0;
         g.l2cuda = d[m].params.cuda_level2 ? 1 : 0;
+        const gpv_grid_info& I = J->info[m];
+        sat_scale_axis(I.bmin[0], I.bmax[0], I.g2[0], g.l2cuda != 0, g.s2x, g.d2x);
+        sat_scale_axis(I.bmin[1], I.bmax[1], I.g2[1], g.l2cuda != 0, g.s2y, g.d2y);
+        sat_scale_axis(I.bmin[2], I.bmax[2], I.g2[2], g.l2cuda != 0, g.s2z, g.d2z);
         g.l1st = d[m].params.l1_stencil ? 1 : 0;
         J->any_stencil = J->any_stencil || g.l1st;
         J->all_stencil = (m == 0 || J->all_stencil) && g.l1st;
@@ -792,7 +796,7 @@ int job_create(gpv_ctx* c, const gpv_mesh_desc* d, int nm, int on_device, Job** 
 
     const size_t Tn = (size_t)std::max<int64_t>(T, 1);
     if ((r = alloc(J, &J->box0, Tn)) || (r = alloc(J, &J->box1, Tn)) || (r = alloc(J, &J->rng, Tn)) ||
-        (r = alloc(J, &J->slab1, Tn)) || (r = alloc(J, &J->slab2, Tn)) ||
+        (r = alloc(J, &J->slab1, Tn)) ||
         (r = alloc(J, &J->sat_items, Tn)) || (r = alloc(J, &J->ray_items, Tn)) ||
         (r = alloc(J, &J->sat_off, Tn + 1)) || (r = alloc(J, &J->ray_off, Tn + 1)) ||
         (r = alloc(J, &J->ctr, 1)) || (r = alloc(J, &J->wcnt, (size_t)W)) ||
@@ -840,7 +844,7 @@ int stage_setup(Job* J)
     launch_fill_u64(reinterpret_cast<uint64_t*>(&J->ctr->bad_input), 0, 1, s);
     if (J->nm > 1) launch_mesh_ids(J->d_off, J->nm, J->T, J->tri_mesh, s);
     launch_tri_setup(J->tris, J->T, J->g[0], J->view(), J->box0, J->box1, J->sat_items, J->rng, J->ray_items,
-                     J->slab1, J->slab2, 3, &J->ctr->bad_input, s);
+                     J->slab1, 3, &J->ctr->bad_input, s);
     TRY(ensure_scan_tmp(J, J->T));
     launch_scan_u32_u64(J->sat_items, J->sat_off, J->T, J->scan64, s);
     launch_scan_u32_u64(J->ray_items, J->ray_off, J->T, J->scan64, s);
@@ -864,12 +868,12 @@ int stage_setup_split(Job* J)
     TRY(alloc(J, &J->scan_ray, scan_tmp_elems(J->T)));
     HIP_TRY(hipEventRecord(J->ev[15], s));
     launch_tri_setup(J->tris, J->T, J->g[0], J->view(), J->box0, J->box1, J->sat_items, J->rng, J->ray_items,
-                     J->slab1, J->slab2, 1, &J->ctr->bad_input, s);
+                     J->slab1, 1, &J->ctr->bad_input, s);
     launch_scan_u32_u64(J->sat_items, J->sat_off, J->T, J->scan64, s);
     HIP_TRY(hipStreamWaitEvent(c->side, J->ev[15], 0));
     if (!J->all_stencil) {   // the ray half feeds only the ray parity
         launch_tri_setup(J->tris, J->T, J->g[0], J->view(), J->box0, J->box1, J->sat_items, J->rng, J->ray_items,
-                         J->slab1, J->slab2, 2, &J->ctr->bad_input, c->side);
+                         J->slab1, 2, &J->ctr->bad_input, c->side);
         launch_scan_u32_u64(J->ray_items, J->ray_off, J->T, J->scan_ray, c->side);
     }
     HIP_TRY(hipGetLastError());
@@ -1170,18 +1174,40 @@ int launch_compact(Job* J)
     return GPV_OK;
 }
 
-// Level2 parity waves of the job; in a batch each mesh's first wave goes to
-// MeshOff::pw0 on the device (main stream, before any parity launch)
-int l2_parity_plan(Job* J)
+// Most voxels of a Level2 SAT group: as many as hold about 56 bin entries (two
+// stagings of 32; 28 entries took 0.33 ms on the torus knot and 0.62 ms on a
+// batch of small meshes where 56 take 0.28 and 0.51, 84 gain nothing more),
+// fewer where that would leave less than 16 waves per CU; one where the bins
+// hold more than tune.l2_group_below.
+int l2_sat_most(const Job* J)
 {
-    int64_t w = 0;
+    if (J->B <= 0 || (int64_t)J->n_pairs >= (int64_t)J->ctx->tune.l2_group_below * J->B) return 1;
+    const int64_t fill = std::max<int64_t>(1, 56 * J->B / std::max<int64_t>(1, (int64_t)J->n_pairs));
+    const int64_t spread = std::max<int64_t>(1, J->B / (int64_t)(16 * std::max(1, J->ctx->num_cu)));
+    return (int)std::min<int64_t>(kL2GroupMax, std::min(fill, spread));
+}
+
+// Level2 parity waves and SAT groups of the job; in a batch each mesh's first
+// ones go to MeshOff::pw0 and sg0 on the device (main stream, before any
+// Level2 launch)
+int l2_plan(Job* J)
+{
+    int64_t w = 0, sg = 0;
+    J->l2s_most = l2_sat_most(J);
     for (int m = 0; m < J->nm; ++m) {
         J->off[m].pw0 = (uint32_t)w;
+        J->off[m].sg0 = (uint32_t)sg;
         w += l2_parity_waves(J->g[m].n2, J->nb(m));
+        if (J->g[m].n2 > 0) {
+            const int64_t c = l2_group_voxels(J->g[m].n2, J->l2s_most);
+            sg += (J->nb(m) + c - 1) / c;
+        }
     }
     J->off[J->nm].pw0 = (uint32_t)w;
+    J->off[J->nm].sg0 = (uint32_t)sg;
     if (w >= (int64_t(1) << 32)) return fail(GPV_ERR_INVALID, "too many Level2 parity waves");
     J->l2p_waves = w;
+    J->l2s_groups = sg;
     if (J->nm > 1) {
         hipStream_t s = J->ctx->stream;
         // the MeshOff staging region was last filled by the size read-back,
@@ -1223,77 +1249,20 @@ int run_l2_parity(Job* J)
     hipStream_t s = J->ctx->stream;
     HIP_TRY(hipEventRecord(J->ev[5], s));
     TRY(alloc_cpass(J));
-    TRY(l2_parity_plan(J));
+    TRY(l2_plan(J));
     TRY(l2_parity_kernels(J, s));
     release(J, J->cpass);
     J->l2p_done = true;
     return GPV_OK;
 }
 
-// group arrays of the Level2 SAT (allocated outside any two-stream region)
-int alloc_l2_groups(Job* J)
-{
-    const size_t n = (size_t)std::max<int64_t>(J->B, 1) + 1;
-    release(J, J->gflag);
-    release(J, J->gidx);
-    release(J, J->gstart);
-    TRY(alloc(J, &J->gflag, n));
-    TRY(alloc(J, &J->gidx, n));
-    TRY(alloc(J, &J->gstart, n));
-    return ensure_scan_tmp(J, J->B);
-}
-
-void release_l2_groups(Job* J)
-{
-    release(J, J->gflag);
-    release(J, J->gidx);
-    release(J, J->gstart);
-}
-
-// whether the Level2 SAT shares waves among voxels: few bin entries per voxel
-bool l2_grouped(const Job* J)
-{
-    if (J->B <= 0 || (int64_t)J->n_pairs >= (int64_t)J->ctx->tune.l2_group_below * J->B) return false;
-    // a group of one voxel (n2 = 16: its 64 words fill the wave's LDS) is
-    // the per-voxel kernel at a lower occupancy
-    for (int m = 0; m < J->nm; ++m)
-        if (J->g[m].n2 > 0 && l2_group_voxels(J->g[m].w2, J->g[m].n2) > 1) return true;
-    return false;
-}
-
-// group formation of the Level2 SAT (main stream, group arrays allocated)
-void l2_sat_groups(Job* J)
-{
-    if (l2_grouped(J))
-        launch_l2_groups(J->boff, J->B, J->g[0], J->view(), J->gflag, J->gidx, J->scan32, J->gstart,
-                         J->ctx->stream);
-}
-
-// the Level2 SAT kernel on the main stream (groups formed)
+// the Level2 SAT kernel on the main stream (groups planned)
 int l2_sat_kernels(Job* J)
 {
     hipStream_t s = J->ctx->stream;
     HIP_TRY(hipEventRecord(J->ev[6], s));
-    // voxels with few bin entries share waves (k_l2_sat_grp); with many one
-    // voxel per wave is faster
-    const bool grouped = l2_grouped(J);
-    // one wave per group, for an upper bound on the group count computed
-    // here (a group starts at a mesh start, at a new 64-entry chunk of first
-    // bin entries, or after a full group), so the grid is sized without
-    // reading the count back; waves past the real count exit
-    int64_t gmax = J->B;
-    if (grouped) {
-        gmax = (int64_t)(J->n_pairs / 64) + 1;
-        for (int m = 0; m < J->nm; ++m) {
-            const int64_t nb = J->nb(m);
-            const int w2 = J->g[m].w2;
-            const int64_t cap = l2_group_voxels(w2, J->g[m].n2);
-            gmax += (nb + cap - 1) / cap + 1;
-        }
-        gmax = std::min<int64_t>(gmax, J->B);
-    }
-    launch_l2_sat(J->tris, J->bidx, J->B, J->boff, J->list, J->pmask, J->slab2, grouped ? J->gstart : nullptr,
-                  J->gidx + J->B, gmax, J->ctx->tune.l2_sat_waves, J->g[0], J->view(), J->sat2, s);
+    launch_l2_sat(J->tris, J->bidx, J->B, J->l2s_groups, J->l2s_most, J->boff, J->list, J->pmask,
+                  J->ctx->tune.l2_sat_waves, J->g[0], J->view(), J->sat2, s);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipEventRecord(J->ev[7], s));
     return GPV_OK;
@@ -1302,10 +1271,8 @@ int l2_sat_kernels(Job* J)
 int run_l2_sat(Job* J)
 {
     if (J->n2max <= 0) return GPV_OK;
-    TRY(alloc_l2_groups(J));
-    l2_sat_groups(J);
+    TRY(l2_plan(J));
     TRY(l2_sat_kernels(J));
-    release_l2_groups(J);
     J->l2s_done = true;
     return GPV_OK;
 }
@@ -1320,11 +1287,7 @@ int run_level2(Job* J)
     gpv_ctx* c = J->ctx;
     hipStream_t s = c->stream;
     TRY(alloc_cpass(J));
-    TRY(alloc_l2_groups(J));
-    TRY(l2_parity_plan(J));
-    // the SAT's small group-formation kernels go first: launched beside the
-    // parity they would wait for its waves to drain
-    l2_sat_groups(J);
+    TRY(l2_plan(J));
     HIP_TRY(hipEventRecord(J->ev[5], s));
     HIP_TRY(hipStreamWaitEvent(c->side, J->ev[5], 0));
     TRY(l2_parity_kernels(J, c->side));
@@ -1333,7 +1296,6 @@ int run_level2(Job* J)
     release(J, J->cpass);
     release(J, J->cs_cnt);
     release(J, J->cs_bucket);
-    release_l2_groups(J);
     J->l2p_done = true;
     J->l2s_done = true;
     return GPV_OK;
@@ -1414,7 +1376,7 @@ int job_finish(Job* J)
         I.ms_normals = ms_nrm;
     }
     // only the result planes stay resident
-    release(J, J->box0); release(J, J->box1); release(J, J->rng); release(J, J->slab1); release(J, J->slab2);
+    release(J, J->box0); release(J, J->box1); release(J, J->rng); release(J, J->slab1);
     release(J, J->pmask);
     release(J, J->sat_items); release(J, J->ray_items); release(J, J->sat_off); release(J, J->ray_off);
     release(J, J->scan64); J->scan32 = nullptr; J->scan_cap = 0; release(J, J->scan_ray);
@@ -1520,14 +1482,14 @@ int64_t predict_run_bytes(const gpv_mesh_desc& d, const gpv_grid_info& I)
     int64_t b = 0;
     b += 4 * (2 * (nx + ny + nz) * (1 + n2) + 1);               // center tables
     b += 36 * T + 4 * T + 4 * B + 4096;                          // soup copy, batch mesh ids, descriptors
-    b += 120 * T + 16 + 2 * scan(std::max(T, W));               // per-triangle set-up, item scans
+    b += 104 * T + 16 + 2 * scan(std::max(T, W));               // per-triangle set-up, item scans
     b += 24 * W + 64 * W;                                        // planes, word counts and prefix, flag bytes
     b += 24 * P + 8 * H;                                         // bin pairs, column entries, ray hits
     b += 8 * ncol + 8 + 48 * H + scan(ncol);                     // parity fill: hits by column, records
     b += 4 * (ncol + 1) + 48 * P + 16 * P + 64 * (ncol / 64 + 1);   // column entries by column, records
     b += 8 * B + 4 + 4 * P + 8 * P + 16 * P + 64 * (B / 64 + 1) + scan(B);   // boundary list, bins, masks
     b += 16 * B * w2;                                            // Level2 planes
-    b += n2 > 0 ? 8 * P * ((n2 * n2 + 63) / 64 + 1) + 12 * (B + 1) : 0;   // Level2 parity bits, SAT groups
+    b += n2 > 0 ? 8 * P * ((n2 * n2 + 63) / 64 + 1) : 0;   // Level2 parity bits
     if (d.params.normals) b += 12 * T + 4 * P + 12 * B + 12 * B * n2 * n2 * n2;
     if (d.params.l1_stencil) b += 12 * T + 8 + scan(T) + 8 * nz * 2 * ny * ((2 * nx + 63) / 64);   // stencil fill
     return b;

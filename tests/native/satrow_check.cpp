@@ -1,0 +1,58 @@
+// Host harness for the row form of the Level2 SAT (gpview_amd/csrc/
+// gpv_satrow.hpp): tests/test_sat_rows.py compares its masks with the
+// reference's SAT.  Test tooling only.
+#include <stdint.h>
+#include "gpv_satrow.hpp"
+
+static bool axis_ok(float a0, float a1, float a2, float c, float h)
+{
+    const float d0 = a0 - c, d1 = a1 - c, d2 = a2 - c;
+    float mn = d0, mx = d0;
+    if (d1 < mn) mn = d1;
+    if (d1 > mx) mx = d1;
+    if (d2 < mn) mn = d2;
+    if (d2 > mx) mx = d2;
+    return !((mn > h) | (mx < -h));
+}
+
+// Case i: triangle tv[9i..], a voxel's sub-center tables cx/cy/cz[n2*i..],
+// grid bounds lo/hi[3i..], sub-voxel g2[3i..], half extents h[3i..].  Per
+// column (q * n2 + p): the layer masks `in` and `may`.  Rows are cut to the
+// boxes whose box-axis predicates hold, as the kernel does.
+extern "C" void satrow_batch(int64_t n, int n2, const float* tv, const float* cx, const float* cy, const float* cz,
+                             const float* lo, const float* hi, const float* g2, const float* h, int cuda_l2,
+                             uint32_t* in, uint32_t* may)
+{
+    for (int64_t i = 0; i < n; ++i) {
+        const float* t = tv + 9 * i;
+        const float *X = cx + n2 * i, *Y = cy + n2 * i, *Z = cz + n2 * i;
+        gpv::SatScale g;
+        gpv::sat_scale_axis(lo[3 * i], hi[3 * i], g2[3 * i], cuda_l2 != 0, g.sx, g.dx);
+        gpv::sat_scale_axis(lo[3 * i + 1], hi[3 * i + 1], g2[3 * i + 1], cuda_l2 != 0, g.sy, g.dy);
+        gpv::sat_scale_axis(lo[3 * i + 2], hi[3 * i + 2], g2[3 * i + 2], cuda_l2 != 0, g.sz, g.dz);
+        int pa = n2, pb = -1, ra = n2, rb = -1;
+        for (int p = 0; p < n2; ++p) {
+            if (axis_ok(t[0], t[3], t[6], X[p], h[3 * i])) { pa = p < pa ? p : pa; pb = p; }
+            if (axis_ok(t[2], t[5], t[8], Z[p], h[3 * i + 2])) { ra = p < ra ? p : ra; rb = p; }
+        }
+        float4 e[gpv::kSatEntry4];
+        bool loose = gpv::sat_entry_part(0, t, X[0], Y[0], Z[0], g, e);
+        loose = gpv::sat_entry_part(1, t, X[0], Y[0], Z[0], g, e) || loose;
+        for (int q = 0; q < n2; ++q) {
+            uint32_t* oi = in + (int64_t)(i * n2 + q) * n2;
+            uint32_t* om = may + (int64_t)(i * n2 + q) * n2;
+            for (int p = 0; p < n2; ++p) oi[p] = om[p] = 0;
+            if (pb < 0 || rb < 0 || !axis_ok(t[1], t[4], t[7], Y[q], h[3 * i + 1])) continue;
+            int p = pa, left = pb - pa + 1;
+            gpv::SatRow s = gpv::sat_row(e, q, ra, rb, loose, p, left);
+            const uint32_t all = ((2u << rb) - 1u) & ~((1u << ra) - 1u);
+            for (int k = 0; k < left; ++k) {
+                gpv::sat_row_column(s, oi[p + k], om[p + k]);
+                if (loose) {
+                    oi[p + k] = 0;
+                    om[p + k] = all;
+                }
+            }
+        }
+    }
+}
