@@ -44,8 +44,8 @@ struct MeshOff {
     uint32_t tri0;
     uint32_t b0;
     uint32_t ptask0;   // first Level1 parity task (16 layers x 64 columns of one row)
-    uint32_t pw0;      // first Level2 parity wave (set on the host once boundary counts are known)
-    uint32_t sg0;      // first Level2 SAT group (set on the host likewise)
+    uint32_t pw0;      // first Level2 parity wave
+    uint32_t sg0;      // first Level2 SAT group (set on the host once boundary counts are known)
 };
 
 // Per-mesh results accumulated on the device.
@@ -194,15 +194,18 @@ void launch_mesh_bins(const uint32_t* boff, int64_t B, const Meshes& M, hipStrea
 void launch_l2_sat(const float* tris, const int32_t* bidx, int64_t B, int64_t ngroups, int gmost, const uint32_t* boff,
                    const uint32_t* list, const uint64_t* pmask, int waves, const GridDev& g0, const Meshes& M,
                    uint64_t* sat2, hipStream_t s);
-// det/u/v pass bits per (column entry, sub-column): stride words per entry
-void launch_col_pass(const float4* rec, const GridDev& g0, const Meshes& M, uint64_t nent, int stride, int waves,
-                     uint64_t* cpass, hipStream_t s);
-// Level2 parity waves of one mesh: one per boundary voxel, one per four when
-// n2 <= 4, none when Level2 is off
-int64_t l2_parity_waves(int n2, int64_t nb);
-// n2max: the largest Level2 resolution of the run
-void launch_l2_parity(const int32_t* bidx, int64_t B, int64_t nwaves, const uint32_t* coff, const float4* rec,
-                      const uint64_t* cpass, int stride, int n2max, int waves, const GridDev& g0, const Meshes& M,
+// Level2 parity: a wave takes l2_parity_columns adjacent columns of a mesh
+// (grids are multiples of four in x): four at n2 <= 4 in runs of at least
+// kL2ParityMany columns, where the shared prologue pays (128 small meshes 0.39
+// ms), one in smaller ones, where the longest wave counts (icosphere 64/4: 24
+// us with four)
+constexpr int64_t kL2ParityMany = 1 << 16;
+__host__ __device__ inline int l2_parity_columns(int n2, bool many) { return many && n2 <= 4 ? 4 : 1; }
+// its waves for a mesh with ncol columns (none when Level2 is off)
+int64_t l2_parity_waves(int n2, int64_t ncol, bool many);
+// n2max, nzmax: the largest Level2 resolution and layer count of the run
+void launch_l2_parity(const uint64_t* bnd, const uint32_t* wprefix, int64_t nwaves, bool many, int n2max, int nzmax,
+                      const uint32_t* coff, const float4* rec, int waves, const GridDev& g0, const Meshes& M,
                       uint64_t* par2, hipStream_t s);
 
 // normals (src/Object.cpp:3219-3253 Level1, 2372-2421 + 2705-2720 Level2)

@@ -8,7 +8,7 @@
 //   compaction + prefix, src/Object.cpp:3270-3279 ... k_popc_words, scan, k_boundary_index
 //   bins by boundary voxel (the CSR of :2137-2219) .. k_ts_count, k_ts_bucket, k_ts_place
 //   Level2 SAT, src/Object.cpp:2344-2424 ............ k_l2_sat
-//   Level2 ray parity, src/Object.cpp:1111-1207 ..... k_ts_* (column entries), k_col_pass, k_l2_parity
+//   Level2 ray parity, src/Object.cpp:1111-1207 ..... k_ts_* (column entries), k_l2_parity
 //   counts, src/Object.cpp:3353-3378 ................ k_count_states
 //   .raw layout, src/Object.cpp:2934-3075 ........... k_export_*
 //
@@ -16,6 +16,7 @@
 // with integer OR / ballot only, so results are deterministic.
 #include "gpv_device.hpp"
 #include "gpv_internal.hpp"
+#include "gpv_parcol.hpp"
 #include "gpv_satrow.hpp"
 #include "gpv_slab.hpp"
 
@@ -31,31 +32,55 @@ __device__ __forceinline__ uint64_t shfl64(uint64_t v, int src)
     return ((uint64_t)hi << 32) | lo;
 }
 
-template <typename T>
-__device__ __forceinline__ T shfl_up_t(T v, unsigned d);
-template <>
-__device__ __forceinline__ uint32_t shfl_up_t<uint32_t>(uint32_t v, unsigned d)
+// Moves across lanes without LDS (DPP and the row swaps): a cross-lane read
+// through LDS waits about a hundred cycles, and the scans and the transpose
+// below are chains of six.
+template <int kCtrl, int kRows, int kBanks>
+__device__ __forceinline__ uint32_t dpp(uint32_t v, uint32_t old)
 {
-    return __shfl_up(v, d);
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)v, kCtrl, kRows, kBanks, false);
 }
-template <>
-__device__ __forceinline__ uint64_t shfl_up_t<uint64_t>(uint64_t v, unsigned d)
+template <int kCtrl, int kRows>
+__device__ __forceinline__ uint32_t dpp_or_0(uint32_t v)
 {
-    const uint32_t lo = __shfl_up((unsigned)(v & 0xffffffffu), d);
-    const uint32_t hi = __shfl_up((unsigned)(v >> 32), d);
-    return ((uint64_t)hi << 32) | lo;
+    return dpp<kCtrl, kRows, 0xf>(v, 0u);
+}
+template <int kCtrl, int kRows>
+__device__ __forceinline__ uint64_t dpp_or_0(uint64_t v)
+{
+    return (uint64_t)dpp_or_0<kCtrl, kRows>((uint32_t)v) |
+           ((uint64_t)dpp_or_0<kCtrl, kRows>((uint32_t)(v >> 32)) << 32);
 }
 
+// inclusive sum over the lanes of a full wave
 template <typename T>
 __device__ __forceinline__ T wave_incl_scan(T x)
 {
-    const unsigned lane = __lane_id();
-#pragma unroll
-    for (unsigned d = 1; d < 64; d <<= 1) {
-        const T y = shfl_up_t<T>(x, d);
-        if (lane >= d) x += y;
-    }
+    x += dpp_or_0<0x111, 0xf>(x);   // row_shr:1, 2, 4, 8: within rows of 16
+    x += dpp_or_0<0x112, 0xf>(x);
+    x += dpp_or_0<0x114, 0xf>(x);
+    x += dpp_or_0<0x118, 0xf>(x);
+    x += dpp_or_0<0x142, 0xa>(x);   // row_bcast:15 into rows 1 and 3
+    x += dpp_or_0<0x143, 0xc>(x);   // row_bcast:31 into rows 2 and 3
     return x;
+}
+
+// the value of lane ^ S
+template <int S>
+__device__ __forceinline__ uint32_t lane_xor(uint32_t v)
+{
+    if constexpr (S == 1) return dpp<0xb1, 0xf, 0xf>(v, v);         // quad_perm 1,0,3,2
+    else if constexpr (S == 2) return dpp<0x4e, 0xf, 0xf>(v, v);    // quad_perm 2,3,0,1
+    else if constexpr (S == 4) {                                    // row_shl:4 / row_shr:4 by banks of four
+        const uint32_t up = dpp<0x104, 0xf, 0x5>(v, v);
+        return dpp<0x114, 0xf, 0xa>(v, up);
+    } else if constexpr (S == 8) return dpp<0x128, 0xf, 0xf>(v, v);  // row_ror:8
+    else {
+        static_assert(S == 16 || S == 32, "lane distance");
+        const auto r = S == 16 ? __builtin_amdgcn_permlane16_swap(v, v, false, false)
+                               : __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        return (__lane_id() & S) ? r[0] : r[1];
+    }
 }
 
 __device__ __forceinline__ uint64_t wave_sum_u64(uint64_t x)
@@ -979,8 +1004,7 @@ struct ColPlace {
         if (!ok) return;
         rec[3 * (uint64_t)pos + 0] = make_float4(m.e1x, m.e1y, m.e1z, m.e2x);
         rec[3 * (uint64_t)pos + 1] = make_float4(m.e2y, m.e2z, m.inv_det, tv[0]);
-        // the last word: the entry's batch-wide column (read by the packed column pass)
-        rec[3 * (uint64_t)pos + 2] = make_float4(tv[1], tv[2], __int_as_float((int)it.z), __uint_as_float(it.x));
+        rec[3 * (uint64_t)pos + 2] = make_float4(tv[1], tv[2], __int_as_float((int)it.z), 0.0f);
     }
 };
 
@@ -1755,23 +1779,28 @@ __device__ __forceinline__ float lane_f(float v, int l)
 
 // Lane l holds row l of a 64x64 bit matrix (bit j = entry (l, j)); returns
 // column l (bit j = entry (j, l)).  Six block swaps of halving size.
+template <int K>
+__device__ __forceinline__ uint64_t transpose_step(uint64_t v)
+{
+    constexpr int s = 32 >> K;
+    constexpr uint64_t masks[6] = {0x00000000FFFFFFFFull, 0x0000FFFF0000FFFFull, 0x00FF00FF00FF00FFull,
+                                   0x0F0F0F0F0F0F0F0Full, 0x3333333333333333ull, 0x5555555555555555ull};
+    constexpr uint64_t m = masks[K];
+    const uint64_t x = (uint64_t)lane_xor<s>((uint32_t)v) | ((uint64_t)lane_xor<s>((uint32_t)(v >> 32)) << 32);
+    // the upper lane of each pair keeps the ~m half
+    const uint64_t lo = (v & m) | ((x & m) << s);
+    const uint64_t hi = (v & ~m) | ((x & ~m) >> s);
+    return (__lane_id() & s) ? hi : lo;
+}
+
 __device__ __forceinline__ uint64_t wave_transpose64(uint64_t v)
 {
-    const int lane = __lane_id();
-    const uint64_t masks[6] = {0x00000000FFFFFFFFull, 0x0000FFFF0000FFFFull, 0x00FF00FF00FF00FFull,
-                               0x0F0F0F0F0F0F0F0Full, 0x3333333333333333ull, 0x5555555555555555ull};
-#pragma unroll
-    for (int k = 0; k < 6; ++k) {
-        const int s = 32 >> k;
-        const uint64_t m = masks[k];
-        const uint64_t x = shfl64(v, lane ^ s);
-        // branch-free select: the upper lane of each pair keeps the ~m half
-        const uint64_t sel = (uint64_t)0 - (uint64_t)((lane >> (5 - k)) & 1);
-        const uint64_t lo = (v & m) | ((x & m) << s);
-        const uint64_t hi = (v & ~m) | ((x & ~m) >> s);
-        v = (lo & ~sel) | (hi & sel);
-    }
-    return v;
+    v = transpose_step<0>(v);
+    v = transpose_step<1>(v);
+    v = transpose_step<2>(v);
+    v = transpose_step<3>(v);
+    v = transpose_step<4>(v);
+    return transpose_step<5>(v);
 }
 
 // LDS of one wave of the Level2 SAT
@@ -2001,7 +2030,7 @@ __global__ __launch_bounds__(64 * W) void k_l2_sat(const float* __restrict__ tri
         }
         return;
     }
-    const float inv = 1.0f / (float)nsc;
+    const float inv = GPV_RCP((float)nsc);
     for (int m = 0; m < w2; ++m) {
         const int s = 64 * m + lane;
         const int r = (int)(((float)s + 0.5f) * inv);   // exact: s + 1/2 is at least 1/512 of n2^2 from a multiple
@@ -2039,617 +2068,439 @@ void launch_l2_sat(const float* tris, const int32_t* bidx, int64_t B, int64_t ng
 }
 
 // ---------------------------------------------------------------------------
-// Level2 ray parity (src/Object.cpp:1111-1207): one wave per boundary voxel
-// (i1, j1, k1).  Candidates are the column's (triangle, zmax) entries with
-// zmax >= k1 -- the deduplicated union of the bins at z' >= k1 -- each with
-// a precomputed MT record (edges, 1/det, V1).  Per chunk of 64 candidates:
-// one coalesced load into LDS; the z-independent det/u/v test runs once per
-// (candidate, sub-column) and leaves a pass bit; t > 1e-6 then runs per
-// sub-voxel only for the passing pairs.
+// Level2 ray parity (src/Object.cpp:1111-1207), by xy columns.  A boundary
+// voxel (i1, j1, k1) takes the triangles of the bins at z' >= k1 in its column,
+// which are the column's (triangle, zmax) entries with zmax >= k1, and each of
+// its sub-voxels counts those whose +z ray test passes.  One wave takes one
+// column (or four adjacent ones, l2_parity_columns): for every (entry, sub-column) pair
+// that the float det/u/v test accepts it finds the number of layers whose
+// t > 1e-6 holds -- the layers below the crossing, bounded by gpv_parcol.hpp,
+// with the float test deciding the few within rounding of it -- and toggles one
+// bit there.  The toggles at or above a layer are then its parity.
+//
+// Pairs, not voxels: an entry's accepted sub-columns are found once for the
+// column (by rows of its xy range, then by the columns each row can accept),
+// where a wave per voxel repeated every entry above each voxel: torus knot
+// 256/8 0.232 -> 0.129 ms alone (1.82e8 -> 0.72e8 instructions), lattice-snapped
+// mesh 512/16 3.90 -> 2.24 ms, 128 small meshes 0.60 -> 0.39 ms.
+//
+// What bounds it: the chain of dependent LDS and global reads of each wave
+// (VALU issue 0.39-0.47), hence one wave per block (an empty column's wave
+// leaves at once; two waves a block took 0.15 ms on the torus knot), 80
+// registers for six waves per SIMD (three waves: 0.18 ms, eight: no gain), scans
+// and transposes without LDS, and 32 staged entries.  Four columns per wave at
+// n2 = 8 took 0.31 ms.
 // ---------------------------------------------------------------------------
-struct ColRec {
-    float e1x, e1y, e1z, e2x, e2y, e2z, inv, v1x, v1y, v1z;
-    int zmax;
+constexpr int L2P_STAGE = 32;    // entries staged at once
+constexpr int L2P_SLOTS = 128;   // boundary voxels of a window, all columns of the wave
+
+// LDS of one wave of the Level2 parity
+template <int KB>
+struct L2PLds {
+    // staged entry: e1, e2x | e2y, e2z, inv, v1x | v1y, dz, mu, delta | l0, cap, column, v1z
+    float4 e[L2P_STAGE][4];
+    // per (column, slot, sub-column) its toggles, in bytes up to n2 = 8 and in
+    // 16 bits above; a column's row past its slots holds the parity of the windows above
+    uint32_t acc[KB / 4];
+    uint32_t slotb[L2P_SLOTS];   // boundary voxel of each slot
+    float ox[16], oy[16];        // origins of the columns (c * n2 + p) and of the row
+    uint8_t win[64];
 };
 
-__device__ __forceinline__ ColRec load_colrec(const float4* __restrict__ rec, uint32_t i)
+// parity waves of a mesh with ncol columns
+int64_t l2_parity_waves(int n2, int64_t ncol, bool many)
 {
-    const float4 a = rec[3 * (uint64_t)i + 0];
-    const float4 b = rec[3 * (uint64_t)i + 1];
-    const float4 c = rec[3 * (uint64_t)i + 2];
-    ColRec r;
-    r.e1x = a.x; r.e1y = a.y; r.e1z = a.z; r.e2x = a.w;
-    r.e2y = b.x; r.e2z = b.y; r.inv = b.z; r.v1x = b.w;
-    r.v1y = c.x; r.v1z = c.y; r.zmax = __float_as_int(c.z);
-    return r;
+    return n2 <= 0 ? 0 : ncol / l2_parity_columns(n2, many);
 }
 
-__device__ __forceinline__ bool colrec_xy(const ColRec& r, float ox, float oy, float& tx, float& ty)
-{
-    MtTri m;
-    m.e1x = r.e1x; m.e1y = r.e1y; m.e1z = r.e1z;
-    m.e2x = r.e2x; m.e2y = r.e2y; m.e2z = r.e2z;
-    m.inv_det = r.inv;
-    return mt_column(m, r.v1x, r.v1y, ox, oy, tx, ty);
-}
-
-// The z-independent half of the MT test (det/u/v, src/TriRayIntersection.cpp:
-// 78-131 with D = +z) depends on the column entry and the sub-column's (x, y)
-// only, so it runs once per (column entry, sub-column) here: one lane per
-// column entry, looping over its column's n2^2 sub-columns
-// (sc = q*n2 + p); entry e's pass bits go to cpass[e * stride + sc / 64], bit
-// sc % 64.  Every boundary voxel of the column then reads them instead of
-// repeating the test.  The entry's last word, cpass[e * stride + stride - 1],
-// is its header: bits 0-31 hold kh + 1 and bits 32-63 zc + 1, where zc is
-// the last layer whose voxels take the entry as a candidate (zmax, or the
-// top layer for the CUDA kernels' whole-column candidates) and kh < zc a
-// layer such that t > 1e-6 holds for every ray origin of the column in
-// layers [0, kh] (t_decided over that box; -1 if none found).  For a voxel at
-// k1 <= kh the entry then flips every layer of each sub-column it passes
-// without a t test.
-// The column entries are packed 64 to a wave across columns (one wave per
-// column would leave most lanes idle: columns hold a few dozen entries).
-// Each lane takes its column from its record and its sub-column origins from
-// the tables.  In a batch a wave's entries can span meshes (they are in
-// column order, and each mesh's columns are contiguous): the wave takes its
-// meshes one after another, each with the lanes whose columns it holds.
-__device__ __forceinline__ void col_pass_entry(const GridDev& g, uint32_t col, const ColRec& r, bool own,
-                                               uint64_t* __restrict__ dst, int stride)
-{
-    const int n2 = g.n2;
-    if (n2 == 0) return;
-    const int i1 = (int)(col % (uint32_t)g.nx), j1 = (int)(col / (uint32_t)g.nx);
-    const float* rx = g.r2x + (int64_t)i1 * n2;
-    const float* ry = g.r2y + (int64_t)j1 * n2;
-    {
-        const int zc = g.l2cuda ? g.nz - 1 : r.zmax;
-        int kh = -1;
-        if (g.r2mono != 0) {
-            const float oxlo = rx[0], oxhi = rx[n2 - 1], oylo = ry[0], oyhi = ry[n2 - 1];
-            const float oz0 = g.r2z[0];
-#pragma unroll
-            for (int d = 8; d >= 1; d >>= 1) {
-                const int k = r.zmax - d;
-                if (k >= 0 && t_decided(r.e1x, r.e1y, r.e1z, r.e2x, r.e2y, r.e2z, r.inv, r.v1x, r.v1y, r.v1z, oxlo, oxhi,
-                                        oylo, oyhi, oz0, g.r2z[(int64_t)k * n2 + n2 - 1], eps_above()) > 0)
-                    kh = k;
-            }
-        }
-        if (own) dst[stride - 1] = (uint64_t)(uint32_t)(kh + 1) | ((uint64_t)(uint32_t)(zc + 1) << 32);
-    }
-    // the lane's sub-column x origins in registers
-    float oxr[16];
-#pragma unroll
-    for (int p = 0; p < 16; ++p) oxr[p] = p < n2 ? rx[p] : 0.0f;
-    uint64_t w = 0;
-    int k = 0, slot = 0;
-    for (int q = 0; q < n2; ++q) {
-        const float oy = ry[q];
-#pragma unroll
-        for (int p = 0; p < 16; ++p) {
-            if (p < n2) {
-                float tx, ty;
-                w |= (uint64_t)colrec_xy(r, oxr[p], oy, tx, ty) << k;
-                if (++k == 64) {
-                    if (own) dst[slot] = w;
-                    ++slot;
-                    w = 0;
-                    k = 0;
-                }
-            }
-        }
-    }
-    if (k && own) dst[slot] = w;
-}
-
-template <bool kM, int CP_WAVES>
-__global__ __launch_bounds__(64 * CP_WAVES) void k_col_pass(const float4* __restrict__ rec, GridDev g0,
-                                                                   Meshes M, uint32_t nent, int stride,
-                                                                   uint64_t* __restrict__ cpass)
-{
-    const uint64_t wbase = ((uint64_t)blockIdx.x * CP_WAVES + (threadIdx.x >> 6)) * 64;
-    if (wbase >= nent) return;
-    const int lane = __lane_id();
-    const uint32_t e = (uint32_t)wbase + (uint32_t)lane;
-    const bool own = e < nent;
-    const uint32_t ei = own ? e : nent - 1;
-    const ColRec r = load_colrec(rec, ei);
-    const uint32_t colb = __float_as_uint(rec[3 * (uint64_t)ei + 2].w);   // batch-wide column
-    uint64_t* dst = cpass + (uint64_t)ei * stride;
-    if constexpr (!kM) {
-        col_pass_entry(g0, colb, r, own, dst, stride);
-    } else {
-        const int lastl = nent - 1 - wbase < 63 ? (int)(nent - 1 - wbase) : 63;
-        const uint32_t cf = (uint32_t)__shfl((int)colb, 0), cl = (uint32_t)__shfl((int)colb, lastl);
-        auto col0 = [](const MeshOff& o) { return (uint64_t)o.col0; };
-        const int mf = wave_mesh_search(M.off, M.nm, cf, col0), ml = wave_mesh_search(M.off, M.nm, cl, col0);
-        for (int m = mf; m <= ml; ++m) {
-            const uint32_t c0 = M.off[m].col0, c1 = M.off[m + 1].col0;
-            if (colb >= c0 && colb < c1) col_pass_entry(M.grids[m], colb - c0, r, own, dst, stride);
-        }
-    }
-}
-
-template <int CW>
-static void launch_col_pass_w(const float4* rec, const GridDev& g0, const Meshes& M, uint64_t nent, int stride,
-                              uint64_t* cpass, hipStream_t s)
-{
-    const uint64_t waves = (nent + 63) / 64;
-    const uint64_t blocks = (waves + CW - 1) / CW;
-    if (M.nm > 1)
-        k_col_pass<true, CW><<<(unsigned)blocks, 64 * CW, 0, s>>>(rec, g0, M, (uint32_t)nent, stride, cpass);
-    else
-        k_col_pass<false, CW><<<(unsigned)blocks, 64 * CW, 0, s>>>(rec, g0, M, (uint32_t)nent, stride, cpass);
-}
-
-void launch_col_pass(const float4* rec, const GridDev& g0, const Meshes& M, uint64_t nent, int stride, int waves,
-                     uint64_t* cpass, hipStream_t s)
-{
-    if (nent == 0) return;
-    if (waves <= 1) launch_col_pass_w<1>(rec, g0, M, nent, stride, cpass, s);
-    else if (waves == 2) launch_col_pass_w<2>(rec, g0, M, nent, stride, cpass, s);
-    else launch_col_pass_w<4>(rec, g0, M, nent, stride, cpass, s);
-}
-
-// How the t test of a column record moves with the ray origin's z, for every
-// sub-column: 0 it passes on a prefix of rising z (or is constant), 1 on a
-// suffix, 2 not known to be monotone.  Rounding is monotone, so each float
-// operation of mt_t_hit is monotone in a monotone operand: tz rises with z,
-// qx = ty e1z - tz e1y moves with -sgn(e1y), qy = tz e1x - tx e1z with
-// sgn(e1x), qz is constant; e2x qx and e2y qy then move with -sgn(e2x)
-// sgn(e1y) and sgn(e2y) sgn(e1x), their left-to-right sum (plus the constant
-// e2z qz) is monotone when those do not oppose, and the product by inv flips
-// it for inv < 0.  That needs every intermediate finite: with the edges,
-// |tx|, |ty| and |v1z| within 2^42, the ray origins within 2^41 and |inv|
-// within 1e7 no product or sum leaves the float range (2^110 at most); the
-// record's part is checked here, the origins' where the search is used.
-// The directions do not depend on (tx, ty).
-__device__ __forceinline__ int sgnf(float x) { return (x > 0.0f) - (x < 0.0f); }
-
-__device__ __forceinline__ int t_run_kind(const ColRec& r)
-{
-    const float lim = 0x1p42f;
-    if (!(fabsf(r.e1x) <= lim && fabsf(r.e1y) <= lim && fabsf(r.e1z) <= lim && fabsf(r.e2x) <= lim &&
-          fabsf(r.e2y) <= lim && fabsf(r.e2z) <= lim && fabsf(r.v1z) <= lim && fabsf(r.inv) <= 1e7f))
-        return 2;
-    const int da = -sgnf(r.e2x) * sgnf(r.e1y), db = sgnf(r.e2y) * sgnf(r.e1x);
-    if (da * db < 0) return 2;
-    return (da ? da : db) * sgnf(r.inv) > 0 ? 1 : 0;
-}
-
-// One boundary voxel (i1, j1, k1) of the Level2 parity.  N2 > 0: the Level2
-// resolution as a compile-time constant (layer loops unrolled, the layer
-// origins held uniform); N2 == 0: any resolution n2 <= 16.  The kernels use
-// it for the resolutions other than 8 (two voxels per wave,
-// l2_parity_pack2_8) and at most 4 (four per wave, l2_parity_pack4).
-template <int N2, bool kRuns = false>
-__device__ __forceinline__ void l2_parity_voxel(int n2_rt, int w2, const GridDev& g, int i1, int j1, int k1,
-                                                uint32_t e0, uint32_t e1, const float4* __restrict__ rec,
-                                                const uint64_t* __restrict__ cpass, int stride, ColRec* cr,
-                                                unsigned long long* acc, float* soz, uint64_t* __restrict__ out)
+// which item range [so, so + P) of the wave's lanes holds item l0 + lane (ranges
+// in lane order); lanes past the last item get some lane's
+__device__ __forceinline__ int wave_item_owner(uint8_t* win, uint32_t so, uint32_t P, uint32_t l0)
 {
     const int lane = __lane_id();
-    const int n2 = N2 > 0 ? N2 : n2_rt;
-    constexpr int NMX = N2 > 0 ? (N2 * N2 + 63) / 64 : 4;   // sub-column slots per lane
-    const int nsc = n2 * n2;
-    const int nm = N2 > 0 ? NMX : (nsc + 63) >> 6;
-    const float* rx = g.r2x + (int64_t)i1 * n2;
-    const float* ry = g.r2y + (int64_t)j1 * n2;
-    const float* rz = g.r2z + (int64_t)k1 * n2;
-    // this lane's sub-columns sc = lane + 64*mm: ray origins
-    float ox[NMX], oy[NMX];
-#pragma unroll
-    for (int mm = 0; mm < NMX; ++mm) {
-        const int sc = lane + 64 * mm;
-        ox[mm] = (mm < nm && sc < nsc) ? rx[sc % n2] : 0.0f;
-        oy[mm] = (mm < nm && sc < nsc) ? ry[sc / n2] : 0.0f;
-    }
-    // layer origins of the sub-voxels: entry r in lane r (and, for a fixed
-    // resolution, in uniform registers)
-    const float ozl = lane < n2 ? rz[lane] : 0.0f;
-    float oz[N2 > 0 ? N2 : 1];
-#pragma unroll
-    for (int rr = 0; rr < (N2 > 0 ? N2 : 1); ++rr) oz[rr] = lane_f(ozl, rr);
-    // resolutions without a fixed layer loop: the layer origins also in LDS,
-    // for per-lane searches along the layers (tables non-decreasing)
-    const bool zruns = kRuns && N2 == 0 && g.r2mono != 0 && n2 >= 8 && fabsf(lane_f(ozl, 0)) <= 0x1p41f &&
-                       fabsf(lane_f(ozl, n2 - 1)) <= 0x1p41f;
-    if (kRuns && N2 == 0 && lane < n2) soz[lane] = ozl;
+    // every range that meets [l0, l0 + 64) marks its first position there (the
+    // one running into the window marks 0; starts are distinct), and an item
+    // takes the mark at the highest marked position up to its own
+    win[lane] = 0xff;
     __builtin_amdgcn_wave_barrier();
-    const uint64_t layers = (1ull << n2) - 1;
-    uint64_t bits = 0;   // bit (mm*n2 + r) for sub-column lane + 64*mm
-    for (uint32_t base = e0; base < e1; base += 64) {
-        const uint32_t i = base + lane;
-        const int k1c = k1;
-        uint64_t row[NMX];   // candidate's det/u/v pass bits over the sub-columns
+    if (P && so < l0 + 64u && so + P > l0) win[so > l0 ? so - l0 : 0u] = (uint8_t)lane;
+    __builtin_amdgcn_wave_barrier();
+    const uint32_t wj = win[lane];
+    const uint64_t marks = __ballot(wj != 0xffu) & ((2ull << lane) - 1ull);
+    const int top = marks ? 63 - __clzll((long long)marks) : 0;
+    const int j = __shfl((int)wj, top) & 63;
+    __builtin_amdgcn_wave_barrier();
+    return j;
+}
+
+// C adjacent columns (i1 .., j1) of a mesh by one wave: 1, or 4 (at n2 <= 4).
+template <int C, int KB>
+__device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB>& L, uint64_t* cb, int nw, const GridDev& g, int i1, int j1,
+                                                       uint64_t word0, uint32_t col0, uint32_t b0,
+                                                       const uint64_t* __restrict__ bnd,
+                                                       const uint32_t* __restrict__ wprefix,
+                                                       const uint32_t* __restrict__ coff,
+                                                       const float4* __restrict__ rec, uint64_t* __restrict__ out)
+{
+    const int lane = __lane_id();
+    const int n2 = g.n2, w2 = g.w2, nsc = n2 * n2, nz = g.nz;
+    const int fb = C == 1 && n2 > 8 ? 2 : 1;
+    uint32_t* pre = reinterpret_cast<uint32_t*>(cb + C * nw);
+    const uint32_t gcol = col0 + (uint32_t)(j1 * g.nx + i1);
+    uint32_t ce[C + 1];   // the columns' first entries
 #pragma unroll
-        for (int mm = 0; mm < NMX; ++mm) row[mm] = 0;
-        bool hit = false;   // every layer's t passes: no t test, no record
-        if (i < e1) {
-            // header (k_col_pass): candidate while k1 <= zc
-            const uint64_t hw = cpass[(uint64_t)i * stride + stride - 1];
-            const int kh = (int)(uint32_t)hw - 1, zc = (int)(uint32_t)(hw >> 32) - 1;
-            if (k1c <= zc) {
+    for (int c = 0; c <= C; ++c) ce[c] = coff[gcol + (uint32_t)c];
+    if (lane < C * n2) L.ox[lane] = g.r2x[i1 * n2 + lane];
+    if (lane < n2) L.oy[lane] = g.r2y[j1 * n2 + lane];
+    // slots of a column per window; one more row carries what lies above it
+    const int Wn = min(KB / (C * nsc * fb) - 1, L2P_SLOTS / C);
+    // the columns' boundary voxels: a bit per layer, their number below each
+    // word of bits, and the boundary index of each slot of the window [lo, hi)
+    const uint64_t word = word0 + (uint64_t)j1 * g.nxw + (uint64_t)(i1 >> 6);
+    const uint64_t plane = (uint64_t)g.ny * g.nxw;
+    const int bit0 = i1 & 63;
+    uint32_t S[C], lo[C], hi[C];
+    auto scan = [&](bool first) {
 #pragma unroll
-                for (int mm = 0; mm < NMX; ++mm)
-                    if (mm < nm) row[mm] = cpass[(uint64_t)i * stride + mm];
-                hit = k1c <= kh;
-                if (!hit) {
-                    ColRec r = load_colrec(rec, i);
-                    if (kRuns) r.zmax = t_run_kind(r);   // the slot is free here: the header holds zc
-                    cr[lane] = r;
+        for (int c = 0; c < C; ++c) S[c] = 0u;
+        for (int kw = 0; kw * 64 < nz; ++kw) {
+            const int k = kw * 64 + lane;
+            uint64_t bits = 0;
+            uint32_t base = 0;
+            if (k < nz) {
+                const uint64_t w = word + (uint64_t)k * plane;
+                bits = bnd[w];
+                base = wprefix[w] - b0;
+            }
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+                const uint64_t m = __ballot((bits >> (bit0 + c)) & 1ull);
+                const uint32_t rank = S[c] + (uint32_t)__popcll(m & lanes_below_mask());
+                if (first && lane == 0) {
+                    cb[c * nw + kw] = m;
+                    pre[c * nw + kw] = S[c];
                 }
+                if (((m >> lane) & 1ull) && rank >= lo[c] && rank < hi[c])
+                    L.slotb[c * Wn + (int)(rank - lo[c])] = base + (uint32_t)__popcll(bits & ((1ull << (bit0 + c)) - 1ull));
+                S[c] += (uint32_t)__popcll(m);
             }
         }
-        const uint64_t all_hit = __ballot(hit);
+    };
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        lo[c] = 0u;
+        hi[c] = (uint32_t)Wn;
+    }
+    scan(true);
+    uint32_t most = 0;
+#pragma unroll
+    for (int c = 0; c < C; ++c) most = max(most, S[c]);
+    if (most == 0) return;
+    const SatScale sc{g.s2x, g.s2y, g.s2z, g.d2x, g.d2y, g.d2z};
+    const float gx = 2.0f * g.h2x, gy = 2.0f * g.h2y, inv_n2 = GPV_RCP((float)n2);
+    const float* rz = g.r2z;
+    uint8_t* a8 = reinterpret_cast<uint8_t*>(L.acc);
+    uint16_t* a16 = reinterpret_cast<uint16_t*>(L.acc);
+    // windows of slots from the top down (one, but for columns of many boundary voxels)
+    for (uint32_t w0 = 0; w0 < most; w0 += (uint32_t)Wn) {
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            hi[c] = S[c] > w0 ? S[c] - w0 : 0u;
+            lo[c] = hi[c] > (uint32_t)Wn ? hi[c] - (uint32_t)Wn : 0u;
+        }
+        if (most > (uint32_t)Wn) {
+            scan(false);
+        }
+        // clear the slots; the row past them keeps the parity of all windows above
+        if (w0 == 0) {
+            for (int i = lane; i < (C * (Wn + 1) * nsc * fb + 3) / 4; i += 64) L.acc[i] = 0u;
+        } else {
+            for (int i = lane; i < C * Wn * nsc; i += 64) {
+                const int c = C == 1 ? 0 : i / (Wn * nsc);
+                const int at = i + c * nsc;
+                if (fb == 2) a16[at] = 0;
+                else a8[at] = 0;
+            }
+        }
         __builtin_amdgcn_wave_barrier();
-        // pass bits per sub-column slot: bit j = candidate j passes at this
-        // lane's sub-column
-        uint64_t pass[NMX];
+        for (uint32_t base = ce[0]; base < ce[C]; base += L2P_STAGE) {
+            const uint32_t i = base + (uint32_t)lane;
+            uint32_t P = 0;   // rows of this lane's entry
+            int q0 = 0;
+            if (lane < L2P_STAGE && i < ce[C]) {
+                const float4 a = rec[3 * (uint64_t)i + 0], b = rec[3 * (uint64_t)i + 1], d = rec[3 * (uint64_t)i + 2];
+                int c = 0;
 #pragma unroll
-        for (int mm = 0; mm < NMX; ++mm) pass[mm] = mm < nm ? wave_transpose64(row[mm]) : 0;
-        // t per sub-voxel for the passing pairs not decided for the voxel
+                for (int k = 1; k < C; ++k) c += (int)(i >= ce[k]);
+                const int zmax = __float_as_int(d.z);
+                ParEntry r;
+                r.e1x = a.x; r.e1y = a.y; r.e1z = a.z; r.e2x = a.w;
+                r.e2y = b.x; r.e2z = b.y; r.inv = b.z; r.v1x = b.w;
+                r.v1y = d.x;
+                r.l0 = zmax * n2;
+                const float ox0 = L.ox[c * n2], oy0 = L.oy[0];
+                par_entry(r, d.y, par_oz(g.bminz, 2.0f * g.h1z, 2.0f * g.h2z, zmax), ox0, oy0, gx, gy, n2, sc);
+                // candidate for the voxels up to zmax (all with the CUDA kernels' whole-column lists)
+                const int cap = (g.l2cuda ? nz : zmax + 1) * n2;
+                bool meets = true;
+                if (most > (uint32_t)Wn) {
+                    // some toggle may fall into this window's slots
+                    uint32_t clo = lo[0], chi = hi[0];
 #pragma unroll
-        for (int mm = 0; mm < NMX; ++mm) {
-            if (__popcll(pass[mm] & all_hit) & 1) bits ^= layers << (mm * n2);
-            for (uint64_t m = pass[mm] & ~all_hit; m; m &= m - 1) {
-                const int j = __ffsll((unsigned long long)m) - 1;
-                const ColRec r = cr[j];
-                const float tx = ox[mm] - r.v1x, ty = oy[mm] - r.v1y;
-                uint32_t hm = 0;   // bit rr: t > 1e-6 at layer rr
-                if constexpr (N2 > 0) {
-#pragma unroll
-                    for (int rr = 0; rr < N2; ++rr)
-                        hm |= (uint32_t)mt_t_hit(r.e1x, r.e1y, r.e1z, r.e2x, r.e2y, r.e2z, r.inv, tx, ty, r.v1z,
-                                                 oz[rr])
-                              << rr;
-                } else {
-                    if (kRuns && zruns && r.zmax < 2 && fabsf(tx) <= 0x1p42f && fabsf(ty) <= 0x1p42f) {
-                        // the passing layers are one run at an end: find its edge
-                        const bool pre = r.zmax == 0;
-                        int lo = 0, hi = n2;
-                        while (lo < hi) {
-                            const int mid = (lo + hi) >> 1;
-                            const bool t = mt_t_hit(r.e1x, r.e1y, r.e1z, r.e2x, r.e2y, r.e2z, r.inv, tx, ty, r.v1z,
-                                                    soz[mid]);
-                            if (t == pre) lo = mid + 1;
-                            else hi = mid;
+                    for (int k = 1; k < C; ++k) {
+                        clo = c == k ? lo[k] : clo;
+                        chi = c == k ? hi[k] : chi;
+                    }
+                    int lmin, lmax;
+                    par_z_range(r, sc.sz, cap, lmin, lmax);
+                    auto upto = [&](int n) -> uint32_t {   // boundary voxels at or below layer n - 1
+                        if (n <= 0) return 0u;
+                        const int k = (int)(((float)(n - 1) + 0.5f) * inv_n2);
+                        return pre[c * nw + (k >> 6)] + (uint32_t)__popcll(cb[c * nw + (k >> 6)] & ((2ull << (k & 63)) - 1ull));
+                    };
+                    meets = upto(lmin) <= chi && upto(lmax) > clo;
+                }
+                const int nq = meets ? par_rows(r, oy0, sc.sy, n2, sc.dy, q0) : 0;
+                P = nq > 0 ? (uint32_t)nq : 0u;
+                L.e[lane][0] = a;
+                L.e[lane][1] = b;
+                L.e[lane][2] = make_float4(d.x, r.dz, r.mu, r.delta);
+                L.e[lane][3] = make_float4(__int_as_float(r.l0), __int_as_float(cap), __int_as_float(c), d.y);
+            }
+            const uint32_t incl = wave_incl_scan<uint32_t>(P);
+            const uint32_t so = incl - P;
+            const uint32_t rows = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+            __builtin_amdgcn_wave_barrier();
+            // the (entry, row) items: the columns each row can accept
+            for (uint32_t l0 = 0; l0 < rows; l0 += 64) {
+                const int j = wave_item_owner(L.win, so, P, l0) & (L2P_STAGE - 1);
+                const int q = __shfl(q0, j) + (int)(l0 + (uint32_t)lane - (uint32_t)__shfl((int)so, j));
+                int p0 = 0, np = 0;
+                if (l0 + (uint32_t)lane < rows) {
+                    const float4 a = L.e[j][0], b = L.e[j][1], d = L.e[j][2];
+                    const int c = C == 1 ? 0 : __float_as_int(L.e[j][3].z);
+                    ParEntry r;
+                    r.e1x = a.x; r.e1y = a.y; r.e2x = a.w;
+                    r.e2y = b.x; r.inv = b.z; r.v1x = b.w;
+                    r.v1y = d.x; r.delta = d.w;
+                    np = par_cols(r, L.ox[c * n2], L.oy[0], gx, gy, n2, q, p0);
+                    np = np > 0 ? np : 0;
+                }
+                const uint32_t pincl = wave_incl_scan<uint32_t>((uint32_t)np);
+                const uint32_t pso = pincl - (uint32_t)np;
+                const uint32_t pairs = (uint32_t)__builtin_amdgcn_readlane((int)pincl, 63);
+                const int pq = p0 | (q << 8) | (j << 16);
+                // the (entry, sub-column) pairs
+                for (uint32_t m0 = 0; m0 < pairs; m0 += 64) {
+                    const int o = wave_item_owner(L.win, pso, (uint32_t)np, m0);
+                    const int v = __shfl(pq, o);
+                    const uint32_t at = m0 + (uint32_t)lane - (uint32_t)__shfl((int)pso, o);
+                    if (m0 + (uint32_t)lane < pairs) {
+                        const int pp = (v & 255) + (int)at, qq = (v >> 8) & 255, jj = v >> 16;
+                        const float4 a = L.e[jj][0], b = L.e[jj][1], d = L.e[jj][2], f = L.e[jj][3];
+                        const int c = C == 1 ? 0 : __float_as_int(f.z);
+                        // the float det/u/v test (mt_column)
+                        const float tx = L.ox[c * n2 + pp] - b.w, ty = L.oy[qq] - d.x;
+                        const float u = (tx * -b.x + ty * a.w) * b.z;
+                        const float vv = (tx * a.y - ty * a.x) * b.z;
+                        int la = 0, lb = 0;
+                        const bool accepted = !((u < 0.f) | (u > 1.f) | (vv < 0.f) | (u + vv > 1.f));
+                        if (accepted) {
+                            ParEntry r;
+                            r.e1z = a.z; r.e2z = b.y; r.dz = d.y; r.mu = d.z;
+                            r.l0 = __float_as_int(f.x);
+                            par_layers(r, u, vv, sc.sz, __float_as_int(f.y), la, lb);
                         }
-                        hm = pre ? (uint32_t)((1ull << lo) - 1) : (uint32_t)(layers & ~((1ull << lo) - 1));
-                    } else {
-                        for (int rr = 0; rr < n2; ++rr)
-                            hm |= (uint32_t)mt_t_hit(r.e1x, r.e1y, r.e1z, r.e2x, r.e2y, r.e2z, r.inv, tx, ty, r.v1z,
-                                                     lane_f(ozl, rr))
-                                  << rr;
+                        uint32_t clo = lo[0], chi = hi[0];
+#pragma unroll
+                        for (int k = 1; k < C; ++k) {
+                            clo = c == k ? lo[k] : clo;
+                            chi = c == k ? hi[k] : chi;
+                        }
+                        const uint32_t sub = (uint32_t)(c * (Wn + 1) * nsc + qq * n2 + pp);
+                        // layers below la pass, none from lb on passes, the float test says
+                        // which of those between do: a toggle wherever that changes
+                        bool pass = accepted;   // whether the layer before passes
+                        for (int l = la; pass || l < lb;) {
+                            int n = lb;         // the next change
+                            for (; l < lb; ++l) {
+                                const int k = (int)(((float)l + 0.5f) * inv_n2);
+                                if (!((cb[c * nw + (k >> 6)] >> (k & 63)) & 1ull)) {
+                                    l = (k + 1) * n2 - 1;   // no boundary voxel here
+                                    continue;
+                                }
+                                if (mt_t_hit(a.x, a.y, a.z, a.w, b.x, b.y, b.z, tx, ty, f.w, rz[l]) != pass) {
+                                    n = l++;
+                                    break;
+                                }
+                            }
+                            // (past lb with the last state `false`: nothing to toggle)
+                            if (n == lb && !pass) break;
+                            pass = !pass;
+                            if (n > 0) {
+                                // `n` layers pass: a toggle at layer n - 1 of its voxel, or at the
+                                // top of the next boundary voxel below
+                                const int k = (int)(((float)(n - 1) + 0.5f) * inv_n2);
+                                const uint64_t bw = cb[c * nw + (k >> 6)];
+                                const uint32_t upto =
+                                    pre[c * nw + (k >> 6)] + (uint32_t)__popcll(bw & ((2ull << (k & 63)) - 1ull));
+                                if (upto > clo && upto <= chi) {
+                                    const int bit = ((bw >> (k & 63)) & 1ull) ? n - 1 - k * n2 : n2 - 1;
+                                    uint32_t sh;
+                                    const uint32_t wi = l2_col_word((upto - 1u - clo) * (uint32_t)nsc + sub, n2, sh);
+                                    atomicXor(&L.acc[wi], 1u << (sh + bit));
+                                }
+                            }
+                        }
                     }
                 }
-                bits ^= (uint64_t)hm << (mm * n2);
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+        // toggles -> parities, from each column's top slot down
+        const uint32_t layers = (1u << n2) - 1u;
+        for (int it = lane; it < C * nsc; it += 64) {
+            const int c = C == 1 ? 0 : it / nsc;
+            const int sub = it - c * nsc;
+            uint32_t n = hi[0] - lo[0];
+#pragma unroll
+            for (int k = 1; k < C; ++k) n = c == k ? hi[k] - lo[k] : n;
+            const int r0 = c * (Wn + 1) * nsc + sub, top = r0 + Wn * nsc;
+            uint32_t above = fb == 2 ? (uint32_t)a16[top] : (uint32_t)a8[top];
+            for (int s = (int)n - 1; s >= 0; --s) {
+                const int at = r0 + s * nsc;
+                uint32_t x = fb == 2 ? (uint32_t)a16[at] : (uint32_t)a8[at];
+                x ^= x >> 1;
+                x ^= x >> 2;
+                x ^= x >> 4;
+                x ^= x >> 8;   // bit r: toggles at r and above
+                const uint32_t y = x ^ (above ? layers : 0u);
+                if (fb == 2) a16[at] = (uint16_t)y;
+                else a8[at] = (uint8_t)y;
+                above ^= x & 1u;
+            }
+            if (fb == 2) a16[top] = (uint16_t)above;
+            else a8[top] = (uint8_t)above;
+        }
+        __builtin_amdgcn_wave_barrier();
+        // the slots' words
+        if (C == 1 && n2 == 8) {
+            const int n = (int)(hi[0] - lo[0]);
+            for (int v0 = 0; v0 < n; v0 += 8) {
+                // bit 8v + r of lane c: layer r of sub-column c of slot v0 + v
+                uint64_t x = 0;
+                for (int v = 0; v < 8 && v0 + v < n; ++v) x |= (uint64_t)a8[(v0 + v) * 64 + lane] << (8 * v);
+                x = wave_transpose64(x);
+                const int v = v0 + (lane >> 3);
+                if (v < n) out[(uint64_t)L.slotb[v] * 8 + (uint64_t)(lane & 7)] = x;
+            }
+        } else if (C == 1 && n2 == 16) {
+            const int n = (int)(hi[0] - lo[0]);
+            for (int v = 0; v < n; ++v) {
+                // bit 16k + r of lane c: layer r of sub-column 64k + c
+                uint64_t x = 0;
+                for (int k = 0; k < 4; ++k) x |= (uint64_t)a16[v * 256 + k * 64 + lane] << (16 * k);
+                out[(uint64_t)L.slotb[v] * 64 + (uint64_t)(4 * (lane & 15) + (lane >> 4))] = wave_transpose64(x);
+            }
+        } else {
+            const float inv = GPV_RCP((float)nsc);
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+                const int n = (int)(hi[c] - lo[c]);
+                // lane t of a run of 64 keeps word t of the column's (slot, word) list
+                for (int t0 = 0; t0 < n * w2; t0 += 64) {
+                    uint64_t mine = 0;
+                    int v = t0 / w2, m = t0 - v * w2;
+                    const int te = min(64, n * w2 - t0);
+                    for (int t = 0; t < te; ++t) {
+                        const int s = 64 * m + lane;
+                        const int r = (int)(((float)s + 0.5f) * inv);   // exact: s + 1/2 is at least 1/512 of n2^2 from a multiple
+                        const int at = (c * (Wn + 1) + v) * nsc + (s - r * nsc);
+                        const uint32_t x = fb == 2 ? (uint32_t)a16[at] : (uint32_t)a8[at];
+                        const uint64_t wd = __ballot(r < n2 && ((x >> r) & 1u));
+                        if (lane == t) mine = wd;
+                        if (++m == w2) {
+                            m = 0;
+                            ++v;
+                        }
+                    }
+                    if (lane < te) {
+                        const int v1 = (t0 + lane) / w2;
+                        out[(uint64_t)L.slotb[c * Wn + v1] * (uint64_t)w2 + (uint64_t)(t0 + lane - v1 * w2)] = mine;
+                    }
+                }
             }
         }
         __builtin_amdgcn_wave_barrier();
     }
-    if (nsc % 64 == 0) {
-        // word r * (nsc / 64) + mm holds layer r of sub-columns 64mm + lane:
-        // one ballot per word, lane w keeps word w, one coalesced store
-        uint64_t mine = 0;
-#pragma unroll
-        for (int mm = 0; mm < NMX; ++mm) {
-            if (mm >= nm) break;
-            for (int r = 0; r < n2; ++r) {
-                const uint64_t wd = __ballot((bits >> (mm * n2 + r)) & 1ull);
-                if (lane == r * nm + mm) mine = wd;
-            }
-        }
-        if (lane < w2) out[lane] = mine;
-        return;
-    }
-    for (int i = lane; i < w2; i += 64) acc[i] = 0ull;
-    __builtin_amdgcn_wave_barrier();
-    for (int mm = 0; mm < nm; ++mm) {
-        const int sc = lane + 64 * mm;
-        if (sc >= nsc) break;
-        for (int r = 0; r < n2; ++r) {
-            if ((bits >> (mm * n2 + r)) & 1ull) {
-                const int s = r * nsc + sc;
-                atomicOr(&acc[s >> 6], 1ull << (s & 63));
-            }
-        }
-    }
-    __builtin_amdgcn_wave_barrier();
-    for (int i = lane; i < w2; i += 64) out[i] = acc[i];
 }
 
-// kM: batch (resolution per mesh, N2 = 0); single mesh: N2 = its resolution
-// when it is 4 or 8 (a kernel of its own, so each keeps its own register
-// budget), else 0
-// Four boundary voxels of one mesh with n2 <= 4 (n2^2 <= 16 sub-columns) in
-// one wave: lane 16v + sc is sub-column sc of voxel v.  Each quarter stages
-// 16 of its own column's candidates per round; a candidate's pass bits sit at
-// bits [16v, 16v + 16) of its lane's row, so one 64x64 transpose gives every
-// lane the pass bits of its own voxel's candidates (the rows of the other
-// quarters have no bits there).  N2 = 4: layers unrolled; 0: any n2 <= 4.
-template <int N2>
-__device__ __forceinline__ void l2_parity_pack4(int n2rt, const GridDev& g, uint32_t col0, int64_t bfirst, int nv,
-                                                const int32_t* __restrict__ bidx, const uint32_t* __restrict__ coff,
-                                                const float4* __restrict__ rec, const uint64_t* __restrict__ cpass,
-                                                int stride, ColRec* cr, uint64_t* __restrict__ out)
+template <bool kM, int KB, int W>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 1 ? 6 : 3))) void k_l2_parity(const uint64_t* __restrict__ bnd,
+                                                      const uint32_t* __restrict__ wprefix, int64_t nwaves, bool many, int nw,
+                                                      const uint32_t* __restrict__ coff,
+                                                      const float4* __restrict__ rec, GridDev g0, Meshes M,
+                                                      uint64_t* __restrict__ par2)
 {
-    const int lane = __lane_id();
-    const int n2 = N2 > 0 ? N2 : n2rt;
-    const int nsc = n2 * n2;
-    const int v = lane >> 4, sc = lane & 15;
-    const bool lv = v < nv;
-    int k1 = 0, ij = 0, i1 = 0, j1 = 0;
-    if (lv) {
-        const int vox = bidx[bfirst + v];
-        const int nxy = g.nx * g.ny;
-        k1 = vox / nxy;
-        ij = vox - k1 * nxy;
-        j1 = ij / g.nx;
-        i1 = ij - j1 * g.nx;
-    }
-    const uint32_t e0 = lv ? coff[col0 + ij] : 0u, e1 = lv ? coff[col0 + ij + 1] : 0u;
-    const bool ls = lv && sc < nsc;
-    const float ox = ls ? g.r2x[(int64_t)i1 * n2 + sc % n2] : 0.0f;
-    const float oy = ls ? g.r2y[(int64_t)j1 * n2 + sc / n2] : 0.0f;
-    float oz[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) oz[r] = (lv && r < n2) ? g.r2z[(int64_t)k1 * n2 + r] : 0.0f;
-    const uint32_t layers = (1u << n2) - 1;
-    // rounds of 16 candidates: the most any quarter needs
-    uint32_t nr = (e1 - e0 + 15) >> 4;
-#pragma unroll
-    for (int d = 16; d <= 32; d <<= 1) {
-        const uint32_t o = (uint32_t)__shfl_xor((int)nr, d);
-        nr = o > nr ? o : nr;
-    }
-    const uint32_t rounds = (uint32_t)__builtin_amdgcn_readfirstlane((int)nr);
-    uint32_t par = 0;   // bit r: parity at layer r of this lane's sub-column
-    for (uint32_t rd = 0; rd < rounds; ++rd) {
-        const uint32_t i = e0 + rd * 16 + (uint32_t)sc;
-        uint64_t row = 0;
-        bool hit = false;   // every layer's t passes for this slot's voxel
-        if (lv && i < e1) {
-            // header (k_col_pass): candidate while k1 <= zc
-            const uint64_t hw = cpass[(uint64_t)i * stride + stride - 1];
-            const int kh = (int)(uint32_t)hw - 1, zc = (int)(uint32_t)(hw >> 32) - 1;
-            if (k1 <= zc) {
-                row = (cpass[(uint64_t)i * stride] & 0xffffull) << (16 * v);
-                hit = k1 <= kh;
-                if (!hit) cr[lane] = load_colrec(rec, i);
-            }
-        }
-        // slot j's flag is for slot j's own voxel, the only one whose lanes
-        // see bit j after the transpose
-        const uint64_t all_hit = __ballot(hit);
-        __builtin_amdgcn_wave_barrier();
-        const uint64_t pm = wave_transpose64(row);
-        if (__popcll(pm & all_hit) & 1) par ^= layers;
-        for (uint64_t m = pm & ~all_hit; m; m &= m - 1) {
-            const int j = __ffsll((unsigned long long)m) - 1;
-            const ColRec r = cr[j];
-            const float tx = ox - r.v1x, ty = oy - r.v1y;
-            uint32_t hm = 0;
-            if constexpr (N2 > 0) {
-#pragma unroll
-                for (int rr = 0; rr < N2; ++rr)
-                    hm |= (uint32_t)mt_t_hit(r.e1x, r.e1y, r.e1z, r.e2x, r.e2y, r.e2z, r.inv, tx, ty, r.v1z, oz[rr])
-                          << rr;
-            } else {
-                for (int rr = 0; rr < n2; ++rr)
-                    hm |= (uint32_t)mt_t_hit(r.e1x, r.e1y, r.e1z, r.e2x, r.e2y, r.e2z, r.inv, tx, ty, r.v1z,
-                                             rr == 0 ? oz[0] : rr == 1 ? oz[1] : rr == 2 ? oz[2] : oz[3])
-                          << rr;
-            }
-            par ^= hm;
-        }
-        __builtin_amdgcn_wave_barrier();
-    }
-    // voxel v's word: bit r*nsc + sc for layer r (n2^3 <= 64, one word)
-    const uint64_t smask = nsc >= 64 ? ~0ull : ((1ull << nsc) - 1);
-    uint64_t word = 0;
-    for (int r = 0; r < n2; ++r) {
-        const uint64_t m = __ballot((par >> r) & 1u);
-        word |= ((m >> (16 * v)) & smask) << (r * nsc);
-    }
-    if (lv && sc == 0) out[v] = word;
-}
-
-// Waves: single mesh, one per boundary voxel, or (n2 <= 4) one per four;
-// batch, per mesh from MeshOff::pw0 likewise.
-// Two boundary voxels of a Level2-8 mesh per wave.  Lanes 32h .. 32h + 31
-// load voxel h's column entries, 32 per round; one 64x64 transpose of their
-// pass-bit rows leaves lane l with sub-column l of both voxels (bit j < 32:
-// voxel 0's slot j passes there; bit j >= 32: voxel 1's slot j - 32), so the
-// two voxels' dependent loads and tests overlap in one wave and share its
-// transposes.  Voxel h's words go to out[8h .. 8h + 7] (word r holds layer r
-// of its 64 sub-columns, bit = sub-column).
-__device__ __forceinline__ void l2_parity_pack2_8(const GridDev& g, uint32_t col0, int64_t bfirst, int nv,
-                                                  const int32_t* __restrict__ bidx, const uint32_t* __restrict__ coff,
-                                                  const float4* __restrict__ rec, const uint64_t* __restrict__ cpass,
-                                                  int stride, ColRec* cr, uint64_t* __restrict__ out)
-{
-    const int lane = __lane_id();
-    const int h = lane >> 5, slot = lane & 31;
-    const int nxy = g.nx * g.ny;
-    int k1v[2];
-    uint32_t e0v[2], e1v[2];
-    float ox[2], oy[2], oz[2][8];
-#pragma unroll
-    for (int hh = 0; hh < 2; ++hh) {
-        const int vox = uniform_i(bidx[bfirst + (hh < nv ? hh : 0)]);
-        const int k1 = vox / nxy;
-        const int ij = vox - k1 * nxy;
-        const int j1 = ij / g.nx;
-        const int i1 = ij - j1 * g.nx;
-        k1v[hh] = k1;
-        e0v[hh] = (uint32_t)uniform_i((int)coff[col0 + ij]);
-        e1v[hh] = hh < nv ? (uint32_t)uniform_i((int)coff[col0 + ij + 1]) : e0v[hh];
-        ox[hh] = g.r2x[(int64_t)i1 * 8 + (lane & 7)];
-        oy[hh] = g.r2y[(int64_t)j1 * 8 + (lane >> 3)];
-#pragma unroll
-        for (int rr = 0; rr < 8; ++rr)
-            oz[hh][rr] = __int_as_float(uniform_i(__float_as_int(g.r2z[(int64_t)k1 * 8 + rr])));
-    }
-    const int k1 = h ? k1v[1] : k1v[0];
-    const uint32_t e0 = h ? e0v[1] : e0v[0], e1 = h ? e1v[1] : e1v[0];
-    const uint32_t n0 = (e1v[0] - e0v[0] + 31) >> 5, n1 = (e1v[1] - e0v[1] + 31) >> 5;
-    const uint32_t rounds = n0 > n1 ? n0 : n1;
-    uint32_t par[2] = {0u, 0u};   // bit r: parity at layer r of sub-column lane of voxel h
-    for (uint32_t rd = 0; rd < rounds; ++rd) {
-        const uint32_t i = e0 + rd * 32 + (uint32_t)slot;
-        uint64_t row = 0;
-        bool hit = false;   // every layer's t passes: no t test, no record
-        if (i < e1) {
-            // header (k_col_pass): candidate while k1 <= zc
-            const uint64_t hw = cpass[(uint64_t)i * stride + stride - 1];
-            const int kh = (int)(uint32_t)hw - 1, zc = (int)(uint32_t)(hw >> 32) - 1;
-            if (k1 <= zc) {
-                row = cpass[(uint64_t)i * stride];
-                hit = k1 <= kh;
-                if (!hit) cr[lane] = load_colrec(rec, i);
-            }
-        }
-        const uint64_t all_hit = __ballot(hit);
-        __builtin_amdgcn_wave_barrier();
-        const uint64_t pm = wave_transpose64(row);
-#pragma unroll
-        for (int hh = 0; hh < 2; ++hh) {
-            const uint64_t mh = pm & (hh ? 0xffffffff00000000ull : 0x00000000ffffffffull);
-            if (__popcll(mh & all_hit) & 1) par[hh] ^= 0xffu;
-            for (uint64_t m = mh & ~all_hit; m; m &= m - 1) {
-                const int j = __ffsll((unsigned long long)m) - 1;
-                const ColRec r = cr[j];
-                const float tx = ox[hh] - r.v1x, ty = oy[hh] - r.v1y;
-                uint32_t hm = 0;
-#pragma unroll
-                for (int rr = 0; rr < 8; ++rr)
-                    hm |= (uint32_t)mt_t_hit(r.e1x, r.e1y, r.e1z, r.e2x, r.e2y, r.e2z, r.inv, tx, ty, r.v1z, oz[hh][rr])
-                          << rr;
-                par[hh] ^= hm;
-            }
-        }
-        __builtin_amdgcn_wave_barrier();
-    }
-    uint64_t mine = 0;
-#pragma unroll
-    for (int hh = 0; hh < 2; ++hh) {
-#pragma unroll
-        for (int r = 0; r < 8; ++r) {
-            const uint64_t wd = __ballot((par[hh] >> r) & 1u);
-            if (lane == hh * 8 + r) mine = wd;
-        }
-    }
-    if (lane < 8 * nv) out[lane] = mine;
-}
-
-// kRuns: some mesh has a resolution above 8 without a fixed layer loop,
-// whose passing layers are found by a search along the run (the other
-// instantiations leave that path out and keep its registers)
-// Eight waves per SIMD (at most 64 VGPRs) for the latency of each voxel's
-// chain of dependent loads.
-template <bool kM, int N2, int L2P_WAVES, bool kRuns>
-__global__ __launch_bounds__(64 * L2P_WAVES) __attribute__((amdgpu_waves_per_eu(8))) void k_l2_parity(const int32_t* __restrict__ bidx, int64_t B,
-                                                              int64_t nwaves, const uint32_t* __restrict__ coff,
-                                                              const float4* __restrict__ rec,
-                                                              const uint64_t* __restrict__ cpass, int stride,
-                                                              GridDev g0, Meshes M, uint64_t* __restrict__ par2)
-{
-    __shared__ unsigned long long s_acc[L2P_WAVES][64];
-    __shared__ ColRec s_rec[L2P_WAVES][64];
-    __shared__ float s_oz[L2P_WAVES][16];
-    const int wv = threadIdx.x >> 6;
-    const int64_t w = (int64_t)blockIdx.x * L2P_WAVES + wv;
-    if (w >= nwaves) return;
+    __shared__ L2PLds<KB> s_l[W];
+    extern __shared__ uint64_t s_cb[];   // per wave: 4 * nw words of column bits, then 4 * nw counts
+    const int wv = uniform_i((int)threadIdx.x >> 6);
+    // runs of 16 blocks (adjacent columns, which share boundary words) to one XCD
+    uint32_t blk = blockIdx.x;
+    if ((gridDim.x & 127u) == 0) blk = ((blk >> 7) << 7) + ((blk & 7u) << 4) + ((blk >> 3) & 15u);
+    const int64_t wave = (int64_t)blk * W + wv;
+    if (wave >= nwaves) return;
+    uint64_t* cb = s_cb + (size_t)wv * 6 * nw;
     int mesh = 0;
-    if constexpr (kM)   // the mesh whose waves hold w
-        mesh = wave_mesh_search(M.off, M.nm, (uint64_t)w, [](const MeshOff& o) { return (uint64_t)o.pw0; });
+    if constexpr (kM)   // the mesh whose waves hold this one
+        mesh = wave_mesh_search(M.off, M.nm, (uint64_t)wave, [](const MeshOff& o) { return (uint64_t)o.pw0; });
     const GridDev& g = grid_of<kM>(g0, M, mesh);
-    const int n2 = g.n2, w2 = g.w2, gnx = g.nx, gny = g.ny;
-    if (kM && n2 == 0) return;
-    const int64_t mb0 = kM ? (int64_t)M.off[mesh].b0 : 0;
-    const int64_t mb1 = kM ? (int64_t)M.off[mesh + 1].b0 : B;
-    const int64_t lw = w - (kM ? (int64_t)M.off[mesh].pw0 : 0);
-    const uint64_t l2w0 = kM ? M.off[mesh].l2w0 : 0;
-    const uint32_t col0 = kM ? M.off[mesh].col0 : 0;
-    if ((N2 == 0 || N2 == 8) && n2 == 8) {
-        const int64_t bfirst = mb0 + 2 * lw;
-        const int nv = (int)(mb1 - bfirst < 2 ? mb1 - bfirst : 2);
-        l2_parity_pack2_8(g, col0, bfirst, nv, bidx, coff, rec, cpass, stride, s_rec[wv],
-                          par2 + l2w0 + (uint64_t)(bfirst - mb0) * 8);
-        return;
-    }
-    if ((N2 == 0 || N2 == 4) && n2 <= 4) {
-        const int64_t bfirst = mb0 + 4 * lw;
-        const int nv = (int)(mb1 - bfirst < 4 ? mb1 - bfirst : 4);
-        uint64_t* out = par2 + l2w0 + (uint64_t)(bfirst - mb0);   // w2 == 1
-        if (n2 == 4)
-            l2_parity_pack4<4>(n2, g, col0, bfirst, nv, bidx, coff, rec, cpass, stride, s_rec[wv], out);
-        else
-            l2_parity_pack4<0>(n2, g, col0, bfirst, nv, bidx, coff, rec, cpass, stride, s_rec[wv], out);
-        return;
-    }
-    const int64_t b = mb0 + lw;
-    uint64_t* out = par2 + l2w0 + (uint64_t)(b - mb0) * w2;
-    const int v = bidx[b];
-    const int nxy = gnx * gny;
-    const int k1 = v / nxy;
-    const int ij = v - k1 * nxy;
-    const int j1 = ij / gnx;
-    const int i1 = ij - j1 * gnx;
-    const uint32_t e0 = coff[col0 + ij], e1 = coff[col0 + ij + 1];
-    // the other resolutions (Level2 8 and at most 4 returned above)
-    if constexpr (N2 == 0)
-        l2_parity_voxel<0, kRuns>(n2, w2, g, i1, j1, k1, e0, e1, rec, cpass, stride, s_rec[wv], s_acc[wv], s_oz[wv],
-                                  out);
+    if (kM && g.n2 == 0) return;
+    const int C = l2_parity_columns(g.n2, many);
+    const int col = (int)(wave - (kM ? (int64_t)M.off[mesh].pw0 : 0)) * C;
+    const int j1 = col / g.nx, i1 = col - j1 * g.nx;
+    const uint64_t word0 = kM ? M.off[mesh].word0 : 0;
+    const uint32_t col0 = kM ? M.off[mesh].col0 : 0, b0 = kM ? M.off[mesh].b0 : 0;
+    uint64_t* out = par2 + (kM ? M.off[mesh].l2w0 : 0);
+    if (C == 4)
+        l2_parity_columns_wave<4>(s_l[wv], cb, nw, g, i1, j1, word0, col0, b0, bnd, wprefix, coff, rec, out);
+    else
+        l2_parity_columns_wave<1>(s_l[wv], cb, nw, g, i1, j1, word0, col0, b0, bnd, wprefix, coff, rec, out);
 }
 
-// waves of the Level2 parity for nb boundary voxels at resolution n2
-int64_t l2_parity_waves(int n2, int64_t nb)
+template <int KB, int W>
+static void launch_l2_parity_w(const uint64_t* bnd, const uint32_t* wprefix, int64_t nwaves, bool many, int nzmax,
+                               const uint32_t* coff, const float4* rec, const GridDev& g0, const Meshes& M,
+                               uint64_t* par2, hipStream_t s)
 {
-    if (n2 <= 0) return 0;
-    return n2 <= 4 ? (nb + 3) / 4 : n2 == 8 ? (nb + 1) / 2 : nb;
-}
-
-template <int PW, bool kRuns>
-static void launch_l2_parity_r(const int32_t* bidx, int64_t B, int64_t nwaves, const uint32_t* coff,
-                               const float4* rec, const uint64_t* cpass, int stride, const GridDev& g0,
-                               const Meshes& M, uint64_t* par2, hipStream_t s)
-{
-    const unsigned blocks = (unsigned)((nwaves + PW - 1) / PW);
-    const dim3 bs(64 * PW);
+    unsigned blocks = (unsigned)((nwaves + W - 1) / W);
+    if (blocks >= 1024) blocks = (blocks + 127u) & ~127u;   // whole rounds of the XCD mapping
+    const int nw = (nzmax + 63) / 64;
+    const size_t lds = (size_t)W * 6 * nw * sizeof(uint64_t);
     if (M.nm > 1)
-        k_l2_parity<true, 0, PW, kRuns><<<blocks, bs, 0, s>>>(bidx, B, nwaves, coff, rec, cpass, stride, g0, M, par2);
-    else if (g0.n2 == 8)
-        k_l2_parity<false, 8, PW, false><<<blocks, bs, 0, s>>>(bidx, B, nwaves, coff, rec, cpass, stride, g0, M,
-                                                                par2);
-    else if (g0.n2 == 4)
-        k_l2_parity<false, 4, PW, false><<<blocks, bs, 0, s>>>(bidx, B, nwaves, coff, rec, cpass, stride, g0, M,
-                                                                par2);
+        k_l2_parity<true, KB, W><<<blocks, 64 * W, lds, s>>>(bnd, wprefix, nwaves, many, nw, coff, rec, g0, M, par2);
     else
-        k_l2_parity<false, 0, PW, kRuns><<<blocks, bs, 0, s>>>(bidx, B, nwaves, coff, rec, cpass, stride, g0, M,
-                                                                par2);
+        k_l2_parity<false, KB, W><<<blocks, 64 * W, lds, s>>>(bnd, wprefix, nwaves, many, nw, coff, rec, g0, M, par2);
 }
 
-template <int PW>
-static void launch_l2_parity_w(const int32_t* bidx, int64_t B, int64_t nwaves, const uint32_t* coff,
-                               const float4* rec, const uint64_t* cpass, int stride, int n2max, const GridDev& g0,
-                               const Meshes& M, uint64_t* par2, hipStream_t s)
+template <int KB>
+static void launch_l2_parity_k(const uint64_t* bnd, const uint32_t* wprefix, int64_t nwaves, bool many, int nzmax,
+                               const uint32_t* coff, const float4* rec, int waves, const GridDev& g0, const Meshes& M,
+                               uint64_t* par2, hipStream_t s)
 {
-    if (n2max > 8)
-        launch_l2_parity_r<PW, true>(bidx, B, nwaves, coff, rec, cpass, stride, g0, M, par2, s);
-    else
-        launch_l2_parity_r<PW, false>(bidx, B, nwaves, coff, rec, cpass, stride, g0, M, par2, s);
+    if (waves <= 1) launch_l2_parity_w<KB, 1>(bnd, wprefix, nwaves, many, nzmax, coff, rec, g0, M, par2, s);
+    else if (waves == 2) launch_l2_parity_w<KB, 2>(bnd, wprefix, nwaves, many, nzmax, coff, rec, g0, M, par2, s);
+    else launch_l2_parity_w<KB, 4>(bnd, wprefix, nwaves, many, nzmax, coff, rec, g0, M, par2, s);
 }
 
-void launch_l2_parity(const int32_t* bidx, int64_t B, int64_t nwaves, const uint32_t* coff, const float4* rec,
-                      const uint64_t* cpass, int stride, int n2max, int waves, const GridDev& g0, const Meshes& M,
+void launch_l2_parity(const uint64_t* bnd, const uint32_t* wprefix, int64_t nwaves, bool many, int n2max, int nzmax,
+                      const uint32_t* coff, const float4* rec, int waves, const GridDev& g0, const Meshes& M,
                       uint64_t* par2, hipStream_t s)
 {
-    if (B <= 0 || nwaves <= 0) return;
-    if (waves <= 1) launch_l2_parity_w<1>(bidx, B, nwaves, coff, rec, cpass, stride, n2max, g0, M, par2, s);
-    else if (waves == 2) launch_l2_parity_w<2>(bidx, B, nwaves, coff, rec, cpass, stride, n2max, g0, M, par2, s);
-    else launch_l2_parity_w<4>(bidx, B, nwaves, coff, rec, cpass, stride, n2max, g0, M, par2, s);
+    if (nwaves <= 0) return;
+    // room for 31 boundary voxels of a column at n2 = 8, 7 at 16
+    if (n2max <= 8) launch_l2_parity_k<2048>(bnd, wprefix, nwaves, many, nzmax, coff, rec, waves, g0, M, par2, s);
+    else launch_l2_parity_k<4096>(bnd, wprefix, nwaves, many, nzmax, coff, rec, waves, g0, M, par2, s);
 }
 
 // ---------------------------------------------------------------------------

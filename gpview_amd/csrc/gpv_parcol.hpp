@@ -1,0 +1,162 @@
+// gpv_parcol.hpp -- the Level2 ray parity by crossings instead of voxel by voxel.
+//
+// For the +z ray of a sub-column (x, y) the Moller-Trumbore test of one column
+// entry (triangle) accepts or rejects by det/u/v, which do not depend on the
+// origin's z, and then passes where t >= eps (src/TriRayIntersection.cpp:
+// 78-131).  In exact arithmetic t falls with the origin's height, so the
+// sub-layers that pass are those below one crossing height; the parity of
+// every voxel of the column follows from the crossings.  The float test is
+// within rounding of that: functions here bound which sub-columns it can
+// accept and below and above which layers it is certain to pass or fail; the
+// kernel runs the reference's float expressions on the rest.
+//
+// U = 2^-24.  e1, e2 are the record's float edges, inv = fl(1/det),
+// N_a = |e1_b e2_c| + |e1_c e2_b|, T = o - v1.
+//
+// Acceptance.  u = fl((Tx px + Ty py) inv) and v likewise lie within
+//   delta = 64 U (1 + |inv| ((|e1y| + |e2y|) tmx + (|e1x| + |e2x|) tmy + N_z))
+// of the barycentric coordinates a, b of the ray's point with respect to the
+// float edges (3 U per numerator, |inv| N_z 3 U and 2 U for the reciprocal, one
+// product; tm bounds |T| over the column), and the formulas below within half of
+// that of a, b.  So an accepted sub-column satisfies a, b >= -delta,
+// a + b <= 1 + 2 delta; delta also carries the deviation of the origin tables from
+// equal steps (SatScale).
+//
+// Crossing.  The float s = e2 . (T x e1) is within 6.1 U B of the exact one, B =
+// sum |T_a| N_a, and t >= eps means s >= eps |det| up to 2 U; |T_a| <=
+// 2 (|e1_a| + |e2_a|) for an accepted ray at its crossing where 64 U N_z <=
+// |det|.  The crossing height taken here, v1z + u e1z + v e2z - eps, is off by at
+// most 3 U |inv| (|Tx| N_x + |Ty| N_y + N_z (|e1z| + |e2z|)) and rounding.  So the
+// float test agrees with the crossing at every height farther from it than
+//   Ez = 64 U |inv| sum (|e1_a| + |e2_a|) N_a + 16 U (|e1z| + |e2z|) + 2^-12 eps
+// (|det| >= 1e-6 by the det test); worse conditioned records get Ez infinite.
+#pragma once
+
+#include "gpv_satrow.hpp"
+
+namespace gpv {
+
+// Ez of a record (z units)
+__host__ __device__ __forceinline__ float par_ez(float e1x, float e1y, float e1z, float e2x, float e2y, float e2z,
+                                                 float inv)
+{
+    constexpr float U = 0x1p-24f;
+    const float nx = fabsf(e1y * e2z) + fabsf(e1z * e2y), ny = fabsf(e1z * e2x) + fabsf(e1x * e2z),
+                nz = fabsf(e1x * e2y) + fabsf(e1y * e2x);
+    const float ai = fabsf(inv);
+    const float sx = fabsf(e1x) + fabsf(e2x), sy = fabsf(e1y) + fabsf(e2y), sz = fabsf(e1z) + fabsf(e2z);
+    const float b = sx * nx + sy * ny + sz * nz;
+    const bool ok = 64.0f * U * nz * ai <= 1.0f && b * ai < 1e30f;
+    return ok ? 64.0f * U * (ai * b) + (16.0f * U * sz + 2.5e-10f) : 3.0e38f;
+}
+
+// A record with its bounds in one column.
+struct ParEntry {
+    float e1x, e1y, e1z, e2x, e2y, e2z, inv, v1x, v1y;
+    float dz;      // v1z - eps less the origin height of layer l0
+    float mu;      // margin of the crossing, in layers
+    float delta;
+    int l0;        // first layer of the record's voxel zmax
+};
+
+// delta of a record; (ox0, oy0) the column's first origin, gx, gy its sub-voxels
+__host__ __device__ __forceinline__ float par_delta(const ParEntry& r, float ox0, float oy0, float gx, float gy, int n2,
+                                                    float devx, float devy)
+{
+    constexpr float U = 0x1p-24f;
+    const float tmx = fabsf(ox0 - r.v1x) + (float)n2 * gx, tmy = fabsf(oy0 - r.v1y) + (float)n2 * gy;
+    const float sx = fabsf(r.e1x) + fabsf(r.e2x), sy = fabsf(r.e1y) + fabsf(r.e2y);
+    const float nz = fabsf(r.e1x * r.e2y) + fabsf(r.e1y * r.e2x);
+    return 64.0f * U + fabsf(r.inv) * (64.0f * U * (sy * tmx + sx * tmy + nz) + (sy * devx * gx + sx * devy * gy));
+}
+
+// the parts of an entry that depend on the column: z1 the record's v1z, oz0 the
+// origin height of layer l0 (from the grid's bounds, par_oz), (ox0, oy0) the column's first origin, gx, gy its
+// sub-voxels
+__host__ __device__ __forceinline__ void par_entry(ParEntry& r, float z1, float oz0, float ox0, float oy0, float gx,
+                                                   float gy, int n2, const SatScale& g)
+{
+    r.dz = (z1 - oz0) - 1.0e-6f;
+    // across voxels the origin table keeps within 5.5 U cmax of equal steps and
+    // oz0 within 4 U cmax of it, together less than 5 dz
+    r.mu = fminf(par_ez(r.e1x, r.e1y, r.e1z, r.e2x, r.e2y, r.e2z, r.inv) * g.sz, 3.0e38f) + 5.0f * g.dz;
+    r.delta = par_delta(r, ox0, oy0, gx, gy, n2, g.dx, g.dy);
+    if (!(g.dx >= 0.0f && g.dy >= 0.0f && g.dz >= 0.0f)) {   // no scale: everything is undecided
+        r.mu = 3.0e38f;
+        r.delta = 3.0e38f;
+    }
+}
+
+// origin height of the first layer of voxel k (bmin + k g, half a sub-voxel up)
+__host__ __device__ __forceinline__ float par_oz(float bmin, float g1, float g2, int k)
+{
+    return bmin + ((float)k * g1 + 0.5f * g2);
+}
+
+// layers that hold every toggle of an entry's accepted sub-columns: between
+// la and lb of par_layers at the ends of the triangle's z range, grown
+__host__ __device__ __forceinline__ void par_z_range(const ParEntry& r, float sz, int cap, int& lmin, int& lmax)
+{
+    const float lo = fminf(fminf(r.e1z, r.e2z), 0.0f), hi = fmaxf(fmaxf(r.e1z, r.e2z), 0.0f);
+    const float grow = 4.0f * r.delta * (fabsf(r.e1z) + fabsf(r.e2z));
+    const float m = r.mu + 0.01f + 1e-6f * (fabsf(r.dz) + hi - lo) * sz;
+    const float a = fmaxf(((lo - grow) + r.dz) * sz + 1.0f - m, -1.0e8f), b = fminf(((hi + grow) + r.dz) * sz + 1.0f + m, 1.0e8f);
+    // a NaN leaves the range whole
+    lmin = a >= -1.0e8f ? r.l0 + (int)floorf(fminf(a, 1.0e8f)) : 0;
+    lmax = b <= 1.0e8f ? r.l0 + (int)floorf(fmaxf(b, -1.0e8f)) : cap;
+    lmin = lmin < 0 ? 0 : lmin > cap ? cap : lmin;
+    lmax = lmax < 0 ? 0 : lmax > cap ? cap : lmax;
+}
+
+// rows [q0, q0 + n) that can hold an accepted sub-column
+__host__ __device__ __forceinline__ int par_rows(const ParEntry& r, float oy0, float sy, int n2, float devy, int& q0)
+{
+    constexpr float U = 0x1p-24f;
+    const float y = (r.v1y - oy0) * sy, a = r.e1y * sy, b = r.e2y * sy;
+    const float lo = y + fminf(fminf(a, b), 0.0f), hi = y + fmaxf(fmaxf(a, b), 0.0f);
+    const float grow = 4.0f * r.delta * (fabsf(a) + fabsf(b)) + 16.0f * U * (fabsf(y) + fabsf(a) + fabsf(b)) + devy + 0.01f;
+    // written so that a NaN leaves the row range whole
+    const float f = fminf(fmaxf(ceilf(lo - grow), 0.0f), (float)n2), g = fminf(fmaxf(floorf(hi + grow), -1.0f), (float)(n2 - 1));
+    q0 = lo - grow >= 0.0f ? (int)f : 0;
+    const int q1 = hi + grow < (float)(n2 - 1) ? (int)g : n2 - 1;
+    return q1 - q0 + 1;
+}
+
+// of a constraint c0 + c1 x >= 0, its bound on x
+__host__ __device__ __forceinline__ void par_bound(float c0, float c1, float& lo, float& hi)
+{
+    const float t = -c0 * GPV_RCP(c1);
+    lo = c1 > 0.0f ? fmaxf(lo, t) : lo;
+    hi = c1 < 0.0f ? fminf(hi, t) : hi;
+}
+
+// columns [p0, p0 + n) of row q that can be accepted
+__host__ __device__ __forceinline__ int par_cols(const ParEntry& r, float ox0, float oy0, float gx, float gy, int n2, int q,
+                                                 int& p0)
+{
+    const float tx = ox0 - r.v1x, ty = (oy0 - r.v1y) + (float)q * gy;
+    const float a0 = (r.e2x * ty - r.e2y * tx) * r.inv, a1 = -(r.e2y * r.inv) * gx;
+    const float b0 = (r.e1y * tx - r.e1x * ty) * r.inv, b1 = (r.e1y * r.inv) * gx;
+    float lo = 0.0f, hi = (float)(n2 - 1);
+    par_bound(a0 + r.delta, a1, lo, hi);
+    par_bound(b0 + r.delta, b1, lo, hi);
+    par_bound((1.0f + 2.0f * r.delta) - (a0 + b0), -(a1 + b1), lo, hi);
+    const float f = fminf(ceilf(lo - 0.01f), 32.0f), g = fmaxf(floorf(hi + 0.01f), -1.0f);
+    p0 = (int)fmaxf(f, 0.0f);
+    return (int)g - p0 + 1;
+}
+
+// The layers an accepted sub-column with coordinates u, v passes: all below
+// `la`, none from `lb` on, both within [0, cap].
+__host__ __device__ __forceinline__ void par_layers(const ParEntry& r, float u, float v, float sz, int cap, int& la, int& lb)
+{
+    // layer l0 + x is at the crossing's height; l passes for l < that, hence + 1
+    const float x = ((u * r.e1z + v * r.e2z) + r.dz) * sz + 1.0f;
+    const float a = floorf(fmaxf(x - r.mu, -1.0e8f)), b = floorf(fminf(x + r.mu, 1.0e8f));
+    la = r.l0 + (int)fminf(a, 1.0e8f);
+    lb = r.l0 + (int)fmaxf(b, -1.0e8f);
+    la = la < 0 ? 0 : la > cap ? cap : la;
+    lb = lb < 0 ? 0 : lb > cap ? cap : lb;
+}
+
+}  // namespace gpv

@@ -210,6 +210,8 @@ void scratch_setup(int device)
     g_scratch_err[device] = hipSuccess;
 }
 
+constexpr int kJobEvents = 17;   // stage events of a job
+
 }  // namespace
 
 struct gpv_ctx {
@@ -226,9 +228,9 @@ struct gpv_ctx {
     float* tab_buf = nullptr;   // pinned staging of a job's center tables
     size_t tab_cap = 0;
     int num_cu = 256;
-    gpv_tune tune{16, 56, 2048, 1, 1, 2, 128};
+    gpv_tune tune{16, 56, 2048, 1, 1, 1, 128};
     std::vector<hipEvent_t> events;   // recycled stage events of finished jobs
-    hipEvent_t na_ev[16] = {};        // stage events of gpv_voxelize_noalloc (created with the context)
+    hipEvent_t na_ev[kJobEvents] = {};   // stage events of gpv_voxelize_noalloc (created with the context)
 };
 
 namespace gpv {
@@ -299,7 +301,6 @@ struct Job {
     bool cols_side = false;
     uint32_t* cs_cnt = nullptr;
     uint4* cs_bucket = nullptr;
-    uint64_t* cpass = nullptr;   // det/u/v pass bits per column entry and sub-column
     int64_t l2p_waves = 0, l2s_groups = 0;   // Level2 parity waves, SAT groups (l2_plan)
     int l2s_most = 1;                        // most voxels of a SAT group
     uint32_t *hcnt = nullptr, *hoff = nullptr;
@@ -310,7 +311,7 @@ struct Job {
     uint32_t* st_cnt = nullptr;
     uint64_t *st_off = nullptr, *st_scan = nullptr, *st_tog = nullptr;
     uint64_t *sat2 = nullptr, *par2 = nullptr;
-    int n2max = 0;
+    int n2max = 0, nzmax = 0;
     // normals (meshes with params.normals): face normals, sorted bins, and the
     // resident results per boundary voxel / per Level2 voxel
     bool any_normals = false;
@@ -325,7 +326,8 @@ struct Job {
     // 4 compaction+bins, 5 L2 parity, 6 L2 SAT start, 7 L2 SAT end, 8 finish,
     // 9 normals start, 10 normals end, 11 L2 parity end, 12 L1 SAT end,
     // 13 ray expansion end, 14 parity fill end, 15 fork of the ray expansion
-    hipEvent_t ev[16] = {};
+    // 16 L2 parity start
+    hipEvent_t ev[kJobEvents] = {};
     std::vector<void*> bufs;
     // gpv_voxelize_noalloc: buffers are carved from the device scratch array
     // (arena != nullptr) instead of the pool, the result planes are the
@@ -624,7 +626,7 @@ int job_create(gpv_ctx* c, const gpv_mesh_desc* d, int nm, int on_device, Job** 
         J->arena = na->arena;
         J->arena_cap = na->arena_cap;
         J->borrowed_events = true;
-        for (int k = 0; k < 16; ++k) J->ev[k] = c->na_ev[k];
+        for (int k = 0; k < kJobEvents; ++k) J->ev[k] = c->na_ev[k];
         J->nb_cap = na->nb_cap;
         J->out_bidx = na->bidx;
         J->out_sat2 = na->l2b;
@@ -662,6 +664,7 @@ int job_create(gpv_ctx* c, const gpv_mesh_desc* d, int nm, int on_device, Job** 
     size_t ntab = 0;
     uint64_t word0 = 0;
     uint32_t col0 = 0, tri0 = 0, ptask0 = 0;
+    int64_t pw0 = 0;
     for (int m = 0; m < nm; ++m) {
         GridDev& g = J->g[m];
         g = grid_dev(J->info[m]);
@@ -677,10 +680,13 @@ int job_create(gpv_ctx* c, const gpv_mesh_desc* d, int nm, int on_device, Job** 
         J->info[m].has_normals = g.normals;
         J->any_normals = J->any_normals || g.normals;
         J->n2max = std::max(J->n2max, g.n2);
+        J->nzmax = std::max(J->nzmax, g.nz);
         J->off[m].word0 = word0;
         J->off[m].col0 = col0;
         J->off[m].tri0 = tri0;
         J->off[m].ptask0 = ptask0;
+        J->off[m].pw0 = (uint32_t)pw0;
+        pw0 += l2_parity_waves(g.n2, (int64_t)g.nx * g.ny, ncol >= kL2ParityMany);
         ptask0 += (uint32_t)l1_parity_tasks(g);
         word0 += (uint64_t)g.nz * g.ny * g.nxw;
         col0 += (uint32_t)(g.nx * g.ny);
@@ -724,6 +730,8 @@ int job_create(gpv_ctx* c, const gpv_mesh_desc* d, int nm, int on_device, Job** 
     J->off[nm].col0 = col0;
     J->off[nm].tri0 = tri0;
     J->off[nm].ptask0 = ptask0;
+    J->off[nm].pw0 = (uint32_t)pw0;   // at most one per column
+    J->l2p_waves = pw0;
     int r;
     if ((r = alloc(J, &J->tables, ntab)) != GPV_OK) return bail(r);
     if (hipMemcpyAsync(J->tables, tab_src, ntab * sizeof(float), hipMemcpyHostToDevice, c->stream) != hipSuccess)
@@ -1104,7 +1112,27 @@ int launch_parity(Job* J)
     return GPV_OK;
 }
 
+// the Level2 planes: allocated before the side stream forks, whose parity
+// writes one of them
+int alloc_level2(Job* J)
+{
+    if (J->out_bidx && J->B > J->nb_cap)
+        return fail(GPV_ERR_TOO_LARGE, "%lld boundary voxels; the result buffers hold %lld", (long long)J->B,
+                    (long long)J->nb_cap);
+    if (J->n2max <= 0) return GPV_OK;
+    release(J, J->sat2);
+    release(J, J->par2);
+    if (J->out_bidx) {   // W2 = B * w2 fits
+        J->sat2 = J->out_sat2;
+        J->par2 = J->out_par2;
+        return GPV_OK;
+    }
+    TRY(alloc(J, &J->sat2, (size_t)std::max<int64_t>(J->W2, 1)));
+    return alloc(J, &J->par2, (size_t)std::max<int64_t>(J->W2, 1));
+}
+
 // boundary index list, bins per boundary voxel, column entries with records
+// (Level2 planes allocated)
 int launch_compact(Job* J)
 {
     hipStream_t s = J->ctx->stream;
@@ -1112,14 +1140,10 @@ int launch_compact(Job* J)
     const size_t Bn = (size_t)std::max<int64_t>(J->B, 1);
     release(J, J->bidx);
     release(J, J->bmesh);
-    if (J->out_bidx) {
-        if (J->B > J->nb_cap)
-            return fail(GPV_ERR_TOO_LARGE, "%lld boundary voxels; the result buffers hold %lld",
-                        (long long)J->B, (long long)J->nb_cap);
+    if (J->out_bidx)
         J->bidx = J->out_bidx;
-    } else {
+    else
         TRY(alloc(J, &J->bidx, Bn));
-    }
     if (J->nm > 1) TRY(alloc(J, &J->bmesh, Bn));
     launch_boundary_index(J->bnd, J->wprefix, J->g[0], J->view(), J->W, J->bidx, s);
     release(J, J->boff);
@@ -1159,17 +1183,6 @@ int launch_compact(Job* J)
     release(J, ts_cnt);
     release(J, ts_bucket);
     HIP_TRY(hipGetLastError());
-    if (J->n2max > 0) {
-        release(J, J->sat2);
-        release(J, J->par2);
-        if (J->out_bidx) {   // W2 = B * w2 fits: B <= nb_cap was checked above
-            J->sat2 = J->out_sat2;
-            J->par2 = J->out_par2;
-        } else {
-            TRY(alloc(J, &J->sat2, (size_t)std::max<int64_t>(J->W2, 1)));
-            TRY(alloc(J, &J->par2, (size_t)std::max<int64_t>(J->W2, 1)));
-        }
-    }
     J->compact_done = true;
     return GPV_OK;
 }
@@ -1187,26 +1200,21 @@ int l2_sat_most(const Job* J)
     return (int)std::min<int64_t>(kL2GroupMax, std::min(fill, spread));
 }
 
-// Level2 parity waves and SAT groups of the job; in a batch each mesh's first
-// ones go to MeshOff::pw0 and sg0 on the device (main stream, before any
-// Level2 launch)
+// Level2 SAT groups of the job; in a batch each mesh's first one goes to
+// MeshOff::sg0 on the device (main stream, before the fork of the side
+// stream's kernels that read the table)
 int l2_plan(Job* J)
 {
-    int64_t w = 0, sg = 0;
+    int64_t sg = 0;
     J->l2s_most = l2_sat_most(J);
     for (int m = 0; m < J->nm; ++m) {
-        J->off[m].pw0 = (uint32_t)w;
         J->off[m].sg0 = (uint32_t)sg;
-        w += l2_parity_waves(J->g[m].n2, J->nb(m));
         if (J->g[m].n2 > 0) {
             const int64_t c = l2_group_voxels(J->g[m].n2, J->l2s_most);
             sg += (J->nb(m) + c - 1) / c;
         }
     }
-    J->off[J->nm].pw0 = (uint32_t)w;
     J->off[J->nm].sg0 = (uint32_t)sg;
-    if (w >= (int64_t(1) << 32)) return fail(GPV_ERR_INVALID, "too many Level2 parity waves");
-    J->l2p_waves = w;
     J->l2s_groups = sg;
     if (J->nm > 1) {
         hipStream_t s = J->ctx->stream;
@@ -1220,27 +1228,16 @@ int l2_plan(Job* J)
     return GPV_OK;
 }
 
-// cpass words per column entry: the pass bits of its sub-columns and a header
-int cpass_stride(const Job* J) { return (J->n2max * J->n2max + 63) / 64 + 1; }
-
-// Level2 parity kernels on stream s (cpass allocated, waves planned)
+// Level2 parity on stream s: it needs the boundary planes and the column entries
 int l2_parity_kernels(Job* J, hipStream_t s)
 {
-    const int stride = cpass_stride(J);
-    const gpv_tune& tu = J->ctx->tune;
-    launch_col_pass(J->crec, J->g[0], J->view(), J->n_cols, stride, tu.l2_parity_waves, J->cpass, s);
-    launch_l2_parity(J->bidx, J->B, J->l2p_waves, J->coff, J->crec, J->cpass, stride, J->n2max, tu.l2_parity_waves,
-                     J->g[0], J->view(), J->par2, s);
+    HIP_TRY(hipEventRecord(J->ev[16], s));
+    if (J->B > 0)
+        launch_l2_parity(J->bnd, J->wprefix, J->l2p_waves, J->ncol >= kL2ParityMany, J->n2max, J->nzmax, J->coff, J->crec,
+                         J->ctx->tune.l2_parity_waves, J->g[0], J->view(), J->par2, s);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipEventRecord(J->ev[11], s));
     return GPV_OK;
-}
-
-int alloc_cpass(Job* J)
-{
-    const int stride = cpass_stride(J);
-    release(J, J->cpass);
-    return alloc(J, &J->cpass, (size_t)std::max<uint64_t>(J->n_cols, 1) * stride);
 }
 
 int run_l2_parity(Job* J)
@@ -1248,10 +1245,7 @@ int run_l2_parity(Job* J)
     if (J->n2max <= 0) return GPV_OK;
     hipStream_t s = J->ctx->stream;
     HIP_TRY(hipEventRecord(J->ev[5], s));
-    TRY(alloc_cpass(J));
-    TRY(l2_plan(J));
     TRY(l2_parity_kernels(J, s));
-    release(J, J->cpass);
     J->l2p_done = true;
     return GPV_OK;
 }
@@ -1277,23 +1271,20 @@ int run_l2_sat(Job* J)
     return GPV_OK;
 }
 
-// Both Level2 stages of the fused pipeline: the parity on the side stream
-// beside the SAT on the main one (they read the same inputs and write
-// different planes).  Nothing is allocated or released between the fork and
-// the join, so the pool's blocks stay in one stream order.
+// The Level2 stages of the fused pipeline: the parity follows the column-entry
+// sort on the side stream (it reads the Level1 planes and the column entries,
+// not the bins), the SAT the bins on the main one.  Nothing is allocated or
+// released between the fork and the join, so the pool's blocks stay in one
+// stream order.
 int run_level2(Job* J)
 {
     if (J->n2max <= 0) return GPV_OK;
     gpv_ctx* c = J->ctx;
     hipStream_t s = c->stream;
-    TRY(alloc_cpass(J));
-    TRY(l2_plan(J));
     HIP_TRY(hipEventRecord(J->ev[5], s));
-    HIP_TRY(hipStreamWaitEvent(c->side, J->ev[5], 0));
     TRY(l2_parity_kernels(J, c->side));
     TRY(l2_sat_kernels(J));
     HIP_TRY(hipStreamWaitEvent(s, J->ev[11], 0));
-    release(J, J->cpass);
     release(J, J->cs_cnt);
     release(J, J->cs_bucket);
     J->l2p_done = true;
@@ -1351,7 +1342,7 @@ int job_finish(Job* J)
     float ms[6] = {el(0, 1), el(1, 12), el(2, 13) + el(3, 14), 0.0f, 0.0f, 0.0f};
     if (J->n2max > 0) {
         ms[3] = el(4, 5);
-        ms[4] = el(5, 11);   // in the fused pipeline the two Level2 stages overlap
+        ms[4] = el(16, 11);   // in the fused pipeline the two Level2 stages overlap
         ms[5] = el(6, 7);
     } else {
         ms[3] = el(4, 8);
@@ -1439,6 +1430,8 @@ int job_run(Job* J)
         // the side stream too) sort there after the fill, beside the bins
         J->cols_side = J->n2max > 0;
         if (J->cols_side) TRY(alloc_cols(J));
+        TRY(alloc_level2(J));
+        if (J->n2max > 0) TRY(l2_plan(J));
         // the main stream's compaction (the critical path) is enqueued first;
         // the side stream waits for the point before it
         HIP_TRY(hipEventRecord(J->ev[3], c->stream));
@@ -1451,6 +1444,7 @@ int job_run(Job* J)
         HIP_TRY(hipStreamWaitEvent(c->stream, J->ev[14], 0));
     } else {
         TRY(launch_parity(J));
+        TRY(alloc_level2(J));
         TRY(launch_compact(J));
         TRY(run_l2_parity(J));
         TRY(run_l2_sat(J));
@@ -1489,7 +1483,6 @@ int64_t predict_run_bytes(const gpv_mesh_desc& d, const gpv_grid_info& I)
     b += 4 * (ncol + 1) + 48 * P + 16 * P + 64 * (ncol / 64 + 1);   // column entries by column, records
     b += 8 * B + 4 + 4 * P + 8 * P + 16 * P + 64 * (B / 64 + 1) + scan(B);   // boundary list, bins, masks
     b += 16 * B * w2;                                            // Level2 planes
-    b += n2 > 0 ? 8 * P * ((n2 * n2 + 63) / 64 + 1) : 0;   // Level2 parity bits
     if (d.params.normals) b += 12 * T + 4 * P + 12 * B + 12 * B * n2 * n2 * n2;
     if (d.params.l1_stencil) b += 12 * T + 8 + scan(T) + 8 * nz * 2 * ny * ((2 * nx + 63) / 64);   // stencil fill
     return b;
@@ -2062,6 +2055,7 @@ int gpv_compact_boundary(gpv_ctx* c, gpv_grid* G)
     TRY(check_staged(c, G));
     if (!G->job->sat_done) return fail(GPV_ERR_STATE, "gpv_classify_tessellation has not completed");
     HIP_TRY(hipSetDevice(c->device));
+    TRY(alloc_level2(G->job));
     return launch_compact(G->job);
 }
 
