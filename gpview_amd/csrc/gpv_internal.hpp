@@ -24,6 +24,7 @@ struct GridDev {
     float bminx, bminy, bminz, bmaxx, bmaxy, bmaxz;
     float h1x, h1y, h1z;   // Level1 half extents
     float h2x, h2y, h2z;   // Level2 half extents
+    float s1x, s1y, s1z, d1x, d1y, d1z;   // Level1 SAT columns: scale and table deviation per axis (SatScale)
     float s2x, s2y, s2z, d2x, d2y, d2z;   // Level2 SAT rows: scale and table deviation per axis (SatScale)
     const float* c1x; const float* c1y; const float* c1z;   // [n]    Level1 SAT centers
     const float* r1x; const float* r1y; const float* r1z;   // [n]    Level1 ray origins
@@ -102,7 +103,7 @@ void launch_fill_u64(uint64_t* p, uint64_t v, int64_t n, hipStream_t s);
 void launch_mesh_ids(const MeshOff* off, int nm, int64_t T, uint32_t* tri_mesh, hipStream_t s);
 // part 1 (and 3) also raise *bad_input for a coordinate outside the domain
 void launch_tri_setup(const float* tris, int64_t T, const GridDev& g0, const Meshes& M, int4* box0, int4* box1,
-                      uint32_t* sat_items, int4* ray_rng, uint32_t* ray_items, double4* slab1, int part,
+                      uint32_t* sat_items, int4* ray_rng, uint32_t* ray_items, int part,
                       unsigned long long* bad_input, hipStream_t s);
 
 // exclusive scan of n u32 into out[0..n] (out[n] = total); tmp sized by
@@ -113,12 +114,12 @@ void launch_scan_u32_u64(const uint32_t* in, uint64_t* out, int64_t n, uint64_t*
 void launch_scan_u32_u32(const uint32_t* in, uint32_t* out, int64_t n, uint32_t* tmp, unsigned int* max_out,
                          hipStream_t s);
 
-// stage: triangles staged per LDS pass (128 or 256)
-void launch_sat_expand(const float* tris, int64_t T, const int4* box0, const int4* box1, const double4* slab1,
-                       const uint64_t* off, const GridDev& g0, const Meshes& M, uint8_t* bbytes, Append64 pairs,
-                       Append64 cols, int blocks, int stage, hipStream_t s);
+void launch_sat_expand(const float* tris, int64_t T, const int4* box0, const int4* box1, const uint64_t* off,
+                       const GridDev& g0, const Meshes& M, uint8_t* bbytes, Append64 pairs, Append64 cols, int blocks,
+                       hipStream_t s);
 // boundary bytes (W * 64) -> boundary bitplane (W words)
 void launch_pack_bytes(const uint8_t* by, int64_t W, uint64_t* bits, hipStream_t s);
+// stage: triangles staged per LDS pass (128 or 256)
 void launch_ray_expand(const float* tris, int64_t T, const int4* ray_rng, const uint64_t* off, const GridDev& g0,
                        const Meshes& M, Append64 hits, int blocks, int stage, hipStream_t s);
 

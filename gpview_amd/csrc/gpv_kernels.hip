@@ -18,7 +18,6 @@
 #include "gpv_internal.hpp"
 #include "gpv_parcol.hpp"
 #include "gpv_satrow.hpp"
-#include "gpv_slab.hpp"
 
 namespace gpv {
 
@@ -312,12 +311,8 @@ void launch_mesh_ids(const MeshOff* off, int nm, int64_t T, uint32_t* tri_mesh, 
 // the mesh's test counter.  Multi-mesh form: one triangle per thread; blocks
 // inside one mesh (tri_mesh is non-decreasing) reduce into that mesh's
 // counter, the few straddling blocks add per lane.
-// Triangles whose index AABB spans at least kZSlabMin Level1 layers also get a
-// plane slab (gpv_slab.hpp) over the centers of that AABB: the Level1 sweep
-// then visits, per column, only the layers the slab can keep.
-constexpr int kZSlabMin = 3;
 
-// kPart: 1 the SAT half (index AABB, items, slabs, test counts), 2 the ray
+// kPart: 1 the SAT half (index AABB, items, test counts), 2 the ray
 // half (column bound, items), 3 both.  The halves share nothing but the
 // vertices, so they can run on two streams.
 template <bool kM, int kPart>
@@ -326,7 +321,6 @@ __global__ __launch_bounds__(256) void k_tri_setup(const float* __restrict__ tri
                                                    uint32_t* __restrict__ sat_items,
                                                    int4* __restrict__ ray_rng,
                                                    uint32_t* __restrict__ ray_items,
-                                                   double4* __restrict__ slab1,
                                                    unsigned long long* __restrict__ bad_input)
 {
     uint64_t tests = 0;
@@ -367,12 +361,6 @@ __global__ __launch_bounds__(256) void k_tri_setup(const float* __restrict__ tri
             const bool any = dd[0] > 0 && dd[1] > 0 && dd[2] > 0;
             sat_items[t] = any ? (uint32_t)(dd[0] * dd[1]) : 0u;
             tests += any ? (uint64_t)dd[0] * dd[1] * dd[2] : 0;
-            if (any && dd[2] >= kZSlabMin) {
-                const double clo[3] = {g.c1x[lo[0]], g.c1y[lo[1]], g.c1z[lo[2]]};
-                const double chi[3] = {g.c1x[lo[0] + dd[0] - 1], g.c1y[lo[1] + dd[1] - 1], g.c1z[lo[2] + dd[2] - 1]};
-                const PlaneSlab sl = plane_slab(tv, g.h1x, g.h1y, g.h1z, clo, chi);
-                slab1[t] = make_double4(sl.nx, sl.ny, sl.nz, sl.lim);
-            }
         }
         if constexpr ((kPart & 2) == 0) continue;
         uint32_t rit = 0;
@@ -410,30 +398,30 @@ __global__ __launch_bounds__(256) void k_tri_setup(const float* __restrict__ tri
 
 template <int kPart>
 static void tri_setup_part(const float* tris, int64_t T, const GridDev& g0, const Meshes& M, int4* box0, int4* box1,
-                           uint32_t* sat_items, int4* ray_rng, uint32_t* ray_items, double4* slab1,
+                           uint32_t* sat_items, int4* ray_rng, uint32_t* ray_items,
                            unsigned long long* bad_input, hipStream_t s)
 {
     if (M.nm > 1)
         k_tri_setup<true, kPart><<<grid_for(T, 256, 1 << 30), 256, 0, s>>>(tris, T, g0, M, box0, box1, sat_items,
-                                                                            ray_rng, ray_items, slab1,
+                                                                            ray_rng, ray_items,
                                                                             bad_input);
     else
         k_tri_setup<false, kPart><<<grid_for(T, 256, 1024), 256, 0, s>>>(tris, T, g0, M, box0, box1, sat_items,
-                                                                          ray_rng, ray_items, slab1,
+                                                                          ray_rng, ray_items,
                                                                           bad_input);
 }
 
 void launch_tri_setup(const float* tris, int64_t T, const GridDev& g0, const Meshes& M, int4* box0, int4* box1,
-                      uint32_t* sat_items, int4* ray_rng, uint32_t* ray_items, double4* slab1,
+                      uint32_t* sat_items, int4* ray_rng, uint32_t* ray_items,
                       int part, unsigned long long* bad_input, hipStream_t s)
 {
     if (T <= 0) return;
     if (part == 1)
-        tri_setup_part<1>(tris, T, g0, M, box0, box1, sat_items, ray_rng, ray_items, slab1, bad_input, s);
+        tri_setup_part<1>(tris, T, g0, M, box0, box1, sat_items, ray_rng, ray_items, bad_input, s);
     else if (part == 2)
-        tri_setup_part<2>(tris, T, g0, M, box0, box1, sat_items, ray_rng, ray_items, slab1, bad_input, s);
+        tri_setup_part<2>(tris, T, g0, M, box0, box1, sat_items, ray_rng, ray_items, bad_input, s);
     else
-        tri_setup_part<3>(tris, T, g0, M, box0, box1, sat_items, ray_rng, ray_items, slab1, bad_input, s);
+        tri_setup_part<3>(tris, T, g0, M, box0, box1, sat_items, ray_rng, ray_items, bad_input, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -754,97 +742,265 @@ __device__ __forceinline__ void expand_items(const float* __restrict__ tris, int
     }
 }
 
-// Level1 SAT: one item = (triangle, xy column of its index-AABB); the lane
-// walks the AABB's z range.  Hits set the voxel's boundary byte, append the
-// (voxel, triangle) bin pair -- key = batch-wide bit index, value = triangle --
-// and the lane's highest hit z becomes the (column, triangle, zmax) entry used
-// by the Level2 parity candidates.
-template <bool kM, int XCAP>
-__global__ __launch_bounds__(expand_threads<kM>()) void k_sat_expand(const float* __restrict__ tris, int64_t T,
-                                                   const int4* __restrict__ box0,
-                                                   const int4* __restrict__ box1,
-                                                   const double4* __restrict__ slab1,
-                                                   const uint64_t* __restrict__ off, GridDev g0, Meshes M,
-                                                   uint8_t* __restrict__ bbytes, Append64 pairs,
-                                                   Append64 cols)
+// which item range [so, so + P) of the wave's lanes holds item l0 + lane (ranges
+// in lane order); lanes past the last item get some lane's
+__device__ __forceinline__ int wave_item_owner(uint8_t* win, uint32_t so, uint32_t P, uint32_t l0)
 {
-    constexpr uint32_t PB = 1536, CB = 768;
-    __shared__ uint64_t s_pk[PB];
-    __shared__ uint32_t s_pv[PB];
-    __shared__ uint64_t s_ck[CB];
-    __shared__ uint32_t s_cv[CB];
-    __shared__ uint32_t s_n[2];
-    __shared__ uint64_t s_gbase;
-    if (threadIdx.x < 2) s_n[threadIdx.x] = 0;
+    const int lane = __lane_id();
+    // every range that meets [l0, l0 + 64) marks its first position there (the
+    // one running into the window marks 0; starts are distinct), and an item
+    // takes the mark at the highest marked position up to its own
+    win[lane] = 0xff;
+    __builtin_amdgcn_wave_barrier();
+    if (P && so < l0 + 64u && so + P > l0) win[so > l0 ? so - l0 : 0u] = (uint8_t)lane;
+    __builtin_amdgcn_wave_barrier();
+    const uint32_t wj = win[lane];
+    const uint64_t marks = __ballot(wj != 0xffu) & ((2ull << lane) - 1ull);
+    const int top = marks ? 63 - __clzll((long long)marks) : 0;
+    const int j = __shfl((int)wj, top) & 63;
+    __builtin_amdgcn_wave_barrier();
+    return j;
+}
+
+// Append buffer of a block in LDS.  n is the same in every thread: a block
+// counts what its waves append before they write, so that it needs no atomic
+// but the one global reservation per flush (those of one counter are taken at
+// 3.7 ns each, whoever makes them: 64-lane blocks with buffers of their own
+// spent 120 of 290 us on them on the torus knot).
+template <uint32_t CAP>
+struct BlockAppend {
+    uint64_t* key;
+    uint32_t* val;
+    uint64_t* gbase;
+    uint32_t n;
+};
+
+template <uint32_t CAP>
+__device__ __forceinline__ void block_flush(BlockAppend<CAP>& L, const Append64& G)
+{
+    if (L.n == 0) return;
+    if (threadIdx.x == 0) *L.gbase = atomicAdd(G.count, (unsigned long long)L.n);
     __syncthreads();
-    const LdsAppend lp{s_pk, s_pv, &s_n[0], PB};
-    const LdsAppend lc{s_ck, s_cv, &s_n[1], CB};
-    expand_items<expand_threads<kM>(), XCAP>(tris, T, off, [&](int64_t t, uint64_t l, const float* tv) {
+    const uint64_t gb = *L.gbase;
+    for (uint32_t i = threadIdx.x; i < L.n; i += blockDim.x)
+        if (gb + i < G.cap) {
+            G.key[gb + i] = L.key[i];
+            G.val[gb + i] = L.val[i];
+        }
+    __syncthreads();
+    L.n = 0;
+}
+
+// the block appends `all` entries, this wave `total` of them after the first
+// `before`, this lane cnt of those after the first `excl`: put(store) hands
+// each to store(key, val).  Reached after a barrier that followed the last writes.
+template <uint32_t CAP, typename P>
+__device__ __forceinline__ void block_put(BlockAppend<CAP>& L, const Append64& G, uint32_t all, uint32_t before,
+                                          uint32_t total, uint32_t excl, P&& put)
+{
+    if (L.n + all > CAP) block_flush(L, G);
+    if (all > CAP) {   // straight to global memory
+        unsigned long long gb = 0;
+        if (__lane_id() == 0 && total) gb = atomicAdd(G.count, (unsigned long long)total);
+        uint64_t idx = shfl64(gb, 0) + excl;
+        put([&](uint64_t key, uint32_t val) {
+            if (idx < G.cap) {
+                G.key[idx] = key;
+                G.val[idx] = val;
+            }
+            ++idx;
+        });
+        return;
+    }
+    uint32_t idx = L.n + before + excl;
+    put([&](uint64_t key, uint32_t val) {
+        L.key[idx] = key;
+        L.val[idx] = val;
+        ++idx;
+    });
+    L.n += all;
+}
+
+// Level1 SAT: one item = (triangle, xy column of its index AABB), one lane per
+// item.  The layers that pass are an interval up to rounding (sat_column): a
+// lane takes its certain layers as a mask and runs the float SAT on the few it
+// cannot decide (7 of 10000 columns of a torus knot, 8 of 100 where triangles
+// span a whole grid).  Hits set the voxel's boundary byte and append the
+// (voxel, triangle) bin pair -- key = batch-wide bit index, value = triangle;
+// the highest one becomes the (column, triangle, zmax) entry used by the
+// Level2 parity candidates.
+//
+// A wave owns a run of items and walks it 64 at a time over a window of 64
+// triangles, whose item offsets one load brings in; columns of more than 64
+// layers take several rounds.  One barrier a round counts what the block appends.
+// What bounds it: VALU issue for a third of the time (760 instructions per 64
+// items, half of them the triangle's coefficients, which too few columns would
+// share on fine meshes), the latency of the gathers and the barrier at four
+// waves a SIMD (117 VGPRs, 37 KB of LDS a block) for the rest.  Against a block of lanes
+// that walked each column's layers with the float SAT inside a plane slab:
+// torus knot 256 (2.9 M columns) 150 -> 95 us, torus 512 (1.9 M) 115 -> 65,
+// drilled plate 512 (13.6 M, triangles up to the grid's size) 1870 -> 490,
+// 48 mixed meshes 1900 -> 1080, 128 small ones 480 -> 350.
+constexpr uint32_t kSatBlocks = 1024, kSatRounds = 12;
+template <bool kM>
+__global__ __launch_bounds__(256) void k_sat_expand(const float* __restrict__ tris, int64_t T,
+                                                    const int4* __restrict__ box0,
+                                                    const int4* __restrict__ box1,
+                                                    const uint64_t* __restrict__ off, GridDev g0, Meshes M,
+                                                    uint8_t* __restrict__ bbytes, Append64 pairs,
+                                                    Append64 cols)
+{
+    constexpr uint32_t PB = 2048, CB = 1024;
+    __shared__ uint64_t s_pk[PB];
+    __shared__ uint64_t s_ck[CB];
+    __shared__ uint32_t s_pv[PB];
+    __shared__ uint32_t s_cv[CB];
+    __shared__ uint64_t s_gb[2];
+    __shared__ uint4 s_tot[2][4];
+    __shared__ uint8_t s_win[4][64];
+    const int lane = __lane_id(), wid = threadIdx.x >> 6;
+    const uint64_t total = off[T];
+    // The blocks that fit on the chip at once, more (up to all) where each still gets
+    // kSatRounds rounds of items: a block costs two atomics and a search (level1
+    // 512: 1024 blocks 66 us, 4096 103 us), and uneven columns ask for many (drilled plate
+    // 512: 749 us with 1024, 489 us with 4096)
+    const uint64_t full = total / (256u * kSatRounds), most = gridDim.x;
+    const uint32_t nb = (uint32_t)(full < kSatBlocks ? (most < kSatBlocks ? most : kSatBlocks) : full < most ? full : most) & ~7u;
+    if (blockIdx.x >= nb) return;
+    const uint64_t per = ((total + 4ull * nb - 1) / (4ull * nb) + 63) / 64 * 64;
+    // workgroups are dealt to the 8 XCDs round-robin and each XCD has its own
+    // L2: the blocks of one XCD take one contiguous run of ranges (nb is a
+    // multiple of 8), so that the bytes of neighbouring voxels mostly stay in one L2
+    const uint64_t bb = (uint64_t)((blockIdx.x % 8u) * (nb / 8u) + blockIdx.x / 8u) * 4u * per;
+    if (bb >= total) return;
+    uint64_t base = bb + (uint64_t)wid * per;
+    const uint64_t b1 = base + per < total ? base + per : total;
+    BlockAppend<PB> lp{s_pk, s_pv, &s_gb[0], 0};
+    BlockAppend<CB> lc{s_ck, s_cv, &s_gb[1], 0};
+    int64_t t0 = base < b1 ? wave_find_segment(off, 0, T, base) : 0;
+    bool pending = false;   // layers left of the items at hand (uniform)
+    float tv[9] = {};
+    int p = 0, q = 0, z0 = 0, zmax = -1, zb = 0;
+    uint32_t t = 0;
+    bool vis = false;
+    SatColumn sc{0, 0, 0, 0};
+    for (uint32_t round = 0;; round ^= 1u) {
+        if (!pending && base < b1) {
+            uint64_t so, eo;
+            uint32_t n;
+            for (;;) {
+                const int64_t tl = t0 + lane < T ? t0 + lane : T;
+                so = off[tl];
+                eo = off[tl + 1 < T ? tl + 1 : T];
+                const uint64_t wend = shfl64(eo, 63);
+                const uint64_t left = (wend < b1 ? wend : b1) - base;
+                n = left < 64 ? (uint32_t)left : 64u;
+                if (n) break;
+                t0 = wave_find_segment(off, t0 + 64, T, base);   // 64 triangles without items
+            }
+            const uint64_t from = so > base ? so : base;
+            const uint32_t P = eo > from ? (uint32_t)(eo - from < 64 ? eo - from : 64) : 0u;
+            const uint32_t rel = from - base < 64 ? (uint32_t)(from - base) : 64u;
+            const int j = wave_item_owner(s_win[wid], rel, P, 0);
+            const uint32_t l = (uint32_t)base + (uint32_t)lane - (uint32_t)__shfl((int)(uint32_t)so, j);
+            t = (uint32_t)(t0 + j);
+            // the triangles that end here are done
+            t0 += __popcll(__ballot(eo <= base + n));
+            base += n;
+            zb = 0;
+            zmax = -1;
+            sc = SatColumn{0, 0, 0, 0};
+            if ((uint32_t)lane < n) {
+                const GridDev& g = grid_of<kM>(g0, M, kM ? (int)M.tri_mesh[t] : 0);
+                const int4 q0 = box0[t];
+                const int4 q1 = box1[t];
+#pragma unroll
+                for (int c = 0; c < 9; ++c) tv[c] = tris[(uint64_t)t * 9 + c];
+                const uint32_t jq = l / (uint32_t)q1.x;
+                const int xi = (int)(l - jq * (uint32_t)q1.x), yi = (int)jq;
+                p = q0.x + xi;
+                q = q0.y + yi;
+                z0 = q0.z;
+                vis = q0.w != 0;
+                const SatScale s1{g.s1x, g.s1y, g.s1z, g.d1x, g.d1y, g.d1z};
+                sc = sat_column(tv, g.c1x[q0.x], g.c1y[q0.y], g.c1z[q0.z], s1, xi, yi, q1.z);
+                zb = sc.am;
+            }
+        }
         const int mesh = kM ? (int)M.tri_mesh[t] : 0;
         const GridDev& g = grid_of<kM>(g0, M, mesh);
-        const uint64_t word0 = kM ? M.off[mesh].word0 : 0;
-        const uint32_t col0 = kM ? M.off[mesh].col0 : 0;
-        const int4 b0 = box0[t];
-        const int4 b1 = box1[t];
-        const int p = b0.x + (int)(l % (uint64_t)b1.x);
-        const int q = b0.y + (int)(l / (uint64_t)b1.x);
-        const float cx = g.c1x[p], cy = g.c1y[q];
-        const float hx = g.h1x, hy = g.h1y, hz = g.h1z;
-        const uint64_t plane = (uint64_t)g.ny * g.nxw;
-        const uint64_t rowword = word0 + (uint64_t)q * g.nxw + (uint64_t)(p >> 6);
-        const float* c1z = g.c1z;
-        int za = b0.z, zb = b0.z + b1.z;
-        if (b1.z >= kZSlabMin) {
-            const double4 sl = slab1[t];
-            slab_layers(sl.x, sl.y, sl.z, sl.w, cx, cy, tv, c1z, b0.z, b0.z + b1.z, za, zb);
-        }
-        // the e x z edge predicates hold or fail for the whole column
-        if (!xy_edges_ok(cx, cy, hx, hy, tv)) zb = za;
-        int zmax = -1;
-        for (int z = za; z < zb; ++z) {
-            const bool hit = tri_box_overlap<true, false>(cx, cy, c1z[z], hx, hy, hz, tv);
-            const uint64_t w = (uint64_t)z * plane + rowword;
-            if (hit) {
-                zmax = z;
-                bbytes[w * 64 + (uint64_t)(p & 63)] = 1;   // every writer stores the same byte value
+        uint64_t hit = 0;
+        if (zb < sc.bm) {
+            const int m = sc.bm - zb, ia = sc.ai - zb, ib = sc.bi - zb;
+            uint64_t und = m < 64 ? (1ull << m) - 1ull : ~0ull;
+            hit = ib <= 0 ? 0ull : ib < 64 ? (1ull << ib) - 1ull : ~0ull;
+            hit &= ia <= 0 ? ~0ull : ia < 64 ? ~0ull << ia : 0ull;
+            und &= ~hit;
+            while (und) {
+                const int z = __ffsll((unsigned long long)und) - 1;
+                und &= und - 1ull;
+                if (tri_box_overlap<true, true>(g.c1x[p], g.c1y[q], g.c1z[z0 + zb + z], g.h1x, g.h1y, g.h1z, tv))
+                    hit |= 1ull << z;
             }
-            lds_append(lp, pairs, hit, w * 64 + (uint64_t)(p & 63), (uint32_t)t);
+            if (hit) zmax = z0 + zb + 63 - __clzll((long long)hit);
         }
-        const bool emit = (zmax >= 0) && (b0.w != 0);
-        lds_append(lc, cols, emit, ((uint64_t)(col0 + (uint32_t)q * g.nx + p) << 32) | (uint64_t)t,
-                   (uint32_t)zmax);
-    }, [&](bool last) {
-        // flush when half full (block-uniform: counters read after a barrier)
+        const int zf = z0 + zb;   // the layer of bit 0
+        zb += 64;
+        pending = __any(zb < sc.bm);
+        const bool emit = !pending && zmax >= 0 && vis;
+        // what the block's waves append this round
+        const uint32_t cnt = (uint32_t)__popcll(hit);
+        const uint32_t incl = wave_incl_scan<uint32_t>(cnt);
+        const uint64_t em = __ballot(emit);
+        if (lane == 63) s_tot[round][wid] = make_uint4(incl, (uint32_t)__popcll(em), pending || base < b1 ? 1u : 0u, 0u);
         __syncthreads();
-        const bool fp = last || s_n[0] >= PB / 2;
-        const bool fc = last || s_n[1] >= CB / 2;
-        if (fp) lds_flush(lp, pairs, &s_gbase);
-        if (fc) lds_flush(lc, cols, &s_gbase);
-    });
+        uint32_t pall = 0, call = 0, pbef = 0, cbef = 0, more = 0;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const uint4 v = s_tot[round][w];
+            pbef += w < wid ? v.x : 0u;
+            cbef += w < wid ? v.y : 0u;
+            pall += v.x;
+            call += v.y;
+            more |= v.z;
+        }
+        block_put(lp, pairs, pall, pbef, (uint32_t)__builtin_amdgcn_readlane((int)incl, 63), incl - cnt, [&](auto&& store) {
+            if (!hit) return;
+            const uint64_t plane = (uint64_t)g.ny * g.nxw;
+            const uint64_t bit0 =
+                ((kM ? M.off[mesh].word0 : 0) + (uint64_t)zf * plane + (uint64_t)q * g.nxw) * 64 + (uint64_t)p;
+            for (uint64_t h = hit; h; h &= h - 1ull) {
+                const uint64_t bit = bit0 + (uint64_t)(__ffsll((unsigned long long)h) - 1) * plane * 64;
+                bbytes[bit] = 1;   // every writer stores the same byte value
+                store(bit, t);
+            }
+        });
+        block_put(lc, cols, call, cbef, (uint32_t)__popcll(em), (uint32_t)__popcll(em & lanes_below_mask()),
+                  [&](auto&& store) {
+                      const uint32_t col0 = kM ? M.off[mesh].col0 : 0;
+                      if (emit)
+                          store(((uint64_t)(col0 + (uint32_t)q * g.nx + p) << 32) | (uint64_t)t, (uint32_t)zmax);
+                  });
+        if (emit) zmax = -1;
+        if (!more) break;
+    }
+    __syncthreads();
+    block_flush(lp, pairs);
+    block_flush(lc, cols);
 }
 
-template <int XC>
-static void launch_sat_expand_x(const float* tris, int64_t T, const int4* box0, const int4* box1,
-                                const double4* slab1, const uint64_t* off, const GridDev& g0, const Meshes& M,
-                                uint8_t* b, Append64 pairs, Append64 cols, int blocks, hipStream_t s)
-{
-    if (M.nm > 1)
-        k_sat_expand<true, XC><<<blocks, expand_threads<true>(), 0, s>>>(tris, T, box0, box1, slab1, off, g0, M, b,
-                                                                        pairs, cols);
-    else
-        k_sat_expand<false, XC><<<blocks, expand_threads<false>(), 0, s>>>(tris, T, box0, box1, slab1, off, g0, M,
-                                                                          b, pairs, cols);
-}
-
-void launch_sat_expand(const float* tris, int64_t T, const int4* box0, const int4* box1, const double4* slab1,
-                       const uint64_t* off, const GridDev& g0, const Meshes& M, uint8_t* b, Append64 pairs,
-                       Append64 cols, int blocks, int stage, hipStream_t s)
+void launch_sat_expand(const float* tris, int64_t T, const int4* box0, const int4* box1, const uint64_t* off,
+                       const GridDev& g0, const Meshes& M, uint8_t* b, Append64 pairs, Append64 cols, int blocks,
+                       hipStream_t s)
 {
     if (T <= 0) return;
-    if (stage <= 128)
-        launch_sat_expand_x<128>(tris, T, box0, box1, slab1, off, g0, M, b, pairs, cols, blocks, s);
+    // a wave to eight triangles, but 2048 (a box of 12 can hold 10^6 columns): empty blocks cost their launch
+    const int64_t want = T / 32 > 512 ? T / 32 : 512;
+    const unsigned nb = (unsigned)(((want < blocks ? want : blocks) + 7) / 8 * 8);
+    if (M.nm > 1)
+        k_sat_expand<true><<<nb, 256, 0, s>>>(tris, T, box0, box1, off, g0, M, b, pairs, cols);
     else
-        launch_sat_expand_x<256>(tris, T, box0, box1, slab1, off, g0, M, b, pairs, cols, blocks, s);
+        k_sat_expand<false><<<nb, 256, 0, s>>>(tris, T, box0, box1, off, g0, M, b, pairs, cols);
 }
 
 // boundary flags (one byte per padded voxel, written without atomics by the
@@ -2111,26 +2267,6 @@ struct L2PLds {
 int64_t l2_parity_waves(int n2, int64_t ncol, bool many)
 {
     return n2 <= 0 ? 0 : ncol / l2_parity_columns(n2, many);
-}
-
-// which item range [so, so + P) of the wave's lanes holds item l0 + lane (ranges
-// in lane order); lanes past the last item get some lane's
-__device__ __forceinline__ int wave_item_owner(uint8_t* win, uint32_t so, uint32_t P, uint32_t l0)
-{
-    const int lane = __lane_id();
-    // every range that meets [l0, l0 + 64) marks its first position there (the
-    // one running into the window marks 0; starts are distinct), and an item
-    // takes the mark at the highest marked position up to its own
-    win[lane] = 0xff;
-    __builtin_amdgcn_wave_barrier();
-    if (P && so < l0 + 64u && so + P > l0) win[so > l0 ? so - l0 : 0u] = (uint8_t)lane;
-    __builtin_amdgcn_wave_barrier();
-    const uint32_t wj = win[lane];
-    const uint64_t marks = __ballot(wj != 0xffu) & ((2ull << lane) - 1ull);
-    const int top = marks ? 63 - __clzll((long long)marks) : 0;
-    const int j = __shfl((int)wj, top) & 63;
-    __builtin_amdgcn_wave_barrier();
-    return j;
 }
 
 // C adjacent columns (i1 .., j1) of a mesh by one wave: 1, or 4 (at n2 <= 4).

@@ -266,7 +266,6 @@ struct Job {
     MeshCtr* mctr = nullptr;
     // per triangle
     int4 *box0 = nullptr, *box1 = nullptr, *rng = nullptr;
-    double4* slab1 = nullptr;   // plane slab of triangles spanning several layers
     uint32_t *sat_items = nullptr, *ray_items = nullptr;
     uint64_t *sat_off = nullptr, *ray_off = nullptr, *scan64 = nullptr;
     uint64_t* scan_ray = nullptr;   // scan temporary of the ray half of the set-up (side stream)
@@ -671,6 +670,9 @@ int job_create(gpv_ctx* c, const gpv_mesh_desc* d, int nm, int on_device, Job** 
         g.normals = d[m].params.normals ? 1 : 0;
         g.l2cuda = d[m].params.cuda_level2 ? 1 : 0;
         const gpv_grid_info& I = J->info[m];
+        sat_scale_axis(I.bmin[0], I.bmax[0], I.g[0], false, g.s1x, g.d1x);
+        sat_scale_axis(I.bmin[1], I.bmax[1], I.g[1], false, g.s1y, g.d1y);
+        sat_scale_axis(I.bmin[2], I.bmax[2], I.g[2], false, g.s1z, g.d1z);
         sat_scale_axis(I.bmin[0], I.bmax[0], I.g2[0], g.l2cuda != 0, g.s2x, g.d2x);
         sat_scale_axis(I.bmin[1], I.bmax[1], I.g2[1], g.l2cuda != 0, g.s2y, g.d2y);
         sat_scale_axis(I.bmin[2], I.bmax[2], I.g2[2], g.l2cuda != 0, g.s2z, g.d2z);
@@ -804,7 +806,6 @@ int job_create(gpv_ctx* c, const gpv_mesh_desc* d, int nm, int on_device, Job** 
 
     const size_t Tn = (size_t)std::max<int64_t>(T, 1);
     if ((r = alloc(J, &J->box0, Tn)) || (r = alloc(J, &J->box1, Tn)) || (r = alloc(J, &J->rng, Tn)) ||
-        (r = alloc(J, &J->slab1, Tn)) ||
         (r = alloc(J, &J->sat_items, Tn)) || (r = alloc(J, &J->ray_items, Tn)) ||
         (r = alloc(J, &J->sat_off, Tn + 1)) || (r = alloc(J, &J->ray_off, Tn + 1)) ||
         (r = alloc(J, &J->ctr, 1)) || (r = alloc(J, &J->wcnt, (size_t)W)) ||
@@ -852,7 +853,7 @@ int stage_setup(Job* J)
     launch_fill_u64(reinterpret_cast<uint64_t*>(&J->ctr->bad_input), 0, 1, s);
     if (J->nm > 1) launch_mesh_ids(J->d_off, J->nm, J->T, J->tri_mesh, s);
     launch_tri_setup(J->tris, J->T, J->g[0], J->view(), J->box0, J->box1, J->sat_items, J->rng, J->ray_items,
-                     J->slab1, 3, &J->ctr->bad_input, s);
+                     3, &J->ctr->bad_input, s);
     TRY(ensure_scan_tmp(J, J->T));
     launch_scan_u32_u64(J->sat_items, J->sat_off, J->T, J->scan64, s);
     launch_scan_u32_u64(J->ray_items, J->ray_off, J->T, J->scan64, s);
@@ -876,12 +877,12 @@ int stage_setup_split(Job* J)
     TRY(alloc(J, &J->scan_ray, scan_tmp_elems(J->T)));
     HIP_TRY(hipEventRecord(J->ev[15], s));
     launch_tri_setup(J->tris, J->T, J->g[0], J->view(), J->box0, J->box1, J->sat_items, J->rng, J->ray_items,
-                     J->slab1, 1, &J->ctr->bad_input, s);
+                     1, &J->ctr->bad_input, s);
     launch_scan_u32_u64(J->sat_items, J->sat_off, J->T, J->scan64, s);
     HIP_TRY(hipStreamWaitEvent(c->side, J->ev[15], 0));
     if (!J->all_stencil) {   // the ray half feeds only the ray parity
         launch_tri_setup(J->tris, J->T, J->g[0], J->view(), J->box0, J->box1, J->sat_items, J->rng, J->ray_items,
-                         J->slab1, 2, &J->ctr->bad_input, c->side);
+                         2, &J->ctr->bad_input, c->side);
         launch_scan_u32_u64(J->ray_items, J->ray_off, J->T, J->scan_ray, c->side);
     }
     HIP_TRY(hipGetLastError());
@@ -903,8 +904,8 @@ int launch_sat_half(Job* J)
     Append64 pa{&J->ctr->pairs, J->pair_key, J->pair_tri, J->pair_cap};
     Append64 co{&J->ctr->colents, J->col_key, J->col_z, J->col_cap};
     J->pairs_ranked = false;   // the sweep appends voxel bits
-    launch_sat_expand(J->tris, J->T, J->box0, J->box1, J->slab1, J->sat_off, J->g[0], J->view(), bbytes, pa, co,
-                      expand_blocks(c), c->tune.expand_stage_tris, s);
+    launch_sat_expand(J->tris, J->T, J->box0, J->box1, J->sat_off, J->g[0], J->view(), bbytes, pa, co,
+                      expand_blocks(c), s);
     launch_pack_bytes(bbytes, J->W, J->bnd, s);
     release(J, bbytes);
     launch_popc_words(J->bnd, J->W, J->wcnt, s);
@@ -1367,7 +1368,7 @@ int job_finish(Job* J)
         I.ms_normals = ms_nrm;
     }
     // only the result planes stay resident
-    release(J, J->box0); release(J, J->box1); release(J, J->rng); release(J, J->slab1);
+    release(J, J->box0); release(J, J->box1); release(J, J->rng);
     release(J, J->pmask);
     release(J, J->sat_items); release(J, J->ray_items); release(J, J->sat_off); release(J, J->ray_off);
     release(J, J->scan64); J->scan32 = nullptr; J->scan_cap = 0; release(J, J->scan_ray);
@@ -1476,7 +1477,7 @@ int64_t predict_run_bytes(const gpv_mesh_desc& d, const gpv_grid_info& I)
     int64_t b = 0;
     b += 4 * (2 * (nx + ny + nz) * (1 + n2) + 1);               // center tables
     b += 36 * T + 4 * T + 4 * B + 4096;                          // soup copy, batch mesh ids, descriptors
-    b += 104 * T + 16 + 2 * scan(std::max(T, W));               // per-triangle set-up, item scans
+    b += 72 * T + 16 + 2 * scan(std::max(T, W));               // per-triangle set-up, item scans
     b += 24 * W + 64 * W;                                        // planes, word counts and prefix, flag bytes
     b += 24 * P + 8 * H;                                         // bin pairs, column entries, ray hits
     b += 8 * ncol + 8 + 48 * H + scan(ncol);                     // parity fill: hits by column, records

@@ -1,4 +1,5 @@
-// gpv_satrow.hpp -- the Level2 SAT decided for whole rows of sub-voxels.
+// gpv_satrow.hpp -- the Level2 SAT decided for whole rows of sub-voxels, the
+// Level1 SAT for whole columns of a triangle's index AABB.
 //
 // The SAT (src/TriBoxIntersection.cpp:135-210) of one triangle against the
 // n2^3 boxes of a boundary voxel is a conjunction of predicates that are
@@ -103,8 +104,12 @@ __host__ __device__ __forceinline__ float4 sat_edge_z(float eu, float ez, bool z
 }
 
 // Part `h` (0 or 1) of the entry of triangle tv in the voxel whose sub-center
-// 0 is c0: 0 writes groups 0-2 and 9, 1 the others (the plane's slopes included).  Two lanes make one
-// entry on the device; `loose` has to be combined from both parts.
+// 0 is c0 (kBox: in the index AABB whose first center is c0, where a box may
+// miss the triangle's extent by the rounding of the index and of the tables):
+// 0 writes groups 0-2 and 9, 1 the others (the plane's slopes included).  Two
+// lanes can make one entry on the device; `loose` has to be combined from both
+// parts.
+template <bool kBox = false>
 __host__ __device__ __forceinline__ bool sat_entry_part(int h, const float* tv, float c0x, float c0y, float c0z,
                                                         const SatScale& g, float4* out)
 {
@@ -119,9 +124,12 @@ __host__ __device__ __forceinline__ bool sat_entry_part(int h, const float* tv, 
     const float e1x = r1x * g.sx, e1y = r1y * g.sy, e1z = r1z * g.sz;
     const float e2x = r2x * g.sx, e2y = r2y * g.sy, e2z = r2z * g.sz;
     // extents: the longest edge of each axis spans the other two
-    const float Ax = fmaxf(fmaxf(fabsf(e0x), fabsf(e1x)), fabsf(e2x)) * 1.00001f + 0.50001f;
-    const float Ay = fmaxf(fmaxf(fabsf(e0y), fabsf(e1y)), fabsf(e2y)) * 1.00001f + 0.50001f;
-    const float Az = fmaxf(fmaxf(fabsf(e0z), fabsf(e1z)), fabsf(e2z)) * 1.00001f + 0.50001f;
+    const float Ax = fmaxf(fmaxf(fabsf(e0x), fabsf(e1x)), fabsf(e2x)) * 1.00001f +
+                     (kBox ? 0.51f + 2.0f * g.dx : 0.50001f);
+    const float Ay = fmaxf(fmaxf(fabsf(e0y), fabsf(e1y)), fabsf(e2y)) * 1.00001f +
+                     (kBox ? 0.51f + 2.0f * g.dy : 0.50001f);
+    const float Az = fmaxf(fmaxf(fabsf(e0z), fabsf(e1z)), fabsf(e2z)) * 1.00001f +
+                     (kBox ? 0.51f + 2.0f * g.dz : 0.50001f);
     const float Nx = e0y * e1z - e0z * e1y, Ny = e0z * e1x - e0x * e1z, Nz = e0x * e1y - e0y * e1x;
     const float rz = GPV_RCP(Az) * (16.0f * U);
     const float zeta = (t0z - c0z) * g.sz + 1.0f, xi = (t0x - c0x) * g.sx, eta = (t0y - c0y) * g.sy;
@@ -257,6 +265,65 @@ __host__ __device__ __forceinline__ void sat_row_column(SatRow& s, uint32_t& in,
     const uint32_t n = ~(~0u << sat_trunc(hii)) & (~0u << sat_trunc(fminf(loi, 16.0f)));
     may = !(u > s.um) ? m : 0u;
     in = u < -s.um ? n : 0u;
+}
+
+// ---------------------------------------------------------------------------
+// The same for one column of a triangle's Level1 index AABB: any number of
+// layers, as index intervals, and the box-axis predicates (whose boxes the
+// AABB only approximates) among the bounded ones.  Their values: the
+// reference's t - c (U A) against ours (3 U A and dev), A at most the extent
+// and half a voxel: 16 U (extent + 1) + 2 dev.
+// ---------------------------------------------------------------------------
+struct SatColumn {
+    int am, ai, bi, bm;   // layers [ai, bi) pass; of [am, bm) the others are undecided; the rest fail
+};
+
+// (x, y): the column in the AABB, whose first center is c0 and which has
+// `layers` layers
+__host__ __device__ __forceinline__ SatColumn sat_column(const float* tv, float c0x, float c0y, float c0z,
+                                                         const SatScale& g, int xi, int yi, int layers)
+{
+    constexpr float U = 0x1p-24f;
+    float4 e[kSatEntry4];
+    bool loose = sat_entry_part<true>(0, tv, c0x, c0y, c0z, g, e);
+    loose = sat_entry_part<true>(1, tv, c0x, c0y, c0z, g, e) || loose;
+    const float x = (float)xi, y = (float)yi, n = (float)layers;
+    // box axes: the triangle's extent, half a voxel more on each side
+    const float x0 = (fminf(fminf(tv[0], tv[3]), tv[6]) - c0x) * g.sx, x1 = (fmaxf(fmaxf(tv[0], tv[3]), tv[6]) - c0x) * g.sx;
+    const float y0 = (fminf(fminf(tv[1], tv[4]), tv[7]) - c0y) * g.sy, y1 = (fmaxf(fmaxf(tv[1], tv[4]), tv[7]) - c0y) * g.sy;
+    const float z0 = (fminf(fminf(tv[2], tv[5]), tv[8]) - c0z) * g.sz, z1 = (fmaxf(fmaxf(tv[2], tv[5]), tv[8]) - c0z) * g.sz;
+    const float far = fmaxf(fmaxf(x0 - x, x - x1), fmaxf(y0 - y, y - y1)) - 0.5f;
+    const float mxy = 16.0f * U * (fmaxf(x1 - x0, y1 - y0) + 1.0f) + 2.0f * fmaxf(g.dx, g.dy);
+    const float mz = 16.0f * U * ((z1 - z0) + 1.0f) + 2.0f * g.dz;
+    float lom = fmaxf(0.0f, (z0 + 0.5f) - mz), loi = fmaxf(0.0f, (z0 + 0.5f) + mz);
+    float him = fminf(n, (z1 + 1.5f) + mz), hii = fminf(n, (z1 + 1.5f) - mz);
+#ifdef __HIP_DEVICE_COMPILE__
+#pragma unroll
+#endif
+    for (int k = 0; k < 6; ++k) {
+        const float4 c = e[k];
+        const float w = c.x * (k < 3 ? y : x) + c.y;
+        lom = fmaxf(lom, w - c.z); loi = fmaxf(loi, w - c.w);
+        him = fminf(him, w + c.z); hii = fminf(hii, w + c.w);
+    }
+    const float4 c6 = e[6], c7 = e[7], c8 = e[8], pl = e[9];
+    const float pw = (c7.w * x + c8.w * y) + pl.x;
+    lom = fmaxf(lom, pw - pl.y); loi = fmaxf(loi, pw - pl.z);
+    him = fminf(him, pw + pl.y); hii = fminf(hii, pw + pl.z);
+    const float u = fmaxf(fmaxf(fabsf((c6.x * x + c7.x * y) + c8.x), fabsf((c6.y * x + c7.y * y) + c8.y)),
+                          fabsf((c6.z * x + c7.z * y) + c8.z)) - 1.0f;
+    SatColumn s;
+    s.am = (int)fminf(lom, n);
+    s.bm = (int)fmaxf(him, 0.0f);
+    s.ai = (int)fminf(loi, n);
+    s.bi = (int)fmaxf(hii, 0.0f);
+    if (!(u < -c6.w) || !(far < -mxy)) s.ai = s.bi = 0;
+    if (u > c6.w || far > mxy) s.am = s.bm = 0;
+    if (loose) {
+        s.am = s.ai = s.bi = 0;
+        s.bm = layers;
+    }
+    return s;
 }
 
 }  // namespace gpv

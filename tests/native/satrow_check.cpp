@@ -56,3 +56,25 @@ extern "C" void satrow_batch(int64_t n, int n2, const float* tv, const float* cx
         }
     }
 }
+
+// Level1: case i's index AABB (lo, dd: 3 ints each) on a grid with centers
+// cx/cy/cz, bounds lo3/hi3 and voxel g1; per column of it in (q, p) order from
+// off[i]: [am, ai, bi, bm).
+extern "C" void satcol_batch(int64_t n, const float* tv, const int32_t* lo, const int32_t* dd, const float* cx,
+                             const float* cy, const float* cz, const float* lo3, const float* hi3, const float* g1,
+                             const int64_t* off, int32_t* out)
+{
+    gpv::SatScale g;
+    gpv::sat_scale_axis(lo3[0], hi3[0], g1[0], false, g.sx, g.dx);
+    gpv::sat_scale_axis(lo3[1], hi3[1], g1[1], false, g.sy, g.dy);
+    gpv::sat_scale_axis(lo3[2], hi3[2], g1[2], false, g.sz, g.dz);
+    for (int64_t i = 0; i < n; ++i) {
+        const int32_t *l = lo + 3 * i, *d = dd + 3 * i;
+        int32_t* o = out + 4 * off[i];
+        for (int q = 0; q < d[1]; ++q)
+            for (int p = 0; p < d[0]; ++p, o += 4) {
+                const gpv::SatColumn s = gpv::sat_column(tv + 9 * i, cx[l[0]], cy[l[1]], cz[l[2]], g, p, q, d[2]);
+                o[0] = s.am; o[1] = s.ai; o[2] = s.bi; o[3] = s.bm;
+            }
+    }
+}

@@ -23,6 +23,9 @@ def rows():
     f32 = np.ctypeslib.ndpointer(dtype=np.float32, flags="C_CONTIGUOUS")
     u32 = np.ctypeslib.ndpointer(dtype=np.uint32, flags="C_CONTIGUOUS")
     L.satrow_batch.argtypes = [ctypes.c_int64, ctypes.c_int] + [f32] * 8 + [ctypes.c_int, u32, u32]
+    i32, i64 = (np.ctypeslib.ndpointer(dtype=d, flags="C_CONTIGUOUS") for d in (np.int32, np.int64))
+    L.satcol_batch.argtypes = [ctypes.c_int64, f32, i32, i32] + [f32] * 6 + [i64, i32]
+    L.satrow_batch.columns = L.satcol_batch
     return L.satrow_batch
 
 
@@ -133,3 +136,90 @@ def test_level2_sat_huge_bin(gv, orc):
         compare_results("huge bin", g.download(), want, 4)
         assert g.info()["max_tris_per_voxel"] > 65536
         g.release()
+
+
+@pytest.mark.parametrize("fam", ["random", "small", "lattice", "near", "axis", "sliver"])
+def test_columns_never_contradict_the_sat(rows, gv, orc, fam):
+    """The same claims for the Level1 columns of a triangle's index AABB."""
+    from test_slab_filter import _index_box
+    rng = np.random.default_rng(70 + ["random", "small", "lattice", "near", "axis", "sliver"].index(fam))
+    hits = left = 0
+    for k, vc in enumerate([256, 64, 8, 512, 33, 100]):
+        size = [1.0, 1e3, 1e-3, 1e8, 1e-8][k % 5]
+        ext = rng.uniform(0.2, 1, 3) * size
+        off = [0.0, 0.5, -1.0, 30.0, 3000.0][(k * 2) % 5] * rng.uniform(-1, 1, 3) * size
+        bmin, bmax = off.astype(np.float32), (off + ext).astype(np.float32)
+        info = gv.grid_derive(bmin, bmax, float((bmax - bmin).max()), vc, 1)
+        nn, g1 = np.array(list(info.n)), np.array(list(info.g), np.float32)
+        tabs = [gv.grid_centers(info, 0, a) for a in range(3)]
+        idx = np.stack([rng.integers(0, nn[a], 500) for a in range(3)], 1)
+        big = g1.astype(float) * [1, 8, 3][k % 3]
+        tv = _triangles(rng, fam, bmin + (idx + 0.5) * g1.astype(float), big, g1.astype(float), 3)
+        lo, hi = _index_box(tv, bmin, bmax, nn)
+        dd = np.maximum(hi - lo + 1, 0)
+        keep = (dd > 0).all(1) & (dd.prod(1) < 40000)
+        tv, lo, dd = (np.ascontiguousarray(x[keep], t) for x, t in ((tv, np.float32), (lo, np.int32), (dd, np.int32)))
+        at = np.concatenate([[0], np.cumsum(dd[:, 0].astype(np.int64) * dd[:, 1])]).astype(np.int64)
+        out = np.zeros((at[-1], 4), np.int32)
+        rows.columns(len(tv), tv.ravel(), lo.ravel(), dd.ravel(), *tabs, np.array(list(info.bmin), np.float32),
+                     np.array(list(info.bmax), np.float32), g1, at, out.ravel())
+        own = np.repeat(np.arange(len(tv)), np.diff(at))
+        loc = np.arange(at[-1]) - at[own]
+        col = np.repeat(np.arange(len(own)), dd[own, 2])
+        z = np.arange(len(col)) - np.repeat(np.cumsum(dd[own, 2]) - dd[own, 2], dd[own, 2])
+        c = np.stack([tabs[0][lo[own, 0] + loc % dd[own, 0]][col], tabs[1][lo[own, 1] + loc // dd[own, 0]][col],
+                      tabs[2][lo[own[col], 2] + z]], 1)
+        h = np.broadcast_to((g1 / np.float32(2)).astype(np.float32), c.shape)
+        hit = orc.tri_box(c, h, tv[own[col]]).astype(bool)
+        am, ai, bi, bm = out[col].T
+        inn, may = (z >= ai) & (z < bi), (z >= am) & (z < bm)
+        assert not np.any(inn & ~hit), f"{vc}: {np.count_nonzero(inn & ~hit)} boxes accepted that the SAT rejects"
+        assert not np.any(hit & ~may), f"{vc}: {np.count_nonzero(hit & ~may)} SAT hits dropped"
+        hits += int(hit.sum())
+        left += int((may & ~inn).sum()) if size == 1.0 and abs(off).max() <= 1 else 0
+    assert hits > 2000
+    if fam in ("random", "small"):
+        assert left < 0.1 * hits    # the float SAT is the exception, not the rule
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["one", "tall", "walls", "empty"])
+def test_level1_sat_columns(gv, orc, kind):
+    """Columns of more than 64 layers (steep slivers; upright walls that
+    overflow a block's append buffer in one round) and long runs of triangles
+    without a column between others, alone and in a batch."""
+    from gpview_amd import workloads
+    rng = np.random.default_rng(5)
+    bmin, bmax = np.zeros(3, np.float32), np.array([0.5, 0.4, 1.0], np.float32)
+    if kind == "one":
+        soup = rng.uniform(0.1, 0.4, (1, 9))
+    elif kind == "tall":        # slivers along z, a few columns each
+        a = np.concatenate([rng.uniform(0.05, 0.35, (300, 2)), rng.uniform(0, 0.2, (300, 1))], 1)
+        b = a + np.concatenate([rng.normal(0, 0.01, (300, 2)), rng.uniform(0.3, 0.8, (300, 1))], 1)
+        soup = np.concatenate([a, b, a + rng.normal(0, 0.02, (300, 3))], 1)
+    elif kind == "walls":       # x = const and slightly tilted, the whole box high and wide
+        x = rng.uniform(0.05, 0.45, (40, 1))
+        e = rng.normal(0, 1e-3, (40, 3)) * (np.arange(40) % 2)[:, None]
+        o, w = np.zeros((40, 1)), np.ones((40, 1))
+        soup = np.concatenate([x + e[:, :1], o, o, x + e[:, 1:2], w * 0.8, o, x + e[:, 2:], o, w * 2], 1)
+    else:                       # only every 500th triangle meets the grid
+        soup = rng.uniform(2, 3, (4000, 9))
+        soup[::500] = rng.uniform(0.05, 0.35, (8, 9))
+    soup = np.ascontiguousarray(soup, np.float32)
+    v, f = gv.mixed(1, 2000, 3)
+    say(f"Level1 SAT columns: {kind}")
+    mms = np.float32(1)
+    mesh = {"soup": soup, "bmin": bmin, "bmax": bmax, "mms": mms, "voxel_count": 150, "voxel_count2": 2, "level2": True,
+            "initial_capacity": 0}
+    other = workloads.mesh_entry(gv, v, f, 20, 2)
+    want = [orc.voxelize(m["soup"], orc.grid_setup(m["bmin"], m["bmax"], m["mms"], m["voxel_count"], 2), orc.ORC_FAST)
+            for m in (mesh, other)]
+    with gv.Context() as c:
+        g = c.voxelize(soup, bmin, bmax, float(mms), 150, 2)
+        compare_results(f"{kind} alone", g.download(), want[0], 2)
+        g.release()
+        grids = c.voxelize_batch([mesh, other, mesh])
+        for w, g in zip([want[0], want[1], want[0]], grids):
+            compare_results(f"{kind} batch", g.download(), w, 2)
+        for g in grids:
+            g.release()
