@@ -129,12 +129,12 @@ void launch_scatter_hits(const float* tris, const uint64_t* key, uint64_t n, con
                          const uint32_t* off, uint32_t* cnt, float4* rec, hipStream_t s);
 // scratch of a two-level counting sort (ts_tiles(nkeys) tiles): total and
 // fill counters [2*tiles + 1], tile offsets [tiles + 1], scan temporary
-// [scan_tmp_elems(tiles)], bucket [items]
+// [scan_tmp_elems(tiles)], bucket (8 bytes a bin pair, 16 a column entry)
 struct TileSortTmp {
     uint32_t* total;
     uint32_t* off;
     uint32_t* scan;
-    uint4* bucket;
+    void* bucket;
 };
 size_t ts_tiles(uint64_t nkeys);
 
@@ -181,19 +181,17 @@ void launch_mesh_bounds(const uint32_t* wprefix, const Meshes& M, hipStream_t s)
 void launch_boundary_index(const uint64_t* bnd, const uint32_t* wprefix, const GridDev& g0, const Meshes& M,
                            int64_t W, int32_t* bidx, hipStream_t s);
 // pairs: key = batch-wide boundary bit index, val = triangle
-// bin pairs -> CSR by boundary rank (boff[B + 1], list, Level2 box-axis
-// masks); B <= 2^27.  The pairs' voxel bits are replaced by their boundary
+// bin pairs -> CSR by boundary rank (boff[B + 1], list); B <= 2^27.  The pairs' voxel bits are replaced by their boundary
 // ranks (ranked: they hold ranks already)
 void launch_bin_pairs(uint64_t* bits, bool ranked, const uint32_t* tri, uint64_t n, const uint64_t* bnd,
                       const uint32_t* wprefix, uint32_t B, const TileSortTmp& tmp, int items_per_block,
-                      uint32_t* boff, unsigned int* max_out, uint32_t* list, const float* tris,
-                      const int32_t* bidx, const GridDev& g0, const Meshes& M, uint64_t* pmask, hipStream_t s);
+                      uint32_t* boff, unsigned int* max_out, uint32_t* list, hipStream_t s);
 // per-mesh bin totals and largest bin (multi-mesh runs)
 void launch_mesh_bins(const uint32_t* boff, int64_t B, const Meshes& M, hipStream_t s);
 
 // ngroups waves of at most gmost voxels each (l2_group_voxels); waves: per block (1, 2, 4)
 void launch_l2_sat(const float* tris, const int32_t* bidx, int64_t B, int64_t ngroups, int gmost, const uint32_t* boff,
-                   const uint32_t* list, const uint64_t* pmask, int waves, const GridDev& g0, const Meshes& M,
+                   const uint32_t* list, int waves, const GridDev& g0, const Meshes& M,
                    uint64_t* sat2, hipStream_t s);
 // Level2 parity: a wave takes l2_parity_columns adjacent columns of a mesh
 // (grids are multiples of four in x): four at n2 <= 4 in runs of at least

@@ -1132,6 +1132,7 @@ void launch_scatter_hits(const float* tris, const uint64_t* key, uint64_t n, con
 
 // column entries -> CSR by column, each with the MT record its candidates need
 struct ColSrc {
+    using Item = uint4;
     const uint64_t* key;
     const uint32_t* zmax;
     __device__ uint32_t sort_key(uint64_t i) const { return (uint32_t)(key[i] >> 32); }
@@ -1147,6 +1148,7 @@ struct ColSrc {
 
 // place(pos, it, ok): loads for any valid item, stores only when ok
 struct ColPlace {
+    using Item = uint4;
     const float* tris;
     float4* rec;
     __device__ void operator()(uint32_t pos, const uint4& it, bool ok) const
@@ -1629,12 +1631,13 @@ __global__ __launch_bounds__(TS_NT) void k_ts_count(Src src, uint64_t n, int shi
         if (s_h[t]) atomicAdd(&tile_total[t], s_h[t]);
 }
 
-// items (16 bytes, .x = key) to their tile's bucket range; the item is built
+// items (.x = key) to their tile's bucket range; the item is built
 // here, where the block reads its inputs in their original order
 template <typename Src>
 __global__ __launch_bounds__(TS_NT) void k_ts_bucket(Src src, uint64_t n, int shift, int ntiles,
                                                      const uint32_t* __restrict__ tile_off,
-                                                     uint32_t* __restrict__ tile_fill, uint4* __restrict__ bucket)
+                                                     uint32_t* __restrict__ tile_fill,
+                                                     typename Src::Item* __restrict__ bucket)
 {
     extern __shared__ uint32_t s_h[];   // [ntiles]: counts, then this block's next slot per tile
     for (int t = threadIdx.x; t < ntiles; t += TS_NT) s_h[t] = 0;
@@ -1647,7 +1650,7 @@ __global__ __launch_bounds__(TS_NT) void k_ts_bucket(Src src, uint64_t n, int sh
         if (s_h[t]) s_h[t] = tile_off[t] + atomicAdd(&tile_fill[t], s_h[t]);
     __syncthreads();
     for (uint64_t i0 = lo + threadIdx.x; i0 < hi; i0 += (uint64_t)TS_U * TS_NT) {
-        uint4 it[TS_U];
+        typename Src::Item it[TS_U];
 #pragma unroll
         for (int u = 0; u < TS_U; ++u) {
             const uint64_t i = i0 + (uint64_t)u * TS_NT;
@@ -1660,7 +1663,7 @@ __global__ __launch_bounds__(TS_NT) void k_ts_bucket(Src src, uint64_t n, int sh
 }
 
 template <typename Place>
-__global__ __launch_bounds__(TS_NT) void k_ts_place(const uint4* __restrict__ bucket,
+__global__ __launch_bounds__(TS_NT) void k_ts_place(const typename Place::Item* __restrict__ bucket,
                                                     const uint32_t* __restrict__ tile_off, int shift,
                                                     uint32_t nkeys, uint32_t* __restrict__ off,
                                                     unsigned int* __restrict__ max_out, Place place)
@@ -1716,7 +1719,7 @@ __global__ __launch_bounds__(TS_NT) void k_ts_place(const uint4* __restrict__ bu
     if (threadIdx.x == 0 && max_out && s_max) atomicMax(max_out, s_max);
     __syncthreads();
     for (uint32_t i0 = b0 + threadIdx.x; i0 < b1; i0 += TS_U * TS_NT) {
-        uint4 it[TS_U];
+        typename Place::Item it[TS_U];
         uint32_t pos[TS_U];
 #pragma unroll
         for (int u = 0; u < TS_U; ++u) {
@@ -1755,6 +1758,7 @@ static void ts_sort(Src src, uint64_t n, uint32_t nkeys, const TileSortTmp& tmp,
         return;
     }
     launch_fill_u32(tmp.total, 0, 2 * (int64_t)ntiles + 1, s);   // total[ntiles], fill[ntiles + 1]
+    typename Src::Item* bucket = static_cast<typename Src::Item*>(tmp.bucket);
     uint32_t* fill = tmp.total + ntiles;
     if (n > 0) {
         const uint64_t ipb = (uint64_t)items_per_block;
@@ -1762,12 +1766,11 @@ static void ts_sort(Src src, uint64_t n, uint32_t nkeys, const TileSortTmp& tmp,
         const size_t lds = (size_t)ntiles * 4;
         k_ts_count<Src><<<blocks, TS_NT, lds, s>>>(src, n, shift, ntiles, tmp.total);
         launch_scan_u32_u32(tmp.total, tmp.off, ntiles, tmp.scan, nullptr, s);
-        k_ts_bucket<Src><<<blocks, TS_NT, lds, s>>>(src, n, shift, ntiles, tmp.off, fill, tmp.bucket);
+        k_ts_bucket<Src><<<blocks, TS_NT, lds, s>>>(src, n, shift, ntiles, tmp.off, fill, bucket);
     } else {
         launch_fill_u32(tmp.off, 0, (int64_t)ntiles + 1, s);
     }
-    k_ts_place<Place><<<ntiles, TS_NT, (size_t)4 << shift, s>>>(tmp.bucket, tmp.off, shift, nkeys, off, max_out,
-                                                              place);
+    k_ts_place<Place><<<ntiles, TS_NT, (size_t)4 << shift, s>>>(bucket, tmp.off, shift, nkeys, off, max_out, place);
 }
 
 size_t ts_tiles(uint64_t nkeys)
@@ -1776,13 +1779,10 @@ size_t ts_tiles(uint64_t nkeys)
     return (size_t)((nkeys + (1u << shift) - 1) >> shift);
 }
 
-// A bin pair sorts by the rank of its voxel among the boundary voxels; its
-// item carries the triangle and the Level2 box-axis masks: bit p of mask x
-// says the SAT's x box-axis predicate holds for the triangle and the Level2
-// sub-index p of that voxel (the same float test the full SAT runs), likewise
-// y, z; packed x | y << 16 | z << 32.
-template <bool kM>
+// A bin pair sorts by the rank of its voxel among the boundary voxels; its item
+// is (rank, triangle).
 struct PairSrc {
+    using Item = uint2;
     // per pair, its voxel's bit in the Level1 grid; the count pass writes the
     // voxel's boundary rank over it (ranked: a repeated compaction, whose
     // pairs hold ranks already), so the bucket pass reads the rank directly
@@ -1791,11 +1791,6 @@ struct PairSrc {
     const uint32_t* tri;
     const uint64_t* bnd;
     const uint32_t* wprefix;
-    const float* tris;
-    const int32_t* bidx;
-    GridDev g0;
-    Meshes M;
-    bool masks;
     __device__ uint32_t count_key(uint64_t i) const
     {
         return ranked ? (uint32_t)bits[i] : rank_of(bnd, wprefix, bits[i]);
@@ -1805,44 +1800,15 @@ struct PairSrc {
         if (!ranked) bits[i] = k;
     }
     __device__ uint32_t sort_key(uint64_t i) const { return (uint32_t)bits[i]; }
-    __device__ uint4 item(uint64_t i) const
-    {
-        const uint32_t b = (uint32_t)bits[i];
-        const uint32_t t = tri[i];
-        const int mesh = kM ? (int)M.bmesh[b] : 0;
-        const GridDev& g = grid_of<kM>(g0, M, mesh);
-        const int n2 = g.n2;
-        if (!masks || n2 == 0) return make_uint4(b, t, 0u, 0u);
-        const int v = bidx[b];
-        const int nxy = g.nx * g.ny;
-        const int k1 = v / nxy;
-        const int ij = v - k1 * nxy;
-        const int j1 = ij / g.nx;
-        const int i1 = ij - j1 * g.nx;
-        const float* tv = tris + 9 * (uint64_t)t;
-        const float a0 = tv[0], a1 = tv[1], a2 = tv[2], a3 = tv[3], a4 = tv[4], a5 = tv[5], a6 = tv[6],
-                    a7 = tv[7], a8 = tv[8];
-        const float* cx = g.c2x + (int64_t)i1 * n2;
-        const float* cy = g.c2y + (int64_t)j1 * n2;
-        const float* cz = g.c2z + (int64_t)k1 * n2;
-        uint32_t mx = 0, my = 0, mz = 0;
-        for (int p = 0; p < n2; ++p) {
-            mx |= (uint32_t)sat_axis_ok(a0, a3, a6, cx[p], g.h2x) << p;
-            my |= (uint32_t)sat_axis_ok(a1, a4, a7, cy[p], g.h2y) << p;
-            mz |= (uint32_t)sat_axis_ok(a2, a5, a8, cz[p], g.h2z) << p;
-        }
-        return make_uint4(b, t, mx | (my << 16), mz);
-    }
+    __device__ uint2 item(uint64_t i) const { return make_uint2((uint32_t)bits[i], tri[i]); }
 };
 
 struct PairPlace {
+    using Item = uint2;
     uint32_t* list;
-    uint64_t* pmask;
-    __device__ void operator()(uint32_t pos, const uint4& it, bool ok) const
+    __device__ void operator()(uint32_t pos, const uint2& it, bool ok) const
     {
-        if (!ok) return;
-        list[pos] = it.y;
-        if (pmask) pmask[pos] = (uint64_t)it.z | ((uint64_t)it.w << 32);
+        if (ok) list[pos] = it.y;
     }
 };
 
@@ -1854,16 +1820,9 @@ void launch_bin_cols(const float* tris, const uint64_t* key, const uint32_t* zma
 
 void launch_bin_pairs(uint64_t* bits, bool ranked, const uint32_t* tri, uint64_t n, const uint64_t* bnd,
                       const uint32_t* wprefix, uint32_t B, const TileSortTmp& tmp, int items_per_block,
-                      uint32_t* boff, unsigned int* max_out, uint32_t* list, const float* tris,
-                      const int32_t* bidx, const GridDev& g0, const Meshes& M, uint64_t* pmask, hipStream_t s)
+                      uint32_t* boff, unsigned int* max_out, uint32_t* list, hipStream_t s)
 {
-    const PairPlace place{list, pmask};
-    if (M.nm > 1)
-        ts_sort(PairSrc<true>{bits, ranked, tri, bnd, wprefix, tris, bidx, g0, M, pmask != nullptr}, n, B, tmp,
-                items_per_block, boff, max_out, place, s);
-    else
-        ts_sort(PairSrc<false>{bits, ranked, tri, bnd, wprefix, tris, bidx, g0, M, pmask != nullptr}, n, B, tmp,
-                items_per_block, boff, max_out, place, s);
+    ts_sort(PairSrc{bits, ranked, tri, bnd, wprefix}, n, B, tmp, items_per_block, boff, max_out, PairPlace{list}, s);
 }
 
 // Per-mesh bin totals (pairs) and largest bin of a batch.  bmesh is
@@ -2003,13 +1962,32 @@ __device__ __forceinline__ void l2_sat_run(uint32_t ent, bool valid, L2Lds& L, c
         atomicOr(&L.acc[w], 1u << (bit + r));
 }
 
+// The boxes of a voxel that pass the SAT's predicate of one box axis, c their
+// n centers: the float test's two halves fl(lo - c) > h and fl(hi - c) < -h (lo, hi
+// the triangle's extent) are monotone along c, so they are those from first to
+// last, found from an estimate.
+__device__ __forceinline__ int l2_axis_first(const float* __restrict__ c, int n, float lo, float h, float est)
+{
+    int k = (int)fminf(fmaxf(est + 0.5f, 0.0f), (float)n);
+    while (k < n && lo - c[k] > h) ++k;
+    while (k > 0 && !(lo - c[k - 1] > h)) --k;
+    return k;
+}
+
+__device__ __forceinline__ int l2_axis_last(const float* __restrict__ c, int n, float hi, float h, float est)
+{
+    int k = (int)fminf(fmaxf(est + 1.5f, 0.0f), (float)n);
+    while (k < n && !(hi - c[k] < -h)) ++k;
+    while (k > 0 && hi - c[k - 1] < -h) --k;
+    return k - 1;
+}
+
 template <bool kM, int W>
 __global__ __launch_bounds__(64 * W) void k_l2_sat(const float* __restrict__ tris, const int32_t* __restrict__ bidx,
                                                    int64_t B, int64_t ngroups, int gmost,
                                                    const uint32_t* __restrict__ boff,
                                                    const uint32_t* __restrict__ list,
-                                                   const uint64_t* __restrict__ pmask, GridDev g0, Meshes M,
-                                                   uint64_t* __restrict__ sat2)
+                                                   GridDev g0, Meshes M, uint64_t* __restrict__ sat2)
 {
     __shared__ L2Lds s_l[W];
     const int wv = threadIdx.x >> 6;
@@ -2059,33 +2037,40 @@ __global__ __launch_bounds__(64 * W) void k_l2_sat(const float* __restrict__ tri
         const int js = lane & (L2_STAGE - 1), h = lane >> 5;
         const uint32_t i = base + (uint32_t)js;
         uint32_t P = 0;   // rows of the entry (lanes below 32)
+        int v = 0, a0 = 0, a1 = -1, az = 0;
+        bool loose = false;
         if (i < e1) {
             const uint64_t t = list[i];
-            const uint64_t mk = pmask[i];
             float tv[9];
 #pragma unroll
             for (int c = 0; c < 9; ++c) tv[c] = tris[t * 9 + c];
-            int v = 0, hi = nv;   // the voxel whose entries hold i: vb[v] <= i < vb[v + 1]
+            int hi = nv;   // the voxel whose entries hold i: vb[v] <= i < vb[v + 1]
             while (hi - v > 1) {
                 const int mid = (v + hi) >> 1;
                 if (L.vb[mid] <= i) v = mid;
                 else hi = mid;
             }
-            const bool loose = sat_entry_part(h, tv, g.c2x[L.ci[v][0]], g.c2y[L.ci[v][1]], g.c2z[L.ci[v][2]], sc, L.e[js]);
-            const uint32_t mx = (uint32_t)(mk & 0xffffu), my = (uint32_t)((mk >> 16) & 0xffffu),
-                           mz = (uint32_t)((mk >> 32) & 0xffffu);
-            const bool any = mx && my && mz;
-            const int pa = __ffs(mx) - 1, pb = 31 - __clz(mx);
-            const int qa = __ffs(my) - 1, qb = 31 - __clz(my);
-            const int ra = __ffs(mz) - 1, rb = 31 - __clz(mz);
-            // the boxes that pass the box-axis predicates are one run per axis
-            // (the tables are monotone); were they not, the rows would be
-            // undecided and the float SAT settle them
-            const bool runs = __popc(mx) == pb - pa + 1 && __popc(my) == qb - qa + 1 && __popc(mz) == rb - ra + 1;
-            const uint64_t bad = __ballot(loose || !runs);
-            if (h == 0 && any) {
-                L.dec[js] = (uint32_t)pa | ((uint32_t)qa << 4) | ((uint32_t)ra << 8) | ((uint32_t)rb << 12) |
-                            ((uint32_t)(pb - pa) << 16) | ((uint32_t)v << 20) |
+            const float *cx = g.c2x + L.ci[v][0], *cy = g.c2y + L.ci[v][1], *cz = g.c2z + L.ci[v][2];
+            loose = sat_entry_part(h, tv, cx[0], cy[0], cz[0], sc, L.e[js]);
+            // box axes: x and the first layer by the lower lane, y and the last by the upper
+            const float lo = h ? fminf(fminf(tv[1], tv[4]), tv[7]) : fminf(fminf(tv[0], tv[3]), tv[6]);
+            const float top = h ? fmaxf(fmaxf(tv[1], tv[4]), tv[7]) : fmaxf(fmaxf(tv[0], tv[3]), tv[6]);
+            const float* c = h ? cy : cx;
+            const float hh = h ? g.h2y : g.h2x, s = h ? sc.sy : sc.sx;
+            a0 = l2_axis_first(c, n2, lo, hh, (lo - c[0]) * s);
+            a1 = l2_axis_last(c, n2, top, hh, (top - c[0]) * s);
+            const float z = h ? fmaxf(fmaxf(tv[2], tv[5]), tv[8]) : fminf(fminf(tv[2], tv[5]), tv[8]);
+            az = h ? l2_axis_last(cz, n2, z, g.h2z, (z - cz[0]) * sc.sz)
+                   : l2_axis_first(cz, n2, z, g.h2z, (z - cz[0]) * sc.sz);
+        }
+        {
+            // the upper lane's run of rows, last layer and looseness
+            const int qa = (int)lane_xor<32>((uint32_t)a0), qb = (int)lane_xor<32>((uint32_t)a1),
+                      rb = (int)lane_xor<32>((uint32_t)az);
+            const uint64_t bad = __ballot(loose);
+            if (h == 0 && a1 >= a0 && qb >= qa && rb >= az) {
+                L.dec[js] = (uint32_t)a0 | ((uint32_t)qa << 4) | ((uint32_t)az << 8) | ((uint32_t)rb << 12) |
+                            ((uint32_t)(a1 - a0) << 16) | ((uint32_t)v << 20) |
                             (((bad >> js) | (bad >> (js + 32))) & 1ull ? 0x80000000u : 0u);
                 P = (uint32_t)(qb - qa + 1);
             }
@@ -2203,24 +2188,24 @@ __global__ __launch_bounds__(64 * W) void k_l2_sat(const float* __restrict__ tri
 
 template <int W>
 static void launch_l2_sat_w(const float* tris, const int32_t* bidx, int64_t B, int64_t ngroups, int gmost,
-                            const uint32_t* boff, const uint32_t* list, const uint64_t* pmask, const GridDev& g0,
+                            const uint32_t* boff, const uint32_t* list, const GridDev& g0,
                             const Meshes& M, uint64_t* sat2, hipStream_t s)
 {
     const unsigned blocks = (unsigned)((ngroups + W - 1) / W);
     if (M.nm > 1)
-        k_l2_sat<true, W><<<blocks, 64 * W, 0, s>>>(tris, bidx, B, ngroups, gmost, boff, list, pmask, g0, M, sat2);
+        k_l2_sat<true, W><<<blocks, 64 * W, 0, s>>>(tris, bidx, B, ngroups, gmost, boff, list, g0, M, sat2);
     else
-        k_l2_sat<false, W><<<blocks, 64 * W, 0, s>>>(tris, bidx, B, ngroups, gmost, boff, list, pmask, g0, M, sat2);
+        k_l2_sat<false, W><<<blocks, 64 * W, 0, s>>>(tris, bidx, B, ngroups, gmost, boff, list, g0, M, sat2);
 }
 
 void launch_l2_sat(const float* tris, const int32_t* bidx, int64_t B, int64_t ngroups, int gmost, const uint32_t* boff,
-                   const uint32_t* list, const uint64_t* pmask, int waves, const GridDev& g0, const Meshes& M,
+                   const uint32_t* list, int waves, const GridDev& g0, const Meshes& M,
                    uint64_t* sat2, hipStream_t s)
 {
     if (B <= 0 || ngroups <= 0) return;
-    if (waves <= 1) launch_l2_sat_w<1>(tris, bidx, B, ngroups, gmost, boff, list, pmask, g0, M, sat2, s);
-    else if (waves == 2) launch_l2_sat_w<2>(tris, bidx, B, ngroups, gmost, boff, list, pmask, g0, M, sat2, s);
-    else launch_l2_sat_w<4>(tris, bidx, B, ngroups, gmost, boff, list, pmask, g0, M, sat2, s);
+    if (waves <= 1) launch_l2_sat_w<1>(tris, bidx, B, ngroups, gmost, boff, list, g0, M, sat2, s);
+    else if (waves == 2) launch_l2_sat_w<2>(tris, bidx, B, ngroups, gmost, boff, list, g0, M, sat2, s);
+    else launch_l2_sat_w<4>(tris, bidx, B, ngroups, gmost, boff, list, g0, M, sat2, s);
 }
 
 // ---------------------------------------------------------------------------

@@ -292,7 +292,6 @@ struct Job {
     int32_t* bidx = nullptr;
     int64_t B = 0, W2 = 0;
     uint32_t *boff = nullptr, *list = nullptr;
-    uint64_t* pmask = nullptr;   // Level2 box-axis masks per bin entry
     uint32_t* coff = nullptr;
     uint32_t* scan_side = nullptr;   // scan temporary of the parity fill (it may run beside compaction)
     float4* crec = nullptr;   // 3 float4 per column entry
@@ -1149,10 +1148,8 @@ int launch_compact(Job* J)
     launch_boundary_index(J->bnd, J->wprefix, J->g[0], J->view(), J->W, J->bidx, s);
     release(J, J->boff);
     release(J, J->list);
-    release(J, J->pmask);
     TRY(alloc(J, &J->boff, (size_t)J->B + 1));
     TRY(alloc(J, &J->list, (size_t)std::max<uint64_t>(J->n_pairs, 1)));
-    if (J->n2max > 0) TRY(alloc(J, &J->pmask, (size_t)std::max<uint64_t>(J->n_pairs, 1)));
     // one scratch for both counting sorts (bins by boundary rank, column
     // entries by column)
     const size_t tiles = J->cols_side ? ts_tiles((uint64_t)J->B)
@@ -1162,7 +1159,8 @@ int launch_compact(Job* J)
     uint4* ts_bucket = nullptr;
     TRY(alloc(J, &ts_cnt, 3 * tiles + 2));
     TRY(alloc(J, &ts_bucket,
-              (size_t)std::max<uint64_t>(J->cols_side ? J->n_pairs : std::max(J->n_pairs, J->n_cols), 1)));
+              (size_t)std::max<uint64_t>(J->cols_side ? (J->n_pairs + 1) / 2
+                                                      : std::max((J->n_pairs + 1) / 2, J->n_cols), 1)));
     TRY(ensure_scan_tmp(J, (int64_t)tiles));
     ts.total = ts_cnt;
     ts.off = ts_cnt + 2 * tiles + 1;
@@ -1170,8 +1168,7 @@ int launch_compact(Job* J)
     ts.bucket = ts_bucket;
     const int ipb = std::max(256, J->ctx->tune.sort_items_per_block);
     launch_bin_pairs(J->pair_key, J->pairs_ranked, J->pair_tri, J->n_pairs, J->bnd, J->wprefix, (uint32_t)J->B, ts,
-                     ipb, J->boff, J->nm > 1 ? nullptr : &J->mctr[0].max_per_voxel, J->list, J->tris, J->bidx,
-                     J->g[0], J->view(), J->pmask, s);
+                     ipb, J->boff, J->nm > 1 ? nullptr : &J->mctr[0].max_per_voxel, J->list, s);
     J->pairs_ranked = true;
     if (J->nm > 1) launch_mesh_bins(J->boff, J->B, J->view(), s);
     if (!J->cols_side) {
@@ -1256,7 +1253,7 @@ int l2_sat_kernels(Job* J)
 {
     hipStream_t s = J->ctx->stream;
     HIP_TRY(hipEventRecord(J->ev[6], s));
-    launch_l2_sat(J->tris, J->bidx, J->B, J->l2s_groups, J->l2s_most, J->boff, J->list, J->pmask,
+    launch_l2_sat(J->tris, J->bidx, J->B, J->l2s_groups, J->l2s_most, J->boff, J->list,
                   J->ctx->tune.l2_sat_waves, J->g[0], J->view(), J->sat2, s);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipEventRecord(J->ev[7], s));
@@ -1369,7 +1366,6 @@ int job_finish(Job* J)
     }
     // only the result planes stay resident
     release(J, J->box0); release(J, J->box1); release(J, J->rng);
-    release(J, J->pmask);
     release(J, J->sat_items); release(J, J->ray_items); release(J, J->sat_off); release(J, J->ray_off);
     release(J, J->scan64); J->scan32 = nullptr; J->scan_cap = 0; release(J, J->scan_ray);
     release(J, J->pair_key); release(J, J->pair_tri); release(J, J->col_key); release(J, J->col_z);
@@ -1482,7 +1478,7 @@ int64_t predict_run_bytes(const gpv_mesh_desc& d, const gpv_grid_info& I)
     b += 24 * P + 8 * H;                                         // bin pairs, column entries, ray hits
     b += 8 * ncol + 8 + 48 * H + scan(ncol);                     // parity fill: hits by column, records
     b += 4 * (ncol + 1) + 48 * P + 16 * P + 64 * (ncol / 64 + 1);   // column entries by column, records
-    b += 8 * B + 4 + 4 * P + 8 * P + 16 * P + 64 * (B / 64 + 1) + scan(B);   // boundary list, bins, masks
+    b += 8 * B + 4 + 4 * P + 8 * P + 64 * (B / 64 + 1) + scan(B);   // boundary list, bins
     b += 16 * B * w2;                                            // Level2 planes
     if (d.params.normals) b += 12 * T + 4 * P + 12 * B + 12 * B * n2 * n2 * n2;
     if (d.params.l1_stencil) b += 12 * T + 8 + scan(T) + 8 * nz * 2 * ny * ((2 * nx + 63) / 64);   // stencil fill
