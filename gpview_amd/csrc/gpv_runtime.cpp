@@ -1269,24 +1269,40 @@ int run_l2_sat(Job* J)
     return GPV_OK;
 }
 
-// The Level2 stages of the fused pipeline: the parity follows the column-entry
-// sort on the side stream (it reads the Level1 planes and the column entries,
-// not the bins), the SAT the bins on the main one.  Nothing is allocated or
-// released between the fork and the join, so the pool's blocks stay in one
-// stream order.
-int run_level2(Job* J)
+// The two streams of the fused pipeline after the read-back.  Main: the bins and
+// the Level2 SAT, which reads them.  Side: the column-entry sort and the Level2
+// parity, which reads its entries and the Level1 planes, then the Level1
+// parity fill, which nothing but the counts waits for.  Enqueued in the order in
+// which their kernels are due: the host takes longer over the side
+// stream's dozen launches than the main one over the bins.  Nothing is allocated
+// or released between the fork and the join, so the pool's blocks stay in
+// one stream order.
+int run_streams(Job* J)
 {
-    if (J->n2max <= 0) return GPV_OK;
     gpv_ctx* c = J->ctx;
     hipStream_t s = c->stream;
-    HIP_TRY(hipEventRecord(J->ev[5], s));
-    TRY(l2_parity_kernels(J, c->side));
-    TRY(l2_sat_kernels(J));
-    HIP_TRY(hipStreamWaitEvent(s, J->ev[11], 0));
+    const bool l2 = J->n2max > 0;
+    TRY(alloc_parity(J));
+    J->cols_side = l2;
+    if (l2) TRY(alloc_cols(J));
+    TRY(alloc_level2(J));
+    if (l2) TRY(l2_plan(J));
+    HIP_TRY(hipEventRecord(J->ev[3], s));
+    TRY(launch_compact(J));
+    HIP_TRY(hipStreamWaitEvent(c->side, J->ev[3], 0));
+    if (l2) {
+        TRY(col_sort_kernels(J, c->side, J->scan_side));
+        HIP_TRY(hipEventRecord(J->ev[5], s));
+        TRY(l2_sat_kernels(J));
+        TRY(l2_parity_kernels(J, c->side));
+        J->l2p_done = true;
+        J->l2s_done = true;
+    }
+    TRY(parity_kernels(J, c->side));
+    J->inout_done = true;
+    HIP_TRY(hipStreamWaitEvent(s, J->ev[14], 0));   // the side stream's last
     release(J, J->cs_cnt);
     release(J, J->cs_bucket);
-    J->l2p_done = true;
-    J->l2s_done = true;
     return GPV_OK;
 }
 
@@ -1337,7 +1353,8 @@ int job_finish(Job* J)
     // fill), compaction + bins, L2 parity, L2 SAT, each on its own stream;
     // stages on the side stream overlap the main one's.  For a batch these
     // are the batch's stage times
-    float ms[6] = {el(0, 1), el(1, 12), el(2, 13) + el(3, 14), 0.0f, 0.0f, 0.0f};
+    const bool side_l2 = J->cols_side;   // the parity fill followed the Level2 parity
+    float ms[6] = {el(0, 1), el(1, 12), el(2, 13) + el(side_l2 ? 11 : 3, 14), 0.0f, 0.0f, 0.0f};
     if (J->n2max > 0) {
         ms[3] = el(4, 5);
         ms[4] = el(16, 11);   // in the fused pipeline the two Level2 stages overlap
@@ -1388,9 +1405,7 @@ int job_run(Job* J)
 {
     gpv_ctx* c = J->ctx;
     // independent stages go beside each other on the side stream: the ray
-    // expansion beside the Level1 SAT, the parity fill and the column-entry
-    // sort beside the bins (and, in run_level2, the Level2 parity beside the
-    // Level2 SAT).  Side-stream work allocates nothing and its buffers are
+    // expansion beside the Level1 SAT, then see run_streams.  Side-stream work allocates nothing and its buffers are
     // allocated before the fork and live until the join, so pool blocks keep
     // one stream order.
     const bool side = c->tune.l2_overlap != 0;
@@ -1422,23 +1437,7 @@ int job_run(Job* J)
     }
     if (needed > 0 || !ray_ok) return fail(GPV_ERR_CAPACITY, "buffer capacity did not converge");
     if (side) {
-        TRY(alloc_parity(J));
-        // the column entries (read only by the Level2 parity, which runs on
-        // the side stream too) sort there after the fill, beside the bins
-        J->cols_side = J->n2max > 0;
-        if (J->cols_side) TRY(alloc_cols(J));
-        TRY(alloc_level2(J));
-        if (J->n2max > 0) TRY(l2_plan(J));
-        // the main stream's compaction (the critical path) is enqueued first;
-        // the side stream waits for the point before it
-        HIP_TRY(hipEventRecord(J->ev[3], c->stream));
-        TRY(launch_compact(J));
-        HIP_TRY(hipStreamWaitEvent(c->side, J->ev[3], 0));
-        TRY(parity_kernels(J, c->side));
-        if (J->cols_side) TRY(col_sort_kernels(J, c->side, J->scan_side));
-        J->inout_done = true;
-        TRY(run_level2(J));
-        HIP_TRY(hipStreamWaitEvent(c->stream, J->ev[14], 0));
+        TRY(run_streams(J));
     } else {
         TRY(launch_parity(J));
         TRY(alloc_level2(J));
