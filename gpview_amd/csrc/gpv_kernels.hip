@@ -1965,21 +1965,21 @@ __device__ __forceinline__ void l2_sat_run(uint32_t ent, bool valid, L2Lds& L, c
 // The boxes of a voxel that pass the SAT's predicate of one box axis, c their
 // n centers: the float test's two halves fl(lo - c) > h and fl(hi - c) < -h (lo, hi
 // the triangle's extent) are monotone along c, so they are those from first to
-// last, found from an estimate.
-__device__ __forceinline__ int l2_axis_first(const float* __restrict__ c, int n, float lo, float h, float est)
+// last, searched from k on.
+__device__ __forceinline__ int l2_axis_first(const float* __restrict__ c, int n, float lo, float h, int k)
 {
-    int k = (int)fminf(fmaxf(est + 0.5f, 0.0f), (float)n);
+    k = k < 0 ? 0 : k < n ? k : n;
     while (k < n && lo - c[k] > h) ++k;
     while (k > 0 && !(lo - c[k - 1] > h)) --k;
     return k;
 }
 
-__device__ __forceinline__ int l2_axis_last(const float* __restrict__ c, int n, float hi, float h, float est)
+__device__ __forceinline__ int l2_axis_last(const float* __restrict__ c, int n, float hi, float h, int k)
 {
-    int k = (int)fminf(fmaxf(est + 1.5f, 0.0f), (float)n);
-    while (k < n && !(hi - c[k] < -h)) ++k;
-    while (k > 0 && hi - c[k - 1] < -h) --k;
-    return k - 1;
+    k = k < -1 ? -1 : k < n ? k : n - 1;
+    while (k + 1 < n && !(hi - c[k + 1] < -h)) ++k;
+    while (k >= 0 && hi - c[k] < -h) --k;
+    return k;
 }
 
 template <bool kM, int W>
@@ -2056,12 +2056,21 @@ __global__ __launch_bounds__(64 * W) void k_l2_sat(const float* __restrict__ tri
             const float lo = h ? fminf(fminf(tv[1], tv[4]), tv[7]) : fminf(fminf(tv[0], tv[3]), tv[6]);
             const float top = h ? fmaxf(fmaxf(tv[1], tv[4]), tv[7]) : fmaxf(fmaxf(tv[0], tv[3]), tv[6]);
             const float* c = h ? cy : cx;
-            const float hh = h ? g.h2y : g.h2x, s = h ? sc.sy : sc.sx;
-            a0 = l2_axis_first(c, n2, lo, hh, (lo - c[0]) * s);
-            a1 = l2_axis_last(c, n2, top, hh, (top - c[0]) * s);
+            const float hh = h ? g.h2y : g.h2x, s = h ? sc.sy : sc.sx, c0 = h ? cy[0] : cx[0];
+            const float dev = h ? sc.dy : sc.dx;
             const float z = h ? fmaxf(fmaxf(tv[2], tv[5]), tv[8]) : fminf(fminf(tv[2], tv[5]), tv[8]);
-            az = h ? l2_axis_last(cz, n2, z, g.h2z, (z - cz[0]) * sc.sz)
-                   : l2_axis_first(cz, n2, z, g.h2z, (z - cz[0]) * sc.sz);
+            bool clear = true;
+            a0 = sat_axis_end((lo - c0) * s, n2, dev, clear);
+            a1 = sat_axis_end((top - c0) * s, n2, dev, clear);
+            az = sat_axis_end((z - cz[0]) * sc.sz, n2, sc.dz, clear);
+            if (!clear) {
+                a0 = l2_axis_first(c, n2, lo, hh, a0);
+                a1 = l2_axis_last(c, n2, top, hh, a1);
+                az = h ? l2_axis_last(cz, n2, z, g.h2z, az) : l2_axis_first(cz, n2, z, g.h2z, az);
+            }
+            a0 = a0 > 0 ? a0 : 0;
+            a1 = a1 < n2 ? a1 : n2 - 1;
+            az = h ? (az < n2 ? az : n2 - 1) : (az > 0 ? az : 0);
         }
         {
             // the upper lane's run of rows, last layer and looseness

@@ -177,6 +177,18 @@ __host__ __device__ __forceinline__ bool sat_entry_part(int h, const float* tv, 
     return loose || !(rmax < 1e20f);
 }
 
+// A box axis: with x the triangle's least (greatest) coordinate in centers from the
+// voxel's sub-center 0, the float predicate's half fl(x - c) > h (< -h) fails
+// for the centers from (up to) floor(x + 1/2) on.  Returns that, within [-2,
+// n + 2]; clear = false where x + 1/2 lies so near an integer that the rounding
+// of the table (dev), of x and of the test (57 U together) could decide.
+__host__ __device__ __forceinline__ int sat_axis_end(float x, int n, float dev, bool& clear)
+{
+    const float y = fminf(fmaxf(x, -2.0f), (float)n + 2.0f) + 0.5f, f = floorf(y);
+    clear = clear && dev >= 0.0f && fabsf((y - f) - 0.5f) < 0.5f - (2.0f * dev + 0x1p-18f);
+    return (int)f;
+}
+
 // One row of an entry, positioned at a column.
 struct SatRow {
     float a0, a1, a2, w0, w1, w2, m0, m1, m2, n0, n1, n2;   // (x, z): slope, center, half widths

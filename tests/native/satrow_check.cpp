@@ -78,3 +78,18 @@ extern "C" void satcol_batch(int64_t n, const float* tv, const int32_t* lo, cons
             }
     }
 }
+
+// The box-axis ends of sat_axis_end: n cases, `m` centers each; lo, hi the
+// triangle's extent, end = {first, last, clear}.
+extern "C" void sataxis_batch(int64_t n, int m, const float* lo, const float* hi, const float* c, const float* bmin,
+                              const float* bmax, const float* g2, int cuda, int32_t* end)
+{
+    for (int64_t i = 0; i < n; ++i) {
+        float s, dev;
+        gpv::sat_scale_axis(bmin[i], bmax[i], g2[i], cuda != 0, s, dev);
+        bool clear = true;
+        end[3 * i] = gpv::sat_axis_end((lo[i] - c[m * i]) * s, m, dev, clear);
+        end[3 * i + 1] = gpv::sat_axis_end((hi[i] - c[m * i]) * s, m, dev, clear);
+        end[3 * i + 2] = clear;
+    }
+}

@@ -26,6 +26,8 @@ def rows():
     i32, i64 = (np.ctypeslib.ndpointer(dtype=d, flags="C_CONTIGUOUS") for d in (np.int32, np.int64))
     L.satcol_batch.argtypes = [ctypes.c_int64, f32, i32, i32] + [f32] * 6 + [i64, i32]
     L.satrow_batch.columns = L.satcol_batch
+    L.sataxis_batch.argtypes = [ctypes.c_int64, ctypes.c_int] + [f32] * 6 + [ctypes.c_int, i32]
+    L.satrow_batch.axis = L.sataxis_batch
     return L.satrow_batch
 
 
@@ -136,6 +138,39 @@ def test_level2_sat_huge_bin(gv, orc):
         compare_results("huge bin", g.download(), want, 4)
         assert g.info()["max_tris_per_voxel"] > 65536
         g.release()
+
+
+@pytest.mark.parametrize("cuda", [False, True])
+def test_box_axis_ends(rows, gv, cuda):
+    """Where the box-axis runs are called clear, they are the float test's."""
+    rng = np.random.default_rng(9 + cuda)
+    clear = total = 0
+    for k, (vc, n2) in enumerate([(256, 8), (512, 16), (64, 4), (8, 4), (33, 5), (512, 1), (100, 7)] * 2):
+        size = [1.0, 1e3, 1e-3, 1e8, 1e-8][k % 5]
+        ext = rng.uniform(0.2, 1, 3) * size
+        off = [0.0, 0.5, -1.0, 30.0, 3000.0][(k * 2) % 5] * rng.uniform(-1, 1, 3) * size
+        bmin, bmax = off.astype(np.float32), (off + ext).astype(np.float32)
+        info = gv.grid_derive(bmin, bmax, float((bmax - bmin).max()), vc, n2)
+        nn, g2 = np.array(list(info.n)), np.array(list(info.g2), np.float32)
+        for a in range(3):
+            n = 4000
+            c = np.ascontiguousarray(gv.grid_centers(info, 2, a, cuda).reshape(nn[a], n2)[rng.integers(0, nn[a], n)])
+            d = float(g2[a])
+            u = rng.integers(-3, 2 * n2 + 3, (n, 2)) * 0.5 + rng.choice([0.0, 1e-7, -1e-7, 1e-5, 0.1], (n, 2))
+            u[::2] = rng.uniform(-3, n2 + 3, (n // 2 + n % 2, 2)) * rng.choice([1, 1000], (n // 2 + n % 2, 1))
+            e = np.sort((c[:, :1] + u * d).astype(np.float32), 1)
+            lo, hi = np.ascontiguousarray(e[:, 0]), np.ascontiguousarray(e[:, 1])
+            h = np.float32(g2[a] / np.float32(2))
+            end = np.zeros((n, 3), np.int32)
+            rows.axis(n, n2, lo, hi, c.ravel(), np.full(n, bmin[a]), np.full(n, bmax[a]), np.full(n, g2[a]), int(cuda), end.ravel())
+            first = (lo[:, None] - c > h).sum(1)              # monotone: the centers that fail come first
+            last = n2 - 1 - (hi[:, None] - c < -h).sum(1)
+            ok = end[:, 2] != 0
+            np.testing.assert_array_equal(np.clip(end[ok, 0], 0, n2), first[ok])
+            np.testing.assert_array_equal(np.clip(end[ok, 1], -1, n2 - 1), last[ok])
+            clear += int(ok.sum()) if size == 1.0 and abs(off).max() <= 1 else 0
+            total += n if size == 1.0 and abs(off).max() <= 1 else 0
+    assert clear > 0.4 * total
 
 
 @pytest.mark.parametrize("fam", ["random", "small", "lattice", "near", "axis", "sliver"])
