@@ -117,8 +117,8 @@ void launch_scan_u32_u32(const uint32_t* in, uint32_t* out, int64_t n, uint32_t*
 void launch_sat_expand(const float* tris, int64_t T, const int4* box0, const int4* box1, const uint64_t* off,
                        const GridDev& g0, const Meshes& M, uint8_t* bbytes, Append64 pairs, Append64 cols, int blocks,
                        hipStream_t s);
-// boundary bytes (W * 64) -> boundary bitplane (W words)
-void launch_pack_bytes(const uint8_t* by, int64_t W, uint64_t* bits, hipStream_t s);
+// boundary bytes (W * 64, aligned to 16) -> boundary bitplane (W words) and its popcounts
+void launch_pack_bytes(const uint8_t* by, int64_t W, uint64_t* bits, uint32_t* cnt, hipStream_t s);
 // stage: triangles staged per LDS pass (128 or 256)
 void launch_ray_expand(const float* tris, int64_t T, const int4* ray_rng, const uint64_t* off, const GridDev& g0,
                        const Meshes& M, Append64 hits, int blocks, int stage, hipStream_t s);
@@ -175,7 +175,6 @@ void launch_l1_stencil(const float* tris, int64_t T, const GridDev& g, uint32_t*
 void launch_l1_parity(const float4* rec, const uint32_t* hoff, const GridDev& g0, const Meshes& M, int64_t NT,
                       uint64_t* ins, hipStream_t s);
 
-void launch_popc_words(const uint64_t* bits, int64_t W, uint32_t* cnt, hipStream_t s);
 // b0 and l2w0 of every mesh (and the totals in entry nm) from the word prefix
 void launch_mesh_bounds(const uint32_t* wprefix, const Meshes& M, hipStream_t s);
 void launch_boundary_index(const uint64_t* bnd, const uint32_t* wprefix, const GridDev& g0, const Meshes& M,

