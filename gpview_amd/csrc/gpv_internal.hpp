@@ -129,7 +129,7 @@ void launch_scatter_hits(const float* tris, const uint64_t* key, uint64_t n, con
                          const uint32_t* off, uint32_t* cnt, float4* rec, hipStream_t s);
 // scratch of a two-level counting sort (ts_tiles(nkeys) tiles): total and
 // fill counters [2*tiles + 1], tile offsets [tiles + 1], scan temporary
-// [scan_tmp_elems(tiles)], bucket (8 bytes a bin pair, 16 a column entry)
+// [scan_tmp_elems(tiles)], bucket (8 bytes a bin pair, 12 a column entry)
 struct TileSortTmp {
     uint32_t* total;
     uint32_t* off;
@@ -149,10 +149,10 @@ __host__ __device__ inline int l2_group_voxels(int n2, int most)
     if (c > kL2GroupMax) c = kL2GroupMax;
     return c < most ? c : most;
 }
-// column entries (key = column << 32 | triangle) -> CSR by column with the MT
-// records; ncol <= 2^27
-void launch_bin_cols(const float* tris, const uint64_t* key, const uint32_t* zmax, uint64_t n, uint32_t ncol,
-                     const TileSortTmp& tmp, int items_per_block, uint32_t* coff, float4* rec, hipStream_t s);
+// column entries (key = column << 32 | triangle) -> CSR by column of (triangle,
+// zmax); ncol <= 2^27
+void launch_bin_cols(const uint64_t* key, const uint32_t* zmax, uint64_t n, uint32_t ncol, const TileSortTmp& tmp,
+                     int items_per_block, uint32_t* coff, uint2* ent, hipStream_t s);
 
 // Level1 parity tasks: L1P_Z consecutive layers of one 64-column row strip
 constexpr int L1P_Z = 16;
@@ -203,8 +203,8 @@ __host__ __device__ inline int l2_parity_columns(int n2, bool many) { return man
 int64_t l2_parity_waves(int n2, int64_t ncol, bool many);
 // n2max, nzmax: the largest Level2 resolution and layer count of the run
 void launch_l2_parity(const uint64_t* bnd, const uint32_t* wprefix, int64_t nwaves, bool many, int n2max, int nzmax,
-                      const uint32_t* coff, const float4* rec, int waves, const GridDev& g0, const Meshes& M,
-                      uint64_t* par2, hipStream_t s);
+                      const uint32_t* coff, const uint2* ent, const float* tris, int waves, const GridDev& g0,
+                      const Meshes& M, uint64_t* par2, hipStream_t s);
 
 // normals (src/Object.cpp:3219-3253 Level1, 2372-2421 + 2705-2720 Level2)
 void launch_face_normals(const float* tris, int64_t T, float* fn, hipStream_t s);

@@ -294,11 +294,11 @@ struct Job {
     uint32_t *boff = nullptr, *list = nullptr;
     uint32_t* coff = nullptr;
     uint32_t* scan_side = nullptr;   // scan temporary of the parity fill (it may run beside compaction)
-    float4* crec = nullptr;   // 3 float4 per column entry
+    uint2* cent = nullptr;    // (triangle, zmax) of the column entries
     // column-entry sort on the side stream (beside the bins): its own scratch
     bool cols_side = false;
     uint32_t* cs_cnt = nullptr;
-    uint4* cs_bucket = nullptr;
+    uint32_t* cs_bucket = nullptr;   // 3 words per column entry
     int64_t l2p_waves = 0, l2s_groups = 0;   // Level2 parity waves, SAT groups (l2_plan)
     int l2s_most = 1;                        // most voxels of a SAT group
     uint32_t *hcnt = nullptr, *hoff = nullptr;
@@ -1064,23 +1064,23 @@ int launch_stencil(Job* J, hipStream_t s)
 int alloc_cols(Job* J)
 {
     release(J, J->coff);
-    release(J, J->crec);
+    release(J, J->cent);
     release(J, J->cs_cnt);
     release(J, J->cs_bucket);
     TRY(alloc(J, &J->coff, (size_t)J->ncol + 1));
-    TRY(alloc(J, &J->crec, (size_t)std::max<uint64_t>(J->n_cols, 1) * 3));
+    TRY(alloc(J, &J->cent, (size_t)std::max<uint64_t>(J->n_cols, 1)));
     TRY(alloc(J, &J->cs_cnt, 3 * ts_tiles((uint64_t)J->ncol) + 2));
-    return alloc(J, &J->cs_bucket, (size_t)std::max<uint64_t>(J->n_cols, 1));
+    return alloc(J, &J->cs_bucket, 3 * (size_t)std::max<uint64_t>(J->n_cols, 1));
 }
 
-// column entries by column with their MT records, on stream s; scan is a
+// column entries by column, on stream s; scan is a
 // scan temporary of at least scan_tmp_elems(ncol) that no other stream uses
 int col_sort_kernels(Job* J, hipStream_t s, uint32_t* scan)
 {
     const size_t tiles = ts_tiles((uint64_t)J->ncol);
     const TileSortTmp ts{J->cs_cnt, J->cs_cnt + 2 * tiles + 1, scan, J->cs_bucket};
     const int ipb = std::max(256, J->ctx->tune.sort_items_per_block);
-    launch_bin_cols(J->tris, J->col_key, J->col_z, J->n_cols, (uint32_t)J->ncol, ts, ipb, J->coff, J->crec, s);
+    launch_bin_cols(J->col_key, J->col_z, J->n_cols, (uint32_t)J->ncol, ts, ipb, J->coff, J->cent, s);
     HIP_TRY(hipGetLastError());
     return GPV_OK;
 }
@@ -1130,7 +1130,7 @@ int alloc_level2(Job* J)
     return alloc(J, &J->par2, (size_t)std::max<int64_t>(J->W2, 1));
 }
 
-// boundary index list, bins per boundary voxel, column entries with records
+// boundary index list, bins per boundary voxel, column entries by column
 // (Level2 planes allocated)
 int launch_compact(Job* J)
 {
@@ -1155,11 +1155,10 @@ int launch_compact(Job* J)
                                       : std::max(ts_tiles((uint64_t)J->B), ts_tiles((uint64_t)J->ncol));
     TileSortTmp ts{};
     uint32_t* ts_cnt = nullptr;
-    uint4* ts_bucket = nullptr;
+    uint32_t* ts_bucket = nullptr;
     TRY(alloc(J, &ts_cnt, 3 * tiles + 2));
     TRY(alloc(J, &ts_bucket,
-              (size_t)std::max<uint64_t>(J->cols_side ? (J->n_pairs + 1) / 2
-                                                      : std::max((J->n_pairs + 1) / 2, J->n_cols), 1)));
+              (size_t)std::max<uint64_t>(J->cols_side ? 2 * J->n_pairs : std::max(2 * J->n_pairs, 3 * J->n_cols), 1)));
     TRY(ensure_scan_tmp(J, (int64_t)tiles));
     ts.total = ts_cnt;
     ts.off = ts_cnt + 2 * tiles + 1;
@@ -1172,10 +1171,10 @@ int launch_compact(Job* J)
     if (J->nm > 1) launch_mesh_bins(J->boff, J->B, J->view(), s);
     if (!J->cols_side) {
         release(J, J->coff);
-        release(J, J->crec);
+        release(J, J->cent);
         TRY(alloc(J, &J->coff, (size_t)J->ncol + 1));
-        TRY(alloc(J, &J->crec, (size_t)std::max<uint64_t>(J->n_cols, 1) * 3));
-        launch_bin_cols(J->tris, J->col_key, J->col_z, J->n_cols, (uint32_t)J->ncol, ts, ipb, J->coff, J->crec, s);
+        TRY(alloc(J, &J->cent, (size_t)std::max<uint64_t>(J->n_cols, 1)));
+        launch_bin_cols(J->col_key, J->col_z, J->n_cols, (uint32_t)J->ncol, ts, ipb, J->coff, J->cent, s);
     }
     release(J, ts_cnt);
     release(J, ts_bucket);
@@ -1230,8 +1229,8 @@ int l2_parity_kernels(Job* J, hipStream_t s)
 {
     HIP_TRY(hipEventRecord(J->ev[16], s));
     if (J->B > 0)
-        launch_l2_parity(J->bnd, J->wprefix, J->l2p_waves, J->ncol >= kL2ParityMany, J->n2max, J->nzmax, J->coff, J->crec,
-                         J->ctx->tune.l2_parity_waves, J->g[0], J->view(), J->par2, s);
+        launch_l2_parity(J->bnd, J->wprefix, J->l2p_waves, J->ncol >= kL2ParityMany, J->n2max, J->nzmax, J->coff, J->cent,
+                         J->tris, J->ctx->tune.l2_parity_waves, J->g[0], J->view(), J->par2, s);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipEventRecord(J->ev[11], s));
     return GPV_OK;
@@ -1386,7 +1385,7 @@ int job_finish(Job* J)
     release(J, J->scan64); J->scan32 = nullptr; J->scan_cap = 0; release(J, J->scan_ray);
     release(J, J->pair_key); release(J, J->pair_tri); release(J, J->col_key); release(J, J->col_z);
     release(J, J->hit_key); release(J, J->wcnt); release(J, J->boff);
-    release(J, J->list); release(J, J->coff); release(J, J->crec); release(J, J->hcnt);
+    release(J, J->list); release(J, J->coff); release(J, J->cent); release(J, J->hcnt);
     release(J, J->cs_cnt); release(J, J->cs_bucket);
     release(J, J->hoff); release(J, J->hrec); release(J, J->scan_side); release(J, J->tri_mesh);
     release(J, J->st_cnt); release(J, J->st_off); release(J, J->st_scan); release(J, J->st_tog);
@@ -1475,7 +1474,7 @@ int64_t predict_run_bytes(const gpv_mesh_desc& d, const gpv_grid_info& I)
     b += 24 * W + 64 * W;                                        // planes, word counts and prefix, flag bytes
     b += 24 * P + 8 * H;                                         // bin pairs, column entries, ray hits
     b += 8 * ncol + 8 + 48 * H + scan(ncol);                     // parity fill: hits by column, records
-    b += 4 * (ncol + 1) + 48 * P + 16 * P + 64 * (ncol / 64 + 1);   // column entries by column, records
+    b += 4 * (ncol + 1) + 8 * P + 12 * P + 64 * (ncol / 64 + 1);   // column entries by column
     b += 8 * B + 4 + 4 * P + 8 * P + 64 * (B / 64 + 1) + scan(B);   // boundary list, bins
     b += 16 * B * w2;                                            // Level2 planes
     if (d.params.normals) b += 12 * T + 4 * P + 12 * B + 12 * B * n2 * n2 * n2;
