@@ -44,7 +44,7 @@ struct MeshOff {
     uint32_t col0;
     uint32_t tri0;
     uint32_t b0;
-    uint32_t ptask0;   // first Level1 parity task (16 layers x 64 columns of one row)
+    uint32_t ptask0;   // first Level1 fill block (L1F_W words of a layer)
     uint32_t pw0;      // first Level2 parity wave
     uint32_t sg0;      // first Level2 SAT group (set on the host once boundary counts are known)
 };
@@ -85,7 +85,6 @@ struct Append64 {
 struct Counters {
     unsigned long long pairs;       // Level1 SAT (voxel, triangle) pairs
     unsigned long long colents;     // (column, triangle, zmax) entries
-    unsigned long long hits;        // (column, triangle) ray hits, Level1
     unsigned long long bad_input;   // nonzero: a vertex coordinate is not finite or beyond +-2^40
 };
 
@@ -119,14 +118,10 @@ void launch_sat_expand(const float* tris, int64_t T, const int4* box0, const int
                        hipStream_t s);
 // boundary bytes (W * 64, aligned to 16) -> boundary bitplane (W words) and its popcounts
 void launch_pack_bytes(const uint8_t* by, int64_t W, uint64_t* bits, uint32_t* cnt, hipStream_t s);
-// stage: triangles staged per LDS pass (128 or 256)
+// XORs the toggles of the accepted ray crossings into the inside plane (cleared by the caller)
 void launch_ray_expand(const float* tris, int64_t T, const int4* ray_rng, const uint64_t* off, const GridDev& g0,
-                       const Meshes& M, Append64 hits, int blocks, int stage, hipStream_t s);
+                       const Meshes& M, uint64_t* ins, int blocks, hipStream_t s);
 
-// counting sort helpers (keys hold a batch-wide column index in the high word)
-void launch_count_keys_hi(const uint64_t* key, uint64_t n, uint32_t* cnt, hipStream_t s);
-void launch_scatter_hits(const float* tris, const uint64_t* key, uint64_t n, const GridDev& g0, const Meshes& M,
-                         const uint32_t* off, uint32_t* cnt, float4* rec, hipStream_t s);
 // scratch of a two-level counting sort (ts_tiles(nkeys) tiles): total and
 // fill counters [2*tiles + 1], tile offsets [tiles + 1], scan temporary
 // [scan_tmp_elems(tiles)], bucket (8 bytes a bin pair, 12 a column entry)
@@ -154,9 +149,9 @@ __host__ __device__ inline int l2_group_voxels(int n2, int most)
 void launch_bin_cols(const uint64_t* key, const uint32_t* zmax, uint64_t n, uint32_t ncol, const TileSortTmp& tmp,
                      int items_per_block, uint32_t* coff, uint2* ent, hipStream_t s);
 
-// Level1 parity tasks: L1P_Z consecutive layers of one 64-column row strip
-constexpr int L1P_Z = 16;
-inline int64_t l1_parity_tasks(const GridDev& g) { return (int64_t)((g.nz + L1P_Z - 1) / L1P_Z) * g.ny * g.nxw; }
+// Level1 fill: a block takes L1F_W words of a mesh's layer, all layers
+constexpr int L1F_W = 16;
+inline int64_t l1_fill_blocks(const GridDev& g) { return ((int64_t)g.ny * g.nxw + L1F_W - 1) / L1F_W; }
 // one mesh's soup (n floats, device memory or page-locked host memory mapped
 // into the device's address space) and its place in the batch's soup
 struct SoupPiece {
@@ -172,8 +167,8 @@ void launch_gather_soups(const SoupPiece* pc, int nm, float* dst, int blocks, bo
 size_t l1_stencil_words(const GridDev& g);
 void launch_l1_stencil(const float* tris, int64_t T, const GridDev& g, uint32_t* cnt, uint64_t* off,
                        uint64_t* scan_tmp, uint64_t* tog, uint64_t* ins, hipStream_t s);
-void launch_l1_parity(const float4* rec, const uint32_t* hoff, const GridDev& g0, const Meshes& M, int64_t NT,
-                      uint64_t* ins, hipStream_t s);
+// toggles -> inside bits, in place, but for the stencil meshes; blocks: l1_fill_blocks of all meshes
+void launch_l1_fill(const GridDev& g0, const Meshes& M, int64_t blocks, uint64_t* ins, hipStream_t s);
 
 // b0 and l2w0 of every mesh (and the totals in entry nm) from the word prefix
 void launch_mesh_bounds(const uint32_t* wprefix, const Meshes& M, hipStream_t s);

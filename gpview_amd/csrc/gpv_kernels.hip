@@ -106,26 +106,6 @@ __device__ __forceinline__ void block_add_u64(uint64_t x, unsigned long long* ds
     }
 }
 
-// Wave-aggregated append: one atomic per wave per call, lanes write at
-// base + rank among the lanes that append.  Must be reached by every active
-// lane of the wave (it may sit inside divergent code).
-__device__ __forceinline__ void wave_append(const Append64& a, bool pred, uint64_t key, uint32_t val)
-{
-    const uint64_t m = __ballot(pred);
-    if (m == 0) return;
-    const int leader = __ffsll((unsigned long long)m) - 1;
-    uint64_t base = 0;
-    if ((int)__lane_id() == leader) base = atomicAdd(a.count, (unsigned long long)__popcll(m));
-    base = shfl64(base, leader);
-    if (pred) {
-        const uint64_t idx = base + (uint64_t)__popcll(m & lanes_below_mask());
-        if (idx < a.cap) {
-            a.key[idx] = key;
-            if (a.val) a.val[idx] = val;
-        }
-    }
-}
-
 // largest t in [0, n) with off[t] <= x, given off[0] <= x < off[n]
 __device__ __forceinline__ int64_t find_segment(const uint64_t* __restrict__ off, int64_t n, uint64_t x)
 {
@@ -583,22 +563,8 @@ void launch_scan_u32_u32(const uint32_t* in, uint32_t* out, int64_t n, uint32_t*
 }
 
 // ---------------------------------------------------------------------------
-// item expansion with LDS staging: a block takes XB consecutive items of the
-// flattened (triangle, sub-range) space; the triangles those items belong to
-// are staged in LDS (offsets + vertices) with one coalesced copy, and each
-// lane finds its triangle by a binary search in LDS.  Falls back to global
-// memory when a block spans more than XCAP triangles (long runs of empty
-// triangles).  Batches use blocks of 512 threads (the many short item runs
-// of small meshes amortise each pass's searches and staging over twice the
-// items: Level1 SAT of the mixed-size stream 11.9 -> 8.7 ms); one mesh uses
-// 256 (with 512 its Level1 SAT beside the ray expansion took 0.21 -> 0.25 ms).
+// item expansion: the flattened (triangle, column) space of the Level1 stages
 // ---------------------------------------------------------------------------
-template <bool kM>
-constexpr int expand_threads()
-{
-    return kM ? 512 : 256;
-}
-
 // 64-ary search by one wave: largest t in [lo, hi) with off[t] <= x, given
 // off[lo] <= x and (hi == n or off[hi] > x).  ~log64 rounds of dependent
 // loads instead of log2.
@@ -617,129 +583,6 @@ __device__ __forceinline__ int64_t wave_find_segment(const uint64_t* __restrict_
         lo = nlo;
     }
     return lo;
-}
-
-// Block-local append buffer in LDS: wave-aggregated LDS atomics, one global
-// reservation per flush.  Entries that do not fit spill straight to the
-// global buffer with a wave-aggregated global atomic.
-struct LdsAppend {
-    uint64_t* key;
-    uint32_t* val;
-    uint32_t* count;
-    uint32_t cap;
-};
-
-__device__ __forceinline__ void lds_append(const LdsAppend& L, const Append64& G, bool pred, uint64_t key,
-                                           uint32_t val)
-{
-    const uint64_t m = __ballot(pred);
-    if (m == 0) return;
-    const int leader = __ffsll((unsigned long long)m) - 1;
-    uint32_t base = 0;
-    if ((int)__lane_id() == leader) base = atomicAdd(L.count, (uint32_t)__popcll(m));
-    base = __shfl(base, leader);
-    const uint32_t idx = base + (uint32_t)__popcll(m & lanes_below_mask());
-    if (pred && idx < L.cap) {
-        L.key[idx] = key;
-        if (L.val) L.val[idx] = val;
-    }
-    wave_append(G, pred && idx >= L.cap, key, val);
-}
-
-// block-synchronous: every thread of the block calls it
-__device__ __forceinline__ void lds_flush(const LdsAppend& L, const Append64& G, uint64_t* s_gbase)
-{
-    __syncthreads();
-    const uint32_t n = *L.count < L.cap ? *L.count : L.cap;
-    if (threadIdx.x == 0 && n) *s_gbase = atomicAdd(G.count, (unsigned long long)n);
-    __syncthreads();
-    if (n) {
-        const uint64_t gb = *s_gbase;
-        for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
-            const uint64_t idx = gb + i;
-            if (idx < G.cap) {
-                G.key[idx] = L.key[i];
-                if (G.val) G.val[idx] = L.val[i];
-            }
-        }
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) *L.count = 0;
-    __syncthreads();
-}
-
-struct NoAfter {
-    __device__ void operator()(bool) const {}
-};
-
-// Each block owns a contiguous range of items, walked XB at a time, so the
-// triangle searches of consecutive iterations start where the last ended.
-// after(last) runs block-synchronously after every iteration.  XCAP: the
-// triangles one pass stages in LDS (the tuned "triangles per LDS batch").
-template <int XB, int XCAP, typename F, typename A>
-__device__ __forceinline__ void expand_items(const float* __restrict__ tris, int64_t T,
-                                             const uint64_t* __restrict__ off, F&& body, A&& after)
-{
-    __shared__ uint64_t s_off[XCAP + 1];
-    __shared__ float s_tv[XCAP * 9];
-    __shared__ int64_t s_t[2];
-    const uint64_t total = off[T];
-    const int tid = threadIdx.x;
-    const uint64_t per = ((total + gridDim.x - 1) / gridDim.x + XB - 1) / XB * XB;
-    // workgroups are dealt to the 8 XCDs round-robin and each XCD has its own
-    // L2: give the blocks of one XCD one contiguous run of ranges, so the
-    // atomics on neighbouring bitplane words mostly stay in one L2
-    const uint32_t G = gridDim.x;
-    const uint32_t lb = (G % 8u == 0u) ? (blockIdx.x % 8u) * (G / 8u) + blockIdx.x / 8u : blockIdx.x;
-    const uint64_t b0 = (uint64_t)lb * per;
-    const uint64_t b1 = b0 + per < total ? b0 + per : total;
-    int64_t lo_hint = 0;
-    for (uint64_t base = b0; base < b1; base += XB) {
-        const uint64_t last = (base + XB < b1 ? base + XB : b1) - 1;
-        if (tid < 64) {
-            const int64_t r = wave_find_segment(off, lo_hint, T, base);
-            if (tid == 0) s_t[0] = r;
-        } else if (tid < 128) {
-            const int64_t r = wave_find_segment(off, lo_hint, T, last);
-            if (tid == 64) s_t[1] = r;
-        }
-        __syncthreads();
-        const int64_t t0 = s_t[0];
-        const int64_t nt = s_t[1] - t0 + 1;
-        lo_hint = s_t[1];
-        const bool staged = nt <= XCAP;
-        if (staged) {
-            for (int k = tid; k <= nt; k += XB) s_off[k] = off[t0 + k];
-            const float* src = tris + t0 * 9;
-            for (int k = tid; k < nt * 9; k += XB) s_tv[k] = src[k];
-        }
-        __syncthreads();
-        const uint64_t item = base + tid;
-        if (item < total) {
-            int64_t t;
-            uint64_t l;
-            float tv[9];
-            if (staged) {
-                int a = 0, b = (int)nt;
-                while (b - a > 1) {
-                    const int m = (a + b) >> 1;
-                    if (s_off[m] <= item) a = m; else b = m;
-                }
-                t = t0 + a;
-                l = item - s_off[a];
-#pragma unroll
-                for (int c = 0; c < 9; ++c) tv[c] = s_tv[a * 9 + c];
-            } else {
-                t = find_segment(off, T, item);
-                l = item - off[t];
-#pragma unroll
-                for (int c = 0; c < 9; ++c) tv[c] = tris[t * 9 + c];
-            }
-            body(t, l, tv);
-        }
-        __syncthreads();
-        after(base + XB >= b1);
-    }
 }
 
 // which item range [so, so + P) of the wave's lanes holds item l0 + lane (ranges
@@ -947,7 +790,7 @@ __global__ __launch_bounds__(256) void k_sat_expand(const float* __restrict__ tr
         const int zf = z0 + zb;   // the layer of bit 0
         zb += 64;
         pending = __any(zb < sc.bm);
-        const bool emit = !pending && zmax >= 0 && vis;
+        const bool emit = !pending && zmax >= 0 && vis && g.n2 > 0;   // only the Level2 parity reads them
         // what the block's waves append this round
         const uint32_t cnt = (uint32_t)__popcll(hit);
         const uint32_t incl = wave_incl_scan<uint32_t>(cnt);
@@ -1034,115 +877,160 @@ void launch_pack_bytes(const uint8_t* by, int64_t W, uint64_t* bits, uint32_t* c
 }
 
 // Level1 ray parity, first half: one item = (triangle, column inside its
-// conservative bound); the exact det/u/v test keeps the (column, triangle)
-// pairs whose ray the reference's MT accepts at some height.
-template <bool kM, int XCAP>
-__global__ __launch_bounds__(expand_threads<kM>()) void k_ray_expand(const float* __restrict__ tris, int64_t T,
-                                                   const int4* __restrict__ rng,
-                                                   const uint64_t* __restrict__ off, GridDev g0, Meshes M,
-                                                   Append64 hits)
+// conservative bound), one lane per item.  Where the reference's ray test accepts
+// the column (det, u, v), the layers that pass are those below one crossing up to
+// rounding (par_l1_layers): a lane XORs one bit into the inside plane at
+// the layer under the crossing, and where the bounds leave layers undecided runs the
+// float t test on them and XORs a bit at each change.  k_l1_fill makes the parity of
+// the toggles above a layer.
+//
+// A wave owns a run of items and walks it 64 at a time over a window of 64
+// triangles; waves share nothing.  What bounds it: the latency of a
+// round's dependent loads (offsets, triangle, origins), hence all waves the chip
+// holds; the atomics are one per crossing.
+template <bool kM>
+__global__ __launch_bounds__(256) void k_ray_expand(const float* __restrict__ tris, int64_t T,
+                                                    const int4* __restrict__ rng, const uint64_t* __restrict__ off,
+                                                    GridDev g0, Meshes M, unsigned long long* __restrict__ ins)
 {
-    constexpr uint32_t HB = 1024;
-    __shared__ uint64_t s_hk[HB];
-    __shared__ uint32_t s_n;
-    __shared__ uint64_t s_gbase;
-    if (threadIdx.x == 0) s_n = 0;
-    __syncthreads();
-    const LdsAppend lh{s_hk, nullptr, &s_n, HB};
-    expand_items<expand_threads<kM>(), XCAP>(tris, T, off, [&](int64_t t, uint64_t l, const float* tv) {
+    __shared__ uint8_t s_win[4][64];
+    const int lane = __lane_id(), wid = threadIdx.x >> 6;
+    const uint64_t total = off[T];
+    const uint32_t nb = gridDim.x;   // a multiple of 8
+    const uint64_t per = ((total + 4ull * nb - 1) / (4ull * nb) + 63) / 64 * 64;
+    // the blocks of one XCD take one contiguous run of ranges
+    uint64_t base = ((uint64_t)((blockIdx.x % 8u) * (nb / 8u) + blockIdx.x / 8u) * 4u + (uint64_t)wid) * per;
+    if (base >= total) return;
+    const uint64_t b1 = base + per < total ? base + per : total;
+    int64_t t0 = wave_find_segment(off, 0, T, base);
+    while (base < b1) {
+        uint64_t so, eo;
+        uint32_t n;
+        for (;;) {
+            const int64_t tl = t0 + lane < T ? t0 + lane : T;
+            so = off[tl];
+            eo = off[tl + 1 < T ? tl + 1 : T];
+            const uint64_t wend = shfl64(eo, 63);
+            const uint64_t left = (wend < b1 ? wend : b1) - base;
+            n = left < 64 ? (uint32_t)left : 64u;
+            if (n) break;
+            t0 = wave_find_segment(off, t0 + 64, T, base);   // 64 triangles without items
+        }
+        const uint64_t from = so > base ? so : base;
+        const uint32_t P = eo > from ? (uint32_t)(eo - from < 64 ? eo - from : 64) : 0u;
+        const uint32_t rel = from - base < 64 ? (uint32_t)(from - base) : 64u;
+        const int o = wave_item_owner(s_win[wid], rel, P, 0);
+        const uint32_t l = (uint32_t)base + (uint32_t)lane - (uint32_t)__shfl((int)(uint32_t)so, o);
+        const uint32_t t = (uint32_t)(t0 + o);
+        // the triangles that end here are done
+        t0 += __popcll(__ballot(eo <= base + n));
+        base += n;
+        if ((uint32_t)lane >= n) continue;
         const int mesh = kM ? (int)M.tri_mesh[t] : 0;
         const GridDev& g = grid_of<kM>(g0, M, mesh);
-        const uint32_t col0 = kM ? M.off[mesh].col0 : 0;
         const int4 r = rng[t];
-        const int i = r.x + (int)(l % (uint64_t)r.z);
-        const int j = r.y + (int)(l / (uint64_t)r.z);
+        float tv[9];
+#pragma unroll
+        for (int c = 0; c < 9; ++c) tv[c] = tris[(uint64_t)t * 9 + c];
+        const uint32_t jq = l / (uint32_t)r.z;
+        const int i = r.x + (int)(l - jq * (uint32_t)r.z), j = r.y + (int)jq;
         MtTri m;
-        bool ok = mt_setup(tv, m);
         float tx, ty;
-        ok = ok && mt_column(m, tv[0], tv[1], g.r1x[i], g.r1y[j], tx, ty);
-        lds_append(lh, hits, ok, ((uint64_t)(col0 + (uint32_t)j * g.nx + i) << 32) | (uint64_t)t, 0);
-    }, [&](bool last) {
-        __syncthreads();
-        if (last || s_n >= HB / 2) lds_flush(lh, hits, &s_gbase);
-    });
-}
-
-template <int XC>
-static void launch_ray_expand_x(const float* tris, int64_t T, const int4* ray_rng, const uint64_t* off,
-                                const GridDev& g0, const Meshes& M, Append64 hits, int blocks, hipStream_t s)
-{
-    if (M.nm > 1)
-        k_ray_expand<true, XC><<<blocks, expand_threads<true>(), 0, s>>>(tris, T, ray_rng, off, g0, M, hits);
-    else
-        k_ray_expand<false, XC><<<blocks, expand_threads<false>(), 0, s>>>(tris, T, ray_rng, off, g0, M, hits);
+        if (!mt_setup(tv, m) || !mt_column(m, tv[0], tv[1], g.r1x[i], g.r1y[j], tx, ty)) continue;
+        // u and v as mt_column has them
+        const float px = 0.0f * m.e2z - m.e2y, py = m.e2x - 0.0f * m.e2z;
+        const float u = (tx * px + ty * py) * m.inv_det, v = (tx * m.e1y - ty * m.e1x) * m.inv_det;
+        int la, lb;
+        par_l1_layers(g.r1z, g.nz, g.bminz, (float)g.nz / (g.bmaxz - g.bminz), tv[2], m.e1z, m.e2z, u, v,
+                      par_ez(m.e1x, m.e1y, m.e1z, m.e2x, m.e2y, m.e2z, m.inv_det), la, lb);
+        const uint64_t plane = (uint64_t)g.ny * g.nxw;
+        unsigned long long* word = ins + (kM ? M.off[mesh].word0 : 0) + (uint64_t)j * g.nxw + (uint32_t)i / 64u;
+        const unsigned long long bit = 1ull << (i & 63);
+        bool in = la > 0;
+        for (int k = la; k < lb; ++k) {
+            const bool hit = mt_t_hit(m.e1x, m.e1y, m.e1z, m.e2x, m.e2y, m.e2z, m.inv_det, tx, ty, tv[2], g.r1z[k]);
+            if (hit != in && k > 0) atomicXor(&word[(uint64_t)(k - 1) * plane], bit);
+            in = hit;
+        }
+        if (in) atomicXor(&word[(uint64_t)(lb - 1) * plane], bit);
+    }
 }
 
 void launch_ray_expand(const float* tris, int64_t T, const int4* ray_rng, const uint64_t* off, const GridDev& g0,
-                       const Meshes& M, Append64 hits, int blocks, int stage, hipStream_t s)
+                       const Meshes& M, uint64_t* ins, int blocks, hipStream_t s)
 {
     if (T <= 0) return;
-    if (stage <= 128)
-        launch_ray_expand_x<128>(tris, T, ray_rng, off, g0, M, hits, blocks, s);
+    unsigned long long* w = reinterpret_cast<unsigned long long*>(ins);
+    // as many blocks as the Level1 SAT's launch: a wave to eight triangles
+    const int64_t want = T / 32 > 512 ? T / 32 : 512;
+    const int64_t cap = blocks < 2048 ? blocks : 2048;
+    const unsigned nb = (unsigned)(((want < cap ? want : cap) + 7) / 8 * 8);
+    if (M.nm > 1)
+        k_ray_expand<true><<<nb, 256, 0, s>>>(tris, T, ray_rng, off, g0, M, w);
     else
-        launch_ray_expand_x<256>(tris, T, ray_rng, off, g0, M, hits, blocks, s);
+        k_ray_expand<false><<<nb, 256, 0, s>>>(tris, T, ray_rng, off, g0, M, w);
+}
+
+// Level1 ray parity, second half: the toggles of a (row word, layer) XORed over the
+// layers from the top down, in place.  A block takes L1F_W words of a mesh's layer
+// (a cache line) in 64 segments of layers: a pass for each segment's XOR, a second (from
+// the cache) to write.  Bound by the plane's read and write; the segments
+// keep enough loads in flight where a layer has few words.
+constexpr int L1F_U = 8;
+template <bool kM>
+__global__ __launch_bounds__(1024) void k_l1_fill(GridDev g0, Meshes M, uint64_t* __restrict__ ins)
+{
+    __shared__ uint64_t s_x[16][L1F_W];
+    const int lane = __lane_id(), wid = uniform_i(threadIdx.x >> 6);
+    const int mesh = kM ? wave_mesh_search(M.off, M.nm, (uint64_t)blockIdx.x, [](const MeshOff& o) { return (uint64_t)o.ptask0; }) : 0;
+    const GridDev& g = grid_of<kM>(g0, M, mesh);
+    if (g.l1st) return;   // the stencil fill writes this mesh's inside bits
+    const int64_t plane = (int64_t)g.ny * g.nxw;
+    const int64_t w = (int64_t)(blockIdx.x - (kM ? M.off[mesh].ptask0 : 0u)) * L1F_W + (lane & (L1F_W - 1));
+    uint64_t* p = ins + (kM ? M.off[mesh].word0 : 0) + w;
+    const int len = (g.nz + 63) / 64;
+    const int z0 = w < plane ? (wid * 4 + lane / L1F_W) * len : g.nz, z1 = z0 + len < g.nz ? z0 + len : g.nz;
+    uint64_t own = 0;
+    for (int z = z0; z < z1; z += L1F_U) {
+        uint64_t v[L1F_U];
+#pragma unroll
+        for (int k = 0; k < L1F_U; ++k) v[k] = z + k < z1 ? p[(z + k) * plane] : 0ull;
+#pragma unroll
+        for (int k = 0; k < L1F_U; ++k) own ^= v[k];
+    }
+    // the segments from the lane's own up to the wave's last, then the later waves'
+    const uint64_t a = shfl64(own, (lane + 16) & 63);
+    uint64_t acc = own ^ (lane < 48 ? a : 0ull);
+    const uint64_t b = shfl64(acc, (lane + 32) & 63);
+    acc ^= lane < 32 ? b : 0ull;
+    if (lane < L1F_W) s_x[wid][lane] = acc;
+    __syncthreads();
+    acc ^= own;
+    for (int k = wid + 1; k < 16; ++k) acc ^= s_x[k][lane & (L1F_W - 1)];
+    for (int z = z1; z > z0; z -= L1F_U) {
+        uint64_t v[L1F_U];
+#pragma unroll
+        for (int k = 0; k < L1F_U; ++k) v[k] = z - 1 - k >= z0 ? p[(z - 1 - k) * plane] : 0ull;
+#pragma unroll
+        for (int k = 0; k < L1F_U; ++k) {
+            acc ^= v[k];
+            if (z - 1 - k >= z0) p[(z - 1 - k) * plane] = acc;
+        }
+    }
+}
+
+void launch_l1_fill(const GridDev& g0, const Meshes& M, int64_t blocks, uint64_t* ins, hipStream_t s)
+{
+    if (blocks <= 0) return;
+    if (M.nm > 1)
+        k_l1_fill<true><<<(unsigned)blocks, 1024, 0, s>>>(g0, M, ins);
+    else
+        k_l1_fill<false><<<(unsigned)blocks, 1024, 0, s>>>(g0, M, ins);
 }
 
 // ---------------------------------------------------------------------------
 // counting sorts by the high 32 bits of a key
 // ---------------------------------------------------------------------------
-__global__ void k_count_keys_hi(const uint64_t* __restrict__ key, uint64_t n, uint32_t* __restrict__ cnt)
-{
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (uint64_t)gridDim.x * blockDim.x)
-        atomicAdd(&cnt[key[i] >> 32], 1u);
-}
-
-void launch_count_keys_hi(const uint64_t* key, uint64_t n,
-                          uint32_t* cnt, hipStream_t s)
-{
-    if (!n) return;
-    k_count_keys_hi<<<grid_for((int64_t)n, 256, 16384), 256, 0, s>>>(key, n, cnt);
-}
-
-template <bool kM>
-__global__ void k_scatter_hits(const float* __restrict__ tris, const uint64_t* __restrict__ key, uint64_t n,
-                               GridDev g0, Meshes M, const uint32_t* __restrict__ off, uint32_t* __restrict__ cnt,
-                               float4* __restrict__ rec)
-{
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (uint64_t)gridDim.x * blockDim.x) {
-        const uint64_t k = key[i];
-        const uint32_t gcol = (uint32_t)(k >> 32);
-        const uint32_t t = (uint32_t)(k & 0xffffffffu);
-        const uint32_t pos = off[gcol] + atomicSub(&cnt[gcol], 1u) - 1u;
-        const int mesh = kM ? (int)M.tri_mesh[t] : 0;
-        const GridDev& g = grid_of<kM>(g0, M, mesh);
-        const uint32_t col = gcol - (kM ? M.off[mesh].col0 : 0u);
-        float tv[9];
-#pragma unroll
-        for (int c = 0; c < 9; ++c) tv[c] = tris[(uint64_t)t * 9 + c];
-        MtTri m;
-        mt_setup(tv, m);
-        const int i1 = (int)(col % (uint32_t)g.nx), j1 = (int)(col / (uint32_t)g.nx);
-        const float tx = g.r1x[i1] - tv[0];
-        const float ty = g.r1y[j1] - tv[1];
-        rec[3 * (uint64_t)pos + 0] = make_float4(m.e1x, m.e1y, m.e1z, m.e2x);
-        rec[3 * (uint64_t)pos + 1] = make_float4(m.e2y, m.e2z, m.inv_det, tx);
-        rec[3 * (uint64_t)pos + 2] = make_float4(ty, tv[2], 0.0f, 0.0f);
-    }
-}
-
-void launch_scatter_hits(const float* tris, const uint64_t* key, uint64_t n, const GridDev& g0, const Meshes& M,
-                         const uint32_t* off, uint32_t* cnt, float4* rec, hipStream_t s)
-{
-    if (!n) return;
-    const int blocks = grid_for((int64_t)n, 256, 16384);
-    if (M.nm > 1)
-        k_scatter_hits<true><<<blocks, 256, 0, s>>>(tris, key, n, g0, M, off, cnt, rec);
-    else
-        k_scatter_hits<false><<<blocks, 256, 0, s>>>(tris, key, n, g0, M, off, cnt, rec);
-}
-
 // column entries -> CSR by column of (triangle, zmax); the Level2 parity, which
 // reads each once, makes the triangle's Moller-Trumbore record itself
 struct ColItem {
@@ -1172,70 +1060,6 @@ struct ColPlace {
         if (ok) ent[pos] = make_uint2(it.t, it.zmax);
     }
 };
-
-// ---------------------------------------------------------------------------
-// Level1 parity: one wave per task = L1P_Z consecutive layers of a 64-column
-// strip of one row; each lane loads its column's accepted (triangle, column)
-// records once and XORs t > 1e-6 over them at each of the task's layers.
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ int wave_mesh_of_task(const MeshOff* __restrict__ off, int nm, uint64_t task)
-{
-    return wave_mesh_search(off, nm, task, [](const MeshOff& o) { return (uint64_t)o.ptask0; });
-}
-
-template <bool kM>
-__global__ __launch_bounds__(256) void k_l1_parity(const float4* __restrict__ rec,
-                                                   const uint32_t* __restrict__ hoff, GridDev g0, Meshes M,
-                                                   uint64_t* __restrict__ ins, int64_t NT)
-{
-    const int64_t task = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    if (task >= NT) return;
-    const int lane = __lane_id();
-    const int mesh = kM ? wave_mesh_of_task(M.off, M.nm, (uint64_t)task) : 0;
-    const GridDev& g = grid_of<kM>(g0, M, mesh);
-    if (g.l1st) return;   // the stencil fill writes this mesh's inside bits
-    const int64_t tl = task - (int64_t)(kM ? M.off[mesh].ptask0 : 0);
-    const uint64_t word0 = kM ? M.off[mesh].word0 : 0;
-    const uint32_t col0 = kM ? M.off[mesh].col0 : 0;
-    const int nxw = g.nxw, ny = g.ny, nx = g.nx, nz = g.nz;
-    const int xw = (int)(tl % nxw);
-    const int64_t rowt = tl / nxw;
-    const int j = (int)(rowt % ny);
-    const int z0 = (int)(rowt / ny) * L1P_Z;
-    const int nzc = nz - z0 < L1P_Z ? nz - z0 : L1P_Z;
-    float oz[L1P_Z];
-#pragma unroll
-    for (int k = 0; k < L1P_Z; ++k) oz[k] = k < nzc ? g.r1z[z0 + k] : 0.0f;
-    const int x = xw * 64 + lane;
-    uint32_t par = 0;   // bit k: parity at layer z0 + k
-    if (x < nx) {
-        const uint32_t c = col0 + (uint32_t)j * nx + x;
-        const uint32_t h1 = hoff[c + 1];
-        for (uint32_t h = hoff[c]; h < h1; ++h) {
-            const float4 a = rec[3 * (uint64_t)h + 0];
-            const float4 b = rec[3 * (uint64_t)h + 1];
-            const float4 d = rec[3 * (uint64_t)h + 2];
-#pragma unroll
-            for (int k = 0; k < L1P_Z; ++k)
-                if (k < nzc) par ^= (uint32_t)mt_t_hit(a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w, d.x, d.y, oz[k]) << k;
-        }
-    }
-    for (int k = 0; k < nzc; ++k) {
-        const uint64_t m = __ballot((par >> k) & 1u);
-        if (lane == 0) ins[word0 + ((uint64_t)(z0 + k) * ny + j) * nxw + xw] = m;
-    }
-}
-
-void launch_l1_parity(const float4* rec, const uint32_t* hoff, const GridDev& g0, const Meshes& M, int64_t NT,
-                      uint64_t* ins, hipStream_t s)
-{
-    if (NT <= 0) return;
-    const int64_t blocks = (NT * 64 + 255) / 256;
-    if (M.nm > 1)
-        k_l1_parity<true><<<(unsigned)blocks, 256, 0, s>>>(rec, hoff, g0, M, ins, NT);
-    else
-        k_l1_parity<false><<<(unsigned)blocks, 256, 0, s>>>(rec, hoff, g0, M, ins, NT);
-}
 
 // ---------------------------------------------------------------------------
 // a batch's device soups gathered into the batch's soup in one launch (one

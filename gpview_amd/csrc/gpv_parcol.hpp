@@ -1,4 +1,4 @@
-// gpv_parcol.hpp -- the Level2 ray parity by crossings instead of voxel by voxel.
+// gpv_parcol.hpp -- the ray parities by crossings instead of voxel by voxel.
 //
 // For the +z ray of a sub-column (x, y) the Moller-Trumbore test of one column
 // entry (triangle) accepts or rejects by det/u/v, which do not depend on the
@@ -157,6 +157,25 @@ __host__ __device__ __forceinline__ void par_layers(const ParEntry& r, float u, 
     lb = r.l0 + (int)fmaxf(b, -1.0e8f);
     la = la < 0 ? 0 : la > cap ? cap : la;
     lb = lb < 0 ? 0 : lb > cap ? cap : lb;
+}
+
+// Level1: the same crossing against the layers of a grid's column.  Layers [0, la)
+// of the ray-origin table r1z (nz, non-decreasing) pass for certain, none from
+// lb on.  The layers are compared as the float test's own T.z = fl(o.z - v1.z), so
+// only the crossing's height over v1 is rounded: Ez twice over covers that.
+// The estimate from the table's ends (zmin, inv_g = layers per z unit) only says where the search begins.
+__host__ __device__ __forceinline__ void par_l1_layers(const float* r1z, int nz, float zmin, float inv_g, float v1z,
+                                                       float e1z, float e2z, float u, float v, float ez, int& la, int& lb)
+{
+    const float zc = (u * e1z + v * e2z) - 1.0e-6f;
+    const float lo = zc - 2.0f * ez, hi = zc + 2.0f * ez;
+    // a NaN starts at 0
+    int k = (int)fminf(fmaxf(((lo + v1z) - zmin) * inv_g + 0.5f, 0.0f), (float)nz);
+    while (k < nz && r1z[k] - v1z < lo) ++k;
+    while (k > 0 && !(r1z[k - 1] - v1z < lo)) --k;
+    la = k;
+    while (k < nz && !(r1z[k] - v1z > hi)) ++k;
+    lb = k;
 }
 
 }  // namespace gpv

@@ -283,9 +283,7 @@ struct Job {
     uint64_t* col_key = nullptr;
     uint32_t* col_z = nullptr;
     uint64_t col_cap = 0;
-    uint64_t* hit_key = nullptr;
-    uint64_t hit_cap = 0;
-    uint64_t n_pairs = 0, n_cols = 0, n_hits = 0;
+    uint64_t n_pairs = 0, n_cols = 0;
     int regrows = 0;
     // compaction and bins
     uint32_t *wcnt = nullptr, *wprefix = nullptr;
@@ -293,7 +291,7 @@ struct Job {
     int64_t B = 0, W2 = 0;
     uint32_t *boff = nullptr, *list = nullptr;
     uint32_t* coff = nullptr;
-    uint32_t* scan_side = nullptr;   // scan temporary of the parity fill (it may run beside compaction)
+    uint32_t* scan_side = nullptr;   // its scan temporary on the side stream (beside the bins)
     uint2* cent = nullptr;    // (triangle, zmax) of the column entries
     // column-entry sort on the side stream (beside the bins): its own scratch
     bool cols_side = false;
@@ -301,8 +299,6 @@ struct Job {
     uint32_t* cs_bucket = nullptr;   // 3 words per column entry
     int64_t l2p_waves = 0, l2s_groups = 0;   // Level2 parity waves, SAT groups (l2_plan)
     int l2s_most = 1;                        // most voxels of a SAT group
-    uint32_t *hcnt = nullptr, *hoff = nullptr;
-    float4* hrec = nullptr;
     // GL-stencil-equivalent Level1 fill (meshes with params.l1_stencil):
     // per-triangle sample counts and offsets, and the slice toggle planes
     bool any_stencil = false, all_stencil = false, stencil_done = false;
@@ -320,11 +316,10 @@ struct Job {
     // progress
     bool setup_done = false, sat_done = false, inout_done = false, compact_done = false,
          l2p_done = false, l2s_done = false, finished = false;
-    // stream events: 0 setup, 1 L1 SAT, 2 ray expansion, 3 parity fill,
+    // stream events: 0 setup, 1 L1 SAT, 2 L1 parity, 3 fork of the Level2 side stream,
     // 4 compaction+bins, 5 L2 parity, 6 L2 SAT start, 7 L2 SAT end, 8 finish,
     // 9 normals start, 10 normals end, 11 L2 parity end, 12 L1 SAT end,
-    // 13 ray expansion end, 14 parity fill end, 15 fork of the ray expansion
-    // 16 L2 parity start
+    // 13 L1 parity end, 15 fork of the L1 parity, 16 L2 parity start
     hipEvent_t ev[kJobEvents] = {};
     std::vector<void*> bufs;
     // gpv_voxelize_noalloc: buffers are carved from the device scratch array
@@ -580,7 +575,7 @@ int job_create(gpv_ctx* c, const gpv_mesh_desc* d, int nm, int on_device, Job** 
     if (nm < 1) return fail(GPV_ERR_INVALID, "a batch needs at least one mesh");
     std::vector<gpv_grid_info> info((size_t)nm);
     int64_t T = 0, W = 0, ncol = 0, vox = 0;
-    uint64_t pair_cap = 0, hit_cap = 0;
+    uint64_t pair_cap = 0;
     for (int m = 0; m < nm; ++m) {
         if (d[m].ntris < 0 || (d[m].ntris > 0 && !d[m].tris))
             return fail(GPV_ERR_INVALID, "mesh %d: bad triangle soup", m);
@@ -601,7 +596,6 @@ int job_create(gpv_ctx* c, const gpv_mesh_desc* d, int nm, int on_device, Job** 
                                ? d[m].params.initial_capacity
                                : std::max<int64_t>(int64_t(1) << 16, 16 * d[m].ntris + 8 * nmax * nmax);
         pair_cap += (uint64_t)pc;
-        hit_cap += (uint64_t)(8 * d[m].ntris + 4 * nx * ny);
     }
     if (T >= (int64_t(1) << 31)) return fail(GPV_ERR_INVALID, "at most 2^31-1 triangles per batch");
     if (ncol > (int64_t(1) << 27)) return fail(GPV_ERR_INVALID, "at most 2^27 xy columns per batch");
@@ -629,10 +623,9 @@ int job_create(gpv_ctx* c, const gpv_mesh_desc* d, int nm, int on_device, Job** 
         J->out_bidx = na->bidx;
         J->out_sat2 = na->l2b;
         J->out_par2 = na->l2i;
-        // bin and hit buffers within a quarter and a sixteenth of the arena;
-        // a larger count regrows (from what is left) like any other run
+        // bin buffers within a quarter of the arena; a larger count regrows
+        // (from what is left) like any other run
         pair_cap = std::min<uint64_t>(pair_cap, na->arena_cap / 4 / 24);
-        hit_cap = std::min<uint64_t>(hit_cap, na->arena_cap / 16 / 8);
     }
     J->ctx = c;
     J->nm = nm;
@@ -688,7 +681,7 @@ int job_create(gpv_ctx* c, const gpv_mesh_desc* d, int nm, int on_device, Job** 
         J->off[m].ptask0 = ptask0;
         J->off[m].pw0 = (uint32_t)pw0;
         pw0 += l2_parity_waves(g.n2, (int64_t)g.nx * g.ny, ncol >= kL2ParityMany);
-        ptask0 += (uint32_t)l1_parity_tasks(g);
+        ptask0 += (uint32_t)l1_fill_blocks(g);
         word0 += (uint64_t)g.nz * g.ny * g.nxw;
         col0 += (uint32_t)(g.nx * g.ny);
         tri0 += (uint32_t)d[m].ntris;
@@ -818,10 +811,8 @@ int job_create(gpv_ctx* c, const gpv_mesh_desc* d, int nm, int on_device, Job** 
     }
     J->pair_cap = pair_cap;
     J->col_cap = J->pair_cap;
-    J->hit_cap = std::max<uint64_t>(hit_cap, 1u << 16);
     if ((r = alloc(J, &J->pair_key, J->pair_cap)) || (r = alloc(J, &J->pair_tri, J->pair_cap)) ||
-        (r = alloc(J, &J->col_key, J->col_cap)) || (r = alloc(J, &J->col_z, J->col_cap)) ||
-        (r = alloc(J, &J->hit_key, J->hit_cap)))
+        (r = alloc(J, &J->col_key, J->col_cap)) || (r = alloc(J, &J->col_z, J->col_cap)))
         return bail(r);
     if (J->any_stencil) {
         // the stencil fill's scratch: one set for the stencil meshes in turn
@@ -917,29 +908,21 @@ int launch_sat_half(Job* J)
 
 int launch_stencil(Job* J, hipStream_t s);
 
-// Level1 ray expansion on stream s (allocates nothing)
+// Level1 parity on stream s (allocates nothing): the rays' toggles, then the fill
 int launch_ray_half(Job* J, hipStream_t s)
 {
     gpv_ctx* c = J->ctx;
     HIP_TRY(hipEventRecord(J->ev[2], s));
-    if (J->all_stencil) {
-        // no ray parity, hence no hits (the counter is cleared on the stream
-        // of the count read-back): the stencil fill takes the ray half's place
-        launch_fill_u64(reinterpret_cast<uint64_t*>(&J->ctr->hits), 0, 1, J->ctx->stream);
-        TRY(launch_stencil(J, s));
-        HIP_TRY(hipEventRecord(J->ev[13], s));
-        return GPV_OK;
+    if (!J->all_stencil) {   // the ray parity skips the stencil meshes
+        launch_fill_u64(J->ins, 0, J->W, s);
+        launch_ray_expand(J->tris, J->T, J->rng, J->ray_off, J->g[0], J->view(), J->ins, expand_blocks(c), s);
+        launch_l1_fill(J->g[0], J->view(), (int64_t)J->off[J->nm].ptask0, J->ins, s);
     }
-    launch_fill_u64(reinterpret_cast<uint64_t*>(&J->ctr->hits), 0, 1, s);
-    Append64 hi{&J->ctr->hits, J->hit_key, nullptr, J->hit_cap};
-    launch_ray_expand(J->tris, J->T, J->rng, J->ray_off, J->g[0], J->view(), hi, expand_blocks(c),
-                      c->tune.expand_stage_tris, s);
+    TRY(launch_stencil(J, s));
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipEventRecord(J->ev[13], s));
     return GPV_OK;
 }
-
-int launch_ray_half(Job* J) { return launch_ray_half(J, J->ctx->stream); }
 
 // one round trip: the counters and, when asked, the boundary offsets
 int read_counts(Job* J, bool with_b)
@@ -1014,35 +997,6 @@ int complete_sat(Job* J, int64_t* needed)
     return GPV_OK;
 }
 
-// after read_counts: false (and a regrown buffer) when the hits overflowed
-int complete_ray(Job* J, bool* ok)
-{
-    const uint64_t nh = hctr(J).hits;
-    *ok = nh <= J->hit_cap && nh < (uint64_t(1) << 32);
-    if (*ok) {
-        J->n_hits = nh;
-        return GPV_OK;
-    }
-    if (nh >= (uint64_t(1) << 32)) return fail(GPV_ERR_CAPACITY, "more than 2^32-1 ray hits; split the batch");
-    release(J, J->hit_key);
-    J->hit_cap = nh + nh / 8 + 1024;
-    return alloc(J, &J->hit_key, J->hit_cap);
-}
-
-// hits grouped by column, then the parity of every Level1 voxel
-// buffers of the parity fill (allocated before it may fork onto the side stream)
-int alloc_parity(Job* J)
-{
-    release(J, J->hcnt);
-    release(J, J->hoff);
-    release(J, J->hrec);
-    release(J, J->scan_side);
-    TRY(alloc(J, &J->hcnt, (size_t)J->ncol));
-    TRY(alloc(J, &J->hoff, (size_t)J->ncol + 1));
-    TRY(alloc(J, &J->hrec, (size_t)std::max<uint64_t>(J->n_hits, 1) * 3));
-    return alloc(J, &J->scan_side, scan_tmp_elems(J->ncol));
-}
-
 // the GL-stencil-equivalent Level1 fill of every mesh that asks for it, on
 // stream s: it reads only the soup and the grid, so the fused pipeline runs
 // it beside the Level1 SAT; it writes the inside bits of those meshes,
@@ -1067,47 +1021,22 @@ int alloc_cols(Job* J)
     release(J, J->cent);
     release(J, J->cs_cnt);
     release(J, J->cs_bucket);
+    release(J, J->scan_side);
+    TRY(alloc(J, &J->scan_side, scan_tmp_elems((int64_t)ts_tiles((uint64_t)J->ncol))));
     TRY(alloc(J, &J->coff, (size_t)J->ncol + 1));
     TRY(alloc(J, &J->cent, (size_t)std::max<uint64_t>(J->n_cols, 1)));
     TRY(alloc(J, &J->cs_cnt, 3 * ts_tiles((uint64_t)J->ncol) + 2));
     return alloc(J, &J->cs_bucket, 3 * (size_t)std::max<uint64_t>(J->n_cols, 1));
 }
 
-// column entries by column, on stream s; scan is a
-// scan temporary of at least scan_tmp_elems(ncol) that no other stream uses
-int col_sort_kernels(Job* J, hipStream_t s, uint32_t* scan)
+// column entries by column, on stream s
+int col_sort_kernels(Job* J, hipStream_t s)
 {
     const size_t tiles = ts_tiles((uint64_t)J->ncol);
-    const TileSortTmp ts{J->cs_cnt, J->cs_cnt + 2 * tiles + 1, scan, J->cs_bucket};
+    const TileSortTmp ts{J->cs_cnt, J->cs_cnt + 2 * tiles + 1, J->scan_side, J->cs_bucket};
     const int ipb = std::max(256, J->ctx->tune.sort_items_per_block);
     launch_bin_cols(J->col_key, J->col_z, J->n_cols, (uint32_t)J->ncol, ts, ipb, J->coff, J->cent, s);
     HIP_TRY(hipGetLastError());
-    return GPV_OK;
-}
-
-// the parity fill on stream s: hits by column, their MT records, the fill
-int parity_kernels(Job* J, hipStream_t s)
-{
-    if (!J->all_stencil) {   // the ray parity skips the stencil meshes
-        launch_fill_u32(J->hcnt, 0, J->ncol, s);
-        launch_count_keys_hi(J->hit_key, J->n_hits, J->hcnt, s);
-        launch_scan_u32_u32(J->hcnt, J->hoff, J->ncol, J->scan_side, nullptr, s);
-        launch_scatter_hits(J->tris, J->hit_key, J->n_hits, J->g[0], J->view(), J->hoff, J->hcnt, J->hrec, s);
-        launch_l1_parity(J->hrec, J->hoff, J->g[0], J->view(), (int64_t)J->off[J->nm].ptask0, J->ins, s);
-    }
-    TRY(launch_stencil(J, s));   // already launched beside the Level1 SAT in the fused pipeline
-    HIP_TRY(hipGetLastError());
-    HIP_TRY(hipEventRecord(J->ev[14], s));
-    return GPV_OK;
-}
-
-int launch_parity(Job* J)
-{
-    hipStream_t s = J->ctx->stream;
-    HIP_TRY(hipEventRecord(J->ev[3], s));
-    TRY(alloc_parity(J));
-    TRY(parity_kernels(J, s));
-    J->inout_done = true;
     return GPV_OK;
 }
 
@@ -1151,14 +1080,15 @@ int launch_compact(Job* J)
     TRY(alloc(J, &J->list, (size_t)std::max<uint64_t>(J->n_pairs, 1)));
     // one scratch for both counting sorts (bins by boundary rank, column
     // entries by column)
-    const size_t tiles = J->cols_side ? ts_tiles((uint64_t)J->B)
+    const bool cols = J->n2max > 0 && !J->cols_side;   // only the Level2 parity reads them
+    const size_t tiles = !cols ? ts_tiles((uint64_t)J->B)
                                       : std::max(ts_tiles((uint64_t)J->B), ts_tiles((uint64_t)J->ncol));
     TileSortTmp ts{};
     uint32_t* ts_cnt = nullptr;
     uint32_t* ts_bucket = nullptr;
     TRY(alloc(J, &ts_cnt, 3 * tiles + 2));
     TRY(alloc(J, &ts_bucket,
-              (size_t)std::max<uint64_t>(J->cols_side ? 2 * J->n_pairs : std::max(2 * J->n_pairs, 3 * J->n_cols), 1)));
+              (size_t)std::max<uint64_t>(!cols ? 2 * J->n_pairs : std::max(2 * J->n_pairs, 3 * J->n_cols), 1)));
     TRY(ensure_scan_tmp(J, (int64_t)tiles));
     ts.total = ts_cnt;
     ts.off = ts_cnt + 2 * tiles + 1;
@@ -1169,7 +1099,7 @@ int launch_compact(Job* J)
                      ipb, J->boff, J->nm > 1 ? nullptr : &J->mctr[0].max_per_voxel, J->list, s);
     J->pairs_ranked = true;
     if (J->nm > 1) launch_mesh_bins(J->boff, J->B, J->view(), s);
-    if (!J->cols_side) {
+    if (cols) {
         release(J, J->coff);
         release(J, J->cent);
         TRY(alloc(J, &J->coff, (size_t)J->ncol + 1));
@@ -1268,37 +1198,35 @@ int run_l2_sat(Job* J)
 }
 
 // The two streams of the fused pipeline after the read-back.  Main: the bins and
-// the Level2 SAT, which reads them.  Side: the column-entry sort and the Level2
-// parity, which reads its entries and the Level1 planes, then the Level1
-// parity fill, which nothing but the counts waits for.  Enqueued in the order in
-// which their kernels are due: the host takes longer over the side
-// stream's dozen launches than the main one over the bins.  Nothing is allocated
+// the Level2 SAT, which reads them.  Side, behind the Level1 parity: the column-entry
+// sort and the Level2 parity, which reads its entries and the boundary plane.
+// Enqueued in the order in which their kernels are due.  Nothing is allocated
 // or released between the fork and the join, so the pool's blocks stay in
 // one stream order.
 int run_streams(Job* J)
 {
     gpv_ctx* c = J->ctx;
     hipStream_t s = c->stream;
-    const bool l2 = J->n2max > 0;
-    TRY(alloc_parity(J));
-    J->cols_side = l2;
-    if (l2) TRY(alloc_cols(J));
-    TRY(alloc_level2(J));
-    if (l2) TRY(l2_plan(J));
-    HIP_TRY(hipEventRecord(J->ev[3], s));
-    TRY(launch_compact(J));
-    HIP_TRY(hipStreamWaitEvent(c->side, J->ev[3], 0));
-    if (l2) {
-        TRY(col_sort_kernels(J, c->side, J->scan_side));
+    J->cols_side = J->n2max > 0;
+    if (J->cols_side) {
+        TRY(alloc_cols(J));
+        TRY(alloc_level2(J));
+        TRY(l2_plan(J));
+        HIP_TRY(hipEventRecord(J->ev[3], s));
+        TRY(launch_compact(J));
+        HIP_TRY(hipStreamWaitEvent(c->side, J->ev[3], 0));
+        TRY(col_sort_kernels(J, c->side));
         HIP_TRY(hipEventRecord(J->ev[5], s));
         TRY(l2_sat_kernels(J));
         TRY(l2_parity_kernels(J, c->side));
         J->l2p_done = true;
         J->l2s_done = true;
+        HIP_TRY(hipStreamWaitEvent(s, J->ev[11], 0));
+    } else {
+        TRY(alloc_level2(J));
+        TRY(launch_compact(J));
+        HIP_TRY(hipStreamWaitEvent(s, J->ev[13], 0));
     }
-    TRY(parity_kernels(J, c->side));
-    J->inout_done = true;
-    HIP_TRY(hipStreamWaitEvent(s, J->ev[14], 0));   // the side stream's last
     release(J, J->cs_cnt);
     release(J, J->cs_bucket);
     return GPV_OK;
@@ -1347,12 +1275,10 @@ int job_finish(Job* J)
         }
         return v;
     };
-    // setup, L1 SAT (+ boundary scan), L1 parity (ray expansion + parity
-    // fill), compaction + bins, L2 parity, L2 SAT, each on its own stream;
+    // setup, L1 SAT (+ boundary scan), L1 parity (or stencil fill), compaction + bins, L2 parity, L2 SAT, each on its own stream;
     // stages on the side stream overlap the main one's.  For a batch these
     // are the batch's stage times
-    const bool side_l2 = J->cols_side;   // the parity fill followed the Level2 parity
-    float ms[6] = {el(0, 1), el(1, 12), el(2, 13) + el(side_l2 ? 11 : 3, 14), 0.0f, 0.0f, 0.0f};
+    float ms[6] = {el(0, 1), el(1, 12), el(2, 13), 0.0f, 0.0f, 0.0f};
     if (J->n2max > 0) {
         ms[3] = el(4, 5);
         ms[4] = el(16, 11);   // in the fused pipeline the two Level2 stages overlap
@@ -1384,10 +1310,10 @@ int job_finish(Job* J)
     release(J, J->sat_items); release(J, J->ray_items); release(J, J->sat_off); release(J, J->ray_off);
     release(J, J->scan64); J->scan32 = nullptr; J->scan_cap = 0; release(J, J->scan_ray);
     release(J, J->pair_key); release(J, J->pair_tri); release(J, J->col_key); release(J, J->col_z);
-    release(J, J->hit_key); release(J, J->wcnt); release(J, J->boff);
-    release(J, J->list); release(J, J->coff); release(J, J->cent); release(J, J->hcnt);
+    release(J, J->wcnt); release(J, J->boff);
+    release(J, J->list); release(J, J->coff); release(J, J->cent);
     release(J, J->cs_cnt); release(J, J->cs_bucket);
-    release(J, J->hoff); release(J, J->hrec); release(J, J->scan_side); release(J, J->tri_mesh);
+    release(J, J->scan_side); release(J, J->tri_mesh);
     release(J, J->st_cnt); release(J, J->st_off); release(J, J->st_scan); release(J, J->st_tog);
     release(J, J->bmesh);
     release(J, J->d_grids); release(J, J->d_off); release(J, J->own_soup); release(J, J->mctr);
@@ -1402,42 +1328,29 @@ int job_finish(Job* J)
 int job_run(Job* J)
 {
     gpv_ctx* c = J->ctx;
-    // independent stages go beside each other on the side stream: the ray
-    // expansion beside the Level1 SAT, then see run_streams.  Side-stream work allocates nothing and its buffers are
+    // independent stages go beside each other on the side stream: the Level1
+    // parity beside the Level1 SAT, then see run_streams.  Side-stream work allocates nothing and its buffers are
     // allocated before the fork and live until the join, so pool blocks keep
     // one stream order.
     const bool side = c->tune.l2_overlap != 0;
     if (side) {
         TRY(stage_setup_split(J));
         TRY(launch_ray_half(J, c->side));
-        TRY(launch_sat_half(J));
-        // the count read-back waits for the ray expansion's hits; in a batch
-        // that mixes the two fills the stencil follows it on the side stream,
-        // after that point (with only stencil meshes it has run in its place)
-        if (!J->all_stencil) HIP_TRY(hipStreamWaitEvent(c->stream, J->ev[13], 0));
-        TRY(launch_stencil(J, c->side));
     } else {
         TRY(stage_setup(J));
+        TRY(launch_ray_half(J, c->stream));
+    }
+    J->inout_done = true;
+    int64_t needed = 1;
+    for (int attempt = 0; attempt < 3 && needed > 0; ++attempt) {
         TRY(launch_sat_half(J));
-        TRY(launch_ray_half(J));
-    }
-    TRY(read_counts(J, true));
-    int64_t needed = 0;
-    bool ray_ok = false;
-    TRY(complete_sat(J, &needed));
-    TRY(complete_ray(J, &ray_ok));
-    for (int attempt = 0; attempt < 2 && (needed > 0 || !ray_ok); ++attempt) {
-        if (needed > 0) TRY(launch_sat_half(J));
-        if (!ray_ok) TRY(launch_ray_half(J));
         TRY(read_counts(J, true));
-        if (needed > 0) TRY(complete_sat(J, &needed));
-        if (!ray_ok) TRY(complete_ray(J, &ray_ok));
+        TRY(complete_sat(J, &needed));
     }
-    if (needed > 0 || !ray_ok) return fail(GPV_ERR_CAPACITY, "buffer capacity did not converge");
+    if (needed > 0) return fail(GPV_ERR_CAPACITY, "buffer capacity did not converge");
     if (side) {
         TRY(run_streams(J));
     } else {
-        TRY(launch_parity(J));
         TRY(alloc_level2(J));
         TRY(launch_compact(J));
         TRY(run_l2_parity(J));
@@ -1464,7 +1377,6 @@ int64_t predict_run_bytes(const gpv_mesh_desc& d, const gpv_grid_info& I)
     const int64_t nmax = std::max(nx, std::max(ny, nz));
     const int64_t P = d.params.initial_capacity > 0 ? d.params.initial_capacity
                                                     : std::max<int64_t>(int64_t(1) << 16, 16 * T + 8 * nmax * nmax);
-    const int64_t H = std::max<int64_t>(8 * T + 4 * ncol, int64_t(1) << 16);
     const int64_t B = std::min(n1, 4 * (nx * ny + ny * nz + nz * nx));
     auto scan = [](int64_t n) { return 8 * (int64_t)scan_tmp_elems(n); };
     int64_t b = 0;
@@ -1472,9 +1384,8 @@ int64_t predict_run_bytes(const gpv_mesh_desc& d, const gpv_grid_info& I)
     b += 36 * T + 4 * T + 4 * B + 4096;                          // soup copy, batch mesh ids, descriptors
     b += 72 * T + 16 + 2 * scan(std::max(T, W));               // per-triangle set-up, item scans
     b += 24 * W + 64 * W;                                        // planes, word counts and prefix, flag bytes
-    b += 24 * P + 8 * H;                                         // bin pairs, column entries, ray hits
-    b += 8 * ncol + 8 + 48 * H + scan(ncol);                     // parity fill: hits by column, records
-    b += 4 * (ncol + 1) + 8 * P + 12 * P + 64 * (ncol / 64 + 1);   // column entries by column
+    b += 24 * P;                                                 // bin pairs, column entries
+    b += 4 * (ncol + 1) + 8 * P + 12 * P + 64 * (ncol / 64 + 1) + scan(ncol);   // column entries by column
     b += 8 * B + 4 + 4 * P + 8 * P + 64 * (B / 64 + 1) + scan(B);   // boundary list, bins
     b += 16 * B * w2;                                            // Level2 planes
     if (d.params.normals) b += 12 * T + 4 * P + 12 * B + 12 * B * n2 * n2 * n2;
@@ -1508,7 +1419,7 @@ int check_staged(gpv_ctx* c, const gpv_grid* G)
 }
 
 // Meshes [lo, hi) as one run.  A run that fails on a per-run limit found
-// after Level1 (bin entries, boundary voxels, ray hits) or on device memory
+// after Level1 (bin entries, boundary voxels) or on device memory
 // is split in halves and each half runs on its own, down to single meshes;
 // a single mesh's failure is returned.  On failure no grid of the range is
 // left behind.
@@ -1864,7 +1775,7 @@ int gpv_ctx_autotune(gpv_ctx* c, const gpv_mesh_desc* d, int nm, int on_device, 
     int st = tune_trial(c, d, nm, on_device, 1, &warm);
     if (st == GPV_OK) st = tune_trial(c, d, nm, on_device, repeats, &base);
     const std::vector<int> expand = {4, 8, 16, 32}, group = {0, 4, 8, 16, 1 << 20}, items = {1024, 2048, 4096, 8192},
-                           overlap = {0, 1}, waves = {1, 2, 4}, stage = {128, 256};
+                           overlap = {0, 1}, waves = {1, 2, 4};
     auto sweep = [&](int gpv_tune::*field, const std::vector<int>& vals) -> int {
         for (int v : vals) {
             if (v == cur.*field) continue;
@@ -1887,7 +1798,6 @@ int gpv_ctx_autotune(gpv_ctx* c, const gpv_mesh_desc* d, int nm, int on_device, 
     if (st == GPV_OK) st = sweep(&gpv_tune::l2_overlap, overlap);
     if (st == GPV_OK) st = sweep(&gpv_tune::l2_sat_waves, waves);
     if (st == GPV_OK) st = sweep(&gpv_tune::l2_parity_waves, waves);
-    if (st == GPV_OK) st = sweep(&gpv_tune::expand_stage_tris, stage);
     if (st != GPV_OK) {
         c->tune = start;
         return st;
@@ -2032,14 +1942,10 @@ int gpv_classify_inout(gpv_ctx* c, gpv_grid* G)
     Job* J = G->job;
     HIP_TRY(hipSetDevice(c->device));
     TRY(stage_setup(J));
-    bool ok = false;
-    for (int attempt = 0; attempt < 2 && !ok; ++attempt) {
-        TRY(launch_ray_half(J));
-        TRY(read_counts(J, false));
-        TRY(complete_ray(J, &ok));
-    }
-    if (!ok) return fail(GPV_ERR_CAPACITY, "ray hit capacity did not converge");
-    return launch_parity(J);
+    TRY(launch_ray_half(J, c->stream));
+    TRY(read_counts(J, false));   // the input domain
+    J->inout_done = true;
+    return GPV_OK;
 }
 
 int gpv_compact_boundary(gpv_ctx* c, gpv_grid* G)

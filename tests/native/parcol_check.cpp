@@ -1,4 +1,4 @@
-// Host harness for the Level2 parity's crossing bounds (gpview_amd/csrc/
+// Host harness for the ray parities' crossing bounds (gpview_amd/csrc/
 // gpv_parcol.hpp): tests/test_parity_columns.py compares them with the float
 // ray test.  Test tooling only.
 #include <stdint.h>
@@ -68,6 +68,42 @@ extern "C" void parcol_batch(int64_t n, int n2, int nl, const float* tv, const f
                     if (l < la ? !hit : l >= lb ? hit : false) ++o[3];
                 }
             }
+        }
+    }
+}
+
+// Level1: case i, triangle tv[9i..] and a column (ox[i], oy[i]) over the layer
+// origins oz[nl] of a grid from zmin to zmax.  out[4i..]: accepted, layers that
+// contradict the certain ones, undecided layers, layers that pass.
+extern "C" void parl1_batch(int64_t n, int nl, const float* tv, const float* ox, const float* oy, const float* oz,
+                            float zmin, float zmax, uint32_t eps_bits, int64_t* out)
+{
+    float eps;
+    __builtin_memcpy(&eps, &eps_bits, 4);
+    for (int64_t i = 0; i < n; ++i) {
+        const float* t = tv + 9 * i;
+        int64_t* o = out + 4 * i;
+        const float e1x = t[3] - t[0], e1y = t[4] - t[1], e1z = t[5] - t[2];
+        const float e2x = t[6] - t[0], e2y = t[7] - t[1], e2z = t[8] - t[2];
+        const float px = 0.0f * e2z - e2y, py = e2x - 0.0f * e2z, pz = 0.0f * e2y - 0.0f * e2x;
+        const float det = e1x * px + e1y * py + e1z * pz;
+        if ((double)det > -1e-6 && (double)det < 1e-6) continue;
+        const float inv = 1.f / det;
+        const float tx = ox[i] - t[0], ty = oy[i] - t[1];
+        const float u = (tx * px + ty * py) * inv, v = (tx * e1y - ty * e1x) * inv;
+        if ((u < 0.f) | (u > 1.f) | (v < 0.f) | (u + v > 1.f)) continue;
+        o[0] = 1;
+        int la, lb;
+        gpv::par_l1_layers(oz, nl, zmin, (float)nl / (zmax - zmin), t[2], e1z, e2z, u, v,
+                           gpv::par_ez(e1x, e1y, e1z, e2x, e2y, e2z, inv), la, lb);
+        o[1] += la < 0 || lb < la || lb > nl;
+        o[2] = lb - la;
+        for (int l = 0; l < nl; ++l) {
+            const float tz = oz[l] - t[2];
+            const float qx = ty * e1z - tz * e1y, qy = tz * e1x - tx * e1z, qz = tx * e1y - ty * e1x;
+            const bool hit = (e2x * qx + e2y * qy + e2z * qz) * inv >= eps;
+            o[1] += l < la ? !hit : l >= lb ? hit : false;
+            o[3] += hit;
         }
     }
 }

@@ -60,6 +60,38 @@ def test_crossings_never_contradict_the_ray_test(columns, gv, fam):
     assert accepted > (100 if fam == "sliver" else 1000)   # most slivers fail the det test
 
 
+@pytest.mark.parametrize("fam", ["random", "small", "lattice", "near", "axis", "sliver"])
+def test_level1_crossings_never_contradict_the_ray_test(columns, gv, fam):
+    """Level1: the certain layers of a column against the float test at every layer."""
+    L = ctypes.CDLL(os.path.join(NATIVE, "libparcol.so"))
+    f32 = np.ctypeslib.ndpointer(dtype=np.float32, flags="C_CONTIGUOUS")
+    L.parl1_batch.argtypes = [ctypes.c_int64, ctypes.c_int] + [f32] * 4 + [ctypes.c_float] * 2 + \
+        [ctypes.c_uint32, np.ctypeslib.ndpointer(dtype=np.int64, flags="C_CONTIGUOUS")]
+    rng = np.random.default_rng(200 + ["random", "small", "lattice", "near", "axis", "sliver"].index(fam))
+    accepted = left = 0
+    for k, vc in enumerate([256, 64, 8, 33, 128, 4, 100, 512, 700]):
+        size = [1.0, 1e3, 10.0, 1.0, 0.1][k % 5]
+        ext = rng.uniform(0.2, 1, 3) * size
+        off = [0.0, 0.5, -1.0, 30.0, 3000.0][(k * 2) % 5] * rng.uniform(-1, 1, 3) * size
+        bmin, bmax = off.astype(np.float32), (off + ext).astype(np.float32)
+        info = gv.grid_derive(bmin, bmax, float((bmax - bmin).max()), vc, 4)
+        nn, g1 = np.array(list(info.n)), np.array(list(info.g), float)
+        tabs = [gv.grid_centers(info, 1, a, False) for a in range(3)]
+        n = int(max(2000, min(20000, 2e7 / nn[2])))
+        idx = np.stack([rng.integers(0, nn[a], n) for a in range(3)], 1)
+        ox, oy = (np.ascontiguousarray(tabs[a][idx[:, a]]) for a in (0, 1))
+        assert np.all(np.diff(tabs[2]) >= 0)
+        tv = _triangles(rng, fam, bmin + (idx + 0.5) * g1, g1, (g1 / 4), 4)
+        out = np.zeros((n, 4), np.int64)
+        L.parl1_batch(n, int(nn[2]), tv.ravel(), ox, oy, tabs[2], float(bmin[2]), float(bmax[2]), EPS_ABOVE, out.ravel())
+        got, wrong, und, _ = out.sum(0)
+        assert wrong == 0, f"{vc}: {wrong} layers contradict the crossing bounds"
+        accepted += int(got)
+        left += int(und)
+    assert accepted > (20 if fam == "sliver" else 500)   # most slivers fail the det test
+    assert left < 20 * accepted
+
+
 def _tall(gv, seed):
     """A steep closed surface: dozens of boundary voxels in its columns."""
     v, f = gv.icosphere(4, 0.4, (0.5, 0.5, 0.5), 0.02, seed=seed)
