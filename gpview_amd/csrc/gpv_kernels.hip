@@ -64,6 +64,18 @@ __device__ __forceinline__ T wave_incl_scan(T x)
     return x;
 }
 
+// inclusive XOR over the lanes of a full wave
+__device__ __forceinline__ uint64_t wave_incl_xor(uint64_t x)
+{
+    x ^= dpp_or_0<0x111, 0xf>(x);
+    x ^= dpp_or_0<0x112, 0xf>(x);
+    x ^= dpp_or_0<0x114, 0xf>(x);
+    x ^= dpp_or_0<0x118, 0xf>(x);
+    x ^= dpp_or_0<0x142, 0xa>(x);
+    x ^= dpp_or_0<0x143, 0xc>(x);
+    return x;
+}
+
 // the value of lane ^ S
 template <int S>
 __device__ __forceinline__ uint32_t lane_xor(uint32_t v)
@@ -343,7 +355,9 @@ __global__ __launch_bounds__(256) void k_tri_setup(const float* __restrict__ tri
             tests += any ? (uint64_t)dd[0] * dd[1] * dd[2] : 0;
         }
         if constexpr ((kPart & 2) == 0) continue;
-        uint32_t rit = 0;
+        // at least one item, so that runs of k_ray_expand with equal items hold equal
+        // work where most triangles have no column (48 mixed meshes 1414 us without)
+        uint32_t rit = 1;
         int4 rr = make_int4(0, 0, 0, 0);
         if (vis) {
             double xlo, xhi, ylo, yhi;
@@ -885,9 +899,10 @@ void launch_pack_bytes(const uint8_t* by, int64_t W, uint64_t* bits, uint32_t* c
 // the toggles above a layer.
 //
 // A wave owns a run of items and walks it 64 at a time over a window of 64
-// triangles; waves share nothing.  What bounds it: the latency of a
+// triangles; waves share nothing.  The crossings of a flat face fall into the same words:
+// lanes next to each other with the same word make one atomic.  What bounds it: the latency of a
 // round's dependent loads (offsets, triangle, origins), hence all waves the chip
-// holds; the atomics are one per crossing.
+// holds.
 template <bool kM>
 __global__ __launch_bounds__(256) void k_ray_expand(const float* __restrict__ tris, int64_t T,
                                                     const int4* __restrict__ rng, const uint64_t* __restrict__ off,
@@ -925,34 +940,45 @@ __global__ __launch_bounds__(256) void k_ray_expand(const float* __restrict__ tr
         // the triangles that end here are done
         t0 += __popcll(__ballot(eo <= base + n));
         base += n;
-        if ((uint32_t)lane >= n) continue;
-        const int mesh = kM ? (int)M.tri_mesh[t] : 0;
-        const GridDev& g = grid_of<kM>(g0, M, mesh);
-        const int4 r = rng[t];
-        float tv[9];
+        uint32_t at = ~0u;   // the word that gets the lane's toggle (planes hold less than 2^26 words)
+        uint64_t bit = 0;
+        if ((uint32_t)lane < n) {
+            const int mesh = kM ? (int)M.tri_mesh[t] : 0;
+            const GridDev& g = grid_of<kM>(g0, M, mesh);
+            const int4 r = rng[t];
+            float tv[9];
 #pragma unroll
-        for (int c = 0; c < 9; ++c) tv[c] = tris[(uint64_t)t * 9 + c];
-        const uint32_t jq = l / (uint32_t)r.z;
-        const int i = r.x + (int)(l - jq * (uint32_t)r.z), j = r.y + (int)jq;
-        MtTri m;
-        float tx, ty;
-        if (!mt_setup(tv, m) || !mt_column(m, tv[0], tv[1], g.r1x[i], g.r1y[j], tx, ty)) continue;
-        // u and v as mt_column has them
-        const float px = 0.0f * m.e2z - m.e2y, py = m.e2x - 0.0f * m.e2z;
-        const float u = (tx * px + ty * py) * m.inv_det, v = (tx * m.e1y - ty * m.e1x) * m.inv_det;
-        int la, lb;
-        par_l1_layers(g.r1z, g.nz, g.bminz, (float)g.nz / (g.bmaxz - g.bminz), tv[2], m.e1z, m.e2z, u, v,
-                      par_ez(m.e1x, m.e1y, m.e1z, m.e2x, m.e2y, m.e2z, m.inv_det), la, lb);
-        const uint64_t plane = (uint64_t)g.ny * g.nxw;
-        unsigned long long* word = ins + (kM ? M.off[mesh].word0 : 0) + (uint64_t)j * g.nxw + (uint32_t)i / 64u;
-        const unsigned long long bit = 1ull << (i & 63);
-        bool in = la > 0;
-        for (int k = la; k < lb; ++k) {
-            const bool hit = mt_t_hit(m.e1x, m.e1y, m.e1z, m.e2x, m.e2y, m.e2z, m.inv_det, tx, ty, tv[2], g.r1z[k]);
-            if (hit != in && k > 0) atomicXor(&word[(uint64_t)(k - 1) * plane], bit);
-            in = hit;
+            for (int c = 0; c < 9; ++c) tv[c] = tris[(uint64_t)t * 9 + c];
+            const uint32_t rz = r.z > 0 ? (uint32_t)r.z : 1u, jq = l / rz;
+            const int i = r.x + (int)(l - jq * rz), j = r.y + (int)jq;
+            MtTri m;
+            float tx, ty;
+            if (r.z > 0 && mt_setup(tv, m) && mt_column(m, tv[0], tv[1], g.r1x[i], g.r1y[j], tx, ty)) {
+                // u and v as mt_column has them
+                const float px = 0.0f * m.e2z - m.e2y, py = m.e2x - 0.0f * m.e2z;
+                const float u = (tx * px + ty * py) * m.inv_det, v = (tx * m.e1y - ty * m.e1x) * m.inv_det;
+                int la, lb;
+                par_l1_layers(g.r1z, g.nz, g.bminz, (float)g.nz / (g.bmaxz - g.bminz), tv[2], m.e1z, m.e2z, u, v,
+                              par_ez(m.e1x, m.e1y, m.e1z, m.e2x, m.e2y, m.e2z, m.inv_det), la, lb);
+                const uint32_t plane = (uint32_t)g.ny * (uint32_t)g.nxw;
+                const uint32_t w0 = (uint32_t)(kM ? M.off[mesh].word0 : 0) + (uint32_t)j * (uint32_t)g.nxw + (uint32_t)i / 64u;
+                bit = 1ull << (i & 63);
+                bool in = la > 0;
+                for (int k = la; k < lb; ++k) {
+                    const bool hit = mt_t_hit(m.e1x, m.e1y, m.e1z, m.e2x, m.e2y, m.e2z, m.inv_det, tx, ty, tv[2], g.r1z[k]);
+                    if (hit != in && k > 0) atomicXor(&ins[w0 + (uint32_t)(k - 1) * plane], (unsigned long long)bit);
+                    in = hit;
+                }
+                if (in) at = w0 + (uint32_t)(lb - 1) * plane;
+            }
         }
-        if (in) atomicXor(&word[(uint64_t)(lb - 1) * plane], bit);
+        // one atomic for each run of lanes with the same word
+        const uint64_t x = wave_incl_xor(at != ~0u ? bit : 0ull);
+        const uint32_t prev = (uint32_t)__shfl((int)at, lane ? lane - 1 : 0), next = (uint32_t)__shfl((int)at, lane < 63 ? lane + 1 : 63);
+        const uint64_t heads = __ballot(lane == 0 || at != prev) & ((2ull << lane) - 1ull);
+        const int first = 63 - __clzll((long long)heads);
+        const uint64_t before = shfl64(x, first ? first - 1 : 0);
+        if (at != ~0u && (lane == 63 || at != next)) atomicXor(&ins[at], (unsigned long long)(x ^ (first ? before : 0ull)));
     }
 }
 
@@ -1223,6 +1249,8 @@ __global__ __launch_bounds__(256) void k_st_toggle(const float* __restrict__ tri
         int64_t t = find_segment(off, T, i0);
         StTri s;
         st_prepare(tris + 9 * t, g, s);
+        int64_t at = -1;   // the word of the last toggles and their bits
+        unsigned long long bits = 0;
         for (uint64_t i = i0; i < i1; ++i) {
             if (off[t + 1] <= i) {
                 do ++t; while (off[t + 1] <= i);
@@ -1233,9 +1261,16 @@ __global__ __launch_bounds__(256) void k_st_toggle(const float* __restrict__ tri
             const int py = s.pylo + (int)(li / bw), px = s.pxlo + (int)(li % bw);
             if (!st_covers(s, px, py)) continue;
             const int k = st_slice(s, g, px, py);
-            if (k < g.nz)
-                atomicXor(&tog[((int64_t)k * H + py) * wpr + (px >> 6)], 1ull << (px & 63));
+            if (k >= g.nz) continue;
+            const int64_t w = ((int64_t)k * H + py) * wpr + (px >> 6);
+            if (w != at) {
+                if (bits) atomicXor(&tog[at], bits);
+                at = w;
+                bits = 0;
+            }
+            bits ^= 1ull << (px & 63);
         }
+        if (bits) atomicXor(&tog[at], bits);
     }
 }
 

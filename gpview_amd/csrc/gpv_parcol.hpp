@@ -23,12 +23,12 @@
 // equal steps (SatScale).
 //
 // Crossing.  The float s = e2 . (T x e1) is within 6.1 U B of the exact one, B =
-// sum |T_a| N_a, and t >= eps means s >= eps |det| up to 2 U; |T_a| <=
+// sum |T_a| N_a, and t >= eps means s >= eps |det| up to 2 U and the det's own 2.1 U N_z; |T_a| <=
 // 2 (|e1_a| + |e2_a|) for an accepted ray at its crossing where 64 U N_z <=
 // |det|.  The crossing height taken here, v1z + u e1z + v e2z - eps, is off by at
 // most 3 U |inv| (|Tx| N_x + |Ty| N_y + N_z (|e1z| + |e2z|)) and rounding.  So the
 // float test agrees with the crossing at every height farther from it than
-//   Ez = 64 U |inv| sum (|e1_a| + |e2_a|) N_a + 16 U (|e1z| + |e2z|) + 2^-12 eps
+//   Ez = 64 U |inv| sum (|e1_a| + |e2_a|) N_a + 16 U (|e1z| + |e2z|) + (2^-12 + 4 U N_z |inv|) eps
 // (|det| >= 1e-6 by the det test); worse conditioned records get Ez infinite.
 #pragma once
 
@@ -47,7 +47,7 @@ __host__ __device__ __forceinline__ float par_ez(float e1x, float e1y, float e1z
     const float sx = fabsf(e1x) + fabsf(e2x), sy = fabsf(e1y) + fabsf(e2y), sz = fabsf(e1z) + fabsf(e2z);
     const float b = sx * nx + sy * ny + sz * nz;
     const bool ok = 64.0f * U * nz * ai <= 1.0f && b * ai < 1e30f;
-    return ok ? 64.0f * U * (ai * b) + (16.0f * U * sz + 2.5e-10f) : 3.0e38f;
+    return ok ? 64.0f * U * (ai * b) + (16.0f * U * sz + 1.0e-6f * (0x1p-12f + 4.0f * U * nz * ai)) : 3.0e38f;
 }
 
 // A record with its bounds in one column.
