@@ -19,9 +19,9 @@ struct GridDev {
     int n2, w2;
     int normals;           // this mesh asks for Level1/Level2 normals
     int l2cuda;            // Level2 in the reference's CUDA arithmetic (gpv_params::cuda_level2)
-    int r2mono;            // each Level2 ray-origin table non-decreasing over its whole length
     int l1st;              // Level1 inside/outside by the GL-stencil-equivalent fill (gpv_params::l1_stencil)
     float bminx, bminy, bminz, bmaxx, bmaxy, bmaxz;
+    float g1x, g1y, g1z, g2x, g2y, g2z;   // voxel sizes of both levels
     float h1x, h1y, h1z;   // Level1 half extents
     float h2x, h2y, h2z;   // Level2 half extents
     float s1x, s1y, s1z, d1x, d1y, d1z;   // Level1 SAT columns: scale and table deviation per axis (SatScale)
@@ -31,6 +31,36 @@ struct GridDev {
     const float* c2x; const float* c2y; const float* c2z;   // [n*n2] Level2 SAT centers
     const float* r2x; const float* r2y; const float* r2z;   // [n*n2] Level2 ray origins
 };
+
+// Floats of a mesh's center tables: [SAT centers x, y, z | ray origins x, y, z] of
+// Level1 (n each), then of Level2 (n * n2 each).
+__host__ __device__ inline int64_t table_floats(const GridDev& g)
+{
+    return 2 * ((int64_t)g.nx + g.ny + g.nz) * (1 + (g.n2 > 0 ? g.n2 : 0));
+}
+
+// Entry k of a center table along one axis (which: 0 Level1 SAT, 1 Level1 ray, 2
+// Level2 SAT, 3 Level2 ray), with the reference's float and double expressions
+// (src/Object.cpp:2329-2331, 743-745, 2369-2391, 1134-1160).  Additions and products
+// only (halving is exact) and no contraction, so host and device agree to the bit.
+__host__ __device__ inline float center_at(int which, int k, float bmin, float g1, float g2, int n2, bool cuda_l2)
+{
+    const float ext1 = (float)((double)g1 / 2.0);
+    if (which == 0) return (float)((k + 0.5) * (double)ext1 * 2 + (double)bmin);
+    if (which == 1) return (float)((double)bmin + (k + 0.5) * (double)g1);
+    const int i = k / n2, p = k - i * n2;
+    const float mid = (float)((i + 0.5) * (double)g1 + (double)bmin);
+    if (cuda_l2) {
+        const float ext2 = (float)((double)g2 / 2.0);
+        const float two_p1 = (float)(2 * p + 1);
+        const float prod = two_p1 * ext2;
+        const float sum = prod + mid;
+        return sum - ext1;
+    }
+    if (which == 2) return (float)((p + 0.5) * (double)g2 + (double)mid - (double)ext1);
+    const float minp = (float)i * g1 + bmin;
+    return (float)((double)minp + (p + 0.5) * (double)g2);
+}
 
 // Where one mesh of a batch lives in the batch-wide arrays.  A batch
 // concatenates the meshes' soups (tri0), Level1 bitplanes (word0), xy
@@ -86,7 +116,10 @@ struct Counters {
     unsigned long long pairs;       // Level1 SAT (voxel, triangle) pairs
     unsigned long long colents;     // (column, triangle, zmax) entries
     unsigned long long bad_input;   // nonzero: a vertex coordinate is not finite or beyond +-2^40
+    unsigned long long done;        // blocks of the state counts that are through
 };
+// page-locked read-back, written by kernels: Counters | B (one mesh) or MeshOff[nm + 1] | MeshCtr[nm]
+constexpr size_t kHOff = 64;
 
 // sets the calling thread's gpv_last_error text and returns code
 int set_error(int code, const char* msg);
@@ -96,13 +129,25 @@ void pool_reset_peak(gpv_ctx* c);
 // ---- launch wrappers (gpv_kernels.hip) ------------------------------------
 // Launchers that take the batch view M and a grid g0 run the single-mesh
 // instantiation (grid g0) when M.nm == 1, the multi-mesh one otherwise.
+// up to kClearMax regions, their sizes in words of 8 bytes in `end`
+constexpr int kClearMax = 5;
+struct ClearList {
+    uint64_t* p[kClearMax];
+    int64_t end[kClearMax];
+};
+// clears them and, unless nullptr, makes one mesh's center tables
+void launch_clear(ClearList L, const GridDev* tables, hipStream_t s);
+// the center tables of a batch
+void launch_tables(const Meshes& M, hipStream_t s);
 void launch_fill_u32(uint32_t* p, uint32_t v, int64_t n, hipStream_t s);
 void launch_fill_u64(uint64_t* p, uint64_t v, int64_t n, hipStream_t s);
 
 void launch_mesh_ids(const MeshOff* off, int nm, int64_t T, uint32_t* tri_mesh, hipStream_t s);
-// part 1 (and 3) also raise *bad_input for a coordinate outside the domain
+// part 1 (and 3) also raise *bad_input for a coordinate outside the domain;
+// *_sums[k]: the items of triangles [256 k, 256 k + 256)
 void launch_tri_setup(const float* tris, int64_t T, const GridDev& g0, const Meshes& M, int4* box0, int4* box1,
-                      uint32_t* sat_items, int4* ray_rng, uint32_t* ray_items, int part,
+                      uint32_t* sat_items, int4* ray_rng, uint32_t* ray_items, uint64_t* sat_sums,
+                      uint64_t* ray_sums, int part,
                       unsigned long long* bad_input, hipStream_t s);
 
 // exclusive scan of n u32 into out[0..n] (out[n] = total); tmp sized by
@@ -112,24 +157,33 @@ size_t scan_tmp_elems(int64_t n);
 void launch_scan_u32_u64(const uint32_t* in, uint64_t* out, int64_t n, uint64_t* tmp, hipStream_t s);
 void launch_scan_u32_u32(const uint32_t* in, uint32_t* out, int64_t n, uint32_t* tmp, unsigned int* max_out,
                          hipStream_t s);
+// item offsets of T triangles from launch_tri_setup's counts and sums; a
+// second set (in2, or nullptr) in the same launch
+void launch_scan_items(const uint32_t* in, uint64_t* out, const uint64_t* sums, const uint32_t* in2, uint64_t* out2,
+                       const uint64_t* sums2, int64_t T, uint64_t* tmp, hipStream_t s);
+// word prefix from launch_pack_bytes's counts and sums (pack_sums(W) of them); pub
+// (or nullptr): the counters and the total go to the page-locked read-back
+size_t pack_sums(int64_t W);
+void launch_scan_words(const uint32_t* in, uint32_t* out, int64_t W, const uint32_t* sums, const Counters* ctr,
+                       uint64_t* pub, uint32_t* tmp, hipStream_t s);
 
 void launch_sat_expand(const float* tris, int64_t T, const int4* box0, const int4* box1, const uint64_t* off,
                        const GridDev& g0, const Meshes& M, uint8_t* bbytes, Append64 pairs, Append64 cols, int blocks,
                        hipStream_t s);
 // boundary bytes (W * 64, aligned to 16) -> boundary bitplane (W words) and its popcounts
-void launch_pack_bytes(const uint8_t* by, int64_t W, uint64_t* bits, uint32_t* cnt, hipStream_t s);
+void launch_pack_bytes(const uint8_t* by, int64_t W, uint64_t* bits, uint32_t* cnt, uint32_t* sums, hipStream_t s);
 // XORs the toggles of the accepted ray crossings into the inside plane (cleared by the caller)
 void launch_ray_expand(const float* tris, int64_t T, const int4* ray_rng, const uint64_t* off, const GridDev& g0,
                        const Meshes& M, uint64_t* ins, int blocks, hipStream_t s);
 
 // scratch of a two-level counting sort (ts_tiles(nkeys) tiles): total and
-// fill counters [2*tiles + 1], tile offsets [tiles + 1], scan temporary
-// [scan_tmp_elems(tiles)], bucket (8 bytes a bin pair, 12 a column entry)
+// fill counters [2*tiles + 1], tile offsets [tiles + 1], bucket (8 bytes a bin
+// pair, 12 a column entry); cleared: the counters hold zeros
 struct TileSortTmp {
     uint32_t* total;
     uint32_t* off;
-    uint32_t* scan;
     void* bucket;
+    bool cleared;
 };
 size_t ts_tiles(uint64_t nkeys);
 
@@ -171,9 +225,11 @@ void launch_l1_stencil(const float* tris, int64_t T, const GridDev& g, uint32_t*
 void launch_l1_fill(const GridDev& g0, const Meshes& M, int64_t blocks, uint64_t* ins, hipStream_t s);
 
 // b0 and l2w0 of every mesh (and the totals in entry nm) from the word prefix
-void launch_mesh_bounds(const uint32_t* wprefix, const Meshes& M, hipStream_t s);
+// and the counters, to the page-locked read-back pub as well
+void launch_mesh_bounds(const uint32_t* wprefix, const Meshes& M, const Counters* ctr, uint64_t* pub, hipStream_t s);
+// also clears nclear words
 void launch_boundary_index(const uint64_t* bnd, const uint32_t* wprefix, const GridDev& g0, const Meshes& M,
-                           int64_t W, int32_t* bidx, hipStream_t s);
+                           int64_t W, int32_t* bidx, uint32_t* clear, int64_t nclear, hipStream_t s);
 // pairs: key = batch-wide boundary bit index, val = triangle
 // bin pairs -> CSR by boundary rank (boff[B + 1], list); B <= 2^27.  The pairs' voxel bits are replaced by their boundary
 // ranks (ranked: they hold ranks already)
@@ -214,8 +270,10 @@ void launch_export_l1_normals(const uint64_t* bnd, const uint32_t* wprefix, uint
                               const GridDev& g, uint8_t* out, hipStream_t s);
 void launch_export_l2_normals(const float* l2n, int64_t n, uint8_t* out, hipStream_t s);
 
+// counts the states (done: a zero counter) and publishes the meshes' counters to pub
 void launch_count_states(const uint64_t* bnd, const uint64_t* ins, int64_t W, const uint64_t* sat2,
-                         const uint64_t* par2, int64_t W2, const Meshes& M, hipStream_t s);
+                         const uint64_t* par2, int64_t W2, const Meshes& M, unsigned long long* done, uint64_t* pub,
+                         hipStream_t s);
 
 // egress of one mesh (pointers already offset to that mesh's words)
 void launch_export_l1(const uint64_t* bnd, const uint64_t* ins, const GridDev& g, uint8_t unit, uint8_t* out,

@@ -225,8 +225,6 @@ struct gpv_ctx {
     Pool pool;
     char* h_buf = nullptr;   // pinned read-back staging
     size_t h_cap = 0;
-    float* tab_buf = nullptr;   // pinned staging of a job's center tables
-    size_t tab_cap = 0;
     int num_cu = 256;
     gpv_tune tune{16, 56, 2048, 1, 1, 1, 128};
     std::vector<hipEvent_t> events;   // recycled stage events of finished jobs
@@ -251,7 +249,6 @@ struct Job {
     int nm = 1;
     std::vector<gpv_grid_info> info;   // [nm]
     std::vector<GridDev> g;            // [nm], device table pointers
-    std::vector<float> h_tab;          // center tables of a no-allocation call (ordinary host memory)
     std::vector<MeshOff> off;          // [nm + 1]
     int64_t T = 0;
     const float* tris = nullptr;
@@ -269,6 +266,11 @@ struct Job {
     uint32_t *sat_items = nullptr, *ray_items = nullptr;
     uint64_t *sat_off = nullptr, *ray_off = nullptr, *scan64 = nullptr;
     uint64_t* scan_ray = nullptr;   // scan temporary of the ray half of the set-up (side stream)
+    uint64_t *sat_sums = nullptr, *ray_sums = nullptr;   // items per 256 triangles
+    uint8_t* bbytes = nullptr;       // boundary flags of the Level1 SAT
+    bool sat_cleared = false;        // flags and counters of the sweep hold zeros
+    bool ins_cleared = false;        // the inside plane holds zeros
+    bool cols_cleared = false;       // the column sort's counters hold zeros
     uint32_t* scan32 = nullptr;
     size_t scan_cap = 0;
     Counters* ctr = nullptr;
@@ -291,7 +293,6 @@ struct Job {
     int64_t B = 0, W2 = 0;
     uint32_t *boff = nullptr, *list = nullptr;
     uint32_t* coff = nullptr;
-    uint32_t* scan_side = nullptr;   // its scan temporary on the side stream (beside the bins)
     uint2* cent = nullptr;    // (triangle, zmax) of the column entries
     // column-entry sort on the side stream (beside the bins): its own scratch
     bool cols_side = false;
@@ -319,7 +320,7 @@ struct Job {
     // stream events: 0 setup, 1 L1 SAT, 2 L1 parity, 3 fork of the Level2 side stream,
     // 4 compaction+bins, 5 L2 parity, 6 L2 SAT start, 7 L2 SAT end, 8 finish,
     // 9 normals start, 10 normals end, 11 L2 parity end, 12 L1 SAT end,
-    // 13 L1 parity end, 15 fork of the L1 parity, 16 L2 parity start
+    // 13 L1 parity end, 14 end of the side stream, 15 fork of the L1 parity, 16 L2 parity start
     hipEvent_t ev[kJobEvents] = {};
     std::vector<void*> bufs;
     // gpv_voxelize_noalloc: buffers are carved from the device scratch array
@@ -452,45 +453,14 @@ size_t table_layout(const gpv_grid_info& I, size_t off[12])
     return pos + 1;
 }
 
-bool fill_tables(const gpv_grid_info& I, bool cuda_l2, float* tab, const size_t off[12])
-{
-    const int n2 = I.n2 > 0 ? I.n2 : 0;
-    for (int a = 0; a < 3; a++) {
-        const float ext1 = (float)((double)I.g[a] / 2.0);
-        for (int p = 0; p < I.n[a]; p++) {
-            tab[off[a] + p] = (float)((p + 0.5) * (double)ext1 * 2 + (double)I.bmin[a]);
-            tab[off[3 + a] + p] = (float)((double)I.bmin[a] + (p + 0.5) * (double)I.g[a]);
-        }
-        for (int i = 0; i < I.n[a] && n2 > 0; i++) {
-            const float mid = (float)((i + 0.5) * (double)I.g[a] + (double)I.bmin[a]);
-            const float minp = (float)i * I.g[a] + I.bmin[a];
-            const float ext2 = (float)((double)I.g2[a] / 2.0);
-            for (int p = 0; p < n2; p++) {
-                if (cuda_l2) {
-                    const float two_p1 = (float)(2 * p + 1);
-                    const float prod = two_p1 * ext2;
-                    const float sum = prod + mid;
-                    const float c = sum - ext1;
-                    tab[off[6 + a] + (size_t)i * n2 + p] = c;
-                    tab[off[9 + a] + (size_t)i * n2 + p] = c;
-                    continue;
-                }
-                tab[off[6 + a] + (size_t)i * n2 + p] =
-                    (float)((p + 0.5) * (double)I.g2[a] + (double)mid - (double)ext1);
-                tab[off[9 + a] + (size_t)i * n2 + p] = (float)((double)minp + (p + 0.5) * (double)I.g2[a]);
-            }
-        }
-    }
-    bool mono = true;
-    for (int a = 0; a < 3; a++)
-        for (size_t k = 1; k < (size_t)I.n[a] * n2; k++) mono = mono && tab[off[9 + a] + k - 1] <= tab[off[9 + a] + k];
-    return mono;
-}
-
-bool build_tables(const gpv_grid_info& I, bool cuda_l2, std::vector<float>& tab, size_t off[12])
+void build_tables(const gpv_grid_info& I, bool cuda_l2, std::vector<float>& tab, size_t off[12])
 {
     tab.assign(table_layout(I, off), 0.0f);
-    return fill_tables(I, cuda_l2, tab.data(), off);
+    const int n2 = I.n2 > 0 ? I.n2 : 0;
+    for (int w = 0; w < 4; w++)
+        for (int a = 0; a < 3; a++)
+            for (int k = 0; k < I.n[a] * (w < 2 ? 1 : n2); k++)
+                tab[off[3 * w + a] + k] = center_at(w, k, I.bmin[a], I.g[a], I.g2[a], n2, cuda_l2);
 }
 
 int expand_blocks(const gpv_ctx* c) { return std::max(1, c->num_cu) * std::max(1, c->tune.expand_blocks_per_cu); }
@@ -508,7 +478,7 @@ int ensure_hbuf(gpv_ctx* c, size_t bytes)
 }
 
 // pinned staging layout: Counters | MeshOff[nm + 1] | MeshCtr[nm]
-constexpr size_t kHOff = 64;
+static_assert(sizeof(Counters) <= kHOff, "the offsets follow the counters");
 size_t hctr_at(int nm) { return (kHOff + sizeof(MeshOff) * (size_t)(nm + 1) + 63) / 64 * 64; }
 
 int ensure_scan_tmp(Job* J, int64_t n)
@@ -545,6 +515,8 @@ GridDev grid_dev(const gpv_grid_info& info)
     g.w2 = info.n2 > 0 ? (info.n2 * info.n2 * info.n2 + 63) / 64 : 0;
     g.bminx = info.bmin[0]; g.bminy = info.bmin[1]; g.bminz = info.bmin[2];
     g.bmaxx = info.bmax[0]; g.bmaxy = info.bmax[1]; g.bmaxz = info.bmax[2];
+    g.g1x = info.g[0]; g.g1y = info.g[1]; g.g1z = info.g[2];
+    g.g2x = info.g2[0]; g.g2y = info.g2[1]; g.g2z = info.g2[2];
     g.h1x = (float)((double)info.g[0] / 2.0); g.h1y = (float)((double)info.g[1] / 2.0);
     g.h1z = (float)((double)info.g[2] / 2.0);
     g.h2x = (float)((double)info.g2[0] / 2.0); g.h2y = (float)((double)info.g2[1] / 2.0);
@@ -690,36 +662,6 @@ int job_create(gpv_ctx* c, const gpv_mesh_desc* d, int nm, int on_device, Job** 
         for (int k = 0; k < 12; ++k) tab_at[(size_t)m * 12 + k] = ntab + o[k];
         ntab += n;
     }
-    // the tables are written straight into the context's page-locked
-    // staging, so their upload is asynchronous (the previous job on this
-    // context has finished); the no-allocation entry point, which may not
-    // grow that staging, uses ordinary host memory instead
-    float* tab_src = nullptr;
-    if (J->arena) {
-        J->h_tab.assign(ntab, 0.0f);
-        tab_src = J->h_tab.data();
-    } else {
-        if (ntab * sizeof(float) > c->tab_cap) {
-            const size_t want = std::max<size_t>(ntab * sizeof(float), 2 * c->tab_cap);
-            if (c->tab_buf) (void)hipHostFree(c->tab_buf);
-            c->tab_buf = nullptr;
-            c->tab_cap = 0;
-            if (hipHostMalloc(reinterpret_cast<void**>(&c->tab_buf), want, hipHostMallocDefault) != hipSuccess) {
-                (void)hipGetLastError();
-                c->tab_buf = nullptr;
-                return bail(fail(GPV_ERR_OOM, "page-locked table staging of %zu bytes failed", want));
-            }
-            c->tab_cap = want;
-        }
-        tab_src = c->tab_buf;
-    }
-    for (int m = 0; m < nm; ++m) {
-        GridDev& g = J->g[m];
-        size_t o[12];
-        table_layout(J->info[m], o);
-        const size_t base = tab_at[(size_t)m * 12];   // the first table starts at offset 0 of the mesh's block
-        g.r2mono = fill_tables(J->info[m], g.l2cuda != 0, tab_src + base, o) ? 1 : 0;
-    }
     J->off[nm].word0 = word0;
     J->off[nm].col0 = col0;
     J->off[nm].tri0 = tri0;
@@ -728,8 +670,6 @@ int job_create(gpv_ctx* c, const gpv_mesh_desc* d, int nm, int on_device, Job** 
     J->l2p_waves = pw0;
     int r;
     if ((r = alloc(J, &J->tables, ntab)) != GPV_OK) return bail(r);
-    if (hipMemcpyAsync(J->tables, tab_src, ntab * sizeof(float), hipMemcpyHostToDevice, c->stream) != hipSuccess)
-        return bail(fail(GPV_ERR_HIP, "table upload failed"));
     for (int m = 0; m < nm; ++m) {
         const float* tb = J->tables;
         const size_t* o = &tab_at[(size_t)m * 12];
@@ -800,6 +740,7 @@ int job_create(gpv_ctx* c, const gpv_mesh_desc* d, int nm, int on_device, Job** 
     if ((r = alloc(J, &J->box0, Tn)) || (r = alloc(J, &J->box1, Tn)) || (r = alloc(J, &J->rng, Tn)) ||
         (r = alloc(J, &J->sat_items, Tn)) || (r = alloc(J, &J->ray_items, Tn)) ||
         (r = alloc(J, &J->sat_off, Tn + 1)) || (r = alloc(J, &J->ray_off, Tn + 1)) ||
+        (r = alloc(J, &J->sat_sums, Tn / 256 + 1)) || (r = alloc(J, &J->ray_sums, Tn / 256 + 1)) ||
         (r = alloc(J, &J->ctr, 1)) || (r = alloc(J, &J->wcnt, (size_t)W)) ||
         (r = alloc(J, &J->wprefix, (size_t)W + 1)))
         return bail(r);
@@ -839,68 +780,95 @@ int stage_setup(Job* J)
     gpv_ctx* c = J->ctx;
     hipStream_t s = c->stream;
     HIP_TRY(hipEventRecord(J->ev[0], s));
-    launch_fill_u64(reinterpret_cast<uint64_t*>(J->mctr), 0, (int64_t)(sizeof(MeshCtr) / 8) * J->nm, s);
-    launch_fill_u64(reinterpret_cast<uint64_t*>(&J->ctr->bad_input), 0, 1, s);
+    launch_clear(ClearList{{reinterpret_cast<uint64_t*>(J->mctr), reinterpret_cast<uint64_t*>(J->ctr)},
+                           {(int64_t)(sizeof(MeshCtr) / 8) * J->nm, (int64_t)(sizeof(Counters) / 8)}},
+                 J->nm > 1 ? nullptr : &J->g[0], s);
+    if (J->nm > 1) launch_tables(J->view(), s);
     if (J->nm > 1) launch_mesh_ids(J->d_off, J->nm, J->T, J->tri_mesh, s);
     launch_tri_setup(J->tris, J->T, J->g[0], J->view(), J->box0, J->box1, J->sat_items, J->rng, J->ray_items,
-                     3, &J->ctr->bad_input, s);
+                     J->sat_sums, J->ray_sums, 3, &J->ctr->bad_input, s);
     TRY(ensure_scan_tmp(J, J->T));
-    launch_scan_u32_u64(J->sat_items, J->sat_off, J->T, J->scan64, s);
-    launch_scan_u32_u64(J->ray_items, J->ray_off, J->T, J->scan64, s);
+    launch_scan_items(J->sat_items, J->sat_off, J->sat_sums, J->ray_items, J->ray_off, J->ray_sums, J->T, J->scan64, s);
     HIP_TRY(hipGetLastError());
     J->setup_done = true;
     return GPV_OK;
 }
 
-// The set-up in two halves: the SAT half on the main stream, the ray half
-// (and, after it, the ray expansion) on the side stream, forked at ev[15].
+// Triangles up to which the set-up is one launch on the main stream before the
+// fork: as two, beside each other, it costs a launch more, which up to here takes
+// longer than the half it hides (three of a wave's 64 triangles a SIMD).
+constexpr int64_t kSetupSplit = int64_t(1) << 16;
+
+// The fused pipeline's set-up: everything cleared in one launch, then the SAT half on
+// the main stream and the ray half on the side stream, forked at ev[15].
 int stage_setup_split(Job* J)
 {
     gpv_ctx* c = J->ctx;
     hipStream_t s = c->stream;
     HIP_TRY(hipEventRecord(J->ev[0], s));
-    launch_fill_u64(reinterpret_cast<uint64_t*>(J->mctr), 0, (int64_t)(sizeof(MeshCtr) / 8) * J->nm, s);
-    launch_fill_u64(reinterpret_cast<uint64_t*>(&J->ctr->bad_input), 0, 1, s);
-    if (J->nm > 1) launch_mesh_ids(J->d_off, J->nm, J->T, J->tri_mesh, s);
     TRY(ensure_scan_tmp(J, J->T));
     release(J, J->scan_ray);
     TRY(alloc(J, &J->scan_ray, scan_tmp_elems(J->T)));
-    HIP_TRY(hipEventRecord(J->ev[15], s));
+    TRY(alloc(J, &J->bbytes, (size_t)J->W * 64));
+    const size_t tiles = ts_tiles((uint64_t)J->ncol);
+    if (J->n2max > 0) TRY(alloc(J, &J->cs_cnt, 3 * tiles + 2));
+    launch_clear(ClearList{{reinterpret_cast<uint64_t*>(J->mctr), reinterpret_cast<uint64_t*>(J->ctr),
+                            reinterpret_cast<uint64_t*>(J->bbytes), J->ins, reinterpret_cast<uint64_t*>(J->cs_cnt)},
+                           {(int64_t)(sizeof(MeshCtr) / 8) * J->nm, (int64_t)(sizeof(Counters) / 8), J->W * 8,
+                            J->all_stencil ? 0 : J->W, J->n2max > 0 ? (int64_t)tiles + 1 : 0}},
+                 J->nm > 1 ? nullptr : &J->g[0], s);
+    if (J->nm > 1) launch_tables(J->view(), s);
+    J->sat_cleared = true;
+    J->ins_cleared = true;
+    J->cols_cleared = true;
+    if (J->nm > 1) launch_mesh_ids(J->d_off, J->nm, J->T, J->tri_mesh, s);
+    const bool one = J->T <= kSetupSplit && !J->all_stencil;
+    if (!one) HIP_TRY(hipEventRecord(J->ev[15], s));
     launch_tri_setup(J->tris, J->T, J->g[0], J->view(), J->box0, J->box1, J->sat_items, J->rng, J->ray_items,
-                     1, &J->ctr->bad_input, s);
-    launch_scan_u32_u64(J->sat_items, J->sat_off, J->T, J->scan64, s);
+                     J->sat_sums, J->ray_sums, one ? 3 : 1, &J->ctr->bad_input, s);
+    launch_scan_items(J->sat_items, J->sat_off, J->sat_sums, one ? J->ray_items : nullptr, J->ray_off, J->ray_sums, J->T,
+                      J->scan64, s);
+    if (one) HIP_TRY(hipEventRecord(J->ev[15], s));
     HIP_TRY(hipStreamWaitEvent(c->side, J->ev[15], 0));
-    if (!J->all_stencil) {   // the ray half feeds only the ray parity
+    if (!one && !J->all_stencil) {   // the ray half feeds only the ray parity
         launch_tri_setup(J->tris, J->T, J->g[0], J->view(), J->box0, J->box1, J->sat_items, J->rng, J->ray_items,
-                         2, &J->ctr->bad_input, c->side);
-        launch_scan_u32_u64(J->ray_items, J->ray_off, J->T, J->scan_ray, c->side);
+                         J->sat_sums, J->ray_sums, 2, &J->ctr->bad_input, c->side);
+        launch_scan_items(J->ray_items, J->ray_off, J->ray_sums, nullptr, nullptr, nullptr, J->T, J->scan_ray, c->side);
     }
     HIP_TRY(hipGetLastError());
     J->setup_done = true;
     return GPV_OK;
 }
 
-// Level1 SAT sweep + the boundary popcount scan (ranks need the final bits)
+// Level1 SAT sweep + the boundary popcount scan (ranks need the final bits); the
+// counters go to the read-back
 int launch_sat_half(Job* J)
 {
     gpv_ctx* c = J->ctx;
     hipStream_t s = c->stream;
     HIP_TRY(hipEventRecord(J->ev[1], s));
     // boundary flags as bytes (plain stores from the SAT), packed to bits after
-    uint8_t* bbytes = nullptr;
-    TRY(alloc(J, &bbytes, (size_t)J->W * 64));
-    launch_fill_u64(reinterpret_cast<uint64_t*>(bbytes), 0, J->W * 8, s);
-    launch_fill_u64(reinterpret_cast<uint64_t*>(&J->ctr->pairs), 0, 2, s);   // pairs, colents
+    if (!J->sat_cleared) {
+        release(J, J->bbytes);
+        TRY(alloc(J, &J->bbytes, (size_t)J->W * 64));
+        launch_clear(ClearList{{reinterpret_cast<uint64_t*>(J->bbytes), reinterpret_cast<uint64_t*>(&J->ctr->pairs)},
+                               {J->W * 8, 2}}, nullptr, s);   // pairs, colents
+    }
+    J->sat_cleared = false;
     Append64 pa{&J->ctr->pairs, J->pair_key, J->pair_tri, J->pair_cap};
     Append64 co{&J->ctr->colents, J->col_key, J->col_z, J->col_cap};
     J->pairs_ranked = false;   // the sweep appends voxel bits
-    launch_sat_expand(J->tris, J->T, J->box0, J->box1, J->sat_off, J->g[0], J->view(), bbytes, pa, co,
-                      expand_blocks(c), s);
-    launch_pack_bytes(bbytes, J->W, J->bnd, J->wcnt, s);
-    release(J, bbytes);
+    uint32_t* sums = nullptr;
+    TRY(alloc(J, &sums, pack_sums(J->W)));
     TRY(ensure_scan_tmp(J, J->W));
-    launch_scan_u32_u32(J->wcnt, J->wprefix, J->W, J->scan32, nullptr, s);
-    if (J->nm > 1) launch_mesh_bounds(J->wprefix, J->view(), s);
+    uint64_t* pub = reinterpret_cast<uint64_t*>(c->h_buf);
+    launch_sat_expand(J->tris, J->T, J->box0, J->box1, J->sat_off, J->g[0], J->view(), J->bbytes, pa, co,
+                      expand_blocks(c), s);
+    launch_pack_bytes(J->bbytes, J->W, J->bnd, J->wcnt, sums, s);
+    launch_scan_words(J->wcnt, J->wprefix, J->W, sums, J->ctr, J->nm > 1 ? nullptr : pub, J->scan32, s);
+    release(J, J->bbytes);
+    release(J, sums);
+    if (J->nm > 1) launch_mesh_bounds(J->wprefix, J->view(), J->ctr, pub, s);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipEventRecord(J->ev[12], s));
     return GPV_OK;
@@ -914,7 +882,8 @@ int launch_ray_half(Job* J, hipStream_t s)
     gpv_ctx* c = J->ctx;
     HIP_TRY(hipEventRecord(J->ev[2], s));
     if (!J->all_stencil) {   // the ray parity skips the stencil meshes
-        launch_fill_u64(J->ins, 0, J->W, s);
+        if (!J->ins_cleared) launch_fill_u64(J->ins, 0, J->W, s);
+        J->ins_cleared = false;
         launch_ray_expand(J->tris, J->T, J->rng, J->ray_off, J->g[0], J->view(), J->ins, expand_blocks(c), s);
         launch_l1_fill(J->g[0], J->view(), (int64_t)J->off[J->nm].ptask0, J->ins, s);
     }
@@ -924,19 +893,13 @@ int launch_ray_half(Job* J, hipStream_t s)
     return GPV_OK;
 }
 
-// one round trip: the counters and, when asked, the boundary offsets
-int read_counts(Job* J, bool with_b)
+// waits for the counters, which launch_sat_half (swept) publishes with the boundary
+// offsets; the others are copied
+int read_counts(Job* J, bool swept)
 {
     gpv_ctx* c = J->ctx;
     hipStream_t s = c->stream;
-    HIP_TRY(hipMemcpyAsync(c->h_buf, J->ctr, sizeof(Counters), hipMemcpyDeviceToHost, s));
-    if (with_b) {
-        if (J->nm > 1)
-            HIP_TRY(hipMemcpyAsync(c->h_buf + kHOff, J->d_off, sizeof(MeshOff) * ((size_t)J->nm + 1),
-                                   hipMemcpyDeviceToHost, s));
-        else
-            HIP_TRY(hipMemcpyAsync(c->h_buf + kHOff, J->wprefix + J->W, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    }
+    if (!swept) HIP_TRY(hipMemcpyAsync(c->h_buf, J->ctr, sizeof(Counters), hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
     // the set-up kernel flags coordinates outside the input domain (NaN and
     // infinities would reach the index AABBs and the pruning bounds, where
@@ -1013,19 +976,16 @@ int launch_stencil(Job* J, hipStream_t s)
     return GPV_OK;
 }
 
-// buffers of the column-entry sort when it runs on the side stream
+// buffers of the column-entry sort when it runs on the side stream (its counters
+// are there since the set-up)
 // (allocated before the fork, released after the Level2 join)
 int alloc_cols(Job* J)
 {
     release(J, J->coff);
     release(J, J->cent);
-    release(J, J->cs_cnt);
     release(J, J->cs_bucket);
-    release(J, J->scan_side);
-    TRY(alloc(J, &J->scan_side, scan_tmp_elems((int64_t)ts_tiles((uint64_t)J->ncol))));
     TRY(alloc(J, &J->coff, (size_t)J->ncol + 1));
     TRY(alloc(J, &J->cent, (size_t)std::max<uint64_t>(J->n_cols, 1)));
-    TRY(alloc(J, &J->cs_cnt, 3 * ts_tiles((uint64_t)J->ncol) + 2));
     return alloc(J, &J->cs_bucket, 3 * (size_t)std::max<uint64_t>(J->n_cols, 1));
 }
 
@@ -1033,7 +993,8 @@ int alloc_cols(Job* J)
 int col_sort_kernels(Job* J, hipStream_t s)
 {
     const size_t tiles = ts_tiles((uint64_t)J->ncol);
-    const TileSortTmp ts{J->cs_cnt, J->cs_cnt + 2 * tiles + 1, J->scan_side, J->cs_bucket};
+    const TileSortTmp ts{J->cs_cnt, J->cs_cnt + 2 * tiles + 1, J->cs_bucket, J->cols_cleared};
+    J->cols_cleared = false;
     const int ipb = std::max(256, J->ctx->tune.sort_items_per_block);
     launch_bin_cols(J->col_key, J->col_z, J->n_cols, (uint32_t)J->ncol, ts, ipb, J->coff, J->cent, s);
     HIP_TRY(hipGetLastError());
@@ -1073,7 +1034,6 @@ int launch_compact(Job* J)
     else
         TRY(alloc(J, &J->bidx, Bn));
     if (J->nm > 1) TRY(alloc(J, &J->bmesh, Bn));
-    launch_boundary_index(J->bnd, J->wprefix, J->g[0], J->view(), J->W, J->bidx, s);
     release(J, J->boff);
     release(J, J->list);
     TRY(alloc(J, &J->boff, (size_t)J->B + 1));
@@ -1089,16 +1049,17 @@ int launch_compact(Job* J)
     TRY(alloc(J, &ts_cnt, 3 * tiles + 2));
     TRY(alloc(J, &ts_bucket,
               (size_t)std::max<uint64_t>(!cols ? 2 * J->n_pairs : std::max(2 * J->n_pairs, 3 * J->n_cols), 1)));
-    TRY(ensure_scan_tmp(J, (int64_t)tiles));
     ts.total = ts_cnt;
     ts.off = ts_cnt + 2 * tiles + 1;
-    ts.scan = J->scan32;
     ts.bucket = ts_bucket;
+    ts.cleared = true;
+    launch_boundary_index(J->bnd, J->wprefix, J->g[0], J->view(), J->W, J->bidx, ts_cnt, 2 * (int64_t)tiles + 1, s);
     const int ipb = std::max(256, J->ctx->tune.sort_items_per_block);
     launch_bin_pairs(J->pair_key, J->pairs_ranked, J->pair_tri, J->n_pairs, J->bnd, J->wprefix, (uint32_t)J->B, ts,
                      ipb, J->boff, J->nm > 1 ? nullptr : &J->mctr[0].max_per_voxel, J->list, s);
     J->pairs_ranked = true;
-    if (J->nm > 1) launch_mesh_bins(J->boff, J->B, J->view(), s);
+    ts.cleared = false;
+    if (J->nm > 1 && !J->cols_side) launch_mesh_bins(J->boff, J->B, J->view(), s);
     if (cols) {
         release(J, J->coff);
         release(J, J->cent);
@@ -1221,7 +1182,14 @@ int run_streams(Job* J)
         TRY(l2_parity_kernels(J, c->side));
         J->l2p_done = true;
         J->l2s_done = true;
-        HIP_TRY(hipStreamWaitEvent(s, J->ev[11], 0));
+        if (J->nm > 1) {
+            // behind the parity, not before the SAT: its few blocks would wait for room beside the parity's
+            HIP_TRY(hipStreamWaitEvent(c->side, J->ev[6], 0));
+            launch_mesh_bins(J->boff, J->B, J->view(), c->side);
+            HIP_TRY(hipGetLastError());
+            HIP_TRY(hipEventRecord(J->ev[14], c->side));
+        }
+        HIP_TRY(hipStreamWaitEvent(s, J->ev[J->nm > 1 ? 14 : 11], 0));
     } else {
         TRY(alloc_level2(J));
         TRY(launch_compact(J));
@@ -1261,10 +1229,11 @@ int job_finish(Job* J)
 {
     gpv_ctx* c = J->ctx;
     hipStream_t s = c->stream;
-    launch_count_states(J->bnd, J->ins, J->W, J->sat2, J->par2, J->W2, J->view(), s);
-    HIP_TRY(hipEventRecord(J->ev[8], s));
     const size_t at = hctr_at(J->nm);
-    HIP_TRY(hipMemcpyAsync(c->h_buf + at, J->mctr, sizeof(MeshCtr) * (size_t)J->nm, hipMemcpyDeviceToHost, s));
+    launch_count_states(J->bnd, J->ins, J->W, J->sat2, J->par2, J->W2, J->view(), &J->ctr->done,
+                        reinterpret_cast<uint64_t*>(c->h_buf + at), s);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipEventRecord(J->ev[8], s));
     HIP_TRY(hipStreamSynchronize(s));
     const MeshCtr* mc = reinterpret_cast<const MeshCtr*>(c->h_buf + at);
     auto el = [&](int a, int b) -> float {
@@ -1313,7 +1282,7 @@ int job_finish(Job* J)
     release(J, J->wcnt); release(J, J->boff);
     release(J, J->list); release(J, J->coff); release(J, J->cent);
     release(J, J->cs_cnt); release(J, J->cs_bucket);
-    release(J, J->scan_side); release(J, J->tri_mesh);
+    release(J, J->sat_sums); release(J, J->ray_sums); release(J, J->bbytes); release(J, J->tri_mesh);
     release(J, J->st_cnt); release(J, J->st_off); release(J, J->st_scan); release(J, J->st_tog);
     release(J, J->bmesh);
     release(J, J->d_grids); release(J, J->d_off); release(J, J->own_soup); release(J, J->mctr);
@@ -1383,7 +1352,8 @@ int64_t predict_run_bytes(const gpv_mesh_desc& d, const gpv_grid_info& I)
     b += 4 * (2 * (nx + ny + nz) * (1 + n2) + 1);               // center tables
     b += 36 * T + 4 * T + 4 * B + 4096;                          // soup copy, batch mesh ids, descriptors
     b += 72 * T + 16 + 2 * scan(std::max(T, W));               // per-triangle set-up, item scans
-    b += 24 * W + 64 * W;                                        // planes, word counts and prefix, flag bytes
+    b += 24 * W + 64 * W + W / 256 + 4;                          // planes, word counts, their sums and prefix, flag bytes
+    b += T / 16 + 16;                                            // sums of the items
     b += 24 * P;                                                 // bin pairs, column entries
     b += 4 * (ncol + 1) + 8 * P + 12 * P + 64 * (ncol / 64 + 1) + scan(ncol);   // column entries by column
     b += 8 * B + 4 + 4 * P + 8 * P + 64 * (B / 64 + 1) + scan(B);   // boundary list, bins
@@ -1675,7 +1645,6 @@ int gpv_ctx_destroy(gpv_ctx* c)
             if (e) (void)hipEventDestroy(e);
         c->pool.trim();
         if (c->h_buf) (void)hipHostFree(c->h_buf);
-        if (c->tab_buf) (void)hipHostFree(c->tab_buf);
         (void)hipStreamDestroy(c->stream);
         (void)hipStreamDestroy(c->side);
         if (c->copy) (void)hipStreamDestroy(c->copy);
