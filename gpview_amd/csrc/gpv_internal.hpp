@@ -275,6 +275,15 @@ void launch_count_states(const uint64_t* bnd, const uint64_t* ins, int64_t W, co
                          const uint64_t* par2, int64_t W2, const Meshes& M, unsigned long long* done, uint64_t* pub,
                          hipStream_t s);
 
+// up to kCopyMax pieces of device memory and their places in page-locked host memory
+constexpr int kCopyMax = 4;
+struct CopyOut {
+    const char* src[kCopyMax];
+    char* dst[kCopyMax];
+    int64_t n[kCopyMax];
+};
+void launch_copy_out(const CopyOut& L, int pieces, hipStream_t s);
+
 // egress of one mesh (pointers already offset to that mesh's words)
 void launch_export_l1(const uint64_t* bnd, const uint64_t* ins, const GridDev& g, uint8_t unit, uint8_t* out,
                       hipStream_t s);

@@ -3138,6 +3138,36 @@ void launch_count_states(const uint64_t* bnd, const uint64_t* ins, int64_t W, co
 }
 
 // ---------------------------------------------------------------------------
+// device memory -> page-locked host memory, a row of blocks per piece: 16 bytes a
+// lane where the source allows it, bytes otherwise (and for the rest)
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void k_copy_out(CopyOut L)
+{
+    const char* src = L.src[0];
+    char* dst = L.dst[0];
+    int64_t n = L.n[0];
+#pragma unroll
+    for (int k = 1; k < kCopyMax; ++k)
+        if ((int)blockIdx.y == k) {
+            src = L.src[k];
+            dst = L.dst[k];
+            n = L.n[k];
+        }
+    const int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
+    const int64_t wide = (reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) & 15 ? 0 : n / 16;
+    for (int64_t i = i0; i < wide; i += stride) reinterpret_cast<uint4*>(dst)[i] = reinterpret_cast<const uint4*>(src)[i];
+    for (int64_t i = wide * 16 + i0; i < n; i += stride) dst[i] = src[i];
+}
+
+void launch_copy_out(const CopyOut& L, int pieces, hipStream_t s)
+{
+    int64_t most = 0;
+    for (int k = 0; k < pieces; ++k) most = L.n[k] > most ? L.n[k] : most;
+    if (pieces <= 0 || most <= 0) return;
+    k_copy_out<<<dim3((unsigned)grid_for((most + 15) / 16, 256, 256), (unsigned)pieces), 256, 0, s>>>(L);
+}
+
+// ---------------------------------------------------------------------------
 // egress: one byte per voxel holding state * unit (unit 1: the 0/1/2 states;
 // unit 127: the .raw bytes uint8(state * 127.0f), src/Object.cpp:3024-3063)
 // and the int32 exclusive boundary prefix per Level1 voxel

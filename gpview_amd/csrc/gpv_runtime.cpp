@@ -5,6 +5,7 @@
 // are computed with the reference's float/double promotions (see the
 // citations per function) and this file is compiled with -ffp-contract=off.
 #include "gpv.h"
+#include "gpv_download.hpp"
 #include "gpv_internal.hpp"
 #include "gpv_satrow.hpp"
 #include "gpv_serve.h"
@@ -223,6 +224,7 @@ struct gpv_ctx {
     hipStream_t side = nullptr;   // second stream: Level2 parity beside the Level2 SAT
     hipStream_t copy = nullptr;   // uploads of a batch's host soups ahead of its runs (created on first use)
     Pool pool;
+    Downloader down;         // results into ordinary host memory
     char* h_buf = nullptr;   // pinned read-back staging
     size_t h_cap = 0;
     int num_cu = 256;
@@ -1643,6 +1645,7 @@ int gpv_ctx_destroy(gpv_ctx* c)
         c->events.clear();
         for (hipEvent_t e : c->na_ev)
             if (e) (void)hipEventDestroy(e);
+        c->down.close();
         c->pool.trim();
         if (c->h_buf) (void)hipHostFree(c->h_buf);
         (void)hipStreamDestroy(c->stream);
@@ -2173,11 +2176,11 @@ int gpv_grid_download_bits(gpv_ctx* c, const gpv_grid* G, uint64_t* l1b, uint64_
     const size_t w1 = (size_t)g.nz * g.ny * g.nxw * 8;
     const size_t w2 = g.n2 > 0 ? (size_t)J->nb(G->m) * g.w2 * 8 : 0;
     hipStream_t s = c->stream;
-    if (l1b && w1) HIP_TRY(hipMemcpyAsync(l1b, J->bnd + o.word0, w1, hipMemcpyDeviceToHost, s));
-    if (l1i && w1) HIP_TRY(hipMemcpyAsync(l1i, J->ins + o.word0, w1, hipMemcpyDeviceToHost, s));
-    if (l2b && w2) HIP_TRY(hipMemcpyAsync(l2b, J->sat2 + o.l2w0, w2, hipMemcpyDeviceToHost, s));
-    if (l2i && w2) HIP_TRY(hipMemcpyAsync(l2i, J->par2 + o.l2w0, w2, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    const Downloader::Piece pieces[4] = {{l1b, J->bnd + o.word0, l1b ? w1 : 0},
+                                         {l1i, J->ins + o.word0, l1i ? w1 : 0},
+                                         {l2b, J->sat2 + o.l2w0, l2b ? w2 : 0},
+                                         {l2i, J->par2 + o.l2w0, l2i ? w2 : 0}};
+    HIP_TRY(c->down.run(pieces, 4, s));
     return GPV_OK;
 }
 
@@ -2197,35 +2200,56 @@ static int download_impl(gpv_ctx* c, const gpv_grid* G, uint8_t unit, uint8_t* l
     const int64_t n1 = J->info[m].n1;
     const int64_t nb = J->nb(m);
     const int64_t n23 = (int64_t)g.n2 * g.n2 * g.n2;
+    // Exports into device memory of their own, then all of them to the host; where
+    // that memory runs out, those made so far go first.
+    Downloader::Piece pieces[4] = {};
+    uint8_t* made[4] = {};
+    int np = 0;
+    auto flush = [&]() -> int {
+        hipError_t e = hipGetLastError();
+        const hipError_t w = c->down.run(pieces, np, s);   // waits, so the memory can go back
+        if (e == hipSuccess) e = w;
+        for (int k = 0; k < np; ++k) release(J, made[k]);
+        np = 0;
+        HIP_TRY(e);
+        return GPV_OK;
+    };
+    auto room = [&](size_t bytes) -> int {
+        int r = alloc(J, &made[np], bytes);
+        if (r == GPV_ERR_OOM && np > 0) {
+            TRY(flush());
+            r = alloc(J, &made[np], bytes);
+        }
+        if (r != GPV_OK) {
+            const std::string keep = g_err;
+            (void)flush();
+            g_err = keep;
+        }
+        return r;
+    };
     if (l1) {
-        uint8_t* d = nullptr;
-        TRY(alloc(J, &d, (size_t)n1));
-        launch_export_l1(J->bnd + o.word0, J->ins + o.word0, g, unit, d, s);
-        HIP_TRY(hipMemcpyAsync(l1, d, (size_t)n1, hipMemcpyDeviceToHost, s));
-        HIP_TRY(hipStreamSynchronize(s));
-        release(J, d);
+        TRY(room((size_t)n1));
+        launch_export_l1(J->bnd + o.word0, J->ins + o.word0, g, unit, made[np], s);
+        pieces[np] = {l1, made[np], (size_t)n1};
+        ++np;
     }
     if (prefix) {
-        int32_t* d = nullptr;
-        TRY(alloc(J, &d, (size_t)n1));
-        launch_export_prefix(J->bnd + o.word0, J->wprefix + o.word0, o.b0, g, d, s);
-        HIP_TRY(hipMemcpyAsync(prefix, d, (size_t)n1 * 4, hipMemcpyDeviceToHost, s));
-        HIP_TRY(hipStreamSynchronize(s));
-        release(J, d);
+        TRY(room((size_t)n1 * 4));
+        launch_export_prefix(J->bnd + o.word0, J->wprefix + o.word0, o.b0, g, reinterpret_cast<int32_t*>(made[np]), s);
+        pieces[np] = {prefix, made[np], (size_t)n1 * 4};
+        ++np;
     }
     if (bidx && nb > 0) {
-        HIP_TRY(hipMemcpyAsync(bidx, J->bidx + o.b0, (size_t)nb * 4, hipMemcpyDeviceToHost, s));
-        HIP_TRY(hipStreamSynchronize(s));
+        pieces[np] = {bidx, J->bidx + o.b0, (size_t)nb * 4};
+        ++np;
     }
     if (l2 && g.n2 > 0 && nb > 0) {
-        uint8_t* d = nullptr;
-        TRY(alloc(J, &d, (size_t)(nb * n23)));
-        launch_export_l2(J->sat2 + o.l2w0, J->par2 + o.l2w0, nb, g, unit, d, s);
-        HIP_TRY(hipMemcpyAsync(l2, d, (size_t)(nb * n23), hipMemcpyDeviceToHost, s));
-        HIP_TRY(hipStreamSynchronize(s));
-        release(J, d);
+        TRY(room((size_t)(nb * n23)));
+        launch_export_l2(J->sat2 + o.l2w0, J->par2 + o.l2w0, nb, g, unit, made[np], s);
+        pieces[np] = {l2, made[np], (size_t)(nb * n23)};
+        ++np;
     }
-    return GPV_OK;
+    return flush();
 }
 
 // states 0 outside / 1 inside / 2 boundary
@@ -2247,13 +2271,10 @@ int gpv_grid_download_normals(gpv_ctx* c, const gpv_grid* G, float* l1n, float* 
     const int64_t nb = J->nb(G->m);
     const int n2 = J->g[G->m].n2;
     const int64_t n23 = (int64_t)n2 * n2 * n2;
-    if (l1n && nb > 0)
-        HIP_TRY(hipMemcpyAsync(l1n, J->l1n + 3 * (size_t)o.b0, (size_t)nb * 3 * sizeof(float), hipMemcpyDeviceToHost,
-                               c->stream));
-    if (l2n && nb > 0 && n23 > 0)
-        HIP_TRY(hipMemcpyAsync(l2n, J->l2n + 3 * (size_t)o.l2n0, (size_t)(nb * n23) * 3 * sizeof(float),
-                               hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    const Downloader::Piece pieces[2] = {
+        {l1n, J->l1n + 3 * (size_t)o.b0, l1n && nb > 0 ? (size_t)nb * 3 * sizeof(float) : 0},
+        {l2n, J->l2n + 3 * (size_t)o.l2n0, l2n && nb > 0 ? (size_t)(nb * n23) * 3 * sizeof(float) : 0}};
+    HIP_TRY(c->down.run(pieces, 2, c->stream));
     return GPV_OK;
 }
 
