@@ -68,8 +68,8 @@ public:
 private:
     static constexpr size_t kAlign = 256;
     static constexpr size_t kSmall = size_t(256) << 10;   // one launch, no threads
-    static constexpr int kChunks = 16;                    // of a round
-    static constexpr size_t kChunkMin = size_t(256) << 10, kChunkMax = size_t(1) << 20;
+    static constexpr int kChunks = 8;                     // of a round
+    static constexpr size_t kChunkMin = size_t(512) << 10, kChunkMax = size_t(2) << 20;
     static constexpr int kHelpers = 3;
     static size_t up(size_t n) { return (n + kAlign - 1) / kAlign * kAlign; }
 

@@ -176,16 +176,39 @@ void launch_pack_bytes(const uint8_t* by, int64_t W, uint64_t* bits, uint32_t* c
 void launch_ray_expand(const float* tris, int64_t T, const int4* ray_rng, const uint64_t* off, const GridDev& g0,
                        const Meshes& M, uint64_t* ins, int blocks, hipStream_t s);
 
-// scratch of a two-level counting sort (ts_tiles(nkeys) tiles): total and
-// fill counters [2*tiles + 1], tile offsets [tiles + 1], bucket (8 bytes a bin
-// pair, 12 a column entry); cleared: the counters hold zeros
-struct TileSortTmp {
-    uint32_t* total;
+// words of scratch of a two-level counting sort with at most nkeys keys, zeros at its start
+size_t ts_words(uint64_t nkeys);
+
+// bin pairs (key = batch-wide boundary bit index, triangle) -> CSR by boundary rank
+// (off[B + 1], list); B <= 2^27.  The pairs' voxel bits are replaced by their
+// boundary ranks (ranked: they hold ranks already); max_out (or nullptr): the largest bin
+struct BinPairs {
+    uint64_t* bits;
+    bool ranked;
+    const uint32_t* tri;
+    uint64_t n;
+    uint32_t B;
+    uint32_t* cnt;   // [ts_words(B)]
+    void* bucket;    // 8 bytes a pair
     uint32_t* off;
-    void* bucket;
-    bool cleared;
+    unsigned int* max_out;
+    uint32_t* list;
 };
-size_t ts_tiles(uint64_t nkeys);
+// column entries (key = column << 32 | triangle) -> CSR by column of (triangle,
+// zmax); ncol <= 2^27, 0: none
+struct BinCols {
+    const uint64_t* key;
+    const uint32_t* zmax;
+    uint64_t n;
+    uint32_t ncol;
+    uint32_t* cnt;   // [ts_words(ncol)]
+    void* bucket;    // 12 bytes an entry
+    uint32_t* off;
+    uint2* ent;
+};
+// both sorts and the boundary index list
+void launch_bins(const BinPairs& P, const BinCols& C, const uint64_t* bnd, const uint32_t* wprefix, const GridDev& g0,
+                 const Meshes& M, int64_t W, int32_t* bidx, int items_per_block, hipStream_t s);
 
 // Level2 SAT voxel groups (k_l2_sat): consecutive boundary voxels of a mesh
 // that share a wave, at most `most` and kL2GroupMax of them, their layer bits
@@ -198,11 +221,6 @@ __host__ __device__ inline int l2_group_voxels(int n2, int most)
     if (c > kL2GroupMax) c = kL2GroupMax;
     return c < most ? c : most;
 }
-// column entries (key = column << 32 | triangle) -> CSR by column of (triangle,
-// zmax); ncol <= 2^27
-void launch_bin_cols(const uint64_t* key, const uint32_t* zmax, uint64_t n, uint32_t ncol, const TileSortTmp& tmp,
-                     int items_per_block, uint32_t* coff, uint2* ent, hipStream_t s);
-
 // Level1 fill: a block takes L1F_W words of a mesh's layer, all layers
 constexpr int L1F_W = 16;
 inline int64_t l1_fill_blocks(const GridDev& g) { return ((int64_t)g.ny * g.nxw + L1F_W - 1) / L1F_W; }
@@ -227,15 +245,6 @@ void launch_l1_fill(const GridDev& g0, const Meshes& M, int64_t blocks, uint64_t
 // b0 and l2w0 of every mesh (and the totals in entry nm) from the word prefix
 // and the counters, to the page-locked read-back pub as well
 void launch_mesh_bounds(const uint32_t* wprefix, const Meshes& M, const Counters* ctr, uint64_t* pub, hipStream_t s);
-// also clears nclear words
-void launch_boundary_index(const uint64_t* bnd, const uint32_t* wprefix, const GridDev& g0, const Meshes& M,
-                           int64_t W, int32_t* bidx, uint32_t* clear, int64_t nclear, hipStream_t s);
-// pairs: key = batch-wide boundary bit index, val = triangle
-// bin pairs -> CSR by boundary rank (boff[B + 1], list); B <= 2^27.  The pairs' voxel bits are replaced by their boundary
-// ranks (ranked: they hold ranks already)
-void launch_bin_pairs(uint64_t* bits, bool ranked, const uint32_t* tri, uint64_t n, const uint64_t* bnd,
-                      const uint32_t* wprefix, uint32_t B, const TileSortTmp& tmp, int items_per_block,
-                      uint32_t* boff, unsigned int* max_out, uint32_t* list, hipStream_t s);
 // per-mesh bin totals and largest bin (multi-mesh runs)
 void launch_mesh_bins(const uint32_t* boff, int64_t B, const Meshes& M, hipStream_t s);
 

@@ -1588,17 +1588,13 @@ void launch_mesh_bounds(const uint32_t* wprefix, const Meshes& M, const Counters
 }
 
 // ascending linear indices (within the mesh) of the boundary voxels, and in a
-// batch the mesh of each
+// batch the mesh of each; block `blk` of `blocks`
 template <bool kM>
-__global__ void k_boundary_index(const uint64_t* __restrict__ bnd, const uint32_t* __restrict__ wprefix,
-                                 GridDev g0, Meshes M, int64_t W, int32_t* __restrict__ bidx,
-                                 uint32_t* __restrict__ clear, int64_t nclear)
+__device__ __forceinline__ void boundary_index(const uint64_t* __restrict__ bnd, const uint32_t* __restrict__ wprefix,
+                                               const GridDev& g0, const Meshes& M, int64_t W, int32_t* __restrict__ bidx,
+                                               uint32_t blk, uint32_t blocks)
 {
-    // the counters of the sort that follows
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nclear; i += (int64_t)gridDim.x * blockDim.x)
-        clear[i] = 0;
-    for (int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; w < W;
-         w += (int64_t)gridDim.x * blockDim.x) {
+    for (int64_t w = (int64_t)blk * blockDim.x + threadIdx.x; w < W; w += (int64_t)blocks * blockDim.x) {
         uint64_t bits = bnd[w];
         if (!bits) continue;
         uint32_t pos = wprefix[w];
@@ -1614,16 +1610,6 @@ __global__ void k_boundary_index(const uint64_t* __restrict__ bnd, const uint32_
             bidx[pos++] = (int32_t)(row * g.nx + xw * 64 + bit);
         }
     }
-}
-
-void launch_boundary_index(const uint64_t* bnd, const uint32_t* wprefix, const GridDev& g0, const Meshes& M,
-                           int64_t W, int32_t* bidx, uint32_t* clear, int64_t nclear, hipStream_t s)
-{
-    const int blocks = grid_for(W, 256, 16384);
-    if (M.nm > 1)
-        k_boundary_index<true><<<blocks, 256, 0, s>>>(bnd, wprefix, g0, M, W, bidx, clear, nclear);
-    else
-        k_boundary_index<false><<<blocks, 256, 0, s>>>(bnd, wprefix, g0, M, W, bidx, clear, nclear);
 }
 
 __device__ __forceinline__ uint32_t rank_of(const uint64_t* __restrict__ bnd,
@@ -1650,9 +1636,58 @@ __device__ __forceinline__ uint32_t rank_of(const uint64_t* __restrict__ bnd,
 constexpr int TS_NT = 256;
 constexpr int TS_U = 4;
 
-__device__ __forceinline__ void ts_range(uint64_t n, uint64_t& lo, uint64_t& hi)
+// A bin pair sorts by the rank of its voxel among the boundary voxels; its item
+// is (rank, triangle).
+struct PairSrc {
+    using Item = uint2;
+    // per pair, its voxel's bit in the Level1 grid; the count pass writes the
+    // voxel's boundary rank over it (ranked: a repeated compaction, whose
+    // pairs hold ranks already), so the bucket pass reads the rank directly
+    uint64_t* bits;
+    bool ranked;
+    const uint32_t* tri;
+    const uint64_t* bnd;
+    const uint32_t* wprefix;
+    __device__ uint32_t count_key(uint64_t i) const
+    {
+        return ranked ? (uint32_t)bits[i] : rank_of(bnd, wprefix, bits[i]);
+    }
+    __device__ void keep_key(uint64_t i, uint32_t k) const
+    {
+        if (!ranked) bits[i] = k;
+    }
+    __device__ uint32_t sort_key(uint64_t i) const { return (uint32_t)bits[i]; }
+    __device__ uint2 item(uint64_t i) const { return make_uint2((uint32_t)bits[i], tri[i]); }
+};
+
+struct PairPlace {
+    using Item = uint2;
+    uint32_t* list;
+    __device__ void operator()(uint32_t pos, const uint2& it, bool ok) const
+    {
+        if (ok) list[pos] = it.y;
+    }
+};
+
+// One sort of a launch: its scratch (total[ntiles], fill[ntiles], done[1], zeros at the
+// start, then off[ntiles + 1]) and the blocks that share its items; none: no sort.
+template <typename Src>
+struct TsSort {
+    Src src;
+    uint64_t n;
+    uint32_t nkeys;
+    int shift, ntiles, blocks;
+    uint32_t* cnt;
+    typename Src::Item* bucket;
+    __device__ uint32_t* total() const { return cnt; }
+    __device__ uint32_t* fill() const { return cnt + ntiles; }
+    __device__ uint32_t* done() const { return cnt + 2 * ntiles; }
+    __device__ uint32_t* off() const { return cnt + 2 * ntiles + 1; }
+};
+
+__device__ __forceinline__ void ts_range(uint64_t n, int blocks, uint64_t& lo, uint64_t& hi)
 {
-    const uint64_t per = (n + gridDim.x - 1) / gridDim.x;
+    const uint64_t per = (n + blocks - 1) / blocks;
     lo = (uint64_t)blockIdx.x * per;
     hi = lo + per < n ? lo + per : n;
 }
@@ -1683,16 +1718,18 @@ __device__ __forceinline__ void ts_histogram(const Src& src, uint64_t lo, uint64
 }
 
 // Tile totals -> tile offsets by one block of NT threads; s_h holds
-// ts_scan_words(ntiles) words, a word in 33 left out so that the threads' runs
-// start in different banks.  Atomic loads: blocks of the same launch added the totals.
-__host__ __device__ inline size_t ts_scan_words(int ntiles) { return (size_t)ntiles + (size_t)ntiles / 32 + 1; }
-__device__ __forceinline__ int ts_at(int t) { return t + (t >> 5); }
+// ts_scan_words(ntiles) words, up to 8192 tiles a word in 33 left out so that the
+// threads' runs start in different banks.  Atomic loads: blocks of the same launch added the totals.
+__host__ __device__ inline int ts_pad(int ntiles) { return ntiles <= 8192 ? 5 : 31; }
+__host__ __device__ inline size_t ts_scan_words(int ntiles) { return (size_t)ntiles + (size_t)(ntiles >> ts_pad(ntiles)); }
 
 template <int NT>
 __device__ __forceinline__ void ts_scan(const uint32_t* __restrict__ total, uint32_t* __restrict__ off, int ntiles,
                                         uint32_t* s_h, uint32_t* s_wave)
 {
     constexpr int U = 8;
+    const int pad = ts_pad(ntiles);
+    auto at = [pad](int t) { return t + (t >> pad); };
     for (int t0 = threadIdx.x; t0 < ntiles; t0 += U * NT) {
         uint32_t v[U];
 #pragma unroll
@@ -1702,12 +1739,12 @@ __device__ __forceinline__ void ts_scan(const uint32_t* __restrict__ total, uint
         }
 #pragma unroll
         for (int u = 0; u < U; ++u)
-            if (t0 + u * NT < ntiles) s_h[ts_at(t0 + u * NT)] = v[u];
+            if (t0 + u * NT < ntiles) s_h[at(t0 + u * NT)] = v[u];
     }
     __syncthreads();
     const int C = (ntiles + NT - 1) / NT, c0 = (int)threadIdx.x * C, c1 = c0 + C < ntiles ? c0 + C : ntiles;
     uint32_t sum = 0;
-    for (int t = c0; t < c1; ++t) sum += s_h[ts_at(t)];
+    for (int t = c0; t < c1; ++t) sum += s_h[at(t)];
     const int lane = __lane_id(), wid = threadIdx.x >> 6;
     const uint32_t inc = wave_incl_scan<uint32_t>(sum);
     if (lane == 63) s_wave[wid] = inc;
@@ -1715,88 +1752,111 @@ __device__ __forceinline__ void ts_scan(const uint32_t* __restrict__ total, uint
     uint32_t run = inc - sum;
     for (int w = 0; w < wid; ++w) run += s_wave[w];
     for (int t = c0; t < c1; ++t) {
-        const uint32_t v = s_h[ts_at(t)];
-        s_h[ts_at(t)] = run;
+        const uint32_t v = s_h[at(t)];
+        s_h[at(t)] = run;
         run += v;
     }
     if (threadIdx.x == NT - 1) off[ntiles] = run;
     __syncthreads();
-    for (int t = threadIdx.x; t < ntiles; t += NT) off[t] = s_h[ts_at(t)];
+    for (int t = threadIdx.x; t < ntiles; t += NT) off[t] = s_h[at(t)];
 }
 
-__global__ __launch_bounds__(1024) void k_ts_scan(const uint32_t* __restrict__ total, uint32_t* __restrict__ off, int ntiles)
+// a block per sort
+template <typename A, typename B>
+__global__ __launch_bounds__(1024) void k_ts_scan(TsSort<A> a, TsSort<B> b)
 {
     extern __shared__ uint32_t s_h[];   // [ts_scan_words(ntiles)]
     __shared__ uint32_t s_wave[16];
-    ts_scan<1024>(total, off, ntiles, s_h, s_wave);
+    if (blockIdx.x == 0 && a.blocks) ts_scan<1024>(a.total(), a.off(), a.ntiles, s_h, s_wave);
+    if (blockIdx.x == 1 && b.blocks) ts_scan<1024>(b.total(), b.off(), b.ntiles, s_h, s_wave);
 }
 
-// done != nullptr: the last block to get through makes the tiles' offsets, and
+// last: the last block of a sort to get through makes the tiles' offsets, and
 // s_h holds ts_scan_words(ntiles)
 template <typename Src>
-__global__ __launch_bounds__(TS_NT) void k_ts_count(Src src, uint64_t n, int shift, int ntiles,
-                                                    uint32_t* __restrict__ tile_total,
-                                                    uint32_t* __restrict__ tile_off, uint32_t* __restrict__ done)
+__device__ __forceinline__ void ts_count(const TsSort<Src>& S, bool last, uint32_t* s_h, uint32_t* s_wave, uint32_t* s_last)
+{
+    if ((int)blockIdx.x >= S.blocks) return;
+    for (int t = threadIdx.x; t < S.ntiles; t += TS_NT) s_h[t] = 0;
+    __syncthreads();
+    uint64_t lo, hi;
+    ts_range(S.n, S.blocks, lo, hi);
+    ts_histogram<true>(S.src, lo, hi, S.shift, s_h);
+    __syncthreads();
+    for (int t = threadIdx.x; t < S.ntiles; t += TS_NT)
+        if (s_h[t]) atomicAdd(&S.total()[t], s_h[t]);
+    if (!last) return;
+    wait_atomics();
+    __syncthreads();
+    if (threadIdx.x == 0) *s_last = atomicAdd(S.done(), 1u) == (uint32_t)S.blocks - 1u ? 1u : 0u;
+    __syncthreads();
+    if (*s_last) ts_scan<TS_NT>(S.total(), S.off(), S.ntiles, s_h, s_wave);
+}
+
+// Row 0 of the grid counts the bin pairs, row 1 the column entries, row 2 makes the
+// boundary index list: they depend on the boundary plane and the appends alone, and
+// one launch costs what each of three does.
+template <bool kM>
+__global__ __launch_bounds__(TS_NT) void k_ts_count(TsSort<PairSrc> a, TsSort<ColSrc> b, bool last, GridDev g0, Meshes M,
+                                                    const uint64_t* __restrict__ bnd, const uint32_t* __restrict__ wprefix,
+                                                    int64_t W, int32_t* __restrict__ bidx)
 {
     extern __shared__ uint32_t s_h[];   // [ntiles]
     __shared__ uint32_t s_wave[TS_NT / 64];
     __shared__ uint32_t s_last;
-    for (int t = threadIdx.x; t < ntiles; t += TS_NT) s_h[t] = 0;
-    __syncthreads();
-    uint64_t lo, hi;
-    ts_range(n, lo, hi);
-    ts_histogram<true>(src, lo, hi, shift, s_h);
-    __syncthreads();
-    for (int t = threadIdx.x; t < ntiles; t += TS_NT)
-        if (s_h[t]) atomicAdd(&tile_total[t], s_h[t]);
-    if (!done) return;
-    wait_atomics();
-    __syncthreads();
-    if (threadIdx.x == 0) s_last = atomicAdd(done, 1u) == gridDim.x - 1 ? 1u : 0u;
-    __syncthreads();
-    if (s_last) ts_scan<TS_NT>(tile_total, tile_off, ntiles, s_h, s_wave);
+    if (blockIdx.y == 0) ts_count(a, last, s_h, s_wave, &s_last);
+    else if (blockIdx.y == 1) ts_count(b, last, s_h, s_wave, &s_last);
+    else boundary_index<kM>(bnd, wprefix, g0, M, W, bidx, blockIdx.x, gridDim.x);
 }
 
 // items (.x = key) to their tile's bucket range; the item is built
 // here, where the block reads its inputs in their original order
 template <typename Src>
-__global__ __launch_bounds__(TS_NT) void k_ts_bucket(Src src, uint64_t n, int shift, int ntiles,
-                                                     const uint32_t* __restrict__ tile_off,
-                                                     uint32_t* __restrict__ tile_fill,
-                                                     typename Src::Item* __restrict__ bucket)
+__device__ __forceinline__ void ts_bucket(const TsSort<Src>& S, uint32_t* s_h)   // counts, then this block's next slot per tile
 {
-    extern __shared__ uint32_t s_h[];   // [ntiles]: counts, then this block's next slot per tile
-    for (int t = threadIdx.x; t < ntiles; t += TS_NT) s_h[t] = 0;
+    if ((int)blockIdx.x >= S.blocks) return;
+    for (int t = threadIdx.x; t < S.ntiles; t += TS_NT) s_h[t] = 0;
     __syncthreads();
     uint64_t lo, hi;
-    ts_range(n, lo, hi);
-    ts_histogram<false>(src, lo, hi, shift, s_h);
+    ts_range(S.n, S.blocks, lo, hi);
+    ts_histogram<false>(S.src, lo, hi, S.shift, s_h);
     __syncthreads();
-    for (int t = threadIdx.x; t < ntiles; t += TS_NT)
-        if (s_h[t]) s_h[t] = tile_off[t] + atomicAdd(&tile_fill[t], s_h[t]);
+    const uint32_t* off = S.off();
+    uint32_t* fill = S.fill();
+    for (int t = threadIdx.x; t < S.ntiles; t += TS_NT)
+        if (s_h[t]) s_h[t] = off[t] + atomicAdd(&fill[t], s_h[t]);
     __syncthreads();
     for (uint64_t i0 = lo + threadIdx.x; i0 < hi; i0 += (uint64_t)TS_U * TS_NT) {
         typename Src::Item it[TS_U];
 #pragma unroll
         for (int u = 0; u < TS_U; ++u) {
             const uint64_t i = i0 + (uint64_t)u * TS_NT;
-            it[u] = src.item(i < hi ? i : i0);
+            it[u] = S.src.item(i < hi ? i : i0);
         }
 #pragma unroll
         for (int u = 0; u < TS_U; ++u)
-            if (i0 + (uint64_t)u * TS_NT < hi) bucket[atomicAdd(&s_h[it[u].x >> shift], 1u)] = it[u];
+            if (i0 + (uint64_t)u * TS_NT < hi) S.bucket[atomicAdd(&s_h[it[u].x >> S.shift], 1u)] = it[u];
     }
 }
 
-template <typename Place>
-__global__ __launch_bounds__(TS_NT) void k_ts_place(const typename Place::Item* __restrict__ bucket,
-                                                    const uint32_t* __restrict__ tile_off, int shift,
-                                                    uint32_t nkeys, uint32_t* __restrict__ off,
-                                                    unsigned int* __restrict__ max_out, Place place)
+__global__ __launch_bounds__(TS_NT) void k_ts_bucket(TsSort<PairSrc> a, TsSort<ColSrc> b)
 {
-    extern __shared__ uint32_t s_c[];   // [2^shift] key counts, then next slots
-    __shared__ uint32_t s_wave[TS_NT / 64];
-    __shared__ uint32_t s_max;
+    extern __shared__ uint32_t s_h[];   // [ntiles]
+    if (blockIdx.y == 0) ts_bucket(a, s_h);
+    else ts_bucket(b, s_h);
+}
+
+template <typename Src, typename Place>
+__device__ __forceinline__ void ts_place(const TsSort<Src>& S, uint32_t* __restrict__ off, unsigned int* __restrict__ max_out,
+                                         const Place& place, uint32_t* s_c /* [2^shift] key counts, then next slots */,
+                                         uint32_t* s_wave, uint32_t* s_maxp)
+{
+    if (!S.blocks || (int)blockIdx.x >= S.ntiles) return;
+    uint32_t& s_max = *s_maxp;
+    const typename Place::Item* __restrict__ bucket = S.bucket;
+    const uint32_t* __restrict__ tile_off = S.off();
+    const int shift = S.shift;
+    const uint32_t nkeys = S.nkeys;
     const uint32_t T = 1u << shift;
     const uint32_t k0 = (uint32_t)blockIdx.x << shift;
     const uint32_t b0 = tile_off[blockIdx.x], b1 = tile_off[blockIdx.x + 1];
@@ -1860,6 +1920,16 @@ __global__ __launch_bounds__(TS_NT) void k_ts_place(const typename Place::Item* 
     }
 }
 
+__global__ __launch_bounds__(TS_NT) void k_ts_place(TsSort<PairSrc> a, uint32_t* boff, unsigned int* max_out, PairPlace pa,
+                                                    TsSort<ColSrc> b, uint32_t* coff, ColPlace pb)
+{
+    extern __shared__ uint32_t s_c[];
+    __shared__ uint32_t s_wave[TS_NT / 64];
+    __shared__ uint32_t s_max;
+    if (blockIdx.y == 0) ts_place(a, boff, max_out, pa, s_c, s_wave, &s_max);
+    else ts_place(b, coff, nullptr, pb, s_c, s_wave, &s_max);
+}
+
 // tile size 2^shift, 2^8 (TS_NT) to 2^13 keys: at most 8192 tiles below 2^26
 // keys, 16384 at 2^27.  The count and bucket passes hold a counter per tile
 // in every block's LDS (32 KiB at 8192 tiles: five blocks per CU, where
@@ -1873,88 +1943,47 @@ int ts_shift(uint64_t nkeys)
     return sh < 8 ? 8 : sh > 13 ? 13 : sh;
 }
 
-template <typename Src, typename Place>
-static void ts_sort(Src src, uint64_t n, uint32_t nkeys, const TileSortTmp& tmp, int items_per_block, uint32_t* off,
-                    unsigned int* max_out, Place place, hipStream_t s)
-{
-    const int shift = ts_shift(nkeys);
-    const int ntiles = (int)((nkeys + (1u << shift) - 1) >> shift);
-    if (ntiles == 0) {   // no keys, hence no items
-        launch_fill_u32(off, 0, 1, s);
-        return;
-    }
-    // total[ntiles], fill[ntiles], done
-    if (!tmp.cleared) launch_fill_u32(tmp.total, 0, 2 * (int64_t)ntiles + 1, s);
-    typename Src::Item* bucket = static_cast<typename Src::Item*>(tmp.bucket);
-    uint32_t* fill = tmp.total + ntiles;
-    if (n > 0) {
-        const uint64_t ipb = (uint64_t)items_per_block;
-        const int blocks = (int)std::min<uint64_t>(2048, std::max<uint64_t>(1, (n + ipb - 1) / ipb));
-        const size_t lds = (size_t)ntiles * 4;
-        // Tile offsets by the count's last block where that is less than the launch it
-        // saves (5 us): the blocks' counter takes 3.7 ns each, and 256 threads a
-        // tile each a round
-        const bool last = blocks <= 256 && ntiles <= 2048;
-        k_ts_count<Src><<<blocks, TS_NT, last ? ts_scan_words(ntiles) * 4 : lds, s>>>(src, n, shift, ntiles, tmp.total, tmp.off,
-                                                                                   last ? fill + ntiles : nullptr);
-        if (!last) k_ts_scan<<<1, 1024, ts_scan_words(ntiles) * 4, s>>>(tmp.total, tmp.off, ntiles);
-        k_ts_bucket<Src><<<blocks, TS_NT, lds, s>>>(src, n, shift, ntiles, tmp.off, fill, bucket);
-    } else {
-        launch_fill_u32(tmp.off, 0, (int64_t)ntiles + 1, s);
-    }
-    k_ts_place<Place><<<ntiles, TS_NT, (size_t)4 << shift, s>>>(bucket, tmp.off, shift, nkeys, off, max_out, place);
-}
-
 size_t ts_tiles(uint64_t nkeys)
 {
     const int shift = ts_shift(nkeys);
     return (size_t)((nkeys + (1u << shift) - 1) >> shift);
 }
 
-// A bin pair sorts by the rank of its voxel among the boundary voxels; its item
-// is (rank, triangle).
-struct PairSrc {
-    using Item = uint2;
-    // per pair, its voxel's bit in the Level1 grid; the count pass writes the
-    // voxel's boundary rank over it (ranked: a repeated compaction, whose
-    // pairs hold ranks already), so the bucket pass reads the rank directly
-    uint64_t* bits;
-    bool ranked;
-    const uint32_t* tri;
-    const uint64_t* bnd;
-    const uint32_t* wprefix;
-    __device__ uint32_t count_key(uint64_t i) const
-    {
-        return ranked ? (uint32_t)bits[i] : rank_of(bnd, wprefix, bits[i]);
-    }
-    __device__ void keep_key(uint64_t i, uint32_t k) const
-    {
-        if (!ranked) bits[i] = k;
-    }
-    __device__ uint32_t sort_key(uint64_t i) const { return (uint32_t)bits[i]; }
-    __device__ uint2 item(uint64_t i) const { return make_uint2((uint32_t)bits[i], tri[i]); }
-};
+// tiles of any sort with at most nkeys keys
+static size_t ts_tiles_most(uint64_t nkeys) { return nkeys <= (1u << 21) ? ts_tiles(nkeys) : nkeys <= (1u << 26) ? 8192 : 16384; }
 
-struct PairPlace {
-    using Item = uint2;
-    uint32_t* list;
-    __device__ void operator()(uint32_t pos, const uint2& it, bool ok) const
-    {
-        if (ok) list[pos] = it.y;
-    }
-};
+size_t ts_words(uint64_t nkeys) { return (3 * ts_tiles_most(nkeys) + 3) / 2 * 2; }
 
-void launch_bin_cols(const uint64_t* key, const uint32_t* zmax, uint64_t n, uint32_t ncol, const TileSortTmp& tmp,
-                     int items_per_block, uint32_t* coff, uint2* ent, hipStream_t s)
+template <typename Src>
+static TsSort<Src> ts_sort(Src src, uint64_t n, uint32_t nkeys, uint32_t* cnt, void* bucket, int items_per_block)
 {
-    ts_sort(ColSrc{key, zmax}, n, ncol, tmp, items_per_block, coff, nullptr, ColPlace{ent}, s);
+    const uint64_t ipb = (uint64_t)items_per_block;
+    const int blocks = nkeys ? (int)std::min<uint64_t>(2048, std::max<uint64_t>(1, (n + ipb - 1) / ipb)) : 0;
+    return TsSort<Src>{src, n, nkeys, ts_shift(nkeys), (int)ts_tiles(nkeys), blocks, cnt, static_cast<typename Src::Item*>(bucket)};
 }
 
-void launch_bin_pairs(uint64_t* bits, bool ranked, const uint32_t* tri, uint64_t n, const uint64_t* bnd,
-                      const uint32_t* wprefix, uint32_t B, const TileSortTmp& tmp, int items_per_block,
-                      uint32_t* boff, unsigned int* max_out, uint32_t* list, hipStream_t s)
+void launch_bins(const BinPairs& P, const BinCols& C, const uint64_t* bnd, const uint32_t* wprefix, const GridDev& g0,
+                 const Meshes& M, int64_t W, int32_t* bidx, int items_per_block, hipStream_t s)
 {
-    ts_sort(PairSrc{bits, ranked, tri, bnd, wprefix}, n, B, tmp, items_per_block, boff, max_out, PairPlace{list}, s);
+    const auto a = ts_sort(PairSrc{P.bits, P.ranked, P.tri, bnd, wprefix}, P.n, P.B, P.cnt, P.bucket, items_per_block);
+    const auto b = ts_sort(ColSrc{C.key, C.zmax}, C.n, C.ncol, C.cnt, C.bucket, items_per_block);
+    const int blocks = std::max(a.blocks, b.blocks), tiles = std::max(a.ntiles, b.ntiles);
+    // Tile offsets by the count's last block where that is less than the launch it
+    // saves (5 us): the blocks' counter takes 3.7 ns each, and 256 threads a
+    // tile each a round
+    const bool last = blocks <= 256 && tiles <= 2048;
+    const size_t lds = last ? ts_scan_words(tiles) * 4 : (size_t)tiles * 4;
+    const dim3 grid((unsigned)std::max(blocks, grid_for(W, TS_NT, 2048)), 3);
+    if (M.nm > 1)
+        k_ts_count<true><<<grid, TS_NT, lds, s>>>(a, b, last, g0, M, bnd, wprefix, W, bidx);
+    else
+        k_ts_count<false><<<grid, TS_NT, lds, s>>>(a, b, last, g0, M, bnd, wprefix, W, bidx);
+    if (!P.B) launch_fill_u32(P.off, 0, 1, s);   // no keys, hence no items
+    if (!blocks) return;
+    if (!last) k_ts_scan<<<2, 1024, ts_scan_words(tiles) * 4, s>>>(a, b);
+    k_ts_bucket<<<dim3((unsigned)blocks, 2), TS_NT, (size_t)tiles * 4, s>>>(a, b);
+    k_ts_place<<<dim3((unsigned)tiles, 2), TS_NT, (size_t)4 << std::max(a.shift, b.shift), s>>>(a, P.off, P.max_out, PairPlace{P.list}, b,
+                                                                                          C.off, ColPlace{C.ent});
 }
 
 // Per-mesh bin totals (pairs) and largest bin of a batch: the blocks of a

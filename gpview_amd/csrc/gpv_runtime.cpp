@@ -270,9 +270,10 @@ struct Job {
     uint64_t* scan_ray = nullptr;   // scan temporary of the ray half of the set-up (side stream)
     uint64_t *sat_sums = nullptr, *ray_sums = nullptr;   // items per 256 triangles
     uint8_t* bbytes = nullptr;       // boundary flags of the Level1 SAT
+    bool sat_timed = false;          // ev[1] is recorded
+    bool one_setup = false;          // both halves of the set-up ran before ev[1]
     bool sat_cleared = false;        // flags and counters of the sweep hold zeros
     bool ins_cleared = false;        // the inside plane holds zeros
-    bool cols_cleared = false;       // the column sort's counters hold zeros
     uint32_t* scan32 = nullptr;
     size_t scan_cap = 0;
     Counters* ctr = nullptr;
@@ -296,10 +297,11 @@ struct Job {
     uint32_t *boff = nullptr, *list = nullptr;
     uint32_t* coff = nullptr;
     uint2* cent = nullptr;    // (triangle, zmax) of the column entries
-    // column-entry sort on the side stream (beside the bins): its own scratch
-    bool cols_side = false;
-    uint32_t* cs_cnt = nullptr;
-    uint32_t* cs_bucket = nullptr;   // 3 words per column entry
+    // scratch of the two sorts: their counters (zeros since the set-up or not) and buckets
+    uint32_t *pair_cnt = nullptr, *col_cnt = nullptr;
+    size_t bin_words = 0;
+    bool bins_cleared = false;
+    bool streams = false;            // the Level2 stages ran on two streams
     int64_t l2p_waves = 0, l2s_groups = 0;   // Level2 parity waves, SAT groups (l2_plan)
     int l2s_most = 1;                        // most voxels of a SAT group
     // GL-stencil-equivalent Level1 fill (meshes with params.l1_stencil):
@@ -319,8 +321,8 @@ struct Job {
     // progress
     bool setup_done = false, sat_done = false, inout_done = false, compact_done = false,
          l2p_done = false, l2s_done = false, finished = false;
-    // stream events: 0 setup, 1 L1 SAT, 2 L1 parity, 3 fork of the Level2 side stream,
-    // 4 compaction+bins, 5 L2 parity, 6 L2 SAT start, 7 L2 SAT end, 8 finish,
+    // stream events: 0 setup, 1 L1 SAT, 2 L1 parity,
+    // 4 compaction+bins, 5 its end (6 where the Level2 parity forks), 6 L2 SAT start, 7 L2 SAT end, 8 finish,
     // 9 normals start, 10 normals end, 11 L2 parity end, 12 L1 SAT end,
     // 13 L1 parity end, 14 end of the side stream, 15 fork of the L1 parity, 16 L2 parity start
     hipEvent_t ev[kJobEvents] = {};
@@ -775,6 +777,17 @@ int job_create(gpv_ctx* c, const gpv_mesh_desc* d, int nm, int on_device, Job** 
     return GPV_OK;
 }
 
+// counters of both sorts, one after the other, for at most `most` boundary voxels
+int alloc_bin_counters(Job* J, uint64_t most)
+{
+    release(J, J->pair_cnt);
+    const size_t a = ts_words(most), b = J->n2max > 0 ? ts_words((uint64_t)J->ncol) : 0;
+    TRY(alloc(J, &J->pair_cnt, a + b));
+    J->col_cnt = J->pair_cnt + a;
+    J->bin_words = a + b;
+    return GPV_OK;
+}
+
 // per-triangle setup shared by the SAT and the ray paths
 int stage_setup(Job* J)
 {
@@ -802,7 +815,8 @@ int stage_setup(Job* J)
 constexpr int64_t kSetupSplit = int64_t(1) << 16;
 
 // The fused pipeline's set-up: everything cleared in one launch, then the SAT half on
-// the main stream and the ray half on the side stream, forked at ev[15].
+// the main stream and the ray half on the side stream, forked at ev[15] (ev[1] where
+// they are one launch).
 int stage_setup_split(Job* J)
 {
     gpv_ctx* c = J->ctx;
@@ -812,26 +826,27 @@ int stage_setup_split(Job* J)
     release(J, J->scan_ray);
     TRY(alloc(J, &J->scan_ray, scan_tmp_elems(J->T)));
     TRY(alloc(J, &J->bbytes, (size_t)J->W * 64));
-    const size_t tiles = ts_tiles((uint64_t)J->ncol);
-    if (J->n2max > 0) TRY(alloc(J, &J->cs_cnt, 3 * tiles + 2));
+    TRY(alloc_bin_counters(J, (uint64_t)std::min<int64_t>(J->W * 64, int64_t(1) << 27)));
     launch_clear(ClearList{{reinterpret_cast<uint64_t*>(J->mctr), reinterpret_cast<uint64_t*>(J->ctr),
-                            reinterpret_cast<uint64_t*>(J->bbytes), J->ins, reinterpret_cast<uint64_t*>(J->cs_cnt)},
+                            reinterpret_cast<uint64_t*>(J->bbytes), J->ins, reinterpret_cast<uint64_t*>(J->pair_cnt)},
                            {(int64_t)(sizeof(MeshCtr) / 8) * J->nm, (int64_t)(sizeof(Counters) / 8), J->W * 8,
-                            J->all_stencil ? 0 : J->W, J->n2max > 0 ? (int64_t)tiles + 1 : 0}},
+                            J->all_stencil ? 0 : J->W, (int64_t)(J->bin_words / 2)}},
                  J->nm > 1 ? nullptr : &J->g[0], s);
     if (J->nm > 1) launch_tables(J->view(), s);
     J->sat_cleared = true;
     J->ins_cleared = true;
-    J->cols_cleared = true;
+    J->bins_cleared = true;
     if (J->nm > 1) launch_mesh_ids(J->d_off, J->nm, J->T, J->tri_mesh, s);
     const bool one = J->T <= kSetupSplit && !J->all_stencil;
-    if (!one) HIP_TRY(hipEventRecord(J->ev[15], s));
+    if (!one) HIP_TRY(hipEventRecord(J->ev[15], s));   // the fork
     launch_tri_setup(J->tris, J->T, J->g[0], J->view(), J->box0, J->box1, J->sat_items, J->rng, J->ray_items,
                      J->sat_sums, J->ray_sums, one ? 3 : 1, &J->ctr->bad_input, s);
     launch_scan_items(J->sat_items, J->sat_off, J->sat_sums, one ? J->ray_items : nullptr, J->ray_off, J->ray_sums, J->T,
                       J->scan64, s);
-    if (one) HIP_TRY(hipEventRecord(J->ev[15], s));
-    HIP_TRY(hipStreamWaitEvent(c->side, J->ev[15], 0));
+    HIP_TRY(hipEventRecord(J->ev[1], s));
+    J->sat_timed = true;
+    J->one_setup = one;
+    HIP_TRY(hipStreamWaitEvent(c->side, J->ev[one ? 1 : 15], 0));
     if (!one && !J->all_stencil) {   // the ray half feeds only the ray parity
         launch_tri_setup(J->tris, J->T, J->g[0], J->view(), J->box0, J->box1, J->sat_items, J->rng, J->ray_items,
                          J->sat_sums, J->ray_sums, 2, &J->ctr->bad_input, c->side);
@@ -848,7 +863,8 @@ int launch_sat_half(Job* J)
 {
     gpv_ctx* c = J->ctx;
     hipStream_t s = c->stream;
-    HIP_TRY(hipEventRecord(J->ev[1], s));
+    if (!J->sat_timed) HIP_TRY(hipEventRecord(J->ev[1], s));
+    J->sat_timed = false;
     // boundary flags as bytes (plain stores from the SAT), packed to bits after
     if (!J->sat_cleared) {
         release(J, J->bbytes);
@@ -882,7 +898,7 @@ int launch_stencil(Job* J, hipStream_t s);
 int launch_ray_half(Job* J, hipStream_t s)
 {
     gpv_ctx* c = J->ctx;
-    HIP_TRY(hipEventRecord(J->ev[2], s));
+    if (!J->one_setup) HIP_TRY(hipEventRecord(J->ev[2], s));
     if (!J->all_stencil) {   // the ray parity skips the stencil meshes
         if (!J->ins_cleared) launch_fill_u64(J->ins, 0, J->W, s);
         J->ins_cleared = false;
@@ -978,31 +994,6 @@ int launch_stencil(Job* J, hipStream_t s)
     return GPV_OK;
 }
 
-// buffers of the column-entry sort when it runs on the side stream (its counters
-// are there since the set-up)
-// (allocated before the fork, released after the Level2 join)
-int alloc_cols(Job* J)
-{
-    release(J, J->coff);
-    release(J, J->cent);
-    release(J, J->cs_bucket);
-    TRY(alloc(J, &J->coff, (size_t)J->ncol + 1));
-    TRY(alloc(J, &J->cent, (size_t)std::max<uint64_t>(J->n_cols, 1)));
-    return alloc(J, &J->cs_bucket, 3 * (size_t)std::max<uint64_t>(J->n_cols, 1));
-}
-
-// column entries by column, on stream s
-int col_sort_kernels(Job* J, hipStream_t s)
-{
-    const size_t tiles = ts_tiles((uint64_t)J->ncol);
-    const TileSortTmp ts{J->cs_cnt, J->cs_cnt + 2 * tiles + 1, J->cs_bucket, J->cols_cleared};
-    J->cols_cleared = false;
-    const int ipb = std::max(256, J->ctx->tune.sort_items_per_block);
-    launch_bin_cols(J->col_key, J->col_z, J->n_cols, (uint32_t)J->ncol, ts, ipb, J->coff, J->cent, s);
-    HIP_TRY(hipGetLastError());
-    return GPV_OK;
-}
-
 // the Level2 planes: allocated before the side stream forks, whose parity
 // writes one of them
 int alloc_level2(Job* J)
@@ -1038,39 +1029,34 @@ int launch_compact(Job* J)
     if (J->nm > 1) TRY(alloc(J, &J->bmesh, Bn));
     release(J, J->boff);
     release(J, J->list);
+    release(J, J->coff);
+    release(J, J->cent);
     TRY(alloc(J, &J->boff, (size_t)J->B + 1));
     TRY(alloc(J, &J->list, (size_t)std::max<uint64_t>(J->n_pairs, 1)));
-    // one scratch for both counting sorts (bins by boundary rank, column
-    // entries by column)
-    const bool cols = J->n2max > 0 && !J->cols_side;   // only the Level2 parity reads them
-    const size_t tiles = !cols ? ts_tiles((uint64_t)J->B)
-                                      : std::max(ts_tiles((uint64_t)J->B), ts_tiles((uint64_t)J->ncol));
-    TileSortTmp ts{};
-    uint32_t* ts_cnt = nullptr;
-    uint32_t* ts_bucket = nullptr;
-    TRY(alloc(J, &ts_cnt, 3 * tiles + 2));
-    TRY(alloc(J, &ts_bucket,
-              (size_t)std::max<uint64_t>(!cols ? 2 * J->n_pairs : std::max(2 * J->n_pairs, 3 * J->n_cols), 1)));
-    ts.total = ts_cnt;
-    ts.off = ts_cnt + 2 * tiles + 1;
-    ts.bucket = ts_bucket;
-    ts.cleared = true;
-    launch_boundary_index(J->bnd, J->wprefix, J->g[0], J->view(), J->W, J->bidx, ts_cnt, 2 * (int64_t)tiles + 1, s);
-    const int ipb = std::max(256, J->ctx->tune.sort_items_per_block);
-    launch_bin_pairs(J->pair_key, J->pairs_ranked, J->pair_tri, J->n_pairs, J->bnd, J->wprefix, (uint32_t)J->B, ts,
-                     ipb, J->boff, J->nm > 1 ? nullptr : &J->mctr[0].max_per_voxel, J->list, s);
-    J->pairs_ranked = true;
-    ts.cleared = false;
-    if (J->nm > 1 && !J->cols_side) launch_mesh_bins(J->boff, J->B, J->view(), s);
+    if (!J->bins_cleared) {
+        TRY(alloc_bin_counters(J, (uint64_t)J->B));
+        launch_fill_u32(J->pair_cnt, 0, (int64_t)J->bin_words, s);
+    }
+    J->bins_cleared = false;
+    // only the Level2 parity reads the column entries
+    const bool cols = J->n2max > 0;
+    uint2* pb = nullptr;
+    uint32_t* cb = nullptr;
+    TRY(alloc(J, &pb, (size_t)std::max<uint64_t>(J->n_pairs, 1)));
     if (cols) {
-        release(J, J->coff);
-        release(J, J->cent);
+        TRY(alloc(J, &cb, 3 * (size_t)std::max<uint64_t>(J->n_cols, 1)));
         TRY(alloc(J, &J->coff, (size_t)J->ncol + 1));
         TRY(alloc(J, &J->cent, (size_t)std::max<uint64_t>(J->n_cols, 1)));
-        launch_bin_cols(J->col_key, J->col_z, J->n_cols, (uint32_t)J->ncol, ts, ipb, J->coff, J->cent, s);
     }
-    release(J, ts_cnt);
-    release(J, ts_bucket);
+    launch_bins(BinPairs{J->pair_key, J->pairs_ranked, J->pair_tri, J->n_pairs, (uint32_t)J->B, J->pair_cnt, pb, J->boff,
+                         J->nm > 1 ? nullptr : &J->mctr[0].max_per_voxel, J->list},
+                BinCols{J->col_key, J->col_z, J->n_cols, cols ? (uint32_t)J->ncol : 0u, J->col_cnt, cb, J->coff, J->cent},
+                J->bnd, J->wprefix, J->g[0], J->view(), J->W, J->bidx, std::max(256, J->ctx->tune.sort_items_per_block), s);
+    J->pairs_ranked = true;
+    if (J->nm > 1 && !J->streams) launch_mesh_bins(J->boff, J->B, J->view(), s);
+    release(J, J->pair_cnt);
+    release(J, pb);
+    release(J, cb);
     HIP_TRY(hipGetLastError());
     J->compact_done = true;
     return GPV_OK;
@@ -1160,45 +1146,34 @@ int run_l2_sat(Job* J)
     return GPV_OK;
 }
 
-// The two streams of the fused pipeline after the read-back.  Main: the bins and
-// the Level2 SAT, which reads them.  Side, behind the Level1 parity: the column-entry
-// sort and the Level2 parity, which reads its entries and the boundary plane.
-// Enqueued in the order in which their kernels are due.  Nothing is allocated
-// or released between the fork and the join, so the pool's blocks stay in
-// one stream order.
+// The fused pipeline after the read-back: the bins and the column entries, then the
+// Level2 SAT, which reads the former, on the main stream and the Level2 parity, which
+// reads the latter, on the side stream, behind the Level1 parity.  Nothing is allocated
+// between the fork and the join, so the pool's blocks stay in one stream order.
 int run_streams(Job* J)
 {
     gpv_ctx* c = J->ctx;
     hipStream_t s = c->stream;
-    J->cols_side = J->n2max > 0;
-    if (J->cols_side) {
-        TRY(alloc_cols(J));
-        TRY(alloc_level2(J));
-        TRY(l2_plan(J));
-        HIP_TRY(hipEventRecord(J->ev[3], s));
-        TRY(launch_compact(J));
-        HIP_TRY(hipStreamWaitEvent(c->side, J->ev[3], 0));
-        TRY(col_sort_kernels(J, c->side));
-        HIP_TRY(hipEventRecord(J->ev[5], s));
-        TRY(l2_sat_kernels(J));
-        TRY(l2_parity_kernels(J, c->side));
-        J->l2p_done = true;
-        J->l2s_done = true;
-        if (J->nm > 1) {
-            // behind the parity, not before the SAT: its few blocks would wait for room beside the parity's
-            HIP_TRY(hipStreamWaitEvent(c->side, J->ev[6], 0));
-            launch_mesh_bins(J->boff, J->B, J->view(), c->side);
-            HIP_TRY(hipGetLastError());
-            HIP_TRY(hipEventRecord(J->ev[14], c->side));
-        }
-        HIP_TRY(hipStreamWaitEvent(s, J->ev[J->nm > 1 ? 14 : 11], 0));
-    } else {
-        TRY(alloc_level2(J));
-        TRY(launch_compact(J));
+    J->streams = J->n2max > 0;
+    TRY(alloc_level2(J));
+    if (J->streams) TRY(l2_plan(J));
+    TRY(launch_compact(J));
+    if (!J->streams) {
         HIP_TRY(hipStreamWaitEvent(s, J->ev[13], 0));
+        return GPV_OK;
     }
-    release(J, J->cs_cnt);
-    release(J, J->cs_bucket);
+    TRY(l2_sat_kernels(J));
+    HIP_TRY(hipStreamWaitEvent(c->side, J->ev[6], 0));   // recorded before the SAT
+    TRY(l2_parity_kernels(J, c->side));
+    J->l2p_done = true;
+    J->l2s_done = true;
+    if (J->nm > 1) {
+        // behind the parity, not before the SAT: its few blocks would wait for room beside the parity's
+        launch_mesh_bins(J->boff, J->B, J->view(), c->side);
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipEventRecord(J->ev[14], c->side));
+    }
+    HIP_TRY(hipStreamWaitEvent(s, J->ev[J->nm > 1 ? 14 : 11], 0));
     return GPV_OK;
 }
 
@@ -1249,9 +1224,9 @@ int job_finish(Job* J)
     // setup, L1 SAT (+ boundary scan), L1 parity (or stencil fill), compaction + bins, L2 parity, L2 SAT, each on its own stream;
     // stages on the side stream overlap the main one's.  For a batch these
     // are the batch's stage times
-    float ms[6] = {el(0, 1), el(1, 12), el(2, 13), 0.0f, 0.0f, 0.0f};
+    float ms[6] = {el(0, 1), el(1, 12), el(J->one_setup ? 1 : 2, 13), 0.0f, 0.0f, 0.0f};
     if (J->n2max > 0) {
-        ms[3] = el(4, 5);
+        ms[3] = el(4, J->streams ? 6 : 5);
         ms[4] = el(16, 11);   // in the fused pipeline the two Level2 stages overlap
         ms[5] = el(6, 7);
     } else {
@@ -1283,7 +1258,7 @@ int job_finish(Job* J)
     release(J, J->pair_key); release(J, J->pair_tri); release(J, J->col_key); release(J, J->col_z);
     release(J, J->wcnt); release(J, J->boff);
     release(J, J->list); release(J, J->coff); release(J, J->cent);
-    release(J, J->cs_cnt); release(J, J->cs_bucket);
+    release(J, J->pair_cnt);
     release(J, J->sat_sums); release(J, J->ray_sums); release(J, J->bbytes); release(J, J->tri_mesh);
     release(J, J->st_cnt); release(J, J->st_off); release(J, J->st_scan); release(J, J->st_tog);
     release(J, J->bmesh);
