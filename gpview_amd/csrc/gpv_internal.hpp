@@ -253,12 +253,13 @@ void launch_l2_sat(const float* tris, const int32_t* bidx, int64_t B, int64_t ng
                    const uint32_t* list, int waves, const GridDev& g0, const Meshes& M,
                    uint64_t* sat2, hipStream_t s);
 // Level2 parity: a wave takes l2_parity_columns adjacent columns of a mesh
-// (grids are multiples of four in x): four at n2 <= 4 in runs of at least
-// kL2ParityMany columns, where the shared prologue pays (128 small meshes 0.39
-// ms), one in smaller ones, where the longest wave counts (icosphere 64/4: 24
+// (grids are multiples of four in x): four at n2 <= 4, two up to 8, in runs of at least
+// kL2ParityMany columns, where the shared prologue and fuller rounds pay (128 small meshes
+// at 64/4 0.39 ms with four; 48 mixed ones 6.09 -> 5.90 ms in all with two at n2 = 8),
+// one in smaller runs, where the longest wave counts (icosphere 64/4: 24
 // us with four)
 constexpr int64_t kL2ParityMany = 1 << 16;
-__host__ __device__ inline int l2_parity_columns(int n2, bool many) { return many && n2 <= 4 ? 4 : 1; }
+__host__ __device__ inline int l2_parity_columns(int n2, bool many) { return !many || n2 > 8 ? 1 : n2 <= 4 ? 4 : 2; }
 // its waves for a mesh with ncol columns (none when Level2 is off)
 int64_t l2_parity_waves(int n2, int64_t ncol, bool many);
 // n2max, nzmax: the largest Level2 resolution and layer count of the run

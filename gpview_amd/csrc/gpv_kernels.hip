@@ -2383,7 +2383,7 @@ void launch_l2_sat(const float* tris, const int32_t* bidx, int64_t B, int64_t ng
 // voxel (i1, j1, k1) takes the triangles of the bins at z' >= k1 in its column,
 // which are the column's (triangle, zmax) entries with zmax >= k1, and each of
 // its sub-voxels counts those whose +z ray test passes.  One wave takes one
-// column (or four adjacent ones, l2_parity_columns): for every (entry, sub-column) pair
+// column (or two or four adjacent ones, l2_parity_columns): for every (entry, sub-column) pair
 // that the float det/u/v test accepts it finds the number of layers whose
 // t > 1e-6 holds -- the layers below the crossing, bounded by gpv_parcol.hpp,
 // with the float test deciding the few within rounding of it -- and toggles one
@@ -2424,7 +2424,7 @@ int64_t l2_parity_waves(int n2, int64_t ncol, bool many)
     return n2 <= 0 ? 0 : ncol / l2_parity_columns(n2, many);
 }
 
-// C adjacent columns (i1 .., j1) of a mesh by one wave: 1, or 4 (at n2 <= 4).
+// C adjacent columns (i1 .., j1) of a mesh by one wave: 1, 2 (at n2 <= 8) or 4 (at n2 <= 4).
 template <int C, int KB>
 __device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB>& L, uint64_t* cb, int nw, const GridDev& g, int i1, int j1,
                                                        uint64_t word0, uint32_t col0, uint32_t b0,
@@ -2681,15 +2681,19 @@ __device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB>& L, uint64_t* 
         }
         __builtin_amdgcn_wave_barrier();
         // the slots' words
-        if (C == 1 && n2 == 8) {
-            const int n = (int)(hi[0] - lo[0]);
-            for (int v0 = 0; v0 < n; v0 += 8) {
-                // bit 8v + r of lane c: layer r of sub-column c of slot v0 + v
-                uint64_t x = 0;
-                for (int v = 0; v < 8 && v0 + v < n; ++v) x |= (uint64_t)a8[(v0 + v) * 64 + lane] << (8 * v);
-                x = wave_transpose64(x);
-                const int v = v0 + (lane >> 3);
-                if (v < n) out[(uint64_t)L.slotb[v] * 8 + (uint64_t)(lane & 7)] = x;
+        if (C <= 2 && n2 == 8) {
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+                const int n = (int)(hi[c] - lo[c]);
+                for (int v0 = 0; v0 < n; v0 += 8) {
+                    // bit 8v + r of lane t: layer r of sub-column t of slot v0 + v
+                    uint64_t x = 0;
+                    for (int v = 0; v < 8 && v0 + v < n; ++v)
+                        x |= (uint64_t)a8[(c * (Wn + 1) + v0 + v) * 64 + lane] << (8 * v);
+                    x = wave_transpose64(x);
+                    const int v = v0 + (lane >> 3);
+                    if (v < n) out[(uint64_t)L.slotb[c * Wn + v] * 8 + (uint64_t)(lane & 7)] = x;
+                }
             }
         } else if (C == 1 && n2 == 16) {
             const int n = (int)(hi[0] - lo[0]);
@@ -2759,7 +2763,9 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 1 ?
     const uint64_t word0 = kM ? M.off[mesh].word0 : 0;
     const uint32_t col0 = kM ? M.off[mesh].col0 : 0, b0 = kM ? M.off[mesh].b0 : 0;
     uint64_t* out = par2 + (kM ? M.off[mesh].l2w0 : 0);
-    if (C == 4)
+    if (C == 2)
+        l2_parity_columns_wave<2>(s_l[wv], cb, nw, g, i1, j1, word0, col0, b0, bnd, wprefix, coff, ent, tris, out);
+    else if (C == 4)
         l2_parity_columns_wave<4>(s_l[wv], cb, nw, g, i1, j1, word0, col0, b0, bnd, wprefix, coff, ent, tris, out);
     else
         l2_parity_columns_wave<1>(s_l[wv], cb, nw, g, i1, j1, word0, col0, b0, bnd, wprefix, coff, ent, tris, out);

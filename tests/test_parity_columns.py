@@ -126,3 +126,21 @@ def test_tall_columns(gv, orc, n2):
         g = c.voxelize(m["soup"], m["bmin"], m["bmax"], m["mms"], 200, n2, cuda_level2=True)
         compare_results(f"tall cuda {n2}", g.download(), orc.voxelize(m["soup"], gc, orc.ORC_FAST), n2)
         g.release()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n2", [4, 5, 8])
+def test_many_columns(gv, orc, n2):
+    """Enough columns for waves of two and four, columns of more boundary voxels
+    than such a wave's window holds among them."""
+    from gpview_amd import workloads
+    v, f = gv.icosphere(4, 0.4, (0.5, 0.5, 0.5), 0.02, seed=9)
+    m = workloads.mesh_entry(gv, v, f, 260, n2)
+    want = orc.voxelize(m["soup"], orc.grid_setup(m["bmin"], m["bmax"], m["mms"], 260, n2), orc.ORC_FAST)
+    per_column = np.bincount(want["bidx"] % (want["l1"].size // 260))
+    assert per_column.size >= 1 << 16 and per_column.max() > 16
+    with gv.Context() as c:
+        say(f"many columns: n2={n2}")
+        g = c.voxelize(m["soup"], m["bmin"], m["bmax"], m["mms"], 260, n2)
+        compare_results(f"many columns {n2}", g.download(), want, n2)
+        g.release()
