@@ -1634,7 +1634,7 @@ __device__ __forceinline__ uint32_t rank_of(const uint64_t* __restrict__ bnd,
 // chains of dependent loads, not bandwidth, bound these passes.
 // ---------------------------------------------------------------------------
 constexpr int TS_NT = 256;
-constexpr int TS_U = 4;
+constexpr int TS_U = 8;   // a block's 2048 items in one round (torus knot 256/8, three passes: 119 -> 110 us with 4 -> 8)
 
 // A bin pair sorts by the rank of its voxel among the boundary voxels; its item
 // is (rank, triangle).
