@@ -250,7 +250,7 @@ void launch_mesh_bins(const uint32_t* boff, int64_t B, const Meshes& M, hipStrea
 
 // ngroups waves of at most gmost voxels each (l2_group_voxels); waves: per block (1, 2, 4)
 void launch_l2_sat(const float* tris, const int32_t* bidx, int64_t B, int64_t ngroups, int gmost, const uint32_t* boff,
-                   const uint32_t* list, int waves, const GridDev& g0, const Meshes& M,
+                   const uint32_t* list, int n2max, int waves, const GridDev& g0, const Meshes& M,
                    uint64_t* sat2, hipStream_t s);
 // Level2 parity: a wave takes l2_parity_columns adjacent columns of a mesh
 // (grids are multiples of four in x): four at n2 <= 4, two up to 8, in runs of at least

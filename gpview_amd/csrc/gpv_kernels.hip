@@ -2027,7 +2027,9 @@ void launch_mesh_bins(const uint32_t* boff, int64_t B, const Meshes& M, hipStrea
 // boundary voxels of a mesh (l2_group_voxels).  Up to 32 bin entries at a time
 // are staged, two lanes each: what the rows of the entry share
 // (gpv_satrow.hpp) goes to LDS.  The lanes then take the (entry, row of
-// sub-voxels) items and walk each row's columns, which gives per column the
+// sub-voxels) items, drop the columns that the (x, y) predicates fail (kPieces: and put
+// what is left of each row in a ring, in pieces of 2, 4 or 8 columns, which keep the
+// lanes of a round about equally long) and walk the others, which gives per column the
 // layers the SAT accepts for certain and those it has to be run on: the
 // first go straight into the wave's accumulator, the others (0.05 per entry
 // on the torus knot, 9 on a lattice-snapped mesh at 512/16) queue for the
@@ -2046,6 +2048,8 @@ void launch_mesh_bins(const uint32_t* boff, int64_t B, const Meshes& M, hipStrea
 // most 64 entries onto fewer than 64 already queued, so it holds 128
 constexpr int L2_QCAP = 128;
 constexpr int L2_STAGE = 32;   // entries staged at once
+// ring of row pieces per wave: a round pushes at most 192 onto fewer than 64
+constexpr uint32_t L2_SEGS = 256;
 
 // value of a float register in lane `l` (l uniform across the wave)
 __device__ __forceinline__ float lane_f(float v, int l)
@@ -2080,6 +2084,7 @@ __device__ __forceinline__ uint64_t wave_transpose64(uint64_t v)
 }
 
 // LDS of one wave of the Level2 SAT
+template <bool kPieces>
 struct L2Lds {
     union {
         float4 e[L2_STAGE][kSatEntry4];                  // staged entries
@@ -2093,6 +2098,7 @@ struct L2Lds {
     uint32_t vb[kL2GroupMax + 1]; // group voxel v: first bin entry
     int ci[kL2GroupMax][3];       // its sub-center 0 in the tables
     uint8_t win[64];              // per round: staged entry starting at each item position
+    uint16_t seg[kPieces ? L2_SEGS : 1];   // ring of row pieces: entry | row << 5 | column << 9 | columns - 1 << 13
 };
 
 // where the layer bits of sub-column `col` lie: word index and first bit
@@ -2105,7 +2111,8 @@ __device__ __forceinline__ uint32_t l2_col_word(uint32_t col, int n2, uint32_t& 
 
 // Full float SAT for queued entries (one per lane); entry = p | q<<4 | r<<8 |
 // v<<12 | j<<16 where v is the voxel in the group and j the bin entry from base.
-__device__ __forceinline__ void l2_sat_run(uint32_t ent, bool valid, L2Lds& L, const GridDev& g,
+template <bool kPieces>
+__device__ __forceinline__ void l2_sat_run(uint32_t ent, bool valid, L2Lds<kPieces>& L, const GridDev& g,
                                            const float* __restrict__ tris, const uint32_t* __restrict__ list,
                                            uint32_t base)
 {
@@ -2143,17 +2150,17 @@ __device__ __forceinline__ int l2_axis_last(const float* __restrict__ c, int n, 
     return k;
 }
 
-template <bool kM, int W>
+template <bool kM, int W, bool kPieces>
 __global__ __launch_bounds__(64 * W) void k_l2_sat(const float* __restrict__ tris, const int32_t* __restrict__ bidx,
                                                    int64_t B, int64_t ngroups, int gmost,
                                                    const uint32_t* __restrict__ boff,
                                                    const uint32_t* __restrict__ list,
                                                    GridDev g0, Meshes M, uint64_t* __restrict__ sat2)
 {
-    __shared__ L2Lds s_l[W];
+    __shared__ L2Lds<kPieces> s_l[W];
     const int wv = threadIdx.x >> 6;
     const int lane = __lane_id();
-    L2Lds& L = s_l[wv];
+    L2Lds<kPieces>& L = s_l[wv];
     const int64_t grp = (int64_t)blockIdx.x * W + wv;
     if (grp >= ngroups) return;
     int mesh = 0;
@@ -2249,49 +2256,91 @@ __global__ __launch_bounds__(64 * W) void k_l2_sat(const float* __restrict__ tri
         const uint32_t so = incl - P;   // this lane's entry: items [so, so + P)
         const uint32_t S = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
         __builtin_amdgcn_wave_barrier();
-        // the chunk's (entry, row) items, 64 per round
-        for (uint32_t l0 = 0; l0 < S; l0 += 64) {
-            // each item's entry: every entry with items in [l0, l0 + 64) marks
-            // its first position there (the one running into the window marks
-            // 0; starts are distinct), and item l takes the mark at the highest
-            // marked position <= l
-            L.win[lane] = 0xff;
-            __builtin_amdgcn_wave_barrier();
-            if (P && so < l0 + 64u && so + P > l0) L.win[so > l0 ? so - l0 : 0u] = (uint8_t)lane;
-            __builtin_amdgcn_wave_barrier();
-            const uint32_t wj = L.win[lane];
-            const uint64_t marks = __ballot(wj != 0xffu) & ((2ull << lane) - 1ull);
-            const int top = marks ? 63 - __clzll((long long)marks) : 0;
-            const int j = __shfl((int)wj, top) & (L2_STAGE - 1);
-            const uint32_t so_j = (uint32_t)__shfl((int)so, j);
-            __builtin_amdgcn_wave_barrier();
-            const uint32_t l = l0 + (uint32_t)lane;
-            // lanes past the last item repeat one with no columns to do
+        // the chunk's (entry, row) items, 64 per round, less the columns that the (x, y)
+        // predicates fail.  kPieces: what is left of each row goes to the ring in pieces
+        // of 2, 4 or 8 columns, and 64 of those make a round
+        uint32_t rh = 0, rt = 0;   // ring head/tail (uniform)
+        for (uint32_t l0 = 0;;) {
+            int j, q, p, left;   // entry, row, first column, columns
+            if (rt - rh < 64 && l0 < S) {
+                // each item's entry: every entry with items in [l0, l0 + 64) marks
+                // its first position there (the one running into the window marks
+                // 0; starts are distinct), and item l takes the mark at the highest
+                // marked position <= l
+                L.win[lane] = 0xff;
+                __builtin_amdgcn_wave_barrier();
+                if (P && so < l0 + 64u && so + P > l0) L.win[so > l0 ? so - l0 : 0u] = (uint8_t)lane;
+                __builtin_amdgcn_wave_barrier();
+                const uint32_t wj = L.win[lane];
+                const uint64_t marks = __ballot(wj != 0xffu) & ((2ull << lane) - 1ull);
+                const int top = marks ? 63 - __clzll((long long)marks) : 0;
+                j = __shfl((int)wj, top) & (L2_STAGE - 1);
+                const uint32_t so_j = (uint32_t)__shfl((int)so, j);
+                __builtin_amdgcn_wave_barrier();
+                const uint32_t l = l0 + (uint32_t)lane;
+                l0 += 64;
+                // lanes past the last item repeat one with no columns to do
+                const uint32_t d = L.dec[j];
+                q = (int)(((d >> 4) & 15) + (l - so_j));
+                p = d & 15;
+                left = (int)((d >> 16) & 15) + 1;   // columns of the row
+                sat_row_range(L.e[j], q, d >> 31 != 0, p, left);
+                left = l < S && left > 0 ? left : 0;
+                if constexpr (kPieces) {
+                    // pieces of each size, in fields of their own (at most 512, 256, 128 in all)
+                    const uint32_t pk = (uint32_t)((left + 1) >> 1) | ((uint32_t)((left + 3) >> 2) << 11) |
+                                        ((uint32_t)((left + 7) >> 3) << 21);
+                    const uint32_t inc = wave_incl_scan<uint32_t>(pk);
+                    const uint32_t tot = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
+                    const uint32_t n2s = tot & 0x7ffu, n4s = (tot >> 11) & 0x3ffu, n8s = tot >> 21;
+                    // the cheapest: a piece costs about 120 instructions, a column 62
+                    uint32_t sh = 3, fs = 21, best = 616u * n8s;
+                    if (n4s <= L2_SEGS - 64 && 368u * n4s <= best) sh = 2, fs = 11, best = 368u * n4s;
+                    if (n2s <= L2_SEGS - 64 && 244u * n2s <= best) sh = 1, fs = 0;
+                    const uint32_t mask = sh == 1 ? 0x7ffu : 0x3ffu;
+                    const uint32_t own = (pk >> fs) & mask, at = rt + (((inc - pk) >> fs) & mask);
+                    for (uint32_t k = 0; __ballot(k < own); ++k)
+                        if (k < own) {
+                            const uint32_t done = k << sh, cnt = min((uint32_t)left - done, 1u << sh);
+                            L.seg[(at + k) % L2_SEGS] = (uint16_t)((uint32_t)j | ((uint32_t)q << 5) | (((uint32_t)p + done) << 9) | ((cnt - 1u) << 13));
+                        }
+                    rt += (tot >> fs) & mask;
+                    __builtin_amdgcn_wave_barrier();
+                    continue;
+                }
+            } else {
+                if constexpr (!kPieces) break;
+                const uint32_t np = rt - rh < 64 ? rt - rh : 64u;
+                if (!np) break;
+                // lanes past the last piece repeat one with no columns to do
+                const uint32_t pc = L.seg[(rh + ((uint32_t)lane < np ? (uint32_t)lane : 0u)) % L2_SEGS];
+                rh += np;
+                j = (int)(pc & 31u);
+                q = (int)((pc >> 5) & 15u);
+                p = (int)((pc >> 9) & 15u);
+                left = (uint32_t)lane < np ? (int)(pc >> 13) + 1 : 0;
+            }
+            asm("" : "+v"(left));   // a plain number to the loop: a compare a column, not the select above
             const uint32_t d = L.dec[j];
-            const int q = ((d >> 4) & 15) + (int)(l - so_j), ra = (d >> 8) & 15, rb = (d >> 12) & 15;
-            const int v = (int)((d >> 20) & 15u);
+            const int ra = (d >> 8) & 15, rb = (d >> 12) & 15, v = (int)((d >> 20) & 15u);
             const bool loose = d >> 31 != 0;
-            int p = d & 15, left = (int)((d >> 16) & 15) + 1;   // columns of the row
-            SatRow row = sat_row(L.e[j], q, ra, rb, loose, p, left);
-            left = l < S ? left : 0;
-            const uint32_t all = ((2u << rb) - 1u) & ~((1u << ra) - 1u);
+            SatRow row = sat_row_at(L.e[j], q, ra, rb, p);
+            if (__ballot(loose)) sat_row_loose(row, loose, ra, rb);
             uint32_t col = (uint32_t)((v * n2 + q) * n2 + p);
             const uint32_t ent = (uint32_t)p | ((uint32_t)q << 4) | ((uint32_t)v << 12) | ((base - qbase + (uint32_t)j) << 16);
-            const bool any_loose = __ballot(loose && left > 0) != 0;
-            for (int k = 0; __ballot(k < left); ++k, ++col) {
-                uint32_t in, may;
-                sat_row_column(row, in, may);
-                if (any_loose) {
-                    in = loose ? 0u : in;
-                    may = loose ? all : may;
-                }
+            for (int k = 0;; ++k, ++col) {
                 const bool on = k < left;
-                in = on ? in : 0u;
-                uint32_t unk = on ? may & ~in : 0u;
-                if (in) {
-                    uint32_t bit;
-                    const uint32_t w = l2_col_word(col, n2, bit);
-                    atomicOr(&L.acc[w], in << bit);
+                if (!__ballot(on)) break;
+                uint32_t unk = 0;
+                if (on) {
+                    uint32_t in, may;
+                    sat_row_column(row, in, may);
+                    unk = may & ~in;
+                    if (in) {
+                        uint32_t bit;
+                        const uint32_t w = l2_col_word(col, n2, bit);
+                        atomicOr(&L.acc[w], in << bit);
+                    }
                 }
                 // the undecided boxes, one layer per lane per pass
                 for (uint64_t m; (m = __ballot(unk != 0)) != 0;) {
@@ -2356,26 +2405,38 @@ __global__ __launch_bounds__(64 * W) void k_l2_sat(const float* __restrict__ tri
     for (int i = lane; i < nv * w2; i += 64) out[i] = L.words[i];
 }
 
-template <int W>
+template <int W, bool kPieces>
 static void launch_l2_sat_w(const float* tris, const int32_t* bidx, int64_t B, int64_t ngroups, int gmost,
-                            const uint32_t* boff, const uint32_t* list, const GridDev& g0,
-                            const Meshes& M, uint64_t* sat2, hipStream_t s)
+                            const uint32_t* boff, const uint32_t* list, const GridDev& g0, const Meshes& M,
+                            uint64_t* sat2, hipStream_t s)
 {
     const unsigned blocks = (unsigned)((ngroups + W - 1) / W);
     if (M.nm > 1)
-        k_l2_sat<true, W><<<blocks, 64 * W, 0, s>>>(tris, bidx, B, ngroups, gmost, boff, list, g0, M, sat2);
+        k_l2_sat<true, W, kPieces><<<blocks, 64 * W, 0, s>>>(tris, bidx, B, ngroups, gmost, boff, list, g0, M, sat2);
     else
-        k_l2_sat<false, W><<<blocks, 64 * W, 0, s>>>(tris, bidx, B, ngroups, gmost, boff, list, g0, M, sat2);
+        k_l2_sat<false, W, kPieces><<<blocks, 64 * W, 0, s>>>(tris, bidx, B, ngroups, gmost, boff, list, g0, M, sat2);
+}
+
+template <bool kPieces>
+static void launch_l2_sat_p(const float* tris, const int32_t* bidx, int64_t B, int64_t ngroups, int gmost,
+                            const uint32_t* boff, const uint32_t* list, int waves, const GridDev& g0, const Meshes& M,
+                            uint64_t* sat2, hipStream_t s)
+{
+    if (waves <= 1) launch_l2_sat_w<1, kPieces>(tris, bidx, B, ngroups, gmost, boff, list, g0, M, sat2, s);
+    else if (waves == 2) launch_l2_sat_w<2, kPieces>(tris, bidx, B, ngroups, gmost, boff, list, g0, M, sat2, s);
+    else launch_l2_sat_w<4, kPieces>(tris, bidx, B, ngroups, gmost, boff, list, g0, M, sat2, s);
 }
 
 void launch_l2_sat(const float* tris, const int32_t* bidx, int64_t B, int64_t ngroups, int gmost, const uint32_t* boff,
-                   const uint32_t* list, int waves, const GridDev& g0, const Meshes& M,
+                   const uint32_t* list, int n2max, int waves, const GridDev& g0, const Meshes& M,
                    uint64_t* sat2, hipStream_t s)
 {
     if (B <= 0 || ngroups <= 0) return;
-    if (waves <= 1) launch_l2_sat_w<1>(tris, bidx, B, ngroups, gmost, boff, list, g0, M, sat2, s);
-    else if (waves == 2) launch_l2_sat_w<2>(tris, bidx, B, ngroups, gmost, boff, list, g0, M, sat2, s);
-    else launch_l2_sat_w<4>(tris, bidx, B, ngroups, gmost, boff, list, g0, M, sat2, s);
+    // Rows in pieces above n2 = 8, where a round of whole rows waits for one of up to 16
+    // columns (lattice-snapped mesh at 512/16: 2.54 -> 2.24 ms alone).  Shorter rows do not
+    // pay for the ring: torus knot 256/8 the same, 128 small meshes at 64/4 2.25 -> 2.29 ms in all
+    if (n2max > 8) launch_l2_sat_p<true>(tris, bidx, B, ngroups, gmost, boff, list, waves, g0, M, sat2, s);
+    else launch_l2_sat_p<false>(tris, bidx, B, ngroups, gmost, boff, list, waves, g0, M, sat2, s);
 }
 
 // ---------------------------------------------------------------------------

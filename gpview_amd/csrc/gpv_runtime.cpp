@@ -1131,7 +1131,7 @@ int l2_sat_kernels(Job* J)
     hipStream_t s = J->ctx->stream;
     HIP_TRY(hipEventRecord(J->ev[6], s));
     launch_l2_sat(J->tris, J->bidx, J->B, J->l2s_groups, J->l2s_most, J->boff, J->list,
-                  J->ctx->tune.l2_sat_waves, J->g[0], J->view(), J->sat2, s);
+                  J->n2max, J->ctx->tune.l2_sat_waves, J->g[0], J->view(), J->sat2, s);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipEventRecord(J->ev[7], s));
     return GPV_OK;

@@ -206,25 +206,31 @@ __host__ __device__ __forceinline__ void sat_x_range(float e, float c, float lim
     hi = fminf(hi, fmaxf(a, b));
 }
 
-// Row q with layers [ra, rb].  Of the columns [p, p + left) it drops those at
-// either end that the (x, y) predicates certainly fail (unless `keep`).
-__host__ __device__ __forceinline__ SatRow sat_row(const float4* e, int q, int ra, int rb, bool keep, int& p, int& left)
+// Row q: of the columns [p, p + left) it drops those at either end that the (x, y)
+// predicates certainly fail (unless `keep`).
+__host__ __device__ __forceinline__ void sat_row_range(const float4* e, int q, bool keep, int& p, int& left)
+{
+    const float4 c6 = e[6], c7 = e[7], c8 = e[8];
+    const float y = (float)q;
+    const float u0 = c7.x * y + c8.x, u1 = c7.y * y + c8.y, u2 = c7.z * y + c8.z;
+    const float lim = 1.0f + c6.w;
+    float lo = (float)p - 0.5f, hi = (float)(p + left) - 0.5f;
+    sat_x_range(c6.x, u0, lim, lo, hi);
+    sat_x_range(c6.y, u1, lim, lo, hi);
+    sat_x_range(c6.z, u2, lim, lo, hi);
+    // columns in [lo - 0.01, hi + 0.01]; both ends lie in (p - 1, p + left) unless the row is empty
+    const int p1 = (int)fminf(fmaxf(lo + 0.99f, 0.0f), 16.0f), pe = (int)fminf(fmaxf(hi + 1.01f, 0.0f), 16.0f);
+    left = keep ? left : pe - p1;
+    p = keep ? p : p1;
+}
+
+// Row q with layers [ra, rb], positioned at column p.
+__host__ __device__ __forceinline__ SatRow sat_row_at(const float4* e, int q, int ra, int rb, int p)
 {
     SatRow s;
     const float4 c6 = e[6], c7 = e[7], c8 = e[8], pl = e[9];
     const float y = (float)q;
     const float u0 = c7.x * y + c8.x, u1 = c7.y * y + c8.y, u2 = c7.z * y + c8.z;
-    {
-        const float lim = 1.0f + c6.w;
-        float lo = (float)p - 0.5f, hi = (float)(p + left) - 0.5f;
-        sat_x_range(c6.x, u0, lim, lo, hi);
-        sat_x_range(c6.y, u1, lim, lo, hi);
-        sat_x_range(c6.z, u2, lim, lo, hi);
-        // columns in [lo - 0.01, hi + 0.01]; both ends lie in (p - 1, p + left) unless the row is empty
-        const int p1 = (int)fminf(fmaxf(lo + 0.99f, 0.0f), 16.0f), pe = (int)fminf(fmaxf(hi + 1.01f, 0.0f), 16.0f);
-        left = keep ? left : pe - p1;
-        p = keep ? p : p1;
-    }
     const float x = (float)p;
     s.lom = s.loi = (float)ra;
     s.him = s.hii = (float)rb + 1.0f;
@@ -249,6 +255,18 @@ __host__ __device__ __forceinline__ SatRow sat_row(const float4* e, int q, int r
     return s;
 }
 
+// A row of a loose entry (nothing of it is bounded): all layers of its columns undecided.
+__host__ __device__ __forceinline__ void sat_row_loose(SatRow& s, bool loose, int ra, int rb)
+{
+    if (!loose) return;
+    s.a0 = s.a1 = s.a2 = s.pa = 0.0f;
+    s.w0 = s.w1 = s.w2 = s.pw = 0.0f;
+    s.m0 = s.m1 = s.m2 = s.pm = 1e30f;
+    s.lom = (float)ra;
+    s.him = (float)rb + 1.0f;
+    s.um = 3e38f;
+}
+
 // truncation that takes anything below 0 to 0
 __host__ __device__ __forceinline__ uint32_t sat_trunc(float x)
 {
@@ -261,7 +279,7 @@ __host__ __device__ __forceinline__ uint32_t sat_trunc(float x)
 #endif
 }
 
-// The current column's layer masks (of an entry that is not loose); steps the
+// The current column's layer masks (sat_row_loose first for a loose entry); steps the
 // row to the next column.
 __host__ __device__ __forceinline__ void sat_row_column(SatRow& s, uint32_t& in, uint32_t& may)
 {

@@ -44,7 +44,8 @@ extern "C" void satrow_batch(int64_t n, int n2, const float* tv, const float* cx
             for (int p = 0; p < n2; ++p) oi[p] = om[p] = 0;
             if (pb < 0 || rb < 0 || !axis_ok(t[1], t[4], t[7], Y[q], h[3 * i + 1])) continue;
             int p = pa, left = pb - pa + 1;
-            gpv::SatRow s = gpv::sat_row(e, q, ra, rb, loose, p, left);
+            gpv::sat_row_range(e, q, loose, p, left);
+            gpv::SatRow s = gpv::sat_row_at(e, q, ra, rb, p);
             const uint32_t all = ((2u << rb) - 1u) & ~((1u << ra) - 1u);
             for (int k = 0; k < left; ++k) {
                 gpv::sat_row_column(s, oi[p + k], om[p + k]);
