@@ -1308,10 +1308,11 @@ int job_run(Job* J)
 
 // Upper bound of the bytes a one-mesh run requests from the pool (every
 // buffer it allocates, as if none were returned before the run ends), with
-// the run's own capacities for the bin and hit buffers and an estimate of
+// the run's own capacities for the bin buffers and an estimate of
 // the boundary voxels: twice the voxels on the faces of the grid's box, to
-// allow for folds.  Exceeded only when the bins regrow or the surface holds
-// more boundary voxels than that.
+// allow for folds, and up to once more for rough surfaces of many triangles
+// (1.3 million jittered ones at 512 hold 2.8 times).  Exceeded only when the bins
+// regrow or the surface holds more boundary voxels than that.
 int64_t predict_run_bytes(const gpv_mesh_desc& d, const gpv_grid_info& I)
 {
     const int64_t nx = I.n[0], ny = I.n[1], nz = I.n[2];
@@ -1323,7 +1324,8 @@ int64_t predict_run_bytes(const gpv_mesh_desc& d, const gpv_grid_info& I)
     const int64_t nmax = std::max(nx, std::max(ny, nz));
     const int64_t P = d.params.initial_capacity > 0 ? d.params.initial_capacity
                                                     : std::max<int64_t>(int64_t(1) << 16, 16 * T + 8 * nmax * nmax);
-    const int64_t B = std::min(n1, 4 * (nx * ny + ny * nz + nz * nx));
+    const int64_t faces = nx * ny + ny * nz + nz * nx;   // half the box's faces
+    const int64_t B = std::min(n1, 4 * faces + 2 * std::min(T, faces));
     auto scan = [](int64_t n) { return 8 * (int64_t)scan_tmp_elems(n); };
     int64_t b = 0;
     b += 4 * (2 * (nx + ny + nz) * (1 + n2) + 1);               // center tables
@@ -1332,8 +1334,9 @@ int64_t predict_run_bytes(const gpv_mesh_desc& d, const gpv_grid_info& I)
     b += 24 * W + 64 * W + W / 256 + 4;                          // planes, word counts, their sums and prefix, flag bytes
     b += T / 16 + 16;                                            // sums of the items
     b += 24 * P;                                                 // bin pairs, column entries
-    b += 4 * (ncol + 1) + 8 * P + 12 * P + 64 * (ncol / 64 + 1) + scan(ncol);   // column entries by column
-    b += 8 * B + 4 + 4 * P + 8 * P + 64 * (B / 64 + 1) + scan(B);   // boundary list, bins
+    b += 4 * (ncol + 1) + 8 * P + 12 * P;                        // column entries by column
+    b += 8 * B + 4 + 4 * P + 8 * P;                              // boundary list, bins
+    b += 4 * (int64_t)(ts_words((uint64_t)std::min<int64_t>(W * 64, int64_t(1) << 27)) + ts_words((uint64_t)ncol));   // their counters
     b += 16 * B * w2;                                            // Level2 planes
     if (d.params.normals) b += 12 * T + 4 * P + 12 * B + 12 * B * n2 * n2 * n2;
     if (d.params.l1_stencil) b += 12 * T + 8 + scan(T) + 8 * nz * 2 * ny * ((2 * nx + 63) / 64);   // stencil fill
