@@ -292,7 +292,7 @@ int gpv_ctx_autotune(gpv_ctx *ctx, const gpv_mesh_desc *meshes, int nmeshes, int
                      gpv_tune *best, float *best_ms);
 
 /* ---- stage entry points (same order PerformVoxelization calls them) ------- */
-/* Allocates the grid, uploads the soup and the center tables: the set-up of
+/* Allocates the grid and uploads the soup: the set-up of
  * PerformVoxelization (src/Object.cpp:3094-3193). */
 int gpv_grid_create(gpv_ctx *ctx, const float *tris, int64_t ntris, int tris_on_device,
                     const float bmin[3], const float bmax[3], float max_model_size,
