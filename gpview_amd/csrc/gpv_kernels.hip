@@ -383,9 +383,8 @@ void launch_mesh_ids(const MeshOff* off, int nm, int64_t T, uint32_t* tri_mesh, 
 // inside one mesh (tri_mesh is non-decreasing) reduce into that mesh's
 // counter, the few straddling blocks add per lane.
 
-// kPart: 1 the SAT half (index AABB, items, test counts), 2 the ray
-// half (column bound, items), 3 both.  The halves share nothing but the
-// vertices, so they can run on two streams.
+// kPart: 1 the SAT half (index AABB, items, test counts), 3 the ray
+// half (column bound, items) as well.
 template <bool kM, int kPart>
 __global__ __launch_bounds__(256) void k_tri_setup(const float* __restrict__ tris, int64_t T, GridDev g0, Meshes M,
                                                    int4* __restrict__ box0, int4* __restrict__ box1,
@@ -409,36 +408,34 @@ __global__ __launch_bounds__(256) void k_tri_setup(const float* __restrict__ tri
             for (int c = 0; c < 9; ++c) tv[c] = tris[t * 9 + c];
             MtTri m;
             const bool vis = mt_setup(tv, m);
-            if constexpr ((kPart & 1) != 0) {
-                // the input domain: finite coordinates within +-2^40, where every
-                // intermediate of the SAT and of the split +z ray test is finite
-                bool bad = false;
+            // the input domain: finite coordinates within +-2^40, where every
+            // intermediate of the SAT and of the split +z ray test is finite
+            bool bad = false;
 #pragma unroll
-                for (int c = 0; c < 9; ++c) bad = bad || !(fabsf(tv[c]) <= 0x1p40f);
-                if (bad) atomicOr(bad_input, 1ull);
-                int lo[3], dd[3];
-                const int n[3] = {g.nx, g.ny, g.nz};
-                const float mn[3] = {g.bminx, g.bminy, g.bminz};
-                const float mx[3] = {g.bmaxx, g.bmaxy, g.bmaxz};
+            for (int c = 0; c < 9; ++c) bad = bad || !(fabsf(tv[c]) <= 0x1p40f);
+            if (bad) atomicOr(bad_input, 1ull);
+            int lo[3], dd[3];
+            const int n[3] = {g.nx, g.ny, g.nz};
+            const float mn[3] = {g.bminx, g.bminy, g.bminz};
+            const float mx[3] = {g.bmaxx, g.bmaxy, g.bmaxz};
 #pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    const int i0 = vertex_index(tv[a], mn[a], mx[a], n[a]);
-                    const int i1 = vertex_index(tv[3 + a], mn[a], mx[a], n[a]);
-                    const int i2 = vertex_index(tv[6 + a], mn[a], mx[a], n[a]);
-                    int l = min(i0, min(i1, i2));
-                    int h = max(i0, max(i1, i2));
-                    l = max(l, 0);
-                    h = min(h, n[a] - 1);
-                    lo[a] = l;
-                    dd[a] = h >= l ? h - l + 1 : 0;
-                }
-                box0[t] = make_int4(lo[0], lo[1], lo[2], vis ? 1 : 0);
-                box1[t] = make_int4(dd[0], dd[1], dd[2], 0);
-                const bool any = dd[0] > 0 && dd[1] > 0 && dd[2] > 0;
-                nsat = any ? (uint32_t)(dd[0] * dd[1]) : 0u;
-                sat_items[t] = nsat;
-                tests += any ? (uint64_t)dd[0] * dd[1] * dd[2] : 0;
+            for (int a = 0; a < 3; ++a) {
+                const int i0 = vertex_index(tv[a], mn[a], mx[a], n[a]);
+                const int i1 = vertex_index(tv[3 + a], mn[a], mx[a], n[a]);
+                const int i2 = vertex_index(tv[6 + a], mn[a], mx[a], n[a]);
+                int l = min(i0, min(i1, i2));
+                int h = max(i0, max(i1, i2));
+                l = max(l, 0);
+                h = min(h, n[a] - 1);
+                lo[a] = l;
+                dd[a] = h >= l ? h - l + 1 : 0;
             }
+            box0[t] = make_int4(lo[0], lo[1], lo[2], vis ? 1 : 0);
+            box1[t] = make_int4(dd[0], dd[1], dd[2], 0);
+            const bool any = dd[0] > 0 && dd[1] > 0 && dd[2] > 0;
+            nsat = any ? (uint32_t)(dd[0] * dd[1]) : 0u;
+            sat_items[t] = nsat;
+            tests += any ? (uint64_t)dd[0] * dd[1] * dd[2] : 0;
             if constexpr ((kPart & 2) != 0) {
                 // at least one item, so that runs of k_ray_expand with equal items hold equal
                 // work where most triangles have no column (48 mixed meshes 1414 us without)
@@ -465,7 +462,7 @@ __global__ __launch_bounds__(256) void k_tri_setup(const float* __restrict__ tri
         }
         // the items of these 256 triangles, for the scan
         const int wid = threadIdx.x >> 6;
-        const uint64_t a = (kPart & 1) != 0 ? wave_sum_u64(nsat) : 0, b = (kPart & 2) != 0 ? wave_sum_u64(nray) : 0;
+        const uint64_t a = wave_sum_u64(nsat), b = kPart == 3 ? wave_sum_u64(nray) : 0;
         if (__lane_id() == 0) {
             s_sum[0][wid] = a;
             s_sum[1][wid] = b;
@@ -477,7 +474,6 @@ __global__ __launch_bounds__(256) void k_tri_setup(const float* __restrict__ tri
         }
         __syncthreads();
     }
-    if constexpr ((kPart & 1) == 0) return;
     if constexpr (!kM) {
         block_add_u64(tests, &M.ctr[0].tests_l1);
     } else {
@@ -513,8 +509,6 @@ void launch_tri_setup(const float* tris, int64_t T, const GridDev& g0, const Mes
     if (T <= 0) return;
     if (part == 1)
         tri_setup_part<1>(tris, T, g0, M, box0, box1, sat_items, ray_rng, ray_items, sat_sums, ray_sums, bad_input, s);
-    else if (part == 2)
-        tri_setup_part<2>(tris, T, g0, M, box0, box1, sat_items, ray_rng, ray_items, sat_sums, ray_sums, bad_input, s);
     else
         tri_setup_part<3>(tris, T, g0, M, box0, box1, sat_items, ray_rng, ray_items, sat_sums, ray_sums, bad_input, s);
 }

@@ -267,11 +267,10 @@ struct Job {
     int4 *box0 = nullptr, *box1 = nullptr, *rng = nullptr;
     uint32_t *sat_items = nullptr, *ray_items = nullptr;
     uint64_t *sat_off = nullptr, *ray_off = nullptr, *scan64 = nullptr;
-    uint64_t* scan_ray = nullptr;   // scan temporary of the ray half of the set-up (side stream)
     uint64_t *sat_sums = nullptr, *ray_sums = nullptr;   // items per 256 triangles
     uint8_t* bbytes = nullptr;       // boundary flags of the Level1 SAT
     bool sat_timed = false;          // ev[1] is recorded
-    bool one_setup = false;          // both halves of the set-up ran before ev[1]
+    bool one_setup = false;          // the Level1 parity starts at ev[1]
     bool sat_cleared = false;        // flags and counters of the sweep hold zeros
     bool ins_cleared = false;        // the inside plane holds zeros
     uint32_t* scan32 = nullptr;
@@ -324,7 +323,7 @@ struct Job {
     // stream events: 0 setup, 1 L1 SAT, 2 L1 parity,
     // 4 compaction+bins, 5 its end (6 where the Level2 parity forks), 6 L2 SAT start, 7 L2 SAT end, 8 finish,
     // 9 normals start, 10 normals end, 11 L2 parity end, 12 L1 SAT end,
-    // 13 L1 parity end, 14 end of the side stream, 15 fork of the L1 parity, 16 L2 parity start
+    // 13 L1 parity end, 14 end of the side stream, 15 fork of the stencil fill, 16 L2 parity start
     hipEvent_t ev[kJobEvents] = {};
     std::vector<void*> bufs;
     // gpv_voxelize_noalloc: buffers are carved from the device scratch array
@@ -809,22 +808,17 @@ int stage_setup(Job* J)
     return GPV_OK;
 }
 
-// Triangles up to which the set-up is one launch on the main stream before the
-// fork: as two, beside each other, it costs a launch more, which up to here takes
-// longer than the half it hides (three of a wave's 64 triangles a SIMD).
-constexpr int64_t kSetupSplit = int64_t(1) << 16;
-
-// The fused pipeline's set-up: everything cleared in one launch, then the SAT half on
-// the main stream and the ray half on the side stream, forked at ev[15] (ev[1] where
-// they are one launch).
+// The fused pipeline's set-up: everything cleared in one launch, then both halves of the
+// set-up in one and both scans in one; the side stream forks behind them at ev[1] (a ray half
+// of its own beside the SAT half took a launch more and as long in all: torus knot 769 against
+// 767 us, 48 mixed meshes 5.86 both, icosphere 64/4 234 against 232).  The
+// stencil fill needs neither half and forks before them, at ev[15].
 int stage_setup_split(Job* J)
 {
     gpv_ctx* c = J->ctx;
     hipStream_t s = c->stream;
     HIP_TRY(hipEventRecord(J->ev[0], s));
     TRY(ensure_scan_tmp(J, J->T));
-    release(J, J->scan_ray);
-    TRY(alloc(J, &J->scan_ray, scan_tmp_elems(J->T)));
     TRY(alloc(J, &J->bbytes, (size_t)J->W * 64));
     TRY(alloc_bin_counters(J, (uint64_t)std::min<int64_t>(J->W * 64, int64_t(1) << 27)));
     launch_clear(ClearList{{reinterpret_cast<uint64_t*>(J->mctr), reinterpret_cast<uint64_t*>(J->ctr),
@@ -837,21 +831,16 @@ int stage_setup_split(Job* J)
     J->ins_cleared = true;
     J->bins_cleared = true;
     if (J->nm > 1) launch_mesh_ids(J->d_off, J->nm, J->T, J->tri_mesh, s);
-    const bool one = J->T <= kSetupSplit && !J->all_stencil;
-    if (!one) HIP_TRY(hipEventRecord(J->ev[15], s));   // the fork
+    const bool rays = !J->all_stencil;   // the ray half feeds only the ray parity
+    if (!rays) HIP_TRY(hipEventRecord(J->ev[15], s));
     launch_tri_setup(J->tris, J->T, J->g[0], J->view(), J->box0, J->box1, J->sat_items, J->rng, J->ray_items,
-                     J->sat_sums, J->ray_sums, one ? 3 : 1, &J->ctr->bad_input, s);
-    launch_scan_items(J->sat_items, J->sat_off, J->sat_sums, one ? J->ray_items : nullptr, J->ray_off, J->ray_sums, J->T,
+                     J->sat_sums, J->ray_sums, rays ? 3 : 1, &J->ctr->bad_input, s);
+    launch_scan_items(J->sat_items, J->sat_off, J->sat_sums, rays ? J->ray_items : nullptr, J->ray_off, J->ray_sums, J->T,
                       J->scan64, s);
     HIP_TRY(hipEventRecord(J->ev[1], s));
     J->sat_timed = true;
-    J->one_setup = one;
-    HIP_TRY(hipStreamWaitEvent(c->side, J->ev[one ? 1 : 15], 0));
-    if (!one && !J->all_stencil) {   // the ray half feeds only the ray parity
-        launch_tri_setup(J->tris, J->T, J->g[0], J->view(), J->box0, J->box1, J->sat_items, J->rng, J->ray_items,
-                         J->sat_sums, J->ray_sums, 2, &J->ctr->bad_input, c->side);
-        launch_scan_items(J->ray_items, J->ray_off, J->ray_sums, nullptr, nullptr, nullptr, J->T, J->scan_ray, c->side);
-    }
+    J->one_setup = rays;
+    HIP_TRY(hipStreamWaitEvent(c->side, J->ev[rays ? 1 : 15], 0));
     HIP_TRY(hipGetLastError());
     J->setup_done = true;
     return GPV_OK;
@@ -1254,7 +1243,7 @@ int job_finish(Job* J)
     // only the result planes stay resident
     release(J, J->box0); release(J, J->box1); release(J, J->rng);
     release(J, J->sat_items); release(J, J->ray_items); release(J, J->sat_off); release(J, J->ray_off);
-    release(J, J->scan64); J->scan32 = nullptr; J->scan_cap = 0; release(J, J->scan_ray);
+    release(J, J->scan64); J->scan32 = nullptr; J->scan_cap = 0;
     release(J, J->pair_key); release(J, J->pair_tri); release(J, J->col_key); release(J, J->col_z);
     release(J, J->wcnt); release(J, J->boff);
     release(J, J->list); release(J, J->coff); release(J, J->cent);

@@ -1,5 +1,5 @@
 """Whole grids on both sides of the sizes where a launch changes its form: the
-one-launch set-up (2^16 triangles), blocks of the flag packing (1024 words) and of
+blocks of the set-up (256 triangles), of the flag packing (1024 words) and of
 the scans (4096), the tile offsets by the count's last block, the Level2
 SAT's rows in pieces (n2 > 8), waves without columns in the ray expansion, and downloads
 in one launch or in chunks.  Against the oracle, every product, bit for bit."""
