@@ -67,3 +67,24 @@ def test_walls_without_columns(gv, orc):
         g = c.voxelize(soup, bmin, bmax, mms, 70, 3)
         compare_results("walls", g.download(), want, 3)
         g.release()
+
+
+def test_download_with_little_memory(gv):
+    """The arrays of a download one after the other where the device memory for
+    their exports does not hold two of them."""
+    v, f = gv.icosphere(4, 0.4, (0.5, 0.5, 0.5), 0.02, seed=24)
+    soup = gv.flatten(v, f)
+    bmin, bmax, mms = gv.mesh_bbox(v)
+    with gv.Context() as c:
+        say("download with little memory")
+        g = c.voxelize(soup, bmin, bmax, mms, 96, 2)
+        want = g.download()
+        n1 = want["l1"].size
+        need = 1 << (4 * n1 - 1).bit_length()
+        assert want["l2"].size <= need
+        c.set_mem_limit(c.pool_stats()["live_bytes"] + need)
+        got = g.download()
+        for k in ("l1", "prefix", "bidx", "l2"):
+            assert np.array_equal(got[k], want[k]), k
+        c.set_mem_limit(0)
+        g.release()
