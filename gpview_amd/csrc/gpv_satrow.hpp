@@ -255,15 +255,21 @@ __host__ __device__ __forceinline__ SatRow sat_row_at(const float4* e, int q, in
     return s;
 }
 
-// A row of a loose entry (nothing of it is bounded): all layers of its columns undecided.
+// A row of a loose entry (nothing of it is bounded): all layers of its columns undecided,
+// none certain.  Every term is set: an entry is loose where its coefficients may be
+// infinite or NaN, those of the (x, y) predicates among them.
 __host__ __device__ __forceinline__ void sat_row_loose(SatRow& s, bool loose, int ra, int rb)
 {
     if (!loose) return;
     s.a0 = s.a1 = s.a2 = s.pa = 0.0f;
     s.w0 = s.w1 = s.w2 = s.pw = 0.0f;
     s.m0 = s.m1 = s.m2 = s.pm = 1e30f;
-    s.lom = (float)ra;
+    s.n0 = s.n1 = s.n2 = s.pn = 0.0f;
+    s.lom = s.loi = (float)ra;
     s.him = (float)rb + 1.0f;
+    s.hii = 0.0f;
+    s.e0 = s.e1 = s.e2 = 0.0f;
+    s.u0 = s.u1 = s.u2 = 0.0f;
     s.um = 3e38f;
 }
 

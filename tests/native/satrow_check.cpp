@@ -58,6 +58,45 @@ extern "C" void satrow_batch(int64_t n, int n2, const float* tv, const float* cx
     }
 }
 
+// The same with every row walked in pieces of `piece` columns, each begun at its own
+// column with sat_row_at and, for a loose entry, sat_row_loose: the kernel's own
+// sequence, with no word of the harness's about loose entries.
+extern "C" void satrow_pieces(int64_t n, int n2, int piece, const float* tv, const float* cx, const float* cy, const float* cz,
+                              const float* lo, const float* hi, const float* g2, const float* h, int cuda_l2,
+                              uint32_t* in, uint32_t* may, uint8_t* is_loose)
+{
+    for (int64_t i = 0; i < n; ++i) {
+        const float* t = tv + 9 * i;
+        const float *X = cx + n2 * i, *Y = cy + n2 * i, *Z = cz + n2 * i;
+        gpv::SatScale g;
+        gpv::sat_scale_axis(lo[3 * i], hi[3 * i], g2[3 * i], cuda_l2 != 0, g.sx, g.dx);
+        gpv::sat_scale_axis(lo[3 * i + 1], hi[3 * i + 1], g2[3 * i + 1], cuda_l2 != 0, g.sy, g.dy);
+        gpv::sat_scale_axis(lo[3 * i + 2], hi[3 * i + 2], g2[3 * i + 2], cuda_l2 != 0, g.sz, g.dz);
+        int pa = n2, pb = -1, ra = n2, rb = -1;
+        for (int p = 0; p < n2; ++p) {
+            if (axis_ok(t[0], t[3], t[6], X[p], h[3 * i])) { pa = p < pa ? p : pa; pb = p; }
+            if (axis_ok(t[2], t[5], t[8], Z[p], h[3 * i + 2])) { ra = p < ra ? p : ra; rb = p; }
+        }
+        float4 e[gpv::kSatEntry4];
+        bool loose = gpv::sat_entry_part(0, t, X[0], Y[0], Z[0], g, e);
+        loose = gpv::sat_entry_part(1, t, X[0], Y[0], Z[0], g, e) || loose;
+        is_loose[i] = loose;
+        for (int q = 0; q < n2; ++q) {
+            uint32_t* oi = in + (int64_t)(i * n2 + q) * n2;
+            uint32_t* om = may + (int64_t)(i * n2 + q) * n2;
+            for (int p = 0; p < n2; ++p) oi[p] = om[p] = 0;
+            if (pb < 0 || rb < 0 || !axis_ok(t[1], t[4], t[7], Y[q], h[3 * i + 1])) continue;
+            int p = pa, left = pb - pa + 1;
+            gpv::sat_row_range(e, q, loose, p, left);
+            for (; left > 0; p += piece, left -= piece) {
+                gpv::SatRow s = gpv::sat_row_at(e, q, ra, rb, p);
+                gpv::sat_row_loose(s, loose, ra, rb);
+                for (int k = 0; k < (left < piece ? left : piece); ++k) gpv::sat_row_column(s, oi[p + k], om[p + k]);
+            }
+        }
+    }
+}
+
 // Level1: case i's index AABB (lo, dd: 3 ints each) on a grid with centers
 // cx/cy/cz, bounds lo3/hi3 and voxel g1; per column of it in (q, p) order from
 // off[i]: [am, ai, bi, bm).
