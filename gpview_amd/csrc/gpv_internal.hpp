@@ -176,7 +176,34 @@ void launch_pack_bytes(const uint8_t* by, int64_t W, uint64_t* bits, uint32_t* c
 void launch_ray_expand(const float* tris, int64_t T, const int4* ray_rng, const uint64_t* off, const GridDev& g0,
                        const Meshes& M, uint64_t* ins, int blocks, hipStream_t s);
 
-// words of scratch of a two-level counting sort with at most nkeys keys, zeros at its start
+// Two-level counting sort: tiles of 2^8 to 2^13 keys, at most 8192 tiles below 2^26
+// keys and 16384 at 2^27.  The count and bucket passes hold a counter per
+// tile in every block's LDS (32 KiB at 8192 tiles: five blocks per CU, where 16384
+// tiles allowed two), the place pass one per key of its tile (at most 32 KiB).
+constexpr int ts_shift(uint64_t nkeys)
+{
+    int lg = 0;
+    while ((1ull << lg) < nkeys) ++lg;
+    const int sh = lg - 13;
+    return sh < 8 ? 8 : sh > 13 ? 13 : sh;
+}
+constexpr size_t ts_tiles(uint64_t nkeys)
+{
+    const int shift = ts_shift(nkeys);
+    return (size_t)((nkeys + (1u << shift) - 1) >> shift);
+}
+// The scan over a sort's tiles by one block lies in LDS, tile t at word t + (t >>
+// ts_pad): up to 8192 tiles a word in 33 is left out so that the threads' runs start in
+// different banks; more fill 64 KiB as they are.
+__host__ __device__ constexpr int ts_pad(int ntiles) { return ntiles <= 8192 ? 5 : 31; }
+__host__ __device__ constexpr size_t ts_scan_words(int ntiles) { return (size_t)ntiles + (size_t)(ntiles >> ts_pad(ntiles)); }
+// LDS words of a launch whose blocks scan one of two sorts' tiles each.  More tiles can
+// take fewer words (8193 with 8192), so the larger need counts, not the larger sort.
+constexpr size_t ts_scan_lds(int a, int b)
+{
+    return ts_scan_words(a) > ts_scan_words(b) ? ts_scan_words(a) : ts_scan_words(b);
+}
+// words of scratch of a sort with at most nkeys keys, zeros at its start
 size_t ts_words(uint64_t nkeys);
 
 // bin pairs (key = batch-wide boundary bit index, triangle) -> CSR by boundary rank

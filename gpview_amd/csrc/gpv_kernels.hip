@@ -1715,11 +1715,7 @@ __device__ __forceinline__ void ts_histogram(const Src& src, uint64_t lo, uint64
 }
 
 // Tile totals -> tile offsets by one block of NT threads; s_h holds
-// ts_scan_words(ntiles) words, up to 8192 tiles a word in 33 left out so that the
-// threads' runs start in different banks.  Atomic loads: blocks of the same launch added the totals.
-__host__ __device__ inline int ts_pad(int ntiles) { return ntiles <= 8192 ? 5 : 31; }
-__host__ __device__ inline size_t ts_scan_words(int ntiles) { return (size_t)ntiles + (size_t)(ntiles >> ts_pad(ntiles)); }
-
+// ts_scan_words(ntiles) words.  Atomic loads: blocks of the same launch added the totals.
 template <int NT>
 __device__ __forceinline__ void ts_scan(const uint32_t* __restrict__ total, uint32_t* __restrict__ off, int ntiles,
                                         uint32_t* s_h, uint32_t* s_wave)
@@ -1927,24 +1923,7 @@ __global__ __launch_bounds__(TS_NT) void k_ts_place(TsSort<PairSrc> a, uint32_t*
     else ts_place(b, coff, nullptr, pb, s_c, s_wave, &s_max);
 }
 
-// tile size 2^shift, 2^8 (TS_NT) to 2^13 keys: at most 8192 tiles below 2^26
-// keys, 16384 at 2^27.  The count and bucket passes hold a counter per tile
-// in every block's LDS (32 KiB at 8192 tiles: five blocks per CU, where
-// 16384 tiles allowed two), the place pass one per key of its tile (at most
-// 32 KiB).
-int ts_shift(uint64_t nkeys)
-{
-    int lg = 0;
-    while ((1ull << lg) < nkeys) ++lg;
-    const int sh = lg - 13;
-    return sh < 8 ? 8 : sh > 13 ? 13 : sh;
-}
-
-size_t ts_tiles(uint64_t nkeys)
-{
-    const int shift = ts_shift(nkeys);
-    return (size_t)((nkeys + (1u << shift) - 1) >> shift);
-}
+static_assert(1u << ts_shift(0) == TS_NT, "ts_place: every thread owns at least one key of a tile");
 
 // tiles of any sort with at most nkeys keys
 static size_t ts_tiles_most(uint64_t nkeys) { return nkeys <= (1u << 21) ? ts_tiles(nkeys) : nkeys <= (1u << 26) ? 8192 : 16384; }
@@ -1969,7 +1948,8 @@ void launch_bins(const BinPairs& P, const BinCols& C, const uint64_t* bnd, const
     // saves (5 us): the blocks' counter takes 3.7 ns each, and 256 threads a
     // tile each a round
     const bool last = blocks <= 256 && tiles <= 2048;
-    const size_t lds = last ? ts_scan_words(tiles) * 4 : (size_t)tiles * 4;
+    const size_t scan = ts_scan_lds(a.ntiles, b.ntiles) * 4;
+    const size_t lds = last ? scan : (size_t)tiles * 4;
     const dim3 grid((unsigned)std::max(blocks, grid_for(W, TS_NT, 2048)), 3);
     if (M.nm > 1)
         k_ts_count<true><<<grid, TS_NT, lds, s>>>(a, b, last, g0, M, bnd, wprefix, W, bidx);
@@ -1977,7 +1957,7 @@ void launch_bins(const BinPairs& P, const BinCols& C, const uint64_t* bnd, const
         k_ts_count<false><<<grid, TS_NT, lds, s>>>(a, b, last, g0, M, bnd, wprefix, W, bidx);
     if (!P.B) launch_fill_u32(P.off, 0, 1, s);   // no keys, hence no items
     if (!blocks) return;
-    if (!last) k_ts_scan<<<2, 1024, ts_scan_words(tiles) * 4, s>>>(a, b);
+    if (!last) k_ts_scan<<<2, 1024, scan, s>>>(a, b);
     k_ts_bucket<<<dim3((unsigned)blocks, 2), TS_NT, (size_t)tiles * 4, s>>>(a, b);
     k_ts_place<<<dim3((unsigned)tiles, 2), TS_NT, (size_t)4 << std::max(a.shift, b.shift), s>>>(a, P.off, P.max_out, PairPlace{P.list}, b,
                                                                                           C.off, ColPlace{C.ent});
