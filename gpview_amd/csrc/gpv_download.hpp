@@ -1,4 +1,4 @@
-// gpv_download.hpp -- results from the device into ordinary host memory.
+// gpv_download.hpp -- results from the device into host memory.
 //
 // hipMemcpyAsync into pageable memory takes 15 to 25 us a call and then moves about
 // 14 GB/s: it stages on one thread, after the copy.  Here kernels write into
@@ -7,6 +7,10 @@
 // threads while the next ones arrive: 6 MB of states 430 -> 290 us, 8 MB of normals 640 ->
 // 400, four small arrays 60 -> 15; six helpers were slower than three.  Staging and threads belong to a context (its
 // lock is held by the caller) and go with it.
+//
+// Page-locked destinations need no staging: larger results are copied straight there, at
+// 52 GB/s (222 MB of states 5.99 -> 4.23 ms, 10 MB 362 -> 248 us).  Small ones
+// stay with the one launch (20 KB in four arrays: 25 us, 65 in four copies).
 #pragma once
 
 #include "gpv_internal.hpp"
@@ -38,12 +42,25 @@ public:
         for (int k = 0; k < count; ++k) total += up(p[k].n);
         if (total == 0) return hipStreamSynchronize(s);
         const bool one = total <= kSmall && count <= kCopyMax;
-        const hipError_t e = open(one ? kSmall : kChunks * kChunkMax);
-        if (e != hipSuccess) {
-            (void)hipStreamSynchronize(s);
-            return e;
+        hipError_t e = hipSuccess;
+        total = 0;
+        staged_.clear();
+        for (int k = 0; k < count && e == hipSuccess; ++k) {
+            if (!p[k].n) continue;
+            if (direct(p[k].dst, one)) {
+                e = hipMemcpyAsync(p[k].dst, p[k].src, p[k].n, hipMemcpyDeviceToHost, s);
+            } else {
+                staged_.push_back(p[k]);
+                total += up(p[k].n);
+            }
         }
-        return one ? small(p, count, s) : large(p, count, total, s);
+        if (e == hipSuccess && total) {
+            const int n = (int)staged_.size();
+            e = open(one ? kSmall : kChunks * kChunkMax);
+            if (e == hipSuccess) return one ? small(staged_.data(), n, s) : large(staged_.data(), n, total, s);
+        }
+        const hipError_t w = hipStreamSynchronize(s);
+        return e == hipSuccess ? w : e;
     }
 
     void close()
@@ -73,6 +90,18 @@ private:
     static constexpr size_t kChunkMin = size_t(512) << 10, kChunkMax = size_t(2) << 20;
     static constexpr int kHelpers = 3;
     static size_t up(size_t n) { return (n + kAlign - 1) / kAlign * kAlign; }
+
+    // Whether the runtime copies to dst: to device memory always, to page-locked
+    // memory where the results are not small.
+    static bool direct(const void* dst, bool one)
+    {
+        hipPointerAttribute_t a{};
+        if (hipPointerGetAttributes(&a, dst) != hipSuccess) {
+            (void)hipGetLastError();   // pageable memory
+            return false;
+        }
+        return a.type == hipMemoryTypeDevice || (!one && a.type != hipMemoryTypeUnregistered);
+    }
 
     hipError_t open(size_t bytes)
     {
@@ -232,6 +261,7 @@ private:
     uint64_t gen_ = 0;      // of the round at hand (mu_)
     int active_ = 0;        // helpers in a round (mu_)
     bool quit_ = false;     // (mu_)
+    std::vector<Piece> staged_;
     std::vector<Piece> items_;   // rewritten only while no helper is active
     std::atomic<int> next_{0}, ready_{0}, done_{0};
     std::atomic<bool> failed_{false};
