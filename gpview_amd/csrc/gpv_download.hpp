@@ -18,8 +18,8 @@
 #include <atomic>
 #include <condition_variable>
 #include <cstring>
+#include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -56,8 +56,12 @@ public:
         }
         if (e == hipSuccess && total) {
             const int n = (int)staged_.size();
-            e = open(one ? kSmall : kChunks * kChunkMax);
-            if (e == hipSuccess) return one ? small(staged_.data(), n, s) : large(staged_.data(), n, total, s);
+            if (open(one ? kSmall : kChunks * kChunkMax) == hipSuccess)
+                return one ? small(staged_.data(), n, s) : large(staged_.data(), n, total, s);
+            // no staging to be had: the runtime's own copies
+            (void)hipGetLastError();
+            for (int k = 0; k < n && e == hipSuccess; ++k)
+                e = hipMemcpyAsync(staged_[k].dst, staged_[k].src, staged_[k].n, hipMemcpyDeviceToHost, s);
         }
         const hipError_t w = hipStreamSynchronize(s);
         return e == hipSuccess ? w : e;
@@ -230,7 +234,7 @@ private:
         started_ = true;
         try {
             while ((int)threads_.size() < kHelpers) threads_.emplace_back([this] { helper(); });
-        } catch (const std::system_error&) {
+        } catch (const std::exception&) {
             // the caller copies alone, or with those that started
         }
     }

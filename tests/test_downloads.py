@@ -82,6 +82,17 @@ def test_device_destinations_are_never_written_by_the_host(down, n):
     assert log["copy_bytes"] >= n
 
 
+@pytest.mark.parametrize("what", ["no_locked", "no_events"])
+@pytest.mark.parametrize("n", [100, SMALL, SMALL + 1, 5 << 20])
+def test_downloads_without_staging(down, n, what):
+    """No page-locked memory or no events left: the download still arrives, leaves no error
+    behind, and the next one has its staging again."""
+    pieces = [(n, PAGEABLE, 0), (n // 2, PAGEABLE, 4)]
+    log = down.run(pieces, **{what: True})
+    assert log["copy_bytes"] in (0, n + n // 2)
+    assert down.run(pieces)["kernel_bytes"] == n + n // 2
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("l1,n2", [(8, 4), (40, 5), (100, 3)])
 def test_page_locked_download(gv, l1, n2):
