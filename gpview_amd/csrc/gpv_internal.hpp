@@ -63,20 +63,25 @@ __host__ __device__ inline float center_at(int which, int k, float bmin, float g
 }
 
 // Where one mesh of a batch lives in the batch-wide arrays.  A batch
-// concatenates the meshes' soups (tri0), Level1 bitplanes (word0), xy
-// columns (col0), boundary voxels (b0) and Level2 words (l2w0); entry nm is
-// the sentinel holding the totals.  b0 and l2w0 are filled on the device
-// once the boundary scan is known.
+// concatenates the meshes' soups (tri0), Level1 bitplanes (word0) and xy
+// columns (col0); entry nm is the sentinel holding the totals.  Set when the run is
+// created and never written again: kernels on both streams read it.
 struct MeshOff {
     uint64_t word0;
-    uint64_t l2w0;
-    uint64_t l2n0;   // first Level2 normal (one per Level2 voxel of meshes with normals)
     uint32_t col0;
     uint32_t tri0;
-    uint32_t b0;
     uint32_t ptask0;   // first Level1 fill block (L1F_W words of a layer)
     uint32_t pw0;      // first Level2 parity wave
-    uint32_t sg0;      // first Level2 SAT group (set on the host once boundary counts are known)
+};
+
+// The same for what follows from the boundary scan, a table of its own because the
+// main stream writes it while the Level1 parity runs on the other one: boundary voxels (b0),
+// Level2 words (l2w0) and normals by the device, SAT groups by the host.
+struct MeshRank {
+    uint64_t l2w0;
+    uint64_t l2n0;   // first Level2 normal (one per Level2 voxel of meshes with normals)
+    uint32_t b0;
+    uint32_t sg0;    // first Level2 SAT group (l2_plan)
 };
 
 // Per-mesh results accumulated on the device.
@@ -95,7 +100,8 @@ struct MeshCtr {
 // 0 and only ctr is used.
 struct Meshes {
     const GridDev* grids;       // [nm]
-    MeshOff* off;               // [nm + 1]
+    const MeshOff* off;         // [nm + 1]
+    MeshRank* rank;             // [nm + 1]
     const uint32_t* tri_mesh;   // [T]  mesh of each triangle (non-decreasing)
     uint32_t* bmesh;            // [B]  mesh of each boundary voxel (non-decreasing)
     MeshCtr* ctr;               // [nm]
@@ -118,7 +124,7 @@ struct Counters {
     unsigned long long bad_input;   // nonzero: a vertex coordinate is not finite or beyond +-2^40
     unsigned long long done;        // blocks of the state counts that are through
 };
-// page-locked read-back, written by kernels: Counters | B (one mesh) or MeshOff[nm + 1] | MeshCtr[nm]
+// page-locked read-back, written by kernels: Counters | B (one mesh) or MeshRank[nm + 1] | MeshCtr[nm]
 constexpr size_t kHOff = 64;
 
 // sets the calling thread's gpv_last_error text and returns code
@@ -269,7 +275,7 @@ void launch_l1_stencil(const float* tris, int64_t T, const GridDev& g, uint32_t*
 // toggles -> inside bits, in place, but for the stencil meshes; blocks: l1_fill_blocks of all meshes
 void launch_l1_fill(const GridDev& g0, const Meshes& M, int64_t blocks, uint64_t* ins, hipStream_t s);
 
-// b0 and l2w0 of every mesh (and the totals in entry nm) from the word prefix
+// b0, l2w0 and l2n0 of every mesh (and the totals in entry nm) from the word prefix
 // and the counters, to the page-locked read-back pub as well
 void launch_mesh_bounds(const uint32_t* wprefix, const Meshes& M, const Counters* ctr, uint64_t* pub, hipStream_t s);
 // per-mesh bin totals and largest bin (multi-mesh runs)

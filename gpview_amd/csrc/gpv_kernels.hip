@@ -166,8 +166,8 @@ __device__ __forceinline__ int uniform_i(int v) { return __builtin_amdgcn_readfi
 // Largest m in [0, nm) with key(off[m]) <= x for a wave-uniform x (given
 // key(off[0]) <= x), by the whole wave: 64 meshes per round of independent
 // loads, so two rounds of latency up to 4096 meshes instead of log2(nm).
-template <typename K>
-__device__ __forceinline__ int wave_mesh_search(const MeshOff* __restrict__ off, int nm, uint64_t x, K key)
+template <typename E, typename K>
+__device__ __forceinline__ int wave_mesh_search(const E* __restrict__ off, int nm, uint64_t x, K key)
 {
     const int lane = __lane_id();
     int lo = 0, hi = nm;   // key(off[lo]) <= x; the answer lies in [lo, hi)
@@ -1558,15 +1558,12 @@ __global__ __launch_bounds__(64) void k_mesh_bounds(const uint32_t* __restrict__
         }
         const uint64_t wi = wave_incl_scan<uint64_t>(w), ni = wave_incl_scan<uint64_t>(nrm);
         if (m <= M.nm) {
-            MeshOff o = M.off[m];
-            o.b0 = b0;
-            o.l2w0 = l2 + wi - w;
-            o.l2n0 = l2n + ni - nrm;
-            M.off[m] = o;
-            uint64_t q[sizeof(MeshOff) / 8];
+            const MeshRank o{l2 + wi - w, l2n + ni - nrm, b0, 0u};
+            M.rank[m] = o;
+            uint64_t q[sizeof(MeshRank) / 8];
             __builtin_memcpy(q, &o, sizeof o);
-            for (int k = 0; k < (int)(sizeof(MeshOff) / 8); ++k)
-                publish(pub + kHOff / 8 + (size_t)m * (sizeof(MeshOff) / 8) + k, q[k]);
+            for (int k = 0; k < (int)(sizeof(MeshRank) / 8); ++k)
+                publish(pub + kHOff / 8 + (size_t)m * (sizeof(MeshRank) / 8) + k, q[k]);
         }
         l2 += shfl64(wi, 63);
         l2n += shfl64(ni, 63);
@@ -1580,7 +1577,7 @@ __global__ __launch_bounds__(64) void k_mesh_bounds(const uint32_t* __restrict__
 
 void launch_mesh_bounds(const uint32_t* wprefix, const Meshes& M, const Counters* ctr, uint64_t* pub, hipStream_t s)
 {
-    static_assert(sizeof(MeshOff) % 8 == 0, "published by words");
+    static_assert(sizeof(MeshRank) % 8 == 0, "published by words");
     k_mesh_bounds<<<1, 64, 0, s>>>(wprefix, M, ctr, pub);
 }
 
@@ -1971,7 +1968,7 @@ __global__ __launch_bounds__(256) void k_mesh_bins(const uint32_t* __restrict__ 
 {
     __shared__ uint32_t s_max[4];
     for (int m = (int)blockIdx.y; m < M.nm; m += (int)gridDim.y) {
-        const uint32_t b0 = M.off[m].b0, b1 = M.off[m + 1].b0;
+        const uint32_t b0 = M.rank[m].b0, b1 = M.rank[m + 1].b0;
         uint32_t mx = 0;
         for (uint32_t b = b0 + blockIdx.x * 256u + threadIdx.x; b < b1; b += gridDim.x * 256u) {
             const uint32_t c = boff[b + 1] - boff[b];
@@ -2142,16 +2139,16 @@ __global__ __launch_bounds__(64 * W) void k_l2_sat(const float* __restrict__ tri
     if (grp >= ngroups) return;
     int mesh = 0;
     if constexpr (kM)
-        mesh = wave_mesh_search(M.off, M.nm, (uint64_t)grp, [](const MeshOff& o) { return (uint64_t)o.sg0; });
+        mesh = wave_mesh_search(M.rank, M.nm, (uint64_t)grp, [](const MeshRank& o) { return (uint64_t)o.sg0; });
     const GridDev& g = grid_of<kM>(g0, M, mesh);
     const int n2 = g.n2, w2 = g.w2, nsc = n2 * n2;
     if (kM && n2 == 0) return;
-    const int64_t mb0 = kM ? (int64_t)M.off[mesh].b0 : 0, mb1 = kM ? (int64_t)M.off[mesh + 1].b0 : B;
+    const int64_t mb0 = kM ? (int64_t)M.rank[mesh].b0 : 0, mb1 = kM ? (int64_t)M.rank[mesh + 1].b0 : B;
     const int G = l2_group_voxels(n2, gmost);
-    const int64_t vb0 = mb0 + (grp - (kM ? (int64_t)M.off[mesh].sg0 : 0)) * G;
+    const int64_t vb0 = mb0 + (grp - (kM ? (int64_t)M.rank[mesh].sg0 : 0)) * G;
     if (vb0 >= mb1) return;
     const int nv = (int)(mb1 - vb0 < G ? mb1 - vb0 : G);
-    uint64_t* out = sat2 + (kM ? M.off[mesh].l2w0 : 0) + (uint64_t)(vb0 - mb0) * w2;
+    uint64_t* out = sat2 + (kM ? M.rank[mesh].l2w0 : 0) + (uint64_t)(vb0 - mb0) * w2;
     for (int i = lane; i < (nv * nsc * (n2 > 8 ? 2 : 1) + 3) / 4; i += 64) L.acc[i] = 0u;
     if (lane <= nv) L.vb[lane] = boff[vb0 + lane];
     if (lane < nv) {
@@ -2799,8 +2796,8 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 1 ?
     const int col = (int)(wave - (kM ? (int64_t)M.off[mesh].pw0 : 0)) * C;
     const int j1 = col / g.nx, i1 = col - j1 * g.nx;
     const uint64_t word0 = kM ? M.off[mesh].word0 : 0;
-    const uint32_t col0 = kM ? M.off[mesh].col0 : 0, b0 = kM ? M.off[mesh].b0 : 0;
-    uint64_t* out = par2 + (kM ? M.off[mesh].l2w0 : 0);
+    const uint32_t col0 = kM ? M.off[mesh].col0 : 0, b0 = kM ? M.rank[mesh].b0 : 0;
+    uint64_t* out = par2 + (kM ? M.rank[mesh].l2w0 : 0);
     if (C == 2)
         l2_parity_columns_wave<2>(s_l[wv], cb, nw, g, i1, j1, word0, col0, b0, bnd, wprefix, coff, ent, tris, out);
     else if (C == 4)
@@ -3000,7 +2997,7 @@ __global__ __launch_bounds__(256) void k_l2_normals(const float* __restrict__ tr
     if (n2 == 0 || (kM && !g.normals)) return;
     const float h2x = g.h2x, h2y = g.h2y, h2z = g.h2z;
     const int S = n2 * n2 * n2;
-    float* out = l2n + 3 * (kM ? M.off[mesh].l2n0 + (uint64_t)(b - M.off[mesh].b0) * S : (uint64_t)b * S);
+    float* out = l2n + 3 * (kM ? M.rank[mesh].l2n0 + (uint64_t)(b - M.rank[mesh].b0) * S : (uint64_t)b * S);
     const int v = bidx[b];
     const int nxy = gnx * gny;
     const int k1 = v / nxy;
@@ -3145,7 +3142,7 @@ __global__ void k_count_states(const uint64_t* __restrict__ bnd, const uint64_t*
     __shared__ uint32_t s_last;
     const int mesh = kM ? (int)blockIdx.y : 0;
     const uint64_t w_lo = kM ? M.off[mesh].word0 : 0, w_hi = kM ? M.off[mesh + 1].word0 : (uint64_t)W;
-    const uint64_t l_lo = kM ? M.off[mesh].l2w0 : 0, l_hi = kM ? M.off[mesh + 1].l2w0 : (uint64_t)W2;
+    const uint64_t l_lo = kM ? M.rank[mesh].l2w0 : 0, l_hi = kM ? M.rank[mesh + 1].l2w0 : (uint64_t)W2;
     uint64_t a = 0, b = 0, c = 0;
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t i = w_lo + (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < w_hi; i += stride)

@@ -252,6 +252,7 @@ struct Job {
     std::vector<gpv_grid_info> info;   // [nm]
     std::vector<GridDev> g;            // [nm], device table pointers
     std::vector<MeshOff> off;          // [nm + 1]
+    std::vector<MeshRank> rank;        // [nm + 1], once the boundary counts are known
     int64_t T = 0;
     const float* tris = nullptr;
     float* own_soup = nullptr;
@@ -260,6 +261,7 @@ struct Job {
     float* tables = nullptr;
     GridDev* d_grids = nullptr;
     MeshOff* d_off = nullptr;
+    MeshRank* d_rank = nullptr;
     uint32_t* tri_mesh = nullptr;
     uint32_t* bmesh = nullptr;
     MeshCtr* mctr = nullptr;
@@ -336,8 +338,8 @@ struct Job {
     int32_t* out_bidx = nullptr;
     uint64_t *out_sat2 = nullptr, *out_par2 = nullptr;
 
-    Meshes view() const { return Meshes{d_grids, d_off, tri_mesh, bmesh, mctr, nm}; }
-    int64_t nb(int m) const { return (int64_t)off[m + 1].b0 - (int64_t)off[m].b0; }
+    Meshes view() const { return Meshes{d_grids, d_off, d_rank, tri_mesh, bmesh, mctr, nm}; }
+    int64_t nb(int m) const { return (int64_t)rank[m + 1].b0 - (int64_t)rank[m].b0; }
 };
 
 }  // namespace gpv
@@ -480,9 +482,9 @@ int ensure_hbuf(gpv_ctx* c, size_t bytes)
     return GPV_OK;
 }
 
-// pinned staging layout: Counters | MeshOff[nm + 1] | MeshCtr[nm]
+// pinned staging layout: Counters | MeshRank[nm + 1] | MeshCtr[nm]
 static_assert(sizeof(Counters) <= kHOff, "the offsets follow the counters");
-size_t hctr_at(int nm) { return (kHOff + sizeof(MeshOff) * (size_t)(nm + 1) + 63) / 64 * 64; }
+size_t hctr_at(int nm) { return (kHOff + sizeof(MeshRank) * (size_t)(nm + 1) + 63) / 64 * 64; }
 
 int ensure_scan_tmp(Job* J, int64_t n)
 {
@@ -626,6 +628,7 @@ int job_create(gpv_ctx* c, const gpv_mesh_desc* d, int nm, int on_device, Job** 
     // per-mesh grids, offsets and the concatenated center tables
     J->g.resize((size_t)nm);
     J->off.assign((size_t)nm + 1, MeshOff{});
+    J->rank.assign((size_t)nm + 1, MeshRank{});
     std::vector<size_t> tab_at((size_t)nm * 12);
     size_t ntab = 0;
     uint64_t word0 = 0;
@@ -730,7 +733,7 @@ int job_create(gpv_ctx* c, const gpv_mesh_desc* d, int nm, int on_device, Job** 
     if ((r = alloc(J, &J->mctr, (size_t)nm)) != GPV_OK) return bail(r);
     if (nm > 1) {
         if ((r = alloc(J, &J->d_grids, (size_t)nm)) || (r = alloc(J, &J->d_off, (size_t)nm + 1)) ||
-            (r = alloc(J, &J->tri_mesh, (size_t)std::max<int64_t>(T, 1))))
+            (r = alloc(J, &J->d_rank, (size_t)nm + 1)) || (r = alloc(J, &J->tri_mesh, (size_t)std::max<int64_t>(T, 1))))
             return bail(r);
         if (hipMemcpyAsync(J->d_grids, J->g.data(), sizeof(GridDev) * (size_t)nm, hipMemcpyHostToDevice,
                            c->stream) != hipSuccess ||
@@ -947,22 +950,22 @@ int complete_sat(Job* J, int64_t* needed)
     J->n_pairs = np;
     J->n_cols = nc;
     if (J->nm > 1) {
-        memcpy(J->off.data(), c->h_buf + kHOff, sizeof(MeshOff) * ((size_t)J->nm + 1));
+        memcpy(J->rank.data(), c->h_buf + kHOff, sizeof(MeshRank) * ((size_t)J->nm + 1));
     } else {
         const uint32_t B = *reinterpret_cast<const uint32_t*>(c->h_buf + kHOff);
-        J->off[0].b0 = 0;
-        J->off[0].l2w0 = 0;
-        J->off[1].b0 = B;
-        J->off[1].l2w0 = (uint64_t)B * (uint64_t)J->g[0].w2;
-        J->off[0].l2n0 = 0;
-        J->off[1].l2n0 = J->g[0].normals ? (uint64_t)B * J->g[0].n2 * J->g[0].n2 * J->g[0].n2 : 0;
+        J->rank[0].b0 = 0;
+        J->rank[0].l2w0 = 0;
+        J->rank[1].b0 = B;
+        J->rank[1].l2w0 = (uint64_t)B * (uint64_t)J->g[0].w2;
+        J->rank[0].l2n0 = 0;
+        J->rank[1].l2n0 = J->g[0].normals ? (uint64_t)B * J->g[0].n2 * J->g[0].n2 * J->g[0].n2 : 0;
     }
-    J->B = J->off[J->nm].b0;
+    J->B = J->rank[J->nm].b0;
     if (J->B > (int64_t(1) << 27))
         return fail(GPV_ERR_INVALID, "%lld boundary voxels: at most 2^27 per batch (split the batch)",
                     (long long)J->B);
-    J->W2 = (int64_t)J->off[J->nm].l2w0;
-    J->NL2 = (int64_t)J->off[J->nm].l2n0;
+    J->W2 = (int64_t)J->rank[J->nm].l2w0;
+    J->NL2 = (int64_t)J->rank[J->nm].l2n0;
     J->sat_done = true;
     return GPV_OK;
 }
@@ -1065,29 +1068,29 @@ int l2_sat_most(const Job* J)
 }
 
 // Level2 SAT groups of the job; in a batch each mesh's first one goes to
-// MeshOff::sg0 on the device (main stream, before the fork of the side
-// stream's kernels that read the table)
+// MeshRank::sg0 on the device (nothing on the side stream reads that table before
+// it waits for ev[6], recorded after this copy)
 int l2_plan(Job* J)
 {
     int64_t sg = 0;
     J->l2s_most = l2_sat_most(J);
     for (int m = 0; m < J->nm; ++m) {
-        J->off[m].sg0 = (uint32_t)sg;
+        J->rank[m].sg0 = (uint32_t)sg;
         if (J->g[m].n2 > 0) {
             const int64_t c = l2_group_voxels(J->g[m].n2, J->l2s_most);
             sg += (J->nb(m) + c - 1) / c;
         }
     }
-    J->off[J->nm].sg0 = (uint32_t)sg;
+    J->rank[J->nm].sg0 = (uint32_t)sg;
     J->l2s_groups = sg;
     if (J->nm > 1) {
         hipStream_t s = J->ctx->stream;
-        // the MeshOff staging region was last filled by the size read-back,
+        // the MeshRank staging region was last filled by the size read-back,
         // which the host has already waited for; a later job refills it only
         // after its own read-back, which this stream orders after this copy
-        MeshOff* h = reinterpret_cast<MeshOff*>(J->ctx->h_buf + kHOff);
-        memcpy(h, J->off.data(), sizeof(MeshOff) * ((size_t)J->nm + 1));
-        HIP_TRY(hipMemcpyAsync(J->d_off, h, sizeof(MeshOff) * ((size_t)J->nm + 1), hipMemcpyHostToDevice, s));
+        MeshRank* h = reinterpret_cast<MeshRank*>(J->ctx->h_buf + kHOff);
+        memcpy(h, J->rank.data(), sizeof(MeshRank) * ((size_t)J->nm + 1));
+        HIP_TRY(hipMemcpyAsync(J->d_rank, h, sizeof(MeshRank) * ((size_t)J->nm + 1), hipMemcpyHostToDevice, s));
     }
     return GPV_OK;
 }
@@ -1251,7 +1254,7 @@ int job_finish(Job* J)
     release(J, J->sat_sums); release(J, J->ray_sums); release(J, J->bbytes); release(J, J->tri_mesh);
     release(J, J->st_cnt); release(J, J->st_off); release(J, J->st_scan); release(J, J->st_tog);
     release(J, J->bmesh);
-    release(J, J->d_grids); release(J, J->d_off); release(J, J->own_soup); release(J, J->mctr);
+    release(J, J->d_grids); release(J, J->d_off); release(J, J->d_rank); release(J, J->own_soup); release(J, J->mctr);
     release(J, J->soup_pieces);
     release(J, J->fnorm); release(J, J->slist);
     J->tris = nullptr;
@@ -2121,11 +2124,12 @@ int gpv_grid_device_views(const gpv_grid* G, const uint64_t** l1b, const uint64_
     if (!G || !G->job) return fail(GPV_ERR_INVALID, "NULL grid");
     const Job* J = G->job;
     const MeshOff& o = J->off[G->m];
+    const MeshRank& rk = J->rank[G->m];
     if (l1b) *l1b = J->bnd ? J->bnd + o.word0 : nullptr;
     if (l1i) *l1i = J->ins ? J->ins + o.word0 : nullptr;
-    if (l2b) *l2b = J->sat2 && J->g[G->m].n2 > 0 ? J->sat2 + o.l2w0 : nullptr;
-    if (l2i) *l2i = J->par2 && J->g[G->m].n2 > 0 ? J->par2 + o.l2w0 : nullptr;
-    if (bidx) *bidx = J->bidx ? J->bidx + o.b0 : nullptr;
+    if (l2b) *l2b = J->sat2 && J->g[G->m].n2 > 0 ? J->sat2 + rk.l2w0 : nullptr;
+    if (l2i) *l2i = J->par2 && J->g[G->m].n2 > 0 ? J->par2 + rk.l2w0 : nullptr;
+    if (bidx) *bidx = J->bidx ? J->bidx + rk.b0 : nullptr;
     return GPV_OK;
 }
 
@@ -2140,13 +2144,14 @@ int gpv_grid_download_bits(gpv_ctx* c, const gpv_grid* G, uint64_t* l1b, uint64_
     HIP_TRY(hipSetDevice(c->device));
     const GridDev& g = J->g[G->m];
     const MeshOff& o = J->off[G->m];
+    const MeshRank& rk = J->rank[G->m];
     const size_t w1 = (size_t)g.nz * g.ny * g.nxw * 8;
     const size_t w2 = g.n2 > 0 ? (size_t)J->nb(G->m) * g.w2 * 8 : 0;
     hipStream_t s = c->stream;
     const Downloader::Piece pieces[4] = {{l1b, J->bnd + o.word0, l1b ? w1 : 0},
                                          {l1i, J->ins + o.word0, l1i ? w1 : 0},
-                                         {l2b, J->sat2 + o.l2w0, l2b ? w2 : 0},
-                                         {l2i, J->par2 + o.l2w0, l2i ? w2 : 0}};
+                                         {l2b, J->sat2 + rk.l2w0, l2b ? w2 : 0},
+                                         {l2i, J->par2 + rk.l2w0, l2i ? w2 : 0}};
     HIP_TRY(c->down.run(pieces, 4, s));
     return GPV_OK;
 }
@@ -2164,6 +2169,7 @@ static int download_impl(gpv_ctx* c, const gpv_grid* G, uint8_t unit, uint8_t* l
     const int m = G->m;
     const GridDev& g = J->g[m];
     const MeshOff& o = J->off[m];
+    const MeshRank& rk = J->rank[m];
     const int64_t n1 = J->info[m].n1;
     const int64_t nb = J->nb(m);
     const int64_t n23 = (int64_t)g.n2 * g.n2 * g.n2;
@@ -2202,17 +2208,17 @@ static int download_impl(gpv_ctx* c, const gpv_grid* G, uint8_t unit, uint8_t* l
     }
     if (prefix) {
         TRY(room((size_t)n1 * 4));
-        launch_export_prefix(J->bnd + o.word0, J->wprefix + o.word0, o.b0, g, reinterpret_cast<int32_t*>(made[np]), s);
+        launch_export_prefix(J->bnd + o.word0, J->wprefix + o.word0, rk.b0, g, reinterpret_cast<int32_t*>(made[np]), s);
         pieces[np] = {prefix, made[np], (size_t)n1 * 4};
         ++np;
     }
     if (bidx && nb > 0) {
-        pieces[np] = {bidx, J->bidx + o.b0, (size_t)nb * 4};
+        pieces[np] = {bidx, J->bidx + rk.b0, (size_t)nb * 4};
         ++np;
     }
     if (l2 && g.n2 > 0 && nb > 0) {
         TRY(room((size_t)(nb * n23)));
-        launch_export_l2(J->sat2 + o.l2w0, J->par2 + o.l2w0, nb, g, unit, made[np], s);
+        launch_export_l2(J->sat2 + rk.l2w0, J->par2 + rk.l2w0, nb, g, unit, made[np], s);
         pieces[np] = {l2, made[np], (size_t)(nb * n23)};
         ++np;
     }
@@ -2234,13 +2240,13 @@ int gpv_grid_download_normals(gpv_ctx* c, const gpv_grid* G, float* l1n, float* 
     if (!J->finished) return fail(GPV_ERR_STATE, "grid is not finished");
     if (!J->g[G->m].normals) return fail(GPV_ERR_STATE, "grid was made without params.normals");
     HIP_TRY(hipSetDevice(c->device));
-    const MeshOff& o = J->off[G->m];
+    const MeshRank& rk = J->rank[G->m];
     const int64_t nb = J->nb(G->m);
     const int n2 = J->g[G->m].n2;
     const int64_t n23 = (int64_t)n2 * n2 * n2;
     const Downloader::Piece pieces[2] = {
-        {l1n, J->l1n + 3 * (size_t)o.b0, l1n && nb > 0 ? (size_t)nb * 3 * sizeof(float) : 0},
-        {l2n, J->l2n + 3 * (size_t)o.l2n0, l2n && nb > 0 ? (size_t)(nb * n23) * 3 * sizeof(float) : 0}};
+        {l1n, J->l1n + 3 * (size_t)rk.b0, l1n && nb > 0 ? (size_t)nb * 3 * sizeof(float) : 0},
+        {l2n, J->l2n + 3 * (size_t)rk.l2n0, l2n && nb > 0 ? (size_t)(nb * n23) * 3 * sizeof(float) : 0}};
     HIP_TRY(c->down.run(pieces, 2, c->stream));
     return GPV_OK;
 }
@@ -2253,19 +2259,20 @@ static int normal_bytes(gpv_ctx* c, const gpv_grid* G, std::vector<uint8_t>& l1b
     const int m = G->m;
     const GridDev& g = J->g[m];
     const MeshOff& o = J->off[m];
+    const MeshRank& rk = J->rank[m];
     const int64_t n1 = J->info[m].n1, nb = J->nb(m);
     const int64_t n23 = (int64_t)g.n2 * g.n2 * g.n2;
     l1b.assign((size_t)n1 * 3, 0);
     uint8_t* d = nullptr;
     TRY(alloc(J, &d, (size_t)n1 * 3));
-    launch_export_l1_normals(J->bnd + o.word0, J->wprefix + o.word0, o.b0, J->l1n + 3 * (size_t)o.b0, g, d, s);
+    launch_export_l1_normals(J->bnd + o.word0, J->wprefix + o.word0, rk.b0, J->l1n + 3 * (size_t)rk.b0, g, d, s);
     HIP_TRY(hipMemcpyAsync(l1b.data(), d, (size_t)n1 * 3, hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
     release(J, d);
     l2b.assign(g.n2 > 0 ? (size_t)(nb * n23 * 3) : 0, 0);
     if (!l2b.empty()) {
         TRY(alloc(J, &d, l2b.size()));
-        launch_export_l2_normals(J->l2n + 3 * (size_t)o.l2n0, (int64_t)l2b.size(), d, s);
+        launch_export_l2_normals(J->l2n + 3 * (size_t)rk.l2n0, (int64_t)l2b.size(), d, s);
         HIP_TRY(hipMemcpyAsync(l2b.data(), d, l2b.size(), hipMemcpyDeviceToHost, s));
         HIP_TRY(hipStreamSynchronize(s));
         release(J, d);

@@ -3,6 +3,8 @@
 // tooling only.
 #include "gpv_internal.hpp"
 
+#include <type_traits>
+
 // the tiles of a counting sort with nkeys keys
 extern "C" int64_t tiles_of(uint64_t nkeys) { return (int64_t)gpv::ts_tiles(nkeys); }
 
@@ -18,4 +20,16 @@ extern "C" int64_t scan_touched_bytes(int n)
         top = at > top ? at : top;
     }
     return 4 * top;
+}
+
+// Whether kernels get a batch's table of offsets read-only, with nothing in it that
+// is known only after the boundary scan: kernels of both streams read it.
+template <typename T, typename = void>
+struct has_ranks : std::false_type {};
+template <typename T>
+struct has_ranks<T, std::void_t<decltype(T::b0)>> : std::true_type {};
+extern "C" int offsets_are_fixed()
+{
+    using Entry = std::remove_pointer_t<decltype(gpv::Meshes::off)>;
+    return std::is_const<Entry>::value && !has_ranks<Entry>::value;
 }

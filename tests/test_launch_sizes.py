@@ -37,3 +37,9 @@ def test_tile_scan_fits_its_lds(launch):
     bad = [(a, b) for a in tiles for b in tiles if max(need[a], need[b]) > launch.scan_lds_bytes(a, b)]
     assert not bad, f"{len(bad)} pairs of tile counts, the first {bad[0]}"
     assert max(launch.scan_lds_bytes(a, b) for a in tiles for b in tiles) <= 65536
+
+
+def test_batch_offsets_are_fixed(launch):
+    """The Level1 parity reads the offsets on its own stream while the boundary scan and
+    the group plan of the main one write theirs: not into the same table."""
+    assert launch.offsets_are_fixed() == 1
