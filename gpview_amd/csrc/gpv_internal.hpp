@@ -1,10 +1,10 @@
 // gpv_internal.hpp -- shared host/device declarations of libgpv (not public).
 #pragma once
 
+#include "gpv.h"
+
 #include <hip/hip_runtime.h>
 #include <stdint.h>
-
-struct gpv_ctx;
 
 namespace gpv {
 
@@ -126,6 +126,23 @@ struct Counters {
 };
 // page-locked read-back, written by kernels: Counters | B (one mesh) or MeshRank[nm + 1] | MeshCtr[nm]
 constexpr size_t kHOff = 64;
+
+// Launch shapes of a new context, and what the autotuner tries of each field: the
+// default and values around it, so that it finds its way back from any start.  Group
+// thresholds count bin entries a voxel; 0 and 2^20 are never and always.
+constexpr gpv_tune kTuneDefault{16, 56, 2048, 1, 1, 1, 128};
+struct TuneField {
+    int gpv_tune::*field;
+    int n, values[6];
+};
+constexpr TuneField kTuneSweep[] = {
+    {&gpv_tune::expand_blocks_per_cu, 4, {4, 8, 16, 32}},
+    {&gpv_tune::l2_group_below, 6, {0, 14, 28, 56, 112, 1 << 20}},
+    {&gpv_tune::sort_items_per_block, 4, {1024, 2048, 4096, 8192}},
+    {&gpv_tune::l2_overlap, 2, {0, 1}},
+    {&gpv_tune::l2_sat_waves, 3, {1, 2, 4}},
+    {&gpv_tune::l2_parity_waves, 3, {1, 2, 4}},
+};
 
 // sets the calling thread's gpv_last_error text and returns code
 int set_error(int code, const char* msg);

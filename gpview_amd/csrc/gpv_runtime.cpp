@@ -228,7 +228,7 @@ struct gpv_ctx {
     char* h_buf = nullptr;   // pinned read-back staging
     size_t h_cap = 0;
     int num_cu = 256;
-    gpv_tune tune{16, 56, 2048, 1, 1, 1, 128};
+    gpv_tune tune = kTuneDefault;
     std::vector<hipEvent_t> events;   // recycled stage events of finished jobs
     hipEvent_t na_ev[kJobEvents] = {};   // stage events of gpv_voxelize_noalloc (created with the context)
 };
@@ -1716,13 +1716,11 @@ int gpv_ctx_autotune(gpv_ctx* c, const gpv_mesh_desc* d, int nm, int on_device, 
     float warm = 0.0f;
     int st = tune_trial(c, d, nm, on_device, 1, &warm);
     if (st == GPV_OK) st = tune_trial(c, d, nm, on_device, repeats, &base);
-    const std::vector<int> expand = {4, 8, 16, 32}, group = {0, 4, 8, 16, 1 << 20}, items = {1024, 2048, 4096, 8192},
-                           overlap = {0, 1}, waves = {1, 2, 4};
-    auto sweep = [&](int gpv_tune::*field, const std::vector<int>& vals) -> int {
-        for (int v : vals) {
-            if (v == cur.*field) continue;
+    auto sweep = [&](const TuneField& f) -> int {
+        for (int k = 0; k < f.n; ++k) {
+            if (f.values[k] == cur.*f.field) continue;
             gpv_tune t = cur;
-            t.*field = v;
+            t.*f.field = f.values[k];
             c->tune = t;
             float ms = 0.0f;
             TRY(tune_trial(c, d, nm, on_device, repeats, &ms));
@@ -1734,12 +1732,8 @@ int gpv_ctx_autotune(gpv_ctx* c, const gpv_mesh_desc* d, int nm, int on_device, 
         c->tune = cur;
         return GPV_OK;
     };
-    if (st == GPV_OK) st = sweep(&gpv_tune::expand_blocks_per_cu, expand);
-    if (st == GPV_OK) st = sweep(&gpv_tune::l2_group_below, group);
-    if (st == GPV_OK) st = sweep(&gpv_tune::sort_items_per_block, items);
-    if (st == GPV_OK) st = sweep(&gpv_tune::l2_overlap, overlap);
-    if (st == GPV_OK) st = sweep(&gpv_tune::l2_sat_waves, waves);
-    if (st == GPV_OK) st = sweep(&gpv_tune::l2_parity_waves, waves);
+    for (const TuneField& f : kTuneSweep)
+        if (st == GPV_OK) st = sweep(f);
     if (st != GPV_OK) {
         c->tune = start;
         return st;

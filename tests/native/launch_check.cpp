@@ -33,3 +33,15 @@ extern "C" int offsets_are_fixed()
     using Entry = std::remove_pointer_t<decltype(gpv::Meshes::off)>;
     return std::is_const<Entry>::value && !has_ranks<Entry>::value;
 }
+
+// how many of the fields that the autotuner sweeps do not try the default
+extern "C" int sweeps_without_default()
+{
+    int bad = 0;
+    for (const gpv::TuneField& f : gpv::kTuneSweep) {
+        bool found = false;
+        for (int k = 0; k < f.n; ++k) found = found || f.values[k] == gpv::kTuneDefault.*f.field;
+        bad += found ? 0 : 1;
+    }
+    return bad;
+}

@@ -43,3 +43,8 @@ def test_batch_offsets_are_fixed(launch):
     """The Level1 parity reads the offsets on its own stream while the boundary scan and
     the group plan of the main one write theirs: not into the same table."""
     assert launch.offsets_are_fixed() == 1
+
+
+def test_autotuner_tries_the_defaults(launch):
+    """From any shapes set by hand the autotuner can come back to the default ones."""
+    assert launch.sweeps_without_default() == 0
