@@ -855,7 +855,8 @@ int launch_sat_half(Job* J)
 {
     gpv_ctx* c = J->ctx;
     hipStream_t s = c->stream;
-    if (!J->sat_timed) HIP_TRY(hipEventRecord(J->ev[1], s));
+    // (a sweep that runs again leaves ev[1] where the Level1 parity starts)
+    if (!J->sat_timed && !J->one_setup) HIP_TRY(hipEventRecord(J->ev[1], s));
     J->sat_timed = false;
     // boundary flags as bytes (plain stores from the SAT), packed to bits after
     if (!J->sat_cleared) {
