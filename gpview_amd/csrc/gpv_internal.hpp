@@ -72,6 +72,8 @@ struct MeshOff {
     uint32_t tri0;
     uint32_t ptask0;   // first Level1 fill block (L1F_W words of a layer)
     uint32_t pw0;      // first Level2 parity wave
+    uint32_t cw0;      // first word of the columns' occupancy (a bit per column, rows padded to words)
+    uint32_t pad;
 };
 
 // The same for what follows from the boundary scan, a table of its own because the
@@ -256,9 +258,10 @@ struct BinCols {
     uint32_t* off;
     uint2* ent;
 };
-// both sorts and the boundary index list
+// both sorts, the boundary index list and (unless nullptr) the bits of the columns that
+// hold boundary voxels, in occ (cleared by the caller)
 void launch_bins(const BinPairs& P, const BinCols& C, const uint64_t* bnd, const uint32_t* wprefix, const GridDev& g0,
-                 const Meshes& M, int64_t W, int32_t* bidx, int items_per_block, hipStream_t s);
+                 const Meshes& M, int64_t W, int32_t* bidx, uint64_t* occ, int items_per_block, hipStream_t s);
 
 // Level2 SAT voxel groups (k_l2_sat): consecutive boundary voxels of a mesh
 // that share a wave, at most `most` and kL2GroupMax of them, their layer bits
@@ -313,8 +316,9 @@ __host__ __device__ inline int l2_parity_columns(int n2, bool many) { return !ma
 // its waves for a mesh with ncol columns (none when Level2 is off)
 int64_t l2_parity_waves(int n2, int64_t ncol, bool many);
 // n2max, nzmax: the largest Level2 resolution and layer count of the run
-void launch_l2_parity(const uint64_t* bnd, const uint32_t* wprefix, int64_t nwaves, bool many, int n2max, int nzmax,
-                      const uint32_t* coff, const uint2* ent, const float* tris, int waves, const GridDev& g0,
+// occ: the columns that hold boundary voxels
+void launch_l2_parity(const uint64_t* bnd, const uint32_t* wprefix, const uint64_t* occ, int64_t nwaves, bool many,
+                      int n2max, int nzmax, const uint32_t* coff, const uint2* ent, const float* tris, int waves, const GridDev& g0,
                       const Meshes& M, uint64_t* par2, hipStream_t s);
 
 // normals (src/Object.cpp:3219-3253 Level1, 2372-2421 + 2705-2720 Level2)

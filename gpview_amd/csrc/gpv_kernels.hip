@@ -1581,12 +1581,12 @@ void launch_mesh_bounds(const uint32_t* wprefix, const Meshes& M, const Counters
     k_mesh_bounds<<<1, 64, 0, s>>>(wprefix, M, ctr, pub);
 }
 
-// ascending linear indices (within the mesh) of the boundary voxels, and in a
-// batch the mesh of each; block `blk` of `blocks`
+// ascending linear indices (within the mesh) of the boundary voxels, in a
+// batch the mesh of each, and the columns that hold any; block `blk` of `blocks`
 template <bool kM>
 __device__ __forceinline__ void boundary_index(const uint64_t* __restrict__ bnd, const uint32_t* __restrict__ wprefix,
                                                const GridDev& g0, const Meshes& M, int64_t W, int32_t* __restrict__ bidx,
-                                               uint32_t blk, uint32_t blocks)
+                                               unsigned long long* __restrict__ occ, uint32_t blk, uint32_t blocks)
 {
     for (int64_t w = (int64_t)blk * blockDim.x + threadIdx.x; w < W; w += (int64_t)blocks * blockDim.x) {
         uint64_t bits = bnd[w];
@@ -1597,6 +1597,9 @@ __device__ __forceinline__ void boundary_index(const uint64_t* __restrict__ bnd,
         const int64_t wl = w - (int64_t)(kM ? M.off[mesh].word0 : 0);
         const int xw = (int)(wl % g.nxw);
         const int64_t row = wl / g.nxw;
+        if (occ)   // an atomic for every word: looking first whether it adds anything costs 45 us at 512 layers
+            atomicOr(occ + (kM ? M.off[mesh].cw0 : 0u) + ((uint32_t)row % (uint32_t)g.ny) * (uint32_t)g.nxw + (uint32_t)xw,
+                     (unsigned long long)bits);
         while (bits) {
             const int bit = __ffsll((unsigned long long)bits) - 1;
             bits &= bits - 1;
@@ -1789,14 +1792,15 @@ __device__ __forceinline__ void ts_count(const TsSort<Src>& S, bool last, uint32
 template <bool kM>
 __global__ __launch_bounds__(TS_NT) void k_ts_count(TsSort<PairSrc> a, TsSort<ColSrc> b, bool last, GridDev g0, Meshes M,
                                                     const uint64_t* __restrict__ bnd, const uint32_t* __restrict__ wprefix,
-                                                    int64_t W, int32_t* __restrict__ bidx)
+                                                    int64_t W, int32_t* __restrict__ bidx,
+                                                    unsigned long long* __restrict__ occ)
 {
     extern __shared__ uint32_t s_h[];   // [ntiles]
     __shared__ uint32_t s_wave[TS_NT / 64];
     __shared__ uint32_t s_last;
     if (blockIdx.y == 0) ts_count(a, last, s_h, s_wave, &s_last);
     else if (blockIdx.y == 1) ts_count(b, last, s_h, s_wave, &s_last);
-    else boundary_index<kM>(bnd, wprefix, g0, M, W, bidx, blockIdx.x, gridDim.x);
+    else boundary_index<kM>(bnd, wprefix, g0, M, W, bidx, occ, blockIdx.x, gridDim.x);
 }
 
 // items (.x = key) to their tile's bucket range; the item is built
@@ -1936,8 +1940,9 @@ static TsSort<Src> ts_sort(Src src, uint64_t n, uint32_t nkeys, uint32_t* cnt, v
 }
 
 void launch_bins(const BinPairs& P, const BinCols& C, const uint64_t* bnd, const uint32_t* wprefix, const GridDev& g0,
-                 const Meshes& M, int64_t W, int32_t* bidx, int items_per_block, hipStream_t s)
+                 const Meshes& M, int64_t W, int32_t* bidx, uint64_t* occ, int items_per_block, hipStream_t s)
 {
+    unsigned long long* oc = reinterpret_cast<unsigned long long*>(occ);
     const auto a = ts_sort(PairSrc{P.bits, P.ranked, P.tri, bnd, wprefix}, P.n, P.B, P.cnt, P.bucket, items_per_block);
     const auto b = ts_sort(ColSrc{C.key, C.zmax}, C.n, C.ncol, C.cnt, C.bucket, items_per_block);
     const int blocks = std::max(a.blocks, b.blocks), tiles = std::max(a.ntiles, b.ntiles);
@@ -1949,9 +1954,9 @@ void launch_bins(const BinPairs& P, const BinCols& C, const uint64_t* bnd, const
     const size_t lds = last ? scan : (size_t)tiles * 4;
     const dim3 grid((unsigned)std::max(blocks, grid_for(W, TS_NT, 2048)), 3);
     if (M.nm > 1)
-        k_ts_count<true><<<grid, TS_NT, lds, s>>>(a, b, last, g0, M, bnd, wprefix, W, bidx);
+        k_ts_count<true><<<grid, TS_NT, lds, s>>>(a, b, last, g0, M, bnd, wprefix, W, bidx, oc);
     else
-        k_ts_count<false><<<grid, TS_NT, lds, s>>>(a, b, last, g0, M, bnd, wprefix, W, bidx);
+        k_ts_count<false><<<grid, TS_NT, lds, s>>>(a, b, last, g0, M, bnd, wprefix, W, bidx, oc);
     if (!P.B) launch_fill_u32(P.off, 0, 1, s);   // no keys, hence no items
     if (!blocks) return;
     if (!last) k_ts_scan<<<2, 1024, scan, s>>>(a, b);
@@ -2430,6 +2435,10 @@ void launch_l2_sat(const float* tris, const int32_t* bidx, int64_t B, int64_t ng
 // 256/8 0.232 -> 0.129 ms alone (1.82e8 -> 0.72e8 instructions), lattice-snapped
 // mesh 512/16 3.90 -> 2.24 ms, 128 small meshes 0.60 -> 0.39 ms.
 //
+// Columns without a boundary voxel are known from the bins' launch, a bit each: their
+// waves leave at once (a scan of 512 layers by every one of 262,144 columns took 0.89 ms
+// of an almost empty grid at 512/16, now 0.06).
+//
 // What bounds it: the chain of dependent LDS and global reads of each wave
 // (VALU issue 0.39-0.47), hence one wave per block (an empty column's wave
 // leaves at once; two waves a block took 0.15 ms on the torus knot), 80
@@ -2462,7 +2471,8 @@ int64_t l2_parity_waves(int n2, int64_t ncol, bool many)
 // C adjacent columns (i1 .., j1) of a mesh by one wave: 1, 2 (at n2 <= 8) or 4 (at n2 <= 4).
 template <int C, int KB>
 __device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB>& L, uint64_t* cb, int nw, const GridDev& g, int i1, int j1,
-                                                       uint64_t word0, uint32_t col0, uint32_t b0,
+                                                       uint64_t word0, uint32_t col0, uint32_t b0, uint32_t cw0,
+                                                       const uint64_t* __restrict__ occ,
                                                        const uint64_t* __restrict__ bnd,
                                                        const uint32_t* __restrict__ wprefix,
                                                        const uint32_t* __restrict__ coff,
@@ -2471,6 +2481,9 @@ __device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB>& L, uint64_t* 
 {
     const int lane = __lane_id();
     const int n2 = g.n2, w2 = g.w2, nsc = n2 * n2, nz = g.nz;
+    const int bit0 = i1 & 63;
+    const uint32_t cword = (uint32_t)j1 * (uint32_t)g.nxw + (uint32_t)(i1 >> 6);
+    if (!((occ[cw0 + cword] >> bit0) & ((1u << C) - 1u))) return;   // no boundary voxel in these columns
     const int fb = C == 1 && n2 > 8 ? 2 : 1;
     uint32_t* pre = reinterpret_cast<uint32_t*>(cb + C * nw);
     const uint32_t gcol = col0 + (uint32_t)(j1 * g.nx + i1);
@@ -2483,9 +2496,8 @@ __device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB>& L, uint64_t* 
     const int Wn = min(KB / (C * nsc * fb) - 1, L2P_SLOTS / C);
     // the columns' boundary voxels: a bit per layer, their number below each
     // word of bits, and the boundary index of each slot of the window [lo, hi)
-    const uint64_t word = word0 + (uint64_t)j1 * g.nxw + (uint64_t)(i1 >> 6);
+    const uint64_t word = word0 + (uint64_t)cword;
     const uint64_t plane = (uint64_t)g.ny * g.nxw;
-    const int bit0 = i1 & 63;
     uint32_t S[C], lo[C], hi[C];
     auto scan = [&](bool first) {
 #pragma unroll
@@ -2522,7 +2534,6 @@ __device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB>& L, uint64_t* 
     uint32_t most = 0;
 #pragma unroll
     for (int c = 0; c < C; ++c) most = max(most, S[c]);
-    if (most == 0) return;
     const SatScale sc{g.s2x, g.s2y, g.s2z, g.d2x, g.d2y, g.d2z};
     const float gx = 2.0f * g.h2x, gy = 2.0f * g.h2y, inv_n2 = GPV_RCP((float)n2);
     const float* rz = g.r2z;
@@ -2773,7 +2784,8 @@ __device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB>& L, uint64_t* 
 
 template <bool kM, int KB, int W>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 1 ? 6 : 3))) void k_l2_parity(const uint64_t* __restrict__ bnd,
-                                                      const uint32_t* __restrict__ wprefix, int64_t nwaves, bool many, int nw,
+                                                      const uint32_t* __restrict__ wprefix,
+                                                      const uint64_t* __restrict__ occ, int64_t nwaves, bool many, int nw,
                                                       const uint32_t* __restrict__ coff,
                                                       const uint2* __restrict__ ent, const float* __restrict__ tris,
                                                       GridDev g0, Meshes M, uint64_t* __restrict__ par2)
@@ -2797,17 +2809,18 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 1 ?
     const int j1 = col / g.nx, i1 = col - j1 * g.nx;
     const uint64_t word0 = kM ? M.off[mesh].word0 : 0;
     const uint32_t col0 = kM ? M.off[mesh].col0 : 0, b0 = kM ? M.rank[mesh].b0 : 0;
+    const uint32_t cw0 = kM ? M.off[mesh].cw0 : 0;
     uint64_t* out = par2 + (kM ? M.rank[mesh].l2w0 : 0);
     if (C == 2)
-        l2_parity_columns_wave<2>(s_l[wv], cb, nw, g, i1, j1, word0, col0, b0, bnd, wprefix, coff, ent, tris, out);
+        l2_parity_columns_wave<2>(s_l[wv], cb, nw, g, i1, j1, word0, col0, b0, cw0, occ, bnd, wprefix, coff, ent, tris, out);
     else if (C == 4)
-        l2_parity_columns_wave<4>(s_l[wv], cb, nw, g, i1, j1, word0, col0, b0, bnd, wprefix, coff, ent, tris, out);
+        l2_parity_columns_wave<4>(s_l[wv], cb, nw, g, i1, j1, word0, col0, b0, cw0, occ, bnd, wprefix, coff, ent, tris, out);
     else
-        l2_parity_columns_wave<1>(s_l[wv], cb, nw, g, i1, j1, word0, col0, b0, bnd, wprefix, coff, ent, tris, out);
+        l2_parity_columns_wave<1>(s_l[wv], cb, nw, g, i1, j1, word0, col0, b0, cw0, occ, bnd, wprefix, coff, ent, tris, out);
 }
 
 template <int KB, int W>
-static void launch_l2_parity_w(const uint64_t* bnd, const uint32_t* wprefix, int64_t nwaves, bool many, int nzmax,
+static void launch_l2_parity_w(const uint64_t* bnd, const uint32_t* wprefix, const uint64_t* occ, int64_t nwaves, bool many, int nzmax,
                                const uint32_t* coff, const uint2* ent, const float* tris, const GridDev& g0, const Meshes& M,
                                uint64_t* par2, hipStream_t s)
 {
@@ -2816,29 +2829,29 @@ static void launch_l2_parity_w(const uint64_t* bnd, const uint32_t* wprefix, int
     const int nw = (nzmax + 63) / 64;
     const size_t lds = (size_t)W * 6 * nw * sizeof(uint64_t);
     if (M.nm > 1)
-        k_l2_parity<true, KB, W><<<blocks, 64 * W, lds, s>>>(bnd, wprefix, nwaves, many, nw, coff, ent, tris, g0, M, par2);
+        k_l2_parity<true, KB, W><<<blocks, 64 * W, lds, s>>>(bnd, wprefix, occ, nwaves, many, nw, coff, ent, tris, g0, M, par2);
     else
-        k_l2_parity<false, KB, W><<<blocks, 64 * W, lds, s>>>(bnd, wprefix, nwaves, many, nw, coff, ent, tris, g0, M, par2);
+        k_l2_parity<false, KB, W><<<blocks, 64 * W, lds, s>>>(bnd, wprefix, occ, nwaves, many, nw, coff, ent, tris, g0, M, par2);
 }
 
 template <int KB>
-static void launch_l2_parity_k(const uint64_t* bnd, const uint32_t* wprefix, int64_t nwaves, bool many, int nzmax,
+static void launch_l2_parity_k(const uint64_t* bnd, const uint32_t* wprefix, const uint64_t* occ, int64_t nwaves, bool many, int nzmax,
                                const uint32_t* coff, const uint2* ent, const float* tris, int waves, const GridDev& g0, const Meshes& M,
                                uint64_t* par2, hipStream_t s)
 {
-    if (waves <= 1) launch_l2_parity_w<KB, 1>(bnd, wprefix, nwaves, many, nzmax, coff, ent, tris, g0, M, par2, s);
-    else if (waves == 2) launch_l2_parity_w<KB, 2>(bnd, wprefix, nwaves, many, nzmax, coff, ent, tris, g0, M, par2, s);
-    else launch_l2_parity_w<KB, 4>(bnd, wprefix, nwaves, many, nzmax, coff, ent, tris, g0, M, par2, s);
+    if (waves <= 1) launch_l2_parity_w<KB, 1>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, g0, M, par2, s);
+    else if (waves == 2) launch_l2_parity_w<KB, 2>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, g0, M, par2, s);
+    else launch_l2_parity_w<KB, 4>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, g0, M, par2, s);
 }
 
-void launch_l2_parity(const uint64_t* bnd, const uint32_t* wprefix, int64_t nwaves, bool many, int n2max, int nzmax,
+void launch_l2_parity(const uint64_t* bnd, const uint32_t* wprefix, const uint64_t* occ, int64_t nwaves, bool many, int n2max, int nzmax,
                       const uint32_t* coff, const uint2* ent, const float* tris, int waves, const GridDev& g0, const Meshes& M,
                       uint64_t* par2, hipStream_t s)
 {
     if (nwaves <= 0) return;
     // room for 31 boundary voxels of a column at n2 = 8, 7 at 16
-    if (n2max <= 8) launch_l2_parity_k<2048>(bnd, wprefix, nwaves, many, nzmax, coff, ent, tris, waves, g0, M, par2, s);
-    else launch_l2_parity_k<4096>(bnd, wprefix, nwaves, many, nzmax, coff, ent, tris, waves, g0, M, par2, s);
+    if (n2max <= 8) launch_l2_parity_k<2048>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, waves, g0, M, par2, s);
+    else launch_l2_parity_k<4096>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, waves, g0, M, par2, s);
 }
 
 // ---------------------------------------------------------------------------

@@ -298,8 +298,11 @@ struct Job {
     uint32_t *boff = nullptr, *list = nullptr;
     uint32_t* coff = nullptr;
     uint2* cent = nullptr;    // (triangle, zmax) of the column entries
-    // scratch of the two sorts: their counters (zeros since the set-up or not) and buckets
+    // scratch of the two sorts, their counters, and behind them the occupancy bits of
+    // the columns (colw words; both zeros since the set-up or not)
     uint32_t *pair_cnt = nullptr, *col_cnt = nullptr;
+    uint64_t* col_occ = nullptr;
+    int64_t colw = 0;
     size_t bin_words = 0;
     bool bins_cleared = false;
     bool streams = false;            // the Level2 stages ran on two streams
@@ -658,6 +661,8 @@ int job_create(gpv_ctx* c, const gpv_mesh_desc* d, int nm, int on_device, Job** 
         J->off[m].tri0 = tri0;
         J->off[m].ptask0 = ptask0;
         J->off[m].pw0 = (uint32_t)pw0;
+        J->off[m].cw0 = (uint32_t)J->colw;
+        J->colw += (int64_t)g.ny * g.nxw;
         pw0 += l2_parity_waves(g.n2, (int64_t)g.nx * g.ny, ncol >= kL2ParityMany);
         ptask0 += (uint32_t)l1_fill_blocks(g);
         word0 += (uint64_t)g.nz * g.ny * g.nxw;
@@ -779,14 +784,17 @@ int job_create(gpv_ctx* c, const gpv_mesh_desc* d, int nm, int on_device, Job** 
     return GPV_OK;
 }
 
-// counters of both sorts, one after the other, for at most `most` boundary voxels
+// counters of both sorts, one after the other, for at most `most` boundary voxels, and
+// the columns' occupancy (the Level2 parity reads it: kept until the run is finished)
 int alloc_bin_counters(Job* J, uint64_t most)
 {
     release(J, J->pair_cnt);
     const size_t a = ts_words(most), b = J->n2max > 0 ? ts_words((uint64_t)J->ncol) : 0;
-    TRY(alloc(J, &J->pair_cnt, a + b));
+    const size_t occ = J->n2max > 0 ? 2 * (size_t)J->colw : 0;
+    TRY(alloc(J, &J->pair_cnt, a + b + occ));
     J->col_cnt = J->pair_cnt + a;
-    J->bin_words = a + b;
+    J->col_occ = occ ? reinterpret_cast<uint64_t*>(J->pair_cnt + a + b) : nullptr;   // ts_words is even
+    J->bin_words = a + b + occ;
     return GPV_OK;
 }
 
@@ -1044,10 +1052,9 @@ int launch_compact(Job* J)
     launch_bins(BinPairs{J->pair_key, J->pairs_ranked, J->pair_tri, J->n_pairs, (uint32_t)J->B, J->pair_cnt, pb, J->boff,
                          J->nm > 1 ? nullptr : &J->mctr[0].max_per_voxel, J->list},
                 BinCols{J->col_key, J->col_z, J->n_cols, cols ? (uint32_t)J->ncol : 0u, J->col_cnt, cb, J->coff, J->cent},
-                J->bnd, J->wprefix, J->g[0], J->view(), J->W, J->bidx, std::max(256, J->ctx->tune.sort_items_per_block), s);
+                J->bnd, J->wprefix, J->g[0], J->view(), J->W, J->bidx, J->col_occ, std::max(256, J->ctx->tune.sort_items_per_block), s);
     J->pairs_ranked = true;
     if (J->nm > 1 && !J->streams) launch_mesh_bins(J->boff, J->B, J->view(), s);
-    release(J, J->pair_cnt);
     release(J, pb);
     release(J, cb);
     HIP_TRY(hipGetLastError());
@@ -1101,7 +1108,7 @@ int l2_parity_kernels(Job* J, hipStream_t s)
 {
     HIP_TRY(hipEventRecord(J->ev[16], s));
     if (J->B > 0)
-        launch_l2_parity(J->bnd, J->wprefix, J->l2p_waves, J->ncol >= kL2ParityMany, J->n2max, J->nzmax, J->coff, J->cent,
+        launch_l2_parity(J->bnd, J->wprefix, J->col_occ, J->l2p_waves, J->ncol >= kL2ParityMany, J->n2max, J->nzmax, J->coff, J->cent,
                          J->tris, J->ctx->tune.l2_parity_waves, J->g[0], J->view(), J->par2, s);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipEventRecord(J->ev[11], s));
@@ -1329,7 +1336,7 @@ int64_t predict_run_bytes(const gpv_mesh_desc& d, const gpv_grid_info& I)
     b += 24 * P;                                                 // bin pairs, column entries
     b += 4 * (ncol + 1) + 8 * P + 12 * P;                        // column entries by column
     b += 8 * B + 4 + 4 * P + 8 * P;                              // boundary list, bins
-    b += 4 * (int64_t)(ts_words((uint64_t)std::min<int64_t>(W * 64, int64_t(1) << 27)) + ts_words((uint64_t)ncol));   // their counters
+    b += 4 * (int64_t)(ts_words((uint64_t)std::min<int64_t>(W * 64, int64_t(1) << 27)) + ts_words((uint64_t)ncol)) + W / nz * 8;   // their counters, the columns' occupancy
     b += 16 * B * w2;                                            // Level2 planes
     if (d.params.normals) b += 12 * T + 4 * P + 12 * B + 12 * B * n2 * n2 * n2;
     if (d.params.l1_stencil) b += 12 * T + 8 + scan(T) + 8 * nz * 2 * ny * ((2 * nx + 63) / 64);   // stencil fill

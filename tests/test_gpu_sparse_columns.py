@@ -1,0 +1,59 @@
+"""Grids in which few columns hold boundary voxels."""
+import numpy as np
+import pytest
+
+from conftest import compare_results, say
+
+pytestmark = pytest.mark.gpu
+
+
+def _cluster(n, size, at, seed):
+    rng = np.random.default_rng(seed)
+    return np.ascontiguousarray(at + size * rng.uniform(0, 1, (n, 9)), np.float32)
+
+
+# one, two and four columns a wave, words with one and several occupied columns, both ends of a row
+@pytest.mark.parametrize("l1,n2", [(64, 16), (132, 9), (256, 8), (256, 5), (256, 4), (260, 1), (20, 4)])
+def test_few_occupied_columns(gv, orc, l1, n2):
+    soup = np.concatenate([_cluster(15, 0.03, a, 40 + k) for k, a in enumerate((0.0, 0.31, 0.5, 0.97))])
+    bmin, bmax, mms = np.zeros(3, np.float32), np.array([1, 0.9, 0.8], np.float32), np.float32(1)
+    want = orc.voxelize(soup, orc.grid_setup(bmin, bmax, mms, l1, n2), orc.ORC_FAST)
+    mesh = {"soup": soup, "bmin": bmin, "bmax": bmax, "mms": mms, "voxel_count": l1, "voxel_count2": n2}
+    other = {"soup": soup[:20], "bmin": bmin, "bmax": bmax, "mms": mms, "voxel_count": 24, "voxel_count2": 3}
+    wother = orc.voxelize(soup[:20], orc.grid_setup(bmin, bmax, mms, 24, 3), orc.ORC_FAST)
+    with gv.Context() as c:
+        say(f"few occupied columns {l1}/{n2}")
+        for _ in range(2):
+            g = c.voxelize(soup, bmin, bmax, mms, l1, n2)
+            compare_results(f"{l1}/{n2}", g.download(), want, n2)
+            g.release()
+        grids = c.voxelize_batch([other, mesh, other])
+        for g, w, n in zip(grids, (wother, want, wother), (3, n2, 3)):
+            compare_results(f"batch {l1}/{n2}", g.download(), w, n)
+            g.release()
+        g = c.create(soup, bmin, bmax, mms, l1, n2)     # the staged form, its bins made twice
+        g.classify_tessellation()
+        g.classify_inout()
+        g.compact_boundary()
+        g.compact_boundary()
+        g.classify_tessellation_level2()
+        g.classify_inout_level2()
+        g.finish()
+        compare_results(f"staged {l1}/{n2}", g.download(), want, n2)
+        g.release()
+
+
+def test_empty_columns_cost_little(gv):
+    """The Level2 parity of 27 boundary voxels in 262,144 columns of 512 layers: 0.89 ms
+    with a scan of every column, 0.05 ms with the occupied ones only."""
+    soup = _cluster(20, 0.005, 0.5, 7)
+    bmin, bmax = np.zeros(3, np.float32), np.ones(3, np.float32)
+    with gv.Context() as c:
+        say("empty columns")
+        ms = []
+        for _ in range(5):
+            g = c.voxelize(soup, bmin, bmax, 1.0, 512, 16)
+            ms.append(g.info()["ms_stage"][4])
+            g.release()
+        say(f"Level2 parity {min(ms):.3f} ms")
+        assert min(ms) < 0.3
