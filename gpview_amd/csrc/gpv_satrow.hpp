@@ -41,7 +41,7 @@
 // (reference 9.2 U A|N| + 21 U A G, here 40 U A|N| + 11 U A G; the last term
 // pays for keeping |N_z| away from zero).  Where a magnitude leaves the range
 // these products need (A above 2^24 sub-voxels, a reciprocal above 1e20, a
-// nearly degenerate triangle), or g2 is outside [2^-40, 2^40], the entry is
+// nearly degenerate triangle other than a segment), or g2 is outside [2^-40, 2^40], the entry is
 // `loose`: every layer asked for is undecided.
 #pragma once
 
@@ -107,11 +107,12 @@ __host__ __device__ __forceinline__ float4 sat_edge_z(float eu, float ez, bool z
 // 0 is c0 (kBox: in the index AABB whose first center is c0, where a box may
 // miss the triangle's extent by the rounding of the index and of the tables):
 // 0 writes groups 0-2 and 9, 1 the others (the plane's slopes included).  Two
-// lanes can make one entry on the device; `loose` has to be combined from both
-// parts.
-template <bool kBox = false>
-__host__ __device__ __forceinline__ bool sat_entry_part(int h, const float* tv, float c0x, float c0y, float c0z,
-                                                        const SatScale& g, float4* out)
+// lanes can make one entry on the device; looseness has to be combined from both
+// parts.  `plane`: the plane cannot be bounded, which makes the entry loose unless the
+// triangle is a segment (sat_segment); returned are the other reasons.
+template <bool kBox>
+__host__ __device__ __forceinline__ bool sat_entry_terms(int h, const float* tv, float c0x, float c0y, float c0z,
+                                                         const SatScale& g, float4* out, bool& plane)
 {
     constexpr float U = 0x1p-24f;
     const float t0x = tv[0], t0y = tv[1], t0z = tv[2], t1x = tv[3], t1y = tv[4], t1z = tv[5], t2x = tv[6],
@@ -152,7 +153,6 @@ __host__ __device__ __forceinline__ bool sat_entry_part(int h, const float* tv, 
     const float r = GPV_RCP(fmaxf(anz, R * rz));
     const float rs = copysignf(r, Nz);
     const float pa = -Nx * rs, pb = -Ny * rs;
-    loose = loose || !(r < 1e12f);
     if (h) {
         // (x, y), over its half width
         const float hn = 0.5f * Nz, ah = fabsf(hn);
@@ -174,7 +174,27 @@ __host__ __device__ __forceinline__ bool sat_entry_part(int h, const float* tv, 
         const float hw = R * r, mp = M * r + g.dz;
         out[9] = make_float4(zeta - (pa * xi + pb * eta), hw + mp, hw - mp, 0.0f);
     }
+    plane = !(r < 1e12f);
     return loose || !(rmax < 1e20f);
+}
+
+// Two vertices the same: the reference's normal is exactly zero (a zero edge, or one the
+// negative of the other) and its plane test passes everywhere.  So is the normal here, its
+// reciprocal infinite, and each of the plane's terms a NaN, which fmaxf and fminf pass over: the
+// plane bounds nothing.
+__host__ __device__ __forceinline__ bool sat_segment(const float* tv)
+{
+    return (tv[0] == tv[3] && tv[1] == tv[4] && tv[2] == tv[5]) || (tv[3] == tv[6] && tv[4] == tv[7] && tv[5] == tv[8]) ||
+           (tv[6] == tv[0] && tv[7] == tv[1] && tv[8] == tv[2]);
+}
+
+// The same, and whether the part makes the entry loose.
+__host__ __device__ __forceinline__ bool sat_entry_part(int h, const float* tv, float c0x, float c0y, float c0z,
+                                                        const SatScale& g, float4* out)
+{
+    bool plane;
+    const bool loose = sat_entry_terms<false>(h, tv, c0x, c0y, c0z, g, out, plane);
+    return loose || (plane && !sat_segment(tv));
 }
 
 // A box axis: with x the triangle's least (greatest) coordinate in centers from the
@@ -321,8 +341,9 @@ __host__ __device__ __forceinline__ SatColumn sat_column(const float* tv, float 
 {
     constexpr float U = 0x1p-24f;
     float4 e[kSatEntry4];
-    bool loose = sat_entry_part<true>(0, tv, c0x, c0y, c0z, g, e);
-    loose = sat_entry_part<true>(1, tv, c0x, c0y, c0z, g, e) || loose;
+    bool plane;   // the same for both parts
+    bool loose = sat_entry_terms<true>(0, tv, c0x, c0y, c0z, g, e, plane);
+    loose = sat_entry_terms<true>(1, tv, c0x, c0y, c0z, g, e, plane) || loose;
     const float x = (float)xi, y = (float)yi, n = (float)layers;
     // box axes: the triangle's extent, half a voxel more on each side
     const float x0 = (fminf(fminf(tv[0], tv[3]), tv[6]) - c0x) * g.sx, x1 = (fmaxf(fmaxf(tv[0], tv[3]), tv[6]) - c0x) * g.sx;
@@ -355,7 +376,7 @@ __host__ __device__ __forceinline__ SatColumn sat_column(const float* tv, float 
     s.bi = (int)fmaxf(hii, 0.0f);
     if (!(u < -c6.w) || !(far < -mxy)) s.ai = s.bi = 0;
     if (u > c6.w || far > mxy) s.am = s.bm = 0;
-    if (loose) {
+    if ((loose || plane) && (loose || !sat_segment(tv))) {
         s.am = s.ai = s.bi = 0;
         s.bm = layers;
     }
