@@ -77,13 +77,12 @@ struct MeshOff {
 };
 
 // The same for what follows from the boundary scan, a table of its own because the
-// main stream writes it while the Level1 parity runs on the other one: boundary voxels (b0),
-// Level2 words (l2w0) and normals by the device, SAT groups by the host.
+// main stream writes it while the Level1 parity runs on the other one.
 struct MeshRank {
     uint64_t l2w0;
     uint64_t l2n0;   // first Level2 normal (one per Level2 voxel of meshes with normals)
     uint32_t b0;
-    uint32_t sg0;    // first Level2 SAT group (l2_plan)
+    uint32_t sg0;    // first Level2 SAT group (k_mesh_groups)
 };
 
 // Per-mesh results accumulated on the device.
@@ -274,6 +273,13 @@ __host__ __device__ inline int l2_group_voxels(int n2, int most)
     if (c > kL2GroupMax) c = kL2GroupMax;
     return c < most ? c : most;
 }
+// groups of a mesh with nb boundary voxels
+__host__ __device__ inline int64_t l2_groups(int n2, int64_t nb, int most)
+{
+    if (n2 <= 0) return 0;
+    const int64_t c = l2_group_voxels(n2, most);
+    return (nb + c - 1) / c;
+}
 // Level1 fill: a block takes L1F_W words of a mesh's layer, all layers
 constexpr int L1F_W = 16;
 inline int64_t l1_fill_blocks(const GridDev& g) { return ((int64_t)g.ny * g.nxw + L1F_W - 1) / L1F_W; }
@@ -298,6 +304,8 @@ void launch_l1_fill(const GridDev& g0, const Meshes& M, int64_t blocks, uint64_t
 // b0, l2w0 and l2n0 of every mesh (and the totals in entry nm) from the word prefix
 // and the counters, to the page-locked read-back pub as well
 void launch_mesh_bounds(const uint32_t* wprefix, const Meshes& M, const Counters* ctr, uint64_t* pub, hipStream_t s);
+// sg0 of every mesh (and the total in entry nm) from b0
+void launch_mesh_groups(const Meshes& M, int most, hipStream_t s);
 // per-mesh bin totals and largest bin (multi-mesh runs)
 void launch_mesh_bins(const uint32_t* boff, int64_t B, const Meshes& M, hipStream_t s);
 

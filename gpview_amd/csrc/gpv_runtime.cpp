@@ -1076,29 +1076,17 @@ int l2_sat_most(const Job* J)
 }
 
 // Level2 SAT groups of the job; in a batch each mesh's first one goes to
-// MeshRank::sg0 on the device (nothing on the side stream reads that table before
-// it waits for ev[6], recorded after this copy)
+// MeshRank::sg0 (nothing on the side stream reads that table before it waits for
+// ev[6], recorded after this launch)
 int l2_plan(Job* J)
 {
     int64_t sg = 0;
     J->l2s_most = l2_sat_most(J);
-    for (int m = 0; m < J->nm; ++m) {
-        J->rank[m].sg0 = (uint32_t)sg;
-        if (J->g[m].n2 > 0) {
-            const int64_t c = l2_group_voxels(J->g[m].n2, J->l2s_most);
-            sg += (J->nb(m) + c - 1) / c;
-        }
-    }
-    J->rank[J->nm].sg0 = (uint32_t)sg;
+    for (int m = 0; m < J->nm; ++m) sg += l2_groups(J->g[m].n2, J->nb(m), J->l2s_most);
     J->l2s_groups = sg;
     if (J->nm > 1) {
-        hipStream_t s = J->ctx->stream;
-        // the MeshRank staging region was last filled by the size read-back,
-        // which the host has already waited for; a later job refills it only
-        // after its own read-back, which this stream orders after this copy
-        MeshRank* h = reinterpret_cast<MeshRank*>(J->ctx->h_buf + kHOff);
-        memcpy(h, J->rank.data(), sizeof(MeshRank) * ((size_t)J->nm + 1));
-        HIP_TRY(hipMemcpyAsync(J->d_rank, h, sizeof(MeshRank) * ((size_t)J->nm + 1), hipMemcpyHostToDevice, s));
+        launch_mesh_groups(J->view(), J->l2s_most, J->ctx->stream);
+        HIP_TRY(hipGetLastError());
     }
     return GPV_OK;
 }
