@@ -2466,19 +2466,20 @@ void launch_l2_sat(const float* tris, const int32_t* bidx, int64_t B, int64_t ng
 // n2 = 8 took 0.31 ms.
 // ---------------------------------------------------------------------------
 constexpr int L2P_STAGE = 32;    // entries staged at once
+constexpr int L2P_SHARE = 4;     // waves that share a column where there are few
 constexpr int L2P_SLOTS = 128;   // boundary voxels of a window, all columns of the wave
 
-// LDS of one wave of the Level2 parity
-template <int KB>
+// LDS of the V waves that take a column (or a few) together in the Level2 parity
+template <int KB, int V>
 struct L2PLds {
-    // staged entry: e1, e2x | e2y, e2z, inv, v1x | v1y, dz, mu, delta | l0, cap, column, v1z
-    float4 e[L2P_STAGE][4];
+    // staged entries of each: e1, e2x | e2y, e2z, inv, v1x | v1y, dz, mu, delta | l0, cap, column, v1z
+    float4 e[V][L2P_STAGE][4];
     // per (column, slot, sub-column) its toggles, in bytes up to n2 = 8 and in
     // 16 bits above; a column's row past its slots holds the parity of the windows above
     uint32_t acc[KB / 4];
     uint32_t slotb[L2P_SLOTS];   // boundary voxel of each slot
     float ox[16], oy[16];        // origins of the columns (c * n2 + p) and of the row
-    uint8_t win[64];
+    uint8_t win[V][64];
 };
 
 // parity waves of a mesh with ncol columns
@@ -2487,9 +2488,18 @@ int64_t l2_parity_waves(int n2, int64_t ncol, bool many)
     return n2 <= 0 ? 0 : ncol / l2_parity_columns(n2, many);
 }
 
-// C adjacent columns (i1 .., j1) of a mesh by one wave: 1, 2 (at n2 <= 8) or 4 (at n2 <= 4).
-template <int C, int KB>
-__device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB>& L, uint64_t* cb, int nw, const GridDev& g, int i1, int j1,
+// between the phases of a column
+template <int V>
+__device__ __forceinline__ void l2_parity_barrier()
+{
+    if constexpr (V > 1) __syncthreads();
+    else __builtin_amdgcn_wave_barrier();
+}
+
+// C adjacent columns (i1 .., j1) of a mesh by one wave: 1, 2 (at n2 <= 8) or 4 (at n2 <= 4);
+// or, V > 1, by the V waves of a block, this one `wv`, which share the entries.
+template <int C, int KB, int V>
+__device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB, V>& L, int wv, uint64_t* cb, int nw, const GridDev& g, int i1, int j1,
                                                        uint64_t word0, uint32_t col0, uint32_t b0, uint32_t cw0,
                                                        const uint64_t* __restrict__ occ,
                                                        const uint64_t* __restrict__ bnd,
@@ -2498,19 +2508,22 @@ __device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB>& L, uint64_t* 
                                                        const uint2* __restrict__ ent, const float* __restrict__ tris,
                                                        uint64_t* __restrict__ out)
 {
-    const int lane = __lane_id();
+    const int lane = __lane_id(), tid = wv * 64 + lane;
+    constexpr int NT = V * 64;
+    float4(*const E)[4] = L.e[wv];
+    uint8_t* const win = L.win[wv];
     const int n2 = g.n2, w2 = g.w2, nsc = n2 * n2, nz = g.nz;
     const int bit0 = i1 & 63;
     const uint32_t cword = (uint32_t)j1 * (uint32_t)g.nxw + (uint32_t)(i1 >> 6);
-    if (!((occ[cw0 + cword] >> bit0) & ((1u << C) - 1u))) return;   // no boundary voxel in these columns
+    if (occ && !((occ[cw0 + cword] >> bit0) & ((1u << C) - 1u))) return;   // no boundary voxel in these columns
     const int fb = C == 1 && n2 > 8 ? 2 : 1;
     uint32_t* pre = reinterpret_cast<uint32_t*>(cb + C * nw);
     const uint32_t gcol = col0 + (uint32_t)(j1 * g.nx + i1);
     uint32_t ce[C + 1];   // the columns' first entries
 #pragma unroll
     for (int c = 0; c <= C; ++c) ce[c] = coff[gcol + (uint32_t)c];
-    if (lane < C * n2) L.ox[lane] = g.r2x[i1 * n2 + lane];
-    if (lane < n2) L.oy[lane] = g.r2y[j1 * n2 + lane];
+    if (tid < C * n2) L.ox[tid] = g.r2x[i1 * n2 + tid];
+    if (tid < n2) L.oy[tid] = g.r2y[j1 * n2 + tid];
     // slots of a column per window; one more row carries what lies above it
     const int Wn = min(KB / (C * nsc * fb) - 1, L2P_SLOTS / C);
     // the columns' boundary voxels: a bit per layer, their number below each
@@ -2534,11 +2547,11 @@ __device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB>& L, uint64_t* 
             for (int c = 0; c < C; ++c) {
                 const uint64_t m = __ballot((bits >> (bit0 + c)) & 1ull);
                 const uint32_t rank = S[c] + (uint32_t)__popcll(m & lanes_below_mask());
-                if (first && lane == 0) {
+                if (first && tid == 0) {
                     cb[c * nw + kw] = m;
                     pre[c * nw + kw] = S[c];
                 }
-                if (((m >> lane) & 1ull) && rank >= lo[c] && rank < hi[c])
+                if (wv == 0 && ((m >> lane) & 1ull) && rank >= lo[c] && rank < hi[c])
                     L.slotb[c * Wn + (int)(rank - lo[c])] = base + (uint32_t)__popcll(bits & ((1ull << (bit0 + c)) - 1ull));
                 S[c] += (uint32_t)__popcll(m);
             }
@@ -2553,6 +2566,7 @@ __device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB>& L, uint64_t* 
     uint32_t most = 0;
 #pragma unroll
     for (int c = 0; c < C; ++c) most = max(most, S[c]);
+    if (most == 0) return;
     const SatScale sc{g.s2x, g.s2y, g.s2z, g.d2x, g.d2y, g.d2z};
     const float gx = 2.0f * g.h2x, gy = 2.0f * g.h2y, inv_n2 = GPV_RCP((float)n2);
     const float* rz = g.r2z;
@@ -2570,17 +2584,17 @@ __device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB>& L, uint64_t* 
         }
         // clear the slots; the row past them keeps the parity of all windows above
         if (w0 == 0) {
-            for (int i = lane; i < (C * (Wn + 1) * nsc * fb + 3) / 4; i += 64) L.acc[i] = 0u;
+            for (int i = tid; i < (C * (Wn + 1) * nsc * fb + 3) / 4; i += NT) L.acc[i] = 0u;
         } else {
-            for (int i = lane; i < C * Wn * nsc; i += 64) {
+            for (int i = tid; i < C * Wn * nsc; i += NT) {
                 const int c = C == 1 ? 0 : i / (Wn * nsc);
                 const int at = i + c * nsc;
                 if (fb == 2) a16[at] = 0;
                 else a8[at] = 0;
             }
         }
-        __builtin_amdgcn_wave_barrier();
-        for (uint32_t base = ce[0]; base < ce[C]; base += L2P_STAGE) {
+        l2_parity_barrier<V>();
+        for (uint32_t base = ce[0] + (uint32_t)wv * L2P_STAGE; base < ce[C]; base += V * L2P_STAGE) {
             const uint32_t i = base + (uint32_t)lane;
             uint32_t P = 0;   // rows of this lane's entry
             int q0 = 0;
@@ -2624,10 +2638,10 @@ __device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB>& L, uint64_t* 
                 }
                 const int nq = meets ? par_rows(r, oy0, sc.sy, n2, sc.dy, q0) : 0;
                 P = nq > 0 ? (uint32_t)nq : 0u;
-                L.e[lane][0] = make_float4(m.e1x, m.e1y, m.e1z, m.e2x);
-                L.e[lane][1] = make_float4(m.e2y, m.e2z, m.inv_det, tv[0]);
-                L.e[lane][2] = make_float4(tv[1], r.dz, r.mu, r.delta);
-                L.e[lane][3] = make_float4(__int_as_float(r.l0), __int_as_float(cap), __int_as_float(c), tv[2]);
+                E[lane][0] = make_float4(m.e1x, m.e1y, m.e1z, m.e2x);
+                E[lane][1] = make_float4(m.e2y, m.e2z, m.inv_det, tv[0]);
+                E[lane][2] = make_float4(tv[1], r.dz, r.mu, r.delta);
+                E[lane][3] = make_float4(__int_as_float(r.l0), __int_as_float(cap), __int_as_float(c), tv[2]);
             }
             const uint32_t incl = wave_incl_scan<uint32_t>(P);
             const uint32_t so = incl - P;
@@ -2635,12 +2649,12 @@ __device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB>& L, uint64_t* 
             __builtin_amdgcn_wave_barrier();
             // the (entry, row) items: the columns each row can accept
             for (uint32_t l0 = 0; l0 < rows; l0 += 64) {
-                const int j = wave_item_owner(L.win, so, P, l0) & (L2P_STAGE - 1);
+                const int j = wave_item_owner(win, so, P, l0) & (L2P_STAGE - 1);
                 const int q = __shfl(q0, j) + (int)(l0 + (uint32_t)lane - (uint32_t)__shfl((int)so, j));
                 int p0 = 0, np = 0;
                 if (l0 + (uint32_t)lane < rows) {
-                    const float4 a = L.e[j][0], b = L.e[j][1], d = L.e[j][2];
-                    const int c = C == 1 ? 0 : __float_as_int(L.e[j][3].z);
+                    const float4 a = E[j][0], b = E[j][1], d = E[j][2];
+                    const int c = C == 1 ? 0 : __float_as_int(E[j][3].z);
                     ParEntry r;
                     r.e1x = a.x; r.e1y = a.y; r.e2x = a.w;
                     r.e2y = b.x; r.inv = b.z; r.v1x = b.w;
@@ -2654,12 +2668,12 @@ __device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB>& L, uint64_t* 
                 const int pq = p0 | (q << 8) | (j << 16);
                 // the (entry, sub-column) pairs
                 for (uint32_t m0 = 0; m0 < pairs; m0 += 64) {
-                    const int o = wave_item_owner(L.win, pso, (uint32_t)np, m0);
+                    const int o = wave_item_owner(win, pso, (uint32_t)np, m0);
                     const int v = __shfl(pq, o);
                     const uint32_t at = m0 + (uint32_t)lane - (uint32_t)__shfl((int)pso, o);
                     if (m0 + (uint32_t)lane < pairs) {
                         const int pp = (v & 255) + (int)at, qq = (v >> 8) & 255, jj = v >> 16;
-                        const float4 a = L.e[jj][0], b = L.e[jj][1], d = L.e[jj][2], f = L.e[jj][3];
+                        const float4 a = E[jj][0], b = E[jj][1], d = E[jj][2], f = E[jj][3];
                         const int c = C == 1 ? 0 : __float_as_int(f.z);
                         // the float det/u/v test (mt_column)
                         const float tx = L.ox[c * n2 + pp] - b.w, ty = L.oy[qq] - d.x;
@@ -2718,10 +2732,10 @@ __device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB>& L, uint64_t* 
                 }
             }
         }
-        __builtin_amdgcn_wave_barrier();
+        l2_parity_barrier<V>();
         // toggles -> parities, from each column's top slot down
         const uint32_t layers = (1u << n2) - 1u;
-        for (int it = lane; it < C * nsc; it += 64) {
+        for (int it = tid; it < C * nsc; it += NT) {
             const int c = C == 1 ? 0 : it / nsc;
             const int sub = it - c * nsc;
             uint32_t n = hi[0] - lo[0];
@@ -2744,13 +2758,13 @@ __device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB>& L, uint64_t* 
             if (fb == 2) a16[top] = (uint16_t)above;
             else a8[top] = (uint8_t)above;
         }
-        __builtin_amdgcn_wave_barrier();
+        l2_parity_barrier<V>();
         // the slots' words
         if (C <= 2 && n2 == 8) {
 #pragma unroll
             for (int c = 0; c < C; ++c) {
                 const int n = (int)(hi[c] - lo[c]);
-                for (int v0 = 0; v0 < n; v0 += 8) {
+                for (int v0 = wv * 8; v0 < n; v0 += 8 * V) {
                     // bit 8v + r of lane t: layer r of sub-column t of slot v0 + v
                     uint64_t x = 0;
                     for (int v = 0; v < 8 && v0 + v < n; ++v)
@@ -2762,7 +2776,7 @@ __device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB>& L, uint64_t* 
             }
         } else if (C == 1 && n2 == 16) {
             const int n = (int)(hi[0] - lo[0]);
-            for (int v = 0; v < n; ++v) {
+            for (int v = wv; v < n; v += V) {
                 // bit 16k + r of lane c: layer r of sub-column 64k + c
                 uint64_t x = 0;
                 for (int k = 0; k < 4; ++k) x |= (uint64_t)a16[v * 256 + k * 64 + lane] << (16 * k);
@@ -2774,7 +2788,7 @@ __device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB>& L, uint64_t* 
             for (int c = 0; c < C; ++c) {
                 const int n = (int)(hi[c] - lo[c]);
                 // lane t of a run of 64 keeps word t of the column's (slot, word) list
-                for (int t0 = 0; t0 < n * w2; t0 += 64) {
+                for (int t0 = wv * 64; t0 < n * w2; t0 += NT) {
                     uint64_t mine = 0;
                     int v = t0 / w2, m = t0 - v * w2;
                     const int te = min(64, n * w2 - t0);
@@ -2797,60 +2811,68 @@ __device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB>& L, uint64_t* 
                 }
             }
         }
-        __builtin_amdgcn_wave_barrier();
+        l2_parity_barrier<V>();
     }
 }
 
-template <bool kM, int KB, int W>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 1 ? 6 : 3))) void k_l2_parity(const uint64_t* __restrict__ bnd,
+// W waves a block: each with columns of its own (V = 1), or all with the same (V = W)
+template <bool kM, int KB, int W, int V>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(V > 1 ? 2 : W == 1 ? 6 : 3))) void k_l2_parity(const uint64_t* __restrict__ bnd,
                                                       const uint32_t* __restrict__ wprefix,
                                                       const uint64_t* __restrict__ occ, int64_t nwaves, bool many, int nw,
                                                       const uint32_t* __restrict__ coff,
                                                       const uint2* __restrict__ ent, const float* __restrict__ tris,
                                                       GridDev g0, Meshes M, uint64_t* __restrict__ par2)
 {
-    __shared__ L2PLds<KB> s_l[W];
-    extern __shared__ uint64_t s_cb[];   // per wave: 4 * nw words of column bits, then 4 * nw counts
-    const int wv = uniform_i((int)threadIdx.x >> 6);
+    static_assert(V == 1 || V == W, "waves of a column");
+    __shared__ L2PLds<KB, V> s_l[W / V];
+    extern __shared__ uint64_t s_cb[];   // per group of waves: 4 * nw words of column bits, then 4 * nw counts
+    const int wid = uniform_i((int)threadIdx.x >> 6), grp = V > 1 ? 0 : wid, wv = V > 1 ? wid : 0;
     // runs of 16 blocks (adjacent columns, which share boundary words) to one XCD
     uint32_t blk = blockIdx.x;
     if ((gridDim.x & 127u) == 0) blk = ((blk >> 7) << 7) + ((blk & 7u) << 4) + ((blk >> 3) & 15u);
-    const int64_t wave = (int64_t)blk * W + wv;
+    const int64_t wave = (int64_t)blk * (W / V) + grp;
     if (wave >= nwaves) return;
-    uint64_t* cb = s_cb + (size_t)wv * 6 * nw;
+    uint64_t* cb = s_cb + (size_t)grp * 6 * nw;
     int mesh = 0;
     if constexpr (kM)   // the mesh whose waves hold this one
         mesh = wave_mesh_search(M.off, M.nm, (uint64_t)wave, [](const MeshOff& o) { return (uint64_t)o.pw0; });
     const GridDev& g = grid_of<kM>(g0, M, mesh);
     if (kM && g.n2 == 0) return;
-    const int C = l2_parity_columns(g.n2, many);
+    const int C = V > 1 ? 1 : l2_parity_columns(g.n2, many);
     const int col = (int)(wave - (kM ? (int64_t)M.off[mesh].pw0 : 0)) * C;
     const int j1 = col / g.nx, i1 = col - j1 * g.nx;
     const uint64_t word0 = kM ? M.off[mesh].word0 : 0;
     const uint32_t col0 = kM ? M.off[mesh].col0 : 0, b0 = kM ? M.rank[mesh].b0 : 0;
     const uint32_t cw0 = kM ? M.off[mesh].cw0 : 0;
     uint64_t* out = par2 + (kM ? M.rank[mesh].l2w0 : 0);
-    if (C == 2)
-        l2_parity_columns_wave<2>(s_l[wv], cb, nw, g, i1, j1, word0, col0, b0, cw0, occ, bnd, wprefix, coff, ent, tris, out);
-    else if (C == 4)
-        l2_parity_columns_wave<4>(s_l[wv], cb, nw, g, i1, j1, word0, col0, b0, cw0, occ, bnd, wprefix, coff, ent, tris, out);
-    else
-        l2_parity_columns_wave<1>(s_l[wv], cb, nw, g, i1, j1, word0, col0, b0, cw0, occ, bnd, wprefix, coff, ent, tris, out);
+    if constexpr (V == 1) {
+        if (C == 2) {
+            l2_parity_columns_wave<2>(s_l[grp], wv, cb, nw, g, i1, j1, word0, col0, b0, cw0, occ, bnd, wprefix, coff, ent, tris, out);
+            return;
+        }
+        if (C == 4) {
+            l2_parity_columns_wave<4>(s_l[grp], wv, cb, nw, g, i1, j1, word0, col0, b0, cw0, occ, bnd, wprefix, coff, ent, tris, out);
+            return;
+        }
+    }
+    l2_parity_columns_wave<1>(s_l[grp], wv, cb, nw, g, i1, j1, word0, col0, b0, cw0, occ, bnd, wprefix, coff, ent, tris, out);
 }
 
-template <int KB, int W>
+template <int KB, int W, int V = 1>
 static void launch_l2_parity_w(const uint64_t* bnd, const uint32_t* wprefix, const uint64_t* occ, int64_t nwaves, bool many, int nzmax,
                                const uint32_t* coff, const uint2* ent, const float* tris, const GridDev& g0, const Meshes& M,
                                uint64_t* par2, hipStream_t s)
 {
-    unsigned blocks = (unsigned)((nwaves + W - 1) / W);
+    constexpr int G = W / V;   // groups of waves a block
+    unsigned blocks = (unsigned)((nwaves + G - 1) / G);
     if (blocks >= 1024) blocks = (blocks + 127u) & ~127u;   // whole rounds of the XCD mapping
     const int nw = (nzmax + 63) / 64;
-    const size_t lds = (size_t)W * 6 * nw * sizeof(uint64_t);
+    const size_t lds = (size_t)G * 6 * nw * sizeof(uint64_t);
     if (M.nm > 1)
-        k_l2_parity<true, KB, W><<<blocks, 64 * W, lds, s>>>(bnd, wprefix, occ, nwaves, many, nw, coff, ent, tris, g0, M, par2);
+        k_l2_parity<true, KB, W, V><<<blocks, 64 * W, lds, s>>>(bnd, wprefix, occ, nwaves, many, nw, coff, ent, tris, g0, M, par2);
     else
-        k_l2_parity<false, KB, W><<<blocks, 64 * W, lds, s>>>(bnd, wprefix, occ, nwaves, many, nw, coff, ent, tris, g0, M, par2);
+        k_l2_parity<false, KB, W, V><<<blocks, 64 * W, lds, s>>>(bnd, wprefix, occ, nwaves, many, nw, coff, ent, tris, g0, M, par2);
 }
 
 template <int KB>
@@ -2868,9 +2890,17 @@ void launch_l2_parity(const uint64_t* bnd, const uint32_t* wprefix, const uint64
                       uint64_t* par2, hipStream_t s)
 {
     if (nwaves <= 0) return;
-    // room for 31 boundary voxels of a column at n2 = 8, 7 at 16
-    if (n2max <= 8) launch_l2_parity_k<2048>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, waves, g0, M, par2, s);
-    else launch_l2_parity_k<4096>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, waves, g0, M, par2, s);
+    // Up to 1,024 columns the chip holds four waves for each, with room for 128 boundary
+    // voxels a window (31 at n2 = 16): a wave to a column left most of it idle, and every
+    // window of a tall column stages all of its entries (rods of 12 x 12 columns: 512 layers at
+    // n2 = 16 816 -> 338 us in all, 2,048 at 8 742 -> 720; 200,000 triangles at 8/16 772 -> 589; eight
+    // waves the same or slower).  More columns: room for 31 voxels at n2 = 8, 7 at 16
+    if (!many && nwaves <= 1024)
+        launch_l2_parity_w<16384, L2P_SHARE, L2P_SHARE>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, g0, M, par2, s);
+    else if (n2max <= 8)
+        launch_l2_parity_k<2048>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, waves, g0, M, par2, s);
+    else
+        launch_l2_parity_k<4096>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, waves, g0, M, par2, s);
 }
 
 // ---------------------------------------------------------------------------

@@ -43,6 +43,30 @@ def test_few_occupied_columns(gv, orc, l1, n2):
         g.release()
 
 
+# columns taken by several waves (up to 1,024 of them) and not; more boundary voxels than one
+# window of a column holds, more entries than the waves stage at once, and few of either
+@pytest.mark.parametrize("thin,l1,n2", [(0.02, 400, 16), (0.02, 400, 8), (0.03, 300, 11), (0.05, 600, 1), (0.05, 600, 4),
+                                        (0.124, 256, 8), (0.14, 256, 8), (0.124, 256, 16), (1, 12, 16), (1, 4, 5)])
+def test_few_tall_columns(gv, orc, thin, l1, n2):
+    v, f = gv.mixed(1, 9000, 51)
+    v = np.asarray(v, np.float64).copy()
+    v[:, :2] *= thin
+    v = v.astype(np.float32)
+    soup = gv.flatten(v, f)
+    bmin, bmax, mms = gv.mesh_bbox(v)
+    want = orc.voxelize(soup, orc.grid_setup(bmin, bmax, mms, l1, n2), orc.ORC_FAST)
+    mesh = {"soup": soup, "bmin": bmin, "bmax": bmax, "mms": mms, "voxel_count": l1, "voxel_count2": n2}
+    with gv.Context() as c:
+        say(f"few tall columns x{thin} {l1}/{n2}")
+        g = c.voxelize(soup, bmin, bmax, mms, l1, n2)
+        say(f"grid {g.info()['n']}, {g.info()['nb']} boundary voxels")
+        compare_results(f"alone {l1}/{n2}", g.download(), want, n2)
+        g.release()
+        for g in c.voxelize_batch([mesh, mesh]):
+            compare_results(f"batch {l1}/{n2}", g.download(), want, n2)
+            g.release()
+
+
 def test_empty_columns_cost_little(gv):
     """The Level2 parity of 27 boundary voxels in 262,144 columns of 512 layers: 0.89 ms
     with a scan of every column, 0.05 ms with the occupied ones only."""
@@ -57,3 +81,21 @@ def test_empty_columns_cost_little(gv):
             g.release()
         say(f"Level2 parity {min(ms):.3f} ms")
         assert min(ms) < 0.3
+
+
+def test_few_columns_share_the_chip(gv):
+    """The Level2 parity of a rod of 12 x 12 columns and 512 layers at n2 = 16: 0.63 ms with
+    a wave to a column, 0.18 ms with four."""
+    v, f = gv.mixed(1, 60000, 31)
+    v = np.asarray(v, np.float32).copy()
+    v[:, :2] *= np.float32(0.02)
+    soup, box = gv.flatten(v, f), gv.mesh_bbox(v)
+    with gv.Context() as c:
+        say("few columns")
+        ms = []
+        for _ in range(5):
+            g = c.voxelize(soup, *box, 512, 16)
+            ms.append(g.info()["ms_stage"][4])
+            g.release()
+        say(f"Level2 parity {min(ms):.3f} ms")
+        assert min(ms) < 0.4
