@@ -42,7 +42,8 @@ __device__ __forceinline__ bool sat_separated(float pa, float pb, float rad)
 // The three edge-axis predicates along e x z (the third AXISTEST of each
 // edge) read only the x and y components of v_i = tri_i - center and of the
 // edges, which depend on (cx, cy) alone: they hold or fail for a whole column
-// of boxes.  Same float expressions as in tri_box_overlap.
+// of boxes.  Same float expressions as in tri_box_overlap.  (No kernel splits the SAT
+// there any more; the device test of the predicates does.)
 __device__ __forceinline__ bool xy_edges_ok(float cx, float cy, float hx, float hy, const float* __restrict__ tv)
 {
     const float v0x = tv[0] - cx, v0y = tv[1] - cy;

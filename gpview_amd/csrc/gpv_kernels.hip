@@ -4,9 +4,9 @@
 //   index AABB, src/Object.cpp:2272-2318 ........... k_tri_setup
 //   Level1 SAT sweep + bins, src/Object.cpp:2256-2342,
 //     cuda/CUDAClassifyTessellation.cu:320-401 ...... k_sat_expand
-//   Level1 ray parity, src/Object.cpp:716-779 ....... k_ray_expand, k_scatter_hits, k_l1_parity
-//   compaction + prefix, src/Object.cpp:3270-3279 ... k_pack_bytes, scan, k_boundary_index
-//   bins by boundary voxel (the CSR of :2137-2219) .. k_ts_count, k_ts_bucket, k_ts_place
+//   Level1 ray parity, src/Object.cpp:716-779 ....... k_ray_expand, k_l1_fill
+//   compaction + prefix, src/Object.cpp:3270-3279 ... k_pack_bytes, scan, k_ts_count (boundary_index)
+//   bins by boundary voxel (the CSR of :2137-2219) .. k_ts_count, k_ts_scan, k_ts_bucket, k_ts_place
 //   Level2 SAT, src/Object.cpp:2344-2424 ............ k_l2_sat
 //   Level2 ray parity, src/Object.cpp:1111-1207 ..... k_ts_* (column entries), k_l2_parity
 //   counts, src/Object.cpp:3353-3378 ................ k_count_states
@@ -688,13 +688,6 @@ static void scan_rec(const TI* in, TO* out, int64_t n, TO* tmp, unsigned int* ma
         k_scan_apply_direct<TI, TO><<<(unsigned)nb, SCAN_NT, 0, s>>>(ScanJob<TI, TO>{in, sums, out, n, 1}, nullptr, nullptr);
         return;
     }
-    if (nb == 1) {
-        // block prefix of the single block is 0
-        if constexpr (sizeof(TO) == 8) launch_fill_u64(reinterpret_cast<uint64_t*>(sums), 0, 1, s);
-        else launch_fill_u32(reinterpret_cast<uint32_t*>(sums), 0, 1, s);
-        k_scan_apply<TI, TO><<<1, SCAN_NT, 0, s>>>(in, n, sums, out);
-        return;
-    }
     // scan the block sums in place (exclusive) into rest, then apply
     scan_rec<TO, TO>(sums, rest, nb, rest + nb + 1, nullptr, s);
     k_scan_apply<TI, TO><<<(unsigned)nb, SCAN_NT, 0, s>>>(in, n, rest, out);
@@ -863,8 +856,8 @@ __device__ __forceinline__ void block_put(BlockAppend<CAP>& L, const Append64& G
 // layers take several rounds.  One barrier a round counts what the block appends.
 // What bounds it: VALU issue for a third of the time (760 instructions per 64
 // items, half of them the triangle's coefficients, which too few columns would
-// share on fine meshes), the latency of the gathers and the barrier at four
-// waves a SIMD (117 VGPRs, 37 KB of LDS a block) for the rest.  Against a block of lanes
+// share on fine meshes), the latency of the gathers and the barrier for the rest: 117
+// VGPRs and 37 KB of LDS a block allow four waves a SIMD, of which 2.4 to 3.1 are there.  Against a block of lanes
 // that walked each column's layers with the float SAT inside a plane slab:
 // torus knot 256 (2.9 M columns) 150 -> 95 us, torus 512 (1.9 M) 115 -> 65,
 // drilled plate 512 (13.6 M, triangles up to the grid's size) 1870 -> 490,
@@ -2454,9 +2447,14 @@ void launch_l2_sat(const float* tris, const int32_t* bidx, int64_t B, int64_t ng
 // 256/8 0.232 -> 0.129 ms alone (1.82e8 -> 0.72e8 instructions), lattice-snapped
 // mesh 512/16 3.90 -> 2.24 ms, 128 small meshes 0.60 -> 0.39 ms.
 //
-// Columns without a boundary voxel are known from the bins' launch, a bit each: their
-// waves leave at once (a scan of 512 layers by every one of 262,144 columns took 0.89 ms
-// of an almost empty grid at 512/16, now 0.06).
+// From 8,192 columns on those without a boundary voxel are known from the bins' launch, a
+// bit each: their waves leave at once (a scan of 512 layers by every one of 262,144
+// columns took 0.89 ms of an almost empty grid at 512/16, now 0.06).
+//
+// A wave per voxel is still the faster way where a column's work is long and columns are
+// few among many (2,000 overlapping triangles of a tenth of a 256/8 grid: 1.05 against 1.8 ms in
+// all), and where coordinates lie so far from the origin that the margins are whole
+// layers (more than about 2e6 sub-voxels: a float no longer tells sub-voxels apart).
 //
 // What bounds it: the chain of dependent LDS and global reads of each wave
 // (VALU issue 0.39-0.47), hence one wave per block (an empty column's wave

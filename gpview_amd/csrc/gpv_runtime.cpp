@@ -439,17 +439,14 @@ int derive_grid(const float bmin[3], const float bmax[3], float mms, const gpv_p
     return GPV_OK;
 }
 
-// Center tables (float, computed in double exactly as the reference does):
+// Center tables (float, computed in double exactly as the reference does, center_at):
 //   L1 SAT  (p + 0.5)*ext*2 + min          src/Object.cpp:2329-2331
 //   L1 ray  min + (i + 0.5)*g              src/Object.cpp:743-745
 //   L2 SAT  (p + 0.5)*g2 + mid - ext1      src/Object.cpp:2369-2371, 2389-2391
 //   L2 ray  minPoint + (p + 0.5)*g2        src/Object.cpp:1134-1136, 1158-1160
 // cuda_l2: both Level2 tables in the CUDA kernels' float expression
 //   (2p+1)*ext2 + mid - ext1               cuda/CUDAClassifyTessellation.cu:423-425, 472-474
-// Returns whether each Level2 ray-origin table is non-decreasing over its
-// whole length (the parity kernels then bound a range of origins by its
-// first and last entries).
-// the twelve tables' offsets; returns the floats they take (plus one)
+// The twelve tables' offsets; returns the floats they take (plus one).
 size_t table_layout(const gpv_grid_info& I, size_t off[12])
 {
     const int n2 = I.n2 > 0 ? I.n2 : 0;
@@ -905,7 +902,9 @@ int launch_ray_half(Job* J, hipStream_t s)
 {
     gpv_ctx* c = J->ctx;
     if (!J->one_setup) HIP_TRY(hipEventRecord(J->ev[2], s));
-    if (!J->all_stencil) {   // the ray parity skips the stencil meshes
+    // where only some meshes take the stencil fill, the toggles of theirs are made too: the
+    // fill leaves them alone and the stencil's votes replace them
+    if (!J->all_stencil) {
         if (!J->ins_cleared) launch_fill_u64(J->ins, 0, J->W, s);
         J->ins_cleared = false;
         launch_ray_expand(J->tris, J->T, J->rng, J->ray_off, J->g[0], J->view(), J->ins, expand_blocks(c), s);

@@ -1,4 +1,6 @@
 // gpv_slab.hpp -- conservative plane-slab filter for the SAT's plane predicate.
+// No kernel uses it any more (gpv_satrow.hpp and gpv_parcol.hpp decide rows, columns
+// and crossings); host tests still check its bounds.
 //
 // The SAT (src/TriBoxIntersection.cpp:135-210) is a conjunction; its plane
 // predicate (planeBoxOverlap, :64-86) is evaluated on float values relative

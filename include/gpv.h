@@ -166,12 +166,12 @@ typedef struct gpv_tune {
                                   when the bins average fewer entries than this per voxel (56);
                                   0 never, a large value always */
     int sort_items_per_block;  /* bin entries per block in the counting sorts (2048) */
-    int l2_overlap;            /* run independent stages on the context's second stream: the ray
-                                  half of the set-up and the ray expansion beside the SAT half and
-                                  the Level1 SAT, the parity fill and the column-entry sort beside
-                                  the bins, the Level2 parity beside the Level2 SAT (1) */
+    int l2_overlap;            /* run independent stages on the context's second stream: the Level1
+                                  ray parity (or stencil fill) beside the Level1 SAT and the bins,
+                                  the Level2 parity beside the Level2 SAT (1) */
     int l2_sat_waves;          /* waves per block of the Level2 SAT: 1, 2 or 4 (1) */
-    int l2_parity_waves;       /* waves per block of the Level2 parity: 1, 2 or 4 (1) */
+    int l2_parity_waves;       /* waves per block of the Level2 parity: 1, 2 or 4 (1); up to 1,024
+                                  columns four waves share one whatever it says */
     int expand_stage_tris;     /* 128 or 256 (128); no kernel stages triangle batches any more,
                                   so it has no effect */
 } gpv_tune;
@@ -319,7 +319,11 @@ int gpv_grid_finish(gpv_ctx *ctx, gpv_grid *grid);
 
 /* ---- results ---------------------------------------------------------------- */
 int gpv_grid_get_info(const gpv_grid *grid, gpv_grid_info *info);
-/* Copies results to host buffers (any may be NULL):
+/* Copies results to host buffers (any may be NULL).  Ordinary memory is
+ * written by the calling thread and, above 256 KiB, up to three threads of the
+ * context from its page-locked staging (256 KiB, 16 MiB from the first larger
+ * download on); larger results go straight into page-locked memory
+ * (gpv_host_alloc).  The same holds for the normals and bits below.
  *   l1_state[n1]        0 outside / 1 inside / 2 boundary, [z][y][x]
  *   prefix[n1]          exclusive boundary prefix sum (Level1BoundaryPrefixSum.raw)
  *   bidx[nb]            boundary Level1 linear indices, ascending
