@@ -323,11 +323,30 @@ constexpr int64_t kL2ParityMany = 1 << 16;
 __host__ __device__ inline int l2_parity_columns(int n2, bool many) { return !many || n2 > 8 ? 1 : n2 <= 4 ? 4 : 2; }
 // its waves for a mesh with ncol columns (none when Level2 is off)
 int64_t l2_parity_waves(int n2, int64_t ncol, bool many);
-// n2max, nzmax: the largest Level2 resolution and layer count of the run
-// occ: the columns that hold boundary voxels
+// Waves whose columns hold more than `above` entries each leave them to a second launch,
+// where several waves share them: a count (zero at the start) and room for `most` of them
+struct L2Heavy {
+    uint32_t* count;
+    uint32_t* list;   // nullptr: no second launch
+    uint32_t above;
+    int64_t most;
+};
+// More than 128 (256: 4.4 ms in place of 2.9 where 2,000 triangles overlap in a tenth of a
+// 512/16 grid) and than four times what the run's columns hold on average: columns that are
+// all alike are better taken by a wave each (400,000 triangles at 64/4 268 -> 302 us in all with
+// 128 alone).  Below 16,384 waves no column outlasts the others by enough to pay for the
+// launch (most = 0).
+inline L2Heavy l2_heavy(uint64_t ncols, int64_t ncol, int64_t nwaves)
+{
+    const uint64_t mean = ncols / (uint64_t)(ncol > 0 ? ncol : 1);
+    const uint64_t above = 4 * mean > 128 ? 4 * mean : 128;
+    return L2Heavy{nullptr, nullptr, (uint32_t)above, nwaves < 16384 ? 0 : (int64_t)(ncols / (above + 1))};
+}
+// n2max, nzmax: the largest Level2 resolution and layer count of the run; occ: the
+// columns that hold boundary voxels (or nullptr)
 void launch_l2_parity(const uint64_t* bnd, const uint32_t* wprefix, const uint64_t* occ, int64_t nwaves, bool many,
-                      int n2max, int nzmax, const uint32_t* coff, const uint2* ent, const float* tris, int waves, const GridDev& g0,
-                      const Meshes& M, uint64_t* par2, hipStream_t s);
+                      int n2max, int nzmax, const uint32_t* coff, const uint2* ent, const float* tris, int waves,
+                      const GridDev& g0, const Meshes& M, const L2Heavy& H, uint64_t* par2, hipStream_t s);
 
 // normals (src/Object.cpp:3219-3253 Level1, 2372-2421 + 2705-2720 Level2)
 void launch_face_normals(const float* tris, int64_t T, float* fn, hipStream_t s);

@@ -2451,10 +2451,9 @@ void launch_l2_sat(const float* tris, const int32_t* bidx, int64_t B, int64_t ng
 // bit each: their waves leave at once (a scan of 512 layers by every one of 262,144
 // columns took 0.89 ms of an almost empty grid at 512/16, now 0.06).
 //
-// A wave per voxel is still the faster way where a column's work is long and columns are
-// few among many (2,000 overlapping triangles of a tenth of a 256/8 grid: 1.05 against 1.8 ms in
-// all), and where coordinates lie so far from the origin that the margins are whole
-// layers (more than about 2e6 sub-voxels: a float no longer tells sub-voxels apart).
+// A wave per voxel is still the faster way where coordinates lie so far from the origin that
+// the margins are whole layers (more than about 2e6 sub-voxels: a float hardly tells sub-voxels
+// apart), and in columns of many thousand layers.
 //
 // What bounds it: the chain of dependent LDS and global reads of each wave
 // (VALU issue 0.39-0.47), hence one wave per block (an empty column's wave
@@ -2497,7 +2496,8 @@ __device__ __forceinline__ void l2_parity_barrier()
 // C adjacent columns (i1 .., j1) of a mesh by one wave: 1, 2 (at n2 <= 8) or 4 (at n2 <= 4);
 // or, V > 1, by the V waves of a block, this one `wv`, which share the entries.
 template <int C, int KB, int V>
-__device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB, V>& L, int wv, uint64_t* cb, int nw, const GridDev& g, int i1, int j1,
+__device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB, V>& L, int wv, uint32_t wave, const L2Heavy& H, uint64_t* cb, int nw,
+                                                       const GridDev& g, int i1, int j1,
                                                        uint64_t word0, uint32_t col0, uint32_t b0, uint32_t cw0,
                                                        const uint64_t* __restrict__ occ,
                                                        const uint64_t* __restrict__ bnd,
@@ -2520,6 +2520,13 @@ __device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB, V>& L, int wv,
     uint32_t ce[C + 1];   // the columns' first entries
 #pragma unroll
     for (int c = 0; c <= C; ++c) ce[c] = coff[gcol + (uint32_t)c];
+    if (V == 1 && H.list && ce[C] - ce[0] > H.above * C) {   // left to the second launch
+        if (lane == 0) {
+            const uint32_t at = atomicAdd(H.count, 1u);
+            if ((int64_t)at < H.most) H.list[at] = wave;
+        }
+        return;
+    }
     if (tid < C * n2) L.ox[tid] = g.r2x[i1 * n2 + tid];
     if (tid < n2) L.oy[tid] = g.r2y[j1 * n2 + tid];
     // slots of a column per window; one more row carries what lies above it
@@ -2813,14 +2820,15 @@ __device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB, V>& L, int wv,
     }
 }
 
-// W waves a block: each with columns of its own (V = 1), or all with the same (V = W)
+// W waves a block: each with columns of its own (V = 1), or all with the same (V = W), those
+// of H's list if there is one
 template <bool kM, int KB, int W, int V>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(V > 1 ? 2 : W == 1 ? 6 : 3))) void k_l2_parity(const uint64_t* __restrict__ bnd,
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(V > 1 ? 5 : W == 1 ? 6 : 3))) void k_l2_parity(const uint64_t* __restrict__ bnd,
                                                       const uint32_t* __restrict__ wprefix,
                                                       const uint64_t* __restrict__ occ, int64_t nwaves, bool many, int nw,
                                                       const uint32_t* __restrict__ coff,
                                                       const uint2* __restrict__ ent, const float* __restrict__ tris,
-                                                      GridDev g0, Meshes M, uint64_t* __restrict__ par2)
+                                                      GridDev g0, Meshes M, L2Heavy H, uint64_t* __restrict__ par2)
 {
     static_assert(V == 1 || V == W, "waves of a column");
     __shared__ L2PLds<KB, V> s_l[W / V];
@@ -2829,76 +2837,85 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(V > 1 ? 
     // runs of 16 blocks (adjacent columns, which share boundary words) to one XCD
     uint32_t blk = blockIdx.x;
     if ((gridDim.x & 127u) == 0) blk = ((blk >> 7) << 7) + ((blk & 7u) << 4) + ((blk >> 3) & 15u);
-    const int64_t wave = (int64_t)blk * (W / V) + grp;
-    if (wave >= nwaves) return;
     uint64_t* cb = s_cb + (size_t)grp * 6 * nw;
-    int mesh = 0;
-    if constexpr (kM)   // the mesh whose waves hold this one
-        mesh = wave_mesh_search(M.off, M.nm, (uint64_t)wave, [](const MeshOff& o) { return (uint64_t)o.pw0; });
-    const GridDev& g = grid_of<kM>(g0, M, mesh);
-    if (kM && g.n2 == 0) return;
-    const int C = V > 1 ? 1 : l2_parity_columns(g.n2, many);
-    const int col = (int)(wave - (kM ? (int64_t)M.off[mesh].pw0 : 0)) * C;
-    const int j1 = col / g.nx, i1 = col - j1 * g.nx;
-    const uint64_t word0 = kM ? M.off[mesh].word0 : 0;
-    const uint32_t col0 = kM ? M.off[mesh].col0 : 0, b0 = kM ? M.rank[mesh].b0 : 0;
-    const uint32_t cw0 = kM ? M.off[mesh].cw0 : 0;
-    uint64_t* out = par2 + (kM ? M.rank[mesh].l2w0 : 0);
-    if constexpr (V == 1) {
-        if (C == 2) {
-            l2_parity_columns_wave<2>(s_l[grp], wv, cb, nw, g, i1, j1, word0, col0, b0, cw0, occ, bnd, wprefix, coff, ent, tris, out);
-            return;
-        }
-        if (C == 4) {
-            l2_parity_columns_wave<4>(s_l[grp], wv, cb, nw, g, i1, j1, word0, col0, b0, cw0, occ, bnd, wprefix, coff, ent, tris, out);
-            return;
-        }
+    const int64_t first = (int64_t)blk * (W / V) + grp;
+    const bool listed = V > 1 && H.list;
+    const int64_t n = listed ? min((int64_t)*H.count, H.most) : nwaves;
+    for (int64_t at = first; at < n; at += listed ? (int64_t)gridDim.x : n) {   // one turn but for a list
+        const int64_t wave = listed ? (int64_t)H.list[at] : at;
+        int mesh = 0;
+        if constexpr (kM)   // the mesh whose waves hold this one
+            mesh = wave_mesh_search(M.off, M.nm, (uint64_t)wave, [](const MeshOff& o) { return (uint64_t)o.pw0; });
+        const GridDev& g = grid_of<kM>(g0, M, mesh);
+        if (kM && g.n2 == 0) continue;
+        const int C = l2_parity_columns(g.n2, many);
+        const int col = (int)(wave - (kM ? (int64_t)M.off[mesh].pw0 : 0)) * C;
+        const int j1 = col / g.nx, i1 = col - j1 * g.nx;
+        const uint64_t word0 = kM ? M.off[mesh].word0 : 0;
+        const uint32_t col0 = kM ? M.off[mesh].col0 : 0, b0 = kM ? M.rank[mesh].b0 : 0;
+        const uint32_t cw0 = kM ? M.off[mesh].cw0 : 0;
+        uint64_t* out = par2 + (kM ? M.rank[mesh].l2w0 : 0);
+        if (C == 2)
+            l2_parity_columns_wave<2>(s_l[grp], wv, (uint32_t)wave, H, cb, nw, g, i1, j1, word0, col0, b0, cw0, occ, bnd, wprefix, coff, ent, tris, out);
+        else if (C == 4)
+            l2_parity_columns_wave<4>(s_l[grp], wv, (uint32_t)wave, H, cb, nw, g, i1, j1, word0, col0, b0, cw0, occ, bnd, wprefix, coff, ent, tris, out);
+        else
+            l2_parity_columns_wave<1>(s_l[grp], wv, (uint32_t)wave, H, cb, nw, g, i1, j1, word0, col0, b0, cw0, occ, bnd, wprefix, coff, ent, tris, out);
     }
-    l2_parity_columns_wave<1>(s_l[grp], wv, cb, nw, g, i1, j1, word0, col0, b0, cw0, occ, bnd, wprefix, coff, ent, tris, out);
 }
 
 template <int KB, int W, int V = 1>
 static void launch_l2_parity_w(const uint64_t* bnd, const uint32_t* wprefix, const uint64_t* occ, int64_t nwaves, bool many, int nzmax,
                                const uint32_t* coff, const uint2* ent, const float* tris, const GridDev& g0, const Meshes& M,
-                               uint64_t* par2, hipStream_t s)
+                               const L2Heavy& H, uint64_t* par2, hipStream_t s)
 {
     constexpr int G = W / V;   // groups of waves a block
-    unsigned blocks = (unsigned)((nwaves + G - 1) / G);
+    // a list is mostly short or empty: no more blocks than the chip holds at once
+    const int64_t n = V > 1 && H.list ? (H.most < 1536 ? H.most : 1536) : nwaves;
+    unsigned blocks = (unsigned)((n + G - 1) / G);
     if (blocks >= 1024) blocks = (blocks + 127u) & ~127u;   // whole rounds of the XCD mapping
     const int nw = (nzmax + 63) / 64;
     const size_t lds = (size_t)G * 6 * nw * sizeof(uint64_t);
     if (M.nm > 1)
-        k_l2_parity<true, KB, W, V><<<blocks, 64 * W, lds, s>>>(bnd, wprefix, occ, nwaves, many, nw, coff, ent, tris, g0, M, par2);
+        k_l2_parity<true, KB, W, V><<<blocks, 64 * W, lds, s>>>(bnd, wprefix, occ, nwaves, many, nw, coff, ent, tris, g0, M, H, par2);
     else
-        k_l2_parity<false, KB, W, V><<<blocks, 64 * W, lds, s>>>(bnd, wprefix, occ, nwaves, many, nw, coff, ent, tris, g0, M, par2);
+        k_l2_parity<false, KB, W, V><<<blocks, 64 * W, lds, s>>>(bnd, wprefix, occ, nwaves, many, nw, coff, ent, tris, g0, M, H, par2);
 }
 
 template <int KB>
 static void launch_l2_parity_k(const uint64_t* bnd, const uint32_t* wprefix, const uint64_t* occ, int64_t nwaves, bool many, int nzmax,
                                const uint32_t* coff, const uint2* ent, const float* tris, int waves, const GridDev& g0, const Meshes& M,
-                               uint64_t* par2, hipStream_t s)
+                               const L2Heavy& H, uint64_t* par2, hipStream_t s)
 {
-    if (waves <= 1) launch_l2_parity_w<KB, 1>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, g0, M, par2, s);
-    else if (waves == 2) launch_l2_parity_w<KB, 2>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, g0, M, par2, s);
-    else launch_l2_parity_w<KB, 4>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, g0, M, par2, s);
+    if (waves <= 1) launch_l2_parity_w<KB, 1>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, g0, M, H, par2, s);
+    else if (waves == 2) launch_l2_parity_w<KB, 2>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, g0, M, H, par2, s);
+    else launch_l2_parity_w<KB, 4>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, g0, M, H, par2, s);
 }
 
 void launch_l2_parity(const uint64_t* bnd, const uint32_t* wprefix, const uint64_t* occ, int64_t nwaves, bool many, int n2max, int nzmax,
                       const uint32_t* coff, const uint2* ent, const float* tris, int waves, const GridDev& g0, const Meshes& M,
-                      uint64_t* par2, hipStream_t s)
+                      const L2Heavy& H, uint64_t* par2, hipStream_t s)
 {
     if (nwaves <= 0) return;
     // Up to 1,024 columns the chip holds four waves for each, with room for 128 boundary
     // voxels a window (31 at n2 = 16): a wave to a column left most of it idle, and every
     // window of a tall column stages all of its entries (rods of 12 x 12 columns: 512 layers at
     // n2 = 16 816 -> 338 us in all, 2,048 at 8 742 -> 720; 200,000 triangles at 8/16 772 -> 589; eight
-    // waves the same or slower).  More columns: room for 31 voxels at n2 = 8, 7 at 16
-    if (!many && nwaves <= 1024)
-        launch_l2_parity_w<16384, L2P_SHARE, L2P_SHARE>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, g0, M, par2, s);
-    else if (n2max <= 8)
-        launch_l2_parity_k<2048>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, waves, g0, M, par2, s);
+    // waves the same or slower)
+    if (nwaves <= 1024) {
+        launch_l2_parity_w<16384, L2P_SHARE, L2P_SHARE>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, g0, M, L2Heavy{}, par2, s);
+        return;
+    }
+    // More columns: a wave takes its own, with room for 31 voxels at n2 = 8 and 7 at 16 (four
+    // waves to each: lattice-snapped mesh at 512/16 1.8 -> 4.3 ms), but for those of many entries,
+    // which would outlast all others: 2,000 overlapping triangles in a tenth of a 256/8 grid
+    // 1.63 -> 0.54 ms, of a 512/16 one 8.1 -> 3.0
+    if (n2max <= 8)
+        launch_l2_parity_k<2048>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, waves, g0, M, H, par2, s);
     else
-        launch_l2_parity_k<4096>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, waves, g0, M, par2, s);
+        launch_l2_parity_k<4096>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, waves, g0, M, H, par2, s);
+    if (H.list)
+        launch_l2_parity_w<16384, L2P_SHARE, L2P_SHARE>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, g0, M, H, par2, s);
 }
 
 // ---------------------------------------------------------------------------

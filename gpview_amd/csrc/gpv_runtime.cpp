@@ -303,6 +303,8 @@ struct Job {
     uint32_t *pair_cnt = nullptr, *col_cnt = nullptr;
     uint64_t* col_occ = nullptr;
     int64_t colw = 0;
+    L2Heavy heavy{};          // columns of many entries; their count lies behind the counters
+    bool heavy_cleared = false;   // and is zero
     size_t bin_words = 0;
     bool bins_cleared = false;
     bool streams = false;            // the Level2 stages ran on two streams
@@ -793,10 +795,11 @@ int alloc_bin_counters(Job* J, uint64_t most)
     const size_t a = ts_words(most), b = J->n2max > 0 ? ts_words((uint64_t)J->ncol) : 0;
     // (fewer columns are sooner scanned than marked: the marks of a tall grid fall on few words)
     const size_t occ = J->n2max > 0 && J->ncol >= kOccupancyMany ? 2 * (size_t)J->colw : 0;
-    TRY(alloc(J, &J->pair_cnt, a + b + occ));
+    TRY(alloc(J, &J->pair_cnt, a + b + occ + 2));
     J->col_cnt = J->pair_cnt + a;
     J->col_occ = occ ? reinterpret_cast<uint64_t*>(J->pair_cnt + a + b) : nullptr;   // ts_words is even
-    J->bin_words = a + b + occ;
+    J->heavy.count = J->pair_cnt + a + b + occ;
+    J->bin_words = a + b + occ + 2;
     return GPV_OK;
 }
 
@@ -1036,6 +1039,7 @@ int launch_compact(Job* J)
     release(J, J->list);
     release(J, J->coff);
     release(J, J->cent);
+    release(J, J->heavy.list);
     TRY(alloc(J, &J->boff, (size_t)J->B + 1));
     TRY(alloc(J, &J->list, (size_t)std::max<uint64_t>(J->n_pairs, 1)));
     if (!J->bins_cleared) {
@@ -1043,6 +1047,7 @@ int launch_compact(Job* J)
         launch_fill_u32(J->pair_cnt, 0, (int64_t)J->bin_words, s);
     }
     J->bins_cleared = false;
+    J->heavy_cleared = true;
     // only the Level2 parity reads the column entries
     const bool cols = J->n2max > 0;
     uint2* pb = nullptr;
@@ -1052,6 +1057,10 @@ int launch_compact(Job* J)
         TRY(alloc(J, &cb, 3 * (size_t)std::max<uint64_t>(J->n_cols, 1)));
         TRY(alloc(J, &J->coff, (size_t)J->ncol + 1));
         TRY(alloc(J, &J->cent, (size_t)std::max<uint64_t>(J->n_cols, 1)));
+        const L2Heavy h = l2_heavy(J->n_cols, J->ncol, J->l2p_waves);
+        J->heavy.above = h.above;
+        J->heavy.most = h.most;
+        if (J->heavy.most > 0) TRY(alloc(J, &J->heavy.list, (size_t)J->heavy.most));
     }
     launch_bins(BinPairs{J->pair_key, J->pairs_ranked, J->pair_tri, J->n_pairs, (uint32_t)J->B, J->pair_cnt, pb, J->boff,
                          J->nm > 1 ? nullptr : &J->mctr[0].max_per_voxel, J->list},
@@ -1099,9 +1108,11 @@ int l2_plan(Job* J)
 int l2_parity_kernels(Job* J, hipStream_t s)
 {
     HIP_TRY(hipEventRecord(J->ev[16], s));
+    if (!J->heavy_cleared) launch_fill_u32(J->heavy.count, 0, 1, s);   // a parity made again
+    J->heavy_cleared = false;
     if (J->B > 0)
         launch_l2_parity(J->bnd, J->wprefix, J->col_occ, J->l2p_waves, J->ncol >= kL2ParityMany, J->n2max, J->nzmax, J->coff, J->cent,
-                         J->tris, J->ctx->tune.l2_parity_waves, J->g[0], J->view(), J->par2, s);
+                         J->tris, J->ctx->tune.l2_parity_waves, J->g[0], J->view(), J->heavy, J->par2, s);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipEventRecord(J->ev[11], s));
     return GPV_OK;
@@ -1249,7 +1260,7 @@ int job_finish(Job* J)
     release(J, J->scan64); J->scan32 = nullptr; J->scan_cap = 0;
     release(J, J->pair_key); release(J, J->pair_tri); release(J, J->col_key); release(J, J->col_z);
     release(J, J->wcnt); release(J, J->boff);
-    release(J, J->list); release(J, J->coff); release(J, J->cent);
+    release(J, J->list); release(J, J->coff); release(J, J->cent); release(J, J->heavy.list);
     release(J, J->pair_cnt);
     release(J, J->sat_sums); release(J, J->ray_sums); release(J, J->bbytes); release(J, J->tri_mesh);
     release(J, J->st_cnt); release(J, J->st_off); release(J, J->st_scan); release(J, J->st_tog);
@@ -1326,7 +1337,7 @@ int64_t predict_run_bytes(const gpv_mesh_desc& d, const gpv_grid_info& I)
     b += 24 * W + 64 * W + W / 256 + 4;                          // planes, word counts, their sums and prefix, flag bytes
     b += T / 16 + 16;                                            // sums of the items
     b += 24 * P;                                                 // bin pairs, column entries
-    b += 4 * (ncol + 1) + 8 * P + 12 * P;                        // column entries by column
+    b += 4 * (ncol + 1) + 8 * P + 12 * P + P / 64;               // column entries by column, columns of many
     b += 8 * B + 4 + 4 * P + 8 * P;                              // boundary list, bins
     b += 4 * (int64_t)(ts_words((uint64_t)std::min<int64_t>(W * 64, int64_t(1) << 27)) + ts_words((uint64_t)ncol)) + W / nz * 8;   // their counters, the columns' occupancy
     b += 16 * B * w2;                                            // Level2 planes
