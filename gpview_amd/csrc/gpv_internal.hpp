@@ -62,6 +62,19 @@ __host__ __device__ inline float center_at(int which, int k, float bmin, float g
     return (float)((double)minp + (p + 0.5) * (double)g2);
 }
 
+// From an eighth of a sub-voxel of table deviation on (SatScale), Level2 positions are taken
+// from the tables themselves (gpv_satrow.hpp, gpv_parcol.hpp), so that a grid's distance from the
+// origin no longer costs float tests: 60,000 triangles at 128/16, deviations 0.09, 0.29, 0.86, 2.9
+// and 29: by the tables 548, 593, 625, 703 and 1168 us in all, by equal steps 488, 700, 1461, 7359 and
+// more than 12,000; at 128/8, 0.14: 336 and 327.
+constexpr float kFarDev = 0x1p-3f;
+
+inline bool level2_far(const GridDev& g)
+{
+    const float d = g.d2x > g.d2y ? g.d2x : g.d2y;
+    return g.n2 > 0 && (d > g.d2z ? d : g.d2z) > kFarDev;
+}
+
 // Where one mesh of a batch lives in the batch-wide arrays.  A batch
 // concatenates the meshes' soups (tri0), Level1 bitplanes (word0) and xy
 // columns (col0); entry nm is the sentinel holding the totals.  Set when the run is
@@ -311,7 +324,7 @@ void launch_mesh_bins(const uint32_t* boff, int64_t B, const Meshes& M, hipStrea
 
 // ngroups waves of at most gmost voxels each (l2_group_voxels); waves: per block (1, 2, 4)
 void launch_l2_sat(const float* tris, const int32_t* bidx, int64_t B, int64_t ngroups, int gmost, const uint32_t* boff,
-                   const uint32_t* list, int n2max, int waves, const GridDev& g0, const Meshes& M,
+                   const uint32_t* list, int n2max, bool far, int waves, const GridDev& g0, const Meshes& M,
                    uint64_t* sat2, hipStream_t s);
 // Level2 parity: a wave takes l2_parity_columns adjacent columns of a mesh
 // (grids are multiples of four in x): four at n2 <= 4, two up to 8, in runs of at least
@@ -346,7 +359,7 @@ inline L2Heavy l2_heavy(uint64_t ncols, int64_t ncol, int64_t nwaves)
 // columns that hold boundary voxels (or nullptr)
 void launch_l2_parity(const uint64_t* bnd, const uint32_t* wprefix, const uint64_t* occ, int64_t nwaves, bool many,
                       int n2max, int nzmax, const uint32_t* coff, const uint2* ent, const float* tris, int waves,
-                      const GridDev& g0, const Meshes& M, const L2Heavy& H, uint64_t* par2, hipStream_t s);
+                      const GridDev& g0, const Meshes& M, const L2Heavy& H, bool far, uint64_t* par2, hipStream_t s);
 
 // normals (src/Object.cpp:3219-3253 Level1, 2372-2421 + 2705-2720 Level2)
 void launch_face_normals(const float* tris, int64_t T, float* fn, hipStream_t s);

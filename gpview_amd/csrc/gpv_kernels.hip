@@ -2074,9 +2074,17 @@ __device__ __forceinline__ uint64_t wave_transpose64(uint64_t v)
     return transpose_step<5>(v);
 }
 
+// the sub-center positions of a group's voxels, far from the origin (gpv_satrow.hpp)
+template <bool kFar>
+struct L2Pos {};
+template <>
+struct L2Pos<true> {
+    float pos[kL2GroupMax][3][16];
+};
+
 // LDS of one wave of the Level2 SAT
-template <bool kPieces>
-struct L2Lds {
+template <bool kPieces, bool kFar>
+struct L2Lds : L2Pos<kFar> {
     union {
         float4 e[L2_STAGE][kSatEntry4];                  // staged entries
         unsigned long long words[kL2GroupBytes / 8];     // output words, once the bins are done
@@ -2102,8 +2110,8 @@ __device__ __forceinline__ uint32_t l2_col_word(uint32_t col, int n2, uint32_t& 
 
 // Full float SAT for queued entries (one per lane); entry = p | q<<4 | r<<8 |
 // v<<12 | j<<16 where v is the voxel in the group and j the bin entry from base.
-template <bool kPieces>
-__device__ __forceinline__ void l2_sat_run(uint32_t ent, bool valid, L2Lds<kPieces>& L, const GridDev& g,
+template <bool kPieces, bool kFar>
+__device__ __forceinline__ void l2_sat_run(uint32_t ent, bool valid, L2Lds<kPieces, kFar>& L, const GridDev& g,
                                            const float* __restrict__ tris, const uint32_t* __restrict__ list,
                                            uint32_t base)
 {
@@ -2141,17 +2149,17 @@ __device__ __forceinline__ int l2_axis_last(const float* __restrict__ c, int n, 
     return k;
 }
 
-template <bool kM, int W, bool kPieces>
+template <bool kM, int W, bool kPieces, bool kFar>
 __global__ __launch_bounds__(64 * W) void k_l2_sat(const float* __restrict__ tris, const int32_t* __restrict__ bidx,
                                                    int64_t B, int64_t ngroups, int gmost,
                                                    const uint32_t* __restrict__ boff,
                                                    const uint32_t* __restrict__ list,
                                                    GridDev g0, Meshes M, uint64_t* __restrict__ sat2)
 {
-    __shared__ L2Lds<kPieces> s_l[W];
+    __shared__ L2Lds<kPieces, kFar> s_l[W];
     const int wv = threadIdx.x >> 6;
     const int lane = __lane_id();
-    L2Lds<kPieces>& L = s_l[wv];
+    L2Lds<kPieces, kFar>& L = s_l[wv];
     const int64_t grp = (int64_t)blockIdx.x * W + wv;
     if (grp >= ngroups) return;
     int mesh = 0;
@@ -2181,6 +2189,16 @@ __global__ __launch_bounds__(64 * W) void k_l2_sat(const float* __restrict__ tri
     }
     __builtin_amdgcn_wave_barrier();
     const SatScale sc{g.s2x, g.s2y, g.s2z, g.d2x, g.d2y, g.d2z};
+    const SatScale se = kFar ? sat_scale_far(sc) : sc;   // of the entries
+    const int half = n2 > 8 ? 8 : 4;
+    if constexpr (kFar) {
+        for (int i = lane; i < nv * 48; i += 64) {
+            const int v = i / 48, a = (i - v * 48) >> 4, p = i & 15;
+            const float* c = (a == 0 ? g.c2x : a == 1 ? g.c2y : g.c2z) + L.ci[v][a];
+            const float s = a == 0 ? sc.sx : a == 1 ? sc.sy : sc.sz;
+            L.pos[v][a][p] = p < n2 ? (c[p] - c[0]) * s + (a == 2 ? 1.0f : 0.0f) : __builtin_inff();
+        }
+    }
     uint32_t qh = 0, qt = 0;   // ring head/tail (uniform)
     const uint32_t e0 = (uint32_t)uniform_i((int)L.vb[0]), e1 = (uint32_t)uniform_i((int)L.vb[nv]);
     uint32_t qbase = e0;       // the bin entry that queued entries count from
@@ -2210,7 +2228,7 @@ __global__ __launch_bounds__(64 * W) void k_l2_sat(const float* __restrict__ tri
                 else hi = mid;
             }
             const float *cx = g.c2x + L.ci[v][0], *cy = g.c2y + L.ci[v][1], *cz = g.c2z + L.ci[v][2];
-            loose = sat_entry_part(h, tv, cx[0], cy[0], cz[0], sc, L.e[js]);
+            loose = sat_entry_part(h, tv, cx[0], cy[0], cz[0], se, L.e[js]);
             // box axes: x and the first layer by the lower lane, y and the last by the upper
             const float lo = h ? fminf(fminf(tv[1], tv[4]), tv[7]) : fminf(fminf(tv[0], tv[3]), tv[6]);
             const float top = h ? fmaxf(fmaxf(tv[1], tv[4]), tv[7]) : fmaxf(fmaxf(tv[0], tv[3]), tv[6]);
@@ -2275,7 +2293,10 @@ __global__ __launch_bounds__(64 * W) void k_l2_sat(const float* __restrict__ tri
                 q = (int)(((d >> 4) & 15) + (l - so_j));
                 p = d & 15;
                 left = (int)((d >> 16) & 15) + 1;   // columns of the row
-                sat_row_range(L.e[j], q, d >> 31 != 0, p, left);
+                if constexpr (kFar) {
+                    const int vj = (int)((d >> 20) & 15u);
+                    sat_row_range_far(L.e[j], L.pos[vj][1][q & 15], L.pos[vj][0], half, d >> 31 != 0, p, left);
+                } else sat_row_range(L.e[j], q, d >> 31 != 0, p, left);
                 left = l < S && left > 0 ? left : 0;
                 if constexpr (kPieces) {
                     // pieces of each size, in fields of their own (at most 512, 256, 128 in all)
@@ -2315,8 +2336,11 @@ __global__ __launch_bounds__(64 * W) void k_l2_sat(const float* __restrict__ tri
             const uint32_t d = L.dec[j];
             const int ra = (d >> 8) & 15, rb = (d >> 12) & 15, v = (int)((d >> 20) & 15u);
             const bool loose = d >> 31 != 0;
-            SatRow row = sat_row_at(L.e[j], q, ra, rb, p);
-            if (__ballot(loose)) sat_row_loose(row, loose, ra, rb);
+            SatRow row;
+            if constexpr (kFar) row = sat_row_xy(L.e[j], L.pos[v][1][q & 15], -1e9f, 1e9f, L.pos[v][0][p & 15]);
+            else row = sat_row_at(L.e[j], q, ra, rb, p);
+            if (__ballot(loose)) sat_row_loose(row, loose, kFar ? -1 : ra, kFar ? 1 << 30 : rb);
+            const uint32_t layers = (2u << rb) - (1u << ra);
             uint32_t col = (uint32_t)((v * n2 + q) * n2 + p);
             const uint32_t ent = (uint32_t)p | ((uint32_t)q << 4) | ((uint32_t)v << 12) | ((base - qbase + (uint32_t)j) << 16);
             for (int k = 0;; ++k, ++col) {
@@ -2325,7 +2349,11 @@ __global__ __launch_bounds__(64 * W) void k_l2_sat(const float* __restrict__ tri
                 uint32_t unk = 0;
                 if (on) {
                     uint32_t in, may;
-                    sat_row_column(row, in, may);
+                    if constexpr (kFar) {
+                        // (the last column takes no step)
+                        const float step = k + 1 < left ? L.pos[v][0][p + k + 1] - L.pos[v][0][p + k] : 0.0f;
+                        sat_row_column_far(row, L.pos[v][2], half, layers, step, in, may);
+                    } else sat_row_column(row, in, may);
                     unk = may & ~in;
                     if (in) {
                         uint32_t bit;
@@ -2396,16 +2424,16 @@ __global__ __launch_bounds__(64 * W) void k_l2_sat(const float* __restrict__ tri
     for (int i = lane; i < nv * w2; i += 64) out[i] = L.words[i];
 }
 
-template <int W, bool kPieces>
+template <int W, bool kPieces, bool kFar = false>
 static void launch_l2_sat_w(const float* tris, const int32_t* bidx, int64_t B, int64_t ngroups, int gmost,
                             const uint32_t* boff, const uint32_t* list, const GridDev& g0, const Meshes& M,
                             uint64_t* sat2, hipStream_t s)
 {
     const unsigned blocks = (unsigned)((ngroups + W - 1) / W);
     if (M.nm > 1)
-        k_l2_sat<true, W, kPieces><<<blocks, 64 * W, 0, s>>>(tris, bidx, B, ngroups, gmost, boff, list, g0, M, sat2);
+        k_l2_sat<true, W, kPieces, kFar><<<blocks, 64 * W, 0, s>>>(tris, bidx, B, ngroups, gmost, boff, list, g0, M, sat2);
     else
-        k_l2_sat<false, W, kPieces><<<blocks, 64 * W, 0, s>>>(tris, bidx, B, ngroups, gmost, boff, list, g0, M, sat2);
+        k_l2_sat<false, W, kPieces, kFar><<<blocks, 64 * W, 0, s>>>(tris, bidx, B, ngroups, gmost, boff, list, g0, M, sat2);
 }
 
 template <bool kPieces>
@@ -2419,10 +2447,16 @@ static void launch_l2_sat_p(const float* tris, const int32_t* bidx, int64_t B, i
 }
 
 void launch_l2_sat(const float* tris, const int32_t* bidx, int64_t B, int64_t ngroups, int gmost, const uint32_t* boff,
-                   const uint32_t* list, int n2max, int waves, const GridDev& g0, const Meshes& M,
+                   const uint32_t* list, int n2max, bool far, int waves, const GridDev& g0, const Meshes& M,
                    uint64_t* sat2, hipStream_t s)
 {
     if (B <= 0 || ngroups <= 0) return;
+    // one wave a block is the default of `waves` as well
+    if (far) {
+        if (n2max > 8) launch_l2_sat_w<1, true, true>(tris, bidx, B, ngroups, gmost, boff, list, g0, M, sat2, s);
+        else launch_l2_sat_w<1, false, true>(tris, bidx, B, ngroups, gmost, boff, list, g0, M, sat2, s);
+        return;
+    }
     // Rows in pieces above n2 = 8, where a round of whole rows waits for one of up to 16
     // columns (lattice-snapped mesh at 512/16: 2.54 -> 2.24 ms alone).  Shorter rows do not
     // pay for the ring: torus knot 256/8 the same, 128 small meshes at 64/4 2.25 -> 2.29 ms in all
@@ -2451,9 +2485,7 @@ void launch_l2_sat(const float* tris, const int32_t* bidx, int64_t B, int64_t ng
 // bit each: their waves leave at once (a scan of 512 layers by every one of 262,144
 // columns took 0.89 ms of an almost empty grid at 512/16, now 0.06).
 //
-// A wave per voxel is still the faster way where coordinates lie so far from the origin that
-// the margins are whole layers (more than about 2e6 sub-voxels: a float hardly tells sub-voxels
-// apart), and in columns of many thousand layers.
+// A wave per voxel is still the faster way in columns of many thousand layers.
 //
 // What bounds it: the chain of dependent LDS and global reads of each wave
 // (VALU issue 0.39-0.47), hence one wave per block (an empty column's wave
@@ -2495,7 +2527,7 @@ __device__ __forceinline__ void l2_parity_barrier()
 
 // C adjacent columns (i1 .., j1) of a mesh by one wave: 1, 2 (at n2 <= 8) or 4 (at n2 <= 4);
 // or, V > 1, by the V waves of a block, this one `wv`, which share the entries.
-template <int C, int KB, int V>
+template <int C, int KB, int V, bool kFar>
 __device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB, V>& L, int wv, uint32_t wave, const L2Heavy& H, uint64_t* cb, int nw,
                                                        const GridDev& g, int i1, int j1,
                                                        uint64_t word0, uint32_t col0, uint32_t b0, uint32_t cw0,
@@ -2575,6 +2607,7 @@ __device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB, V>& L, int wv,
     const SatScale sc{g.s2x, g.s2y, g.s2z, g.d2x, g.d2y, g.d2z};
     const float gx = 2.0f * g.h2x, gy = 2.0f * g.h2y, inv_n2 = GPV_RCP((float)n2);
     const float* rz = g.r2z;
+    const bool scaled = sc.dx >= 0.0f && sc.dy >= 0.0f && sc.dz >= 0.0f;
     uint8_t* a8 = reinterpret_cast<uint8_t*>(L.acc);
     uint16_t* a16 = reinterpret_cast<uint16_t*>(L.acc);
     // windows of slots from the top down (one, but for columns of many boundary voxels)
@@ -2623,6 +2656,12 @@ __device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB, V>& L, int wv,
                 par_entry(r, tv[2], par_oz(g.bminz, 2.0f * g.h1z, 2.0f * g.h2z, zmax), ox0, oy0, gx, gy, n2, sc);
                 // candidate for the voxels up to zmax (all with the CUDA kernels' whole-column lists)
                 const int cap = (g.l2cuda ? nz : zmax + 1) * n2;
+                float ez = 0.0f;
+                if constexpr (kFar) {
+                    ez = scaled ? par_ez(m.e1x, m.e1y, m.e1z, m.e2x, m.e2y, m.e2z, m.inv_det) : 3.0e38f;
+                    r.delta = par_delta_far(r, ox0, oy0, gx, gy, n2, sc);
+                    r.mu = par_mu_far(ez, sc, nz * n2);
+                }
                 bool meets = true;
                 if (most > (uint32_t)Wn) {
                     // some toggle may fall into this window's slots
@@ -2641,11 +2680,11 @@ __device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB, V>& L, int wv,
                     };
                     meets = upto(lmin) <= chi && upto(lmax) > clo;
                 }
-                const int nq = meets ? par_rows(r, oy0, sc.sy, n2, sc.dy, q0) : 0;
+                const int nq = !meets ? 0 : kFar ? par_rows_far(r, L.oy, sc.sy, n2, q0) : par_rows(r, oy0, sc.sy, n2, sc.dy, q0);
                 P = nq > 0 ? (uint32_t)nq : 0u;
                 E[lane][0] = make_float4(m.e1x, m.e1y, m.e1z, m.e2x);
                 E[lane][1] = make_float4(m.e2y, m.e2z, m.inv_det, tv[0]);
-                E[lane][2] = make_float4(tv[1], r.dz, r.mu, r.delta);
+                E[lane][2] = make_float4(tv[1], r.dz, kFar ? ez : r.mu, r.delta);   // (the pairs make mu of ez)
                 E[lane][3] = make_float4(__int_as_float(r.l0), __int_as_float(cap), __int_as_float(c), tv[2]);
             }
             const uint32_t incl = wave_incl_scan<uint32_t>(P);
@@ -2664,7 +2703,8 @@ __device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB, V>& L, int wv,
                     r.e1x = a.x; r.e1y = a.y; r.e2x = a.w;
                     r.e2y = b.x; r.inv = b.z; r.v1x = b.w;
                     r.v1y = d.x; r.delta = d.w;
-                    np = par_cols(r, L.ox[c * n2], L.oy[0], gx, gy, n2, q, p0);
+                    np = kFar ? par_cols_far(r, L.ox + c * n2, L.oy[q], gx, n2, p0)
+                              : par_cols(r, L.ox[c * n2], L.oy[0], gx, gy, n2, q, p0);
                     np = np > 0 ? np : 0;
                 }
                 const uint32_t pincl = wave_incl_scan<uint32_t>((uint32_t)np);
@@ -2690,7 +2730,12 @@ __device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB, V>& L, int wv,
                             ParEntry r;
                             r.e1z = a.z; r.e2z = b.y; r.dz = d.y; r.mu = d.z;
                             r.l0 = __float_as_int(f.x);
+                            if (kFar) r.mu = par_mu_far(d.z, sc, nz * n2);
                             par_layers(r, u, vv, sc.sz, __float_as_int(f.y), la, lb);
+                            if (kFar && lb - la > 1) {
+                                const float zc = (u * a.z + vv * b.y) - 1.0e-6f;
+                                par_narrow(rz, n2, inv_n2, f.w, zc - 2.0f * d.z, zc + 2.0f * d.z, la, lb);
+                            }
                         }
                         uint32_t clo = lo[0], chi = hi[0];
 #pragma unroll
@@ -2822,8 +2867,8 @@ __device__ __forceinline__ void l2_parity_columns_wave(L2PLds<KB, V>& L, int wv,
 
 // W waves a block: each with columns of its own (V = 1), or all with the same (V = W), those
 // of H's list if there is one
-template <bool kM, int KB, int W, int V>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(V > 1 ? 5 : W == 1 ? 6 : 3))) void k_l2_parity(const uint64_t* __restrict__ bnd,
+template <bool kM, int KB, int W, int V, bool kFar>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(V > 1 || kFar ? 5 : W == 1 ? 6 : 3))) void k_l2_parity(const uint64_t* __restrict__ bnd,
                                                       const uint32_t* __restrict__ wprefix,
                                                       const uint64_t* __restrict__ occ, int64_t nwaves, bool many, int nw,
                                                       const uint32_t* __restrict__ coff,
@@ -2856,15 +2901,15 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(V > 1 ? 
         const uint32_t cw0 = kM ? M.off[mesh].cw0 : 0;
         uint64_t* out = par2 + (kM ? M.rank[mesh].l2w0 : 0);
         if (C == 2)
-            l2_parity_columns_wave<2>(s_l[grp], wv, (uint32_t)wave, H, cb, nw, g, i1, j1, word0, col0, b0, cw0, occ, bnd, wprefix, coff, ent, tris, out);
+            l2_parity_columns_wave<2, KB, V, kFar>(s_l[grp], wv, (uint32_t)wave, H, cb, nw, g, i1, j1, word0, col0, b0, cw0, occ, bnd, wprefix, coff, ent, tris, out);
         else if (C == 4)
-            l2_parity_columns_wave<4>(s_l[grp], wv, (uint32_t)wave, H, cb, nw, g, i1, j1, word0, col0, b0, cw0, occ, bnd, wprefix, coff, ent, tris, out);
+            l2_parity_columns_wave<4, KB, V, kFar>(s_l[grp], wv, (uint32_t)wave, H, cb, nw, g, i1, j1, word0, col0, b0, cw0, occ, bnd, wprefix, coff, ent, tris, out);
         else
-            l2_parity_columns_wave<1>(s_l[grp], wv, (uint32_t)wave, H, cb, nw, g, i1, j1, word0, col0, b0, cw0, occ, bnd, wprefix, coff, ent, tris, out);
+            l2_parity_columns_wave<1, KB, V, kFar>(s_l[grp], wv, (uint32_t)wave, H, cb, nw, g, i1, j1, word0, col0, b0, cw0, occ, bnd, wprefix, coff, ent, tris, out);
     }
 }
 
-template <int KB, int W, int V = 1>
+template <int KB, int W, int V = 1, bool kFar = false>
 static void launch_l2_parity_w(const uint64_t* bnd, const uint32_t* wprefix, const uint64_t* occ, int64_t nwaves, bool many, int nzmax,
                                const uint32_t* coff, const uint2* ent, const float* tris, const GridDev& g0, const Meshes& M,
                                const L2Heavy& H, uint64_t* par2, hipStream_t s)
@@ -2877,24 +2922,25 @@ static void launch_l2_parity_w(const uint64_t* bnd, const uint32_t* wprefix, con
     const int nw = (nzmax + 63) / 64;
     const size_t lds = (size_t)G * 6 * nw * sizeof(uint64_t);
     if (M.nm > 1)
-        k_l2_parity<true, KB, W, V><<<blocks, 64 * W, lds, s>>>(bnd, wprefix, occ, nwaves, many, nw, coff, ent, tris, g0, M, H, par2);
+        k_l2_parity<true, KB, W, V, kFar><<<blocks, 64 * W, lds, s>>>(bnd, wprefix, occ, nwaves, many, nw, coff, ent, tris, g0, M, H, par2);
     else
-        k_l2_parity<false, KB, W, V><<<blocks, 64 * W, lds, s>>>(bnd, wprefix, occ, nwaves, many, nw, coff, ent, tris, g0, M, H, par2);
+        k_l2_parity<false, KB, W, V, kFar><<<blocks, 64 * W, lds, s>>>(bnd, wprefix, occ, nwaves, many, nw, coff, ent, tris, g0, M, H, par2);
 }
 
 template <int KB>
 static void launch_l2_parity_k(const uint64_t* bnd, const uint32_t* wprefix, const uint64_t* occ, int64_t nwaves, bool many, int nzmax,
                                const uint32_t* coff, const uint2* ent, const float* tris, int waves, const GridDev& g0, const Meshes& M,
-                               const L2Heavy& H, uint64_t* par2, hipStream_t s)
+                               const L2Heavy& H, bool far, uint64_t* par2, hipStream_t s)
 {
-    if (waves <= 1) launch_l2_parity_w<KB, 1>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, g0, M, H, par2, s);
+    if (far) launch_l2_parity_w<KB, 1, 1, true>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, g0, M, H, par2, s);
+    else if (waves <= 1) launch_l2_parity_w<KB, 1>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, g0, M, H, par2, s);
     else if (waves == 2) launch_l2_parity_w<KB, 2>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, g0, M, H, par2, s);
     else launch_l2_parity_w<KB, 4>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, g0, M, H, par2, s);
 }
 
 void launch_l2_parity(const uint64_t* bnd, const uint32_t* wprefix, const uint64_t* occ, int64_t nwaves, bool many, int n2max, int nzmax,
                       const uint32_t* coff, const uint2* ent, const float* tris, int waves, const GridDev& g0, const Meshes& M,
-                      const L2Heavy& H, uint64_t* par2, hipStream_t s)
+                      const L2Heavy& H, bool far, uint64_t* par2, hipStream_t s)
 {
     if (nwaves <= 0) return;
     // Up to 1,024 columns the chip holds four waves for each, with room for 128 boundary
@@ -2902,8 +2948,12 @@ void launch_l2_parity(const uint64_t* bnd, const uint32_t* wprefix, const uint64
     // window of a tall column stages all of its entries (rods of 12 x 12 columns: 512 layers at
     // n2 = 16 816 -> 338 us in all, 2,048 at 8 742 -> 720; 200,000 triangles at 8/16 772 -> 589; eight
     // waves the same or slower)
+    auto share = [&](const L2Heavy& list) {
+        if (far) launch_l2_parity_w<16384, L2P_SHARE, L2P_SHARE, true>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, g0, M, list, par2, s);
+        else launch_l2_parity_w<16384, L2P_SHARE, L2P_SHARE>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, g0, M, list, par2, s);
+    };
     if (nwaves <= 1024) {
-        launch_l2_parity_w<16384, L2P_SHARE, L2P_SHARE>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, g0, M, L2Heavy{}, par2, s);
+        share(L2Heavy{});
         return;
     }
     // More columns: a wave takes its own, with room for 31 voxels at n2 = 8 and 7 at 16 (four
@@ -2911,11 +2961,10 @@ void launch_l2_parity(const uint64_t* bnd, const uint32_t* wprefix, const uint64
     // which would outlast all others: 2,000 overlapping triangles in a tenth of a 256/8 grid
     // 1.63 -> 0.54 ms, of a 512/16 one 8.1 -> 3.0
     if (n2max <= 8)
-        launch_l2_parity_k<2048>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, waves, g0, M, H, par2, s);
+        launch_l2_parity_k<2048>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, waves, g0, M, H, far, par2, s);
     else
-        launch_l2_parity_k<4096>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, waves, g0, M, H, par2, s);
-    if (H.list)
-        launch_l2_parity_w<16384, L2P_SHARE, L2P_SHARE>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, g0, M, H, par2, s);
+        launch_l2_parity_k<4096>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, waves, g0, M, H, far, par2, s);
+    if (H.list) share(H);
 }
 
 // ---------------------------------------------------------------------------

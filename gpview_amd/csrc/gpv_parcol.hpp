@@ -159,6 +159,101 @@ __host__ __device__ __forceinline__ void par_layers(const ParEntry& r, float u, 
     lb = lb < 0 ? 0 : lb > cap ? cap : lb;
 }
 
+// ---------------------------------------------------------------------------
+// Grids far from the origin (as for the SAT, gpv_satrow.hpp: the tables' deviation from
+// equal steps is whole sub-voxels).  These take the origins themselves: `delta`
+// without the deviation, rows and columns by the tables (within a voxel
+// non-decreasing), and of par_layers' [la, lb) the layers that Level1's comparison
+// decides (par_l1_layers).
+// ---------------------------------------------------------------------------
+__host__ __device__ __forceinline__ float par_delta_far(const ParEntry& r, float ox0, float oy0, float gx, float gy, int n2,
+                                                        const SatScale& g)
+{
+    const float wide = fminf(2.0f * fmaxf(g.dx, g.dy) + 1.0f, 1e8f);   // the column is at most n2 and this wide
+    const SatScale f = sat_scale_far(g);
+    return f.dx >= 0.0f && f.dy >= 0.0f ? par_delta(r, ox0, oy0, gx, gy, n2 + (int)wide, f.dx, f.dy) : 3.0e38f;
+}
+
+// margin of the crossing in layers, of `layers` in the grid.  The origins lie within 2 U cmax + U ext
+// of bmin + k g1 + (r + 1/2) g2 (8 U cmax in the CUDA kernels' expression), par_oz within U cmax + 2 U ext, and
+// g1 within U of n2 g2: with ext = `layers` g2, less than 1.5 dz and 4 U `layers` together.
+__host__ __device__ __forceinline__ float par_mu_far(float ez, const SatScale& g, int layers)
+{
+    const bool ok = g.dx >= 0.0f && g.dy >= 0.0f && g.dz >= 0.0f;
+    return ok ? fminf(ez * g.sz, 3.0e38f) + (1.5f * g.dz + 0x1p-21f * (float)layers) : 3.0e38f;
+}
+
+// rows [q0, q0 + n) that can hold an accepted sub-column; oy: the column's n2 origins
+__host__ __device__ __forceinline__ int par_rows_far(const ParEntry& r, const float* oy, float sy, int n2, int& q0)
+{
+    constexpr float U = 0x1p-24f;
+    const float y = (r.v1y - oy[0]) * sy, a = r.e1y * sy, b = r.e2y * sy;
+    const float lo = y + fminf(fminf(a, b), 0.0f), hi = y + fmaxf(fmaxf(a, b), 0.0f);
+    const float grow = 4.0f * r.delta * (fabsf(a) + fabsf(b)) + 16.0f * U * (fabsf(y) + fabsf(a) + fabsf(b)) + 0.01f;
+    // written so that a NaN leaves the row range whole
+    int f = 0, n = n2;
+    while (f < n2 && (oy[f] - oy[0]) * sy < lo - grow) ++f;
+    while (n > f && (oy[n - 1] - oy[0]) * sy > hi + grow) --n;
+    q0 = f;
+    return n - f;
+}
+
+// columns [p0, p0 + n) of the row at height oyq that can be accepted; ox: the column's n2 origins
+__host__ __device__ __forceinline__ int par_cols_far(const ParEntry& r, const float* ox, float oyq, float gx, int n2, int& p0)
+{
+    const float tx = ox[0] - r.v1x, ty = oyq - r.v1y;
+    const float a0 = (r.e2x * ty - r.e2y * tx) * r.inv, a1 = -(r.e2y * r.inv) * gx;
+    const float b0 = (r.e1y * tx - r.e1x * ty) * r.inv, b1 = (r.e1y * r.inv) * gx;
+    float lo = 0.0f, hi = 1e30f;
+    par_bound(a0 + r.delta, a1, lo, hi);
+    par_bound(b0 + r.delta, b1, lo, hi);
+    par_bound((1.0f + 2.0f * r.delta) - (a0 + b0), -(a1 + b1), lo, hi);
+    lo = (lo - 0.01f) * gx;
+    hi = (hi + 0.01f) * gx;
+    int f = 0, n = n2;
+    while (f < n2 && ox[f] - ox[0] < lo) ++f;
+    while (n > f && ox[n - 1] - ox[0] > hi) --n;
+    p0 = f;
+    return n - f;
+}
+
+// Of the layers [la, lb) of the origin table rz, those at the lower end that pass for
+// certain and those at the upper end that do not, taken off: a layer passes where
+// rz - v1z < lo and does not where it is > hi.  Across voxels the table may step back,
+// so each voxel's layers are searched by themselves.
+__host__ __device__ __forceinline__ void par_narrow(const float* rz, int n2, float inv_n2, float v1z, float lo, float hi,
+                                                    int& la, int& lb)
+{
+    while (la < lb) {
+        const int end = ((int)(((float)la + 0.5f) * inv_n2) + 1) * n2, e = end < lb ? end : lb;
+        if (rz[e - 1] - v1z < lo) {
+            la = e;
+            continue;
+        }
+        int b = e - 1;
+        while (la < b) {
+            const int m = (la + b) >> 1;
+            if (rz[m] - v1z < lo) la = m + 1;
+            else b = m;
+        }
+        break;
+    }
+    while (lb > la) {
+        const int beg = (int)(((float)(lb - 1) + 0.5f) * inv_n2) * n2, s = beg > la ? beg : la;
+        if (rz[s] - v1z > hi) {
+            lb = s;
+            continue;
+        }
+        int a = s + 1;
+        while (a < lb) {
+            const int m = (a + lb) >> 1;
+            if (rz[m] - v1z > hi) lb = m;
+            else a = m + 1;
+        }
+        break;
+    }
+}
+
 // Level1: the same crossing against the layers of a grid's column.  Layers [0, la)
 // of the ray-origin table r1z (nz, non-decreasing) pass for certain, none from
 // lb on.  The layers are compared as the float test's own T.z = fl(o.z - v1.z), so

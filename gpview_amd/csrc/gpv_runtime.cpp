@@ -317,6 +317,7 @@ struct Job {
     uint64_t *st_off = nullptr, *st_scan = nullptr, *st_tog = nullptr;
     uint64_t *sat2 = nullptr, *par2 = nullptr;
     int n2max = 0, nzmax = 0;
+    bool far2 = false;            // some mesh's Level2 tables deviate from equal steps (level2_far)
     // normals (meshes with params.normals): face normals, sorted bins, and the
     // resident results per boundary voxel / per Level2 voxel
     bool any_normals = false;
@@ -654,6 +655,7 @@ int job_create(gpv_ctx* c, const gpv_mesh_desc* d, int nm, int on_device, Job** 
         J->info[m].has_normals = g.normals;
         J->any_normals = J->any_normals || g.normals;
         J->n2max = std::max(J->n2max, g.n2);
+        J->far2 = J->far2 || level2_far(g);
         J->nzmax = std::max(J->nzmax, g.nz);
         J->off[m].word0 = word0;
         J->off[m].col0 = col0;
@@ -1112,7 +1114,7 @@ int l2_parity_kernels(Job* J, hipStream_t s)
     J->heavy_cleared = false;
     if (J->B > 0)
         launch_l2_parity(J->bnd, J->wprefix, J->col_occ, J->l2p_waves, J->ncol >= kL2ParityMany, J->n2max, J->nzmax, J->coff, J->cent,
-                         J->tris, J->ctx->tune.l2_parity_waves, J->g[0], J->view(), J->heavy, J->par2, s);
+                         J->tris, J->ctx->tune.l2_parity_waves, J->g[0], J->view(), J->heavy, J->far2, J->par2, s);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipEventRecord(J->ev[11], s));
     return GPV_OK;
@@ -1134,7 +1136,7 @@ int l2_sat_kernels(Job* J)
     hipStream_t s = J->ctx->stream;
     HIP_TRY(hipEventRecord(J->ev[6], s));
     launch_l2_sat(J->tris, J->bidx, J->B, J->l2s_groups, J->l2s_most, J->boff, J->list,
-                  J->n2max, J->ctx->tune.l2_sat_waves, J->g[0], J->view(), J->sat2, s);
+                  J->n2max, J->far2, J->ctx->tune.l2_sat_waves, J->g[0], J->view(), J->sat2, s);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipEventRecord(J->ev[7], s));
     return GPV_OK;

@@ -244,16 +244,14 @@ __host__ __device__ __forceinline__ void sat_row_range(const float4* e, int q, b
     p = keep ? p : p1;
 }
 
-// Row q with layers [ra, rb], positioned at column p.
-__host__ __device__ __forceinline__ SatRow sat_row_at(const float4* e, int q, int ra, int rb, int p)
+// The row at height y with layers from `zlo` below `zhi`, positioned at x.
+__host__ __device__ __forceinline__ SatRow sat_row_xy(const float4* e, float y, float zlo, float zhi, float x)
 {
     SatRow s;
     const float4 c6 = e[6], c7 = e[7], c8 = e[8], pl = e[9];
-    const float y = (float)q;
     const float u0 = c7.x * y + c8.x, u1 = c7.y * y + c8.y, u2 = c7.z * y + c8.z;
-    const float x = (float)p;
-    s.lom = s.loi = (float)ra;
-    s.him = s.hii = (float)rb + 1.0f;
+    s.lom = s.loi = zlo;
+    s.him = s.hii = zhi;
 #ifdef __HIP_DEVICE_COMPILE__
 #pragma unroll
 #endif
@@ -275,6 +273,12 @@ __host__ __device__ __forceinline__ SatRow sat_row_at(const float4* e, int q, in
     return s;
 }
 
+// Row q with layers [ra, rb], positioned at column p.
+__host__ __device__ __forceinline__ SatRow sat_row_at(const float4* e, int q, int ra, int rb, int p)
+{
+    return sat_row_xy(e, (float)q, (float)ra, (float)rb + 1.0f, (float)p);
+}
+
 // A row of a loose entry (nothing of it is bounded): all layers of its columns undecided,
 // none certain.  Every term is set: an entry is loose where its coefficients may be
 // infinite or NaN, those of the (x, y) predicates among them.
@@ -291,6 +295,50 @@ __host__ __device__ __forceinline__ void sat_row_loose(SatRow& s, bool loose, in
     s.e0 = s.e1 = s.e2 = 0.0f;
     s.u0 = s.u1 = s.u2 = 0.0f;
     s.um = 3e38f;
+}
+
+// ---------------------------------------------------------------------------
+// Grids far from the origin.  There a float hardly tells one sub-center from the
+// next, `dev` is whole sub-voxels, and rows that count positions in equal steps
+// leave most boxes undecided.  These take the sub-centers themselves instead: the voxel's
+// positions X, Y (from its first center, in sub-voxels) and Z (one up, as the
+// entry's layers), 16 each, non-decreasing (within a voxel every step of the tables' expressions
+// is monotone), infinite past n2.  What `dev` paid for is gone but for the
+// positions' own rounding, 3 U of at most 16 + 2 dev.  A row steps by
+// slope * (X[p + 1] - X[p]), two roundings more per addition: at most 4 U S.
+// ---------------------------------------------------------------------------
+__host__ __device__ __forceinline__ SatScale sat_scale_far(SatScale g)
+{
+    // (dev < 0 stays what it is: loose)
+    g.dx = g.dx >= 0.0f ? 0x1p-24f * (256.0f + 32.0f * g.dx) : g.dx;
+    g.dy = g.dy >= 0.0f ? 0x1p-24f * (256.0f + 32.0f * g.dy) : g.dy;
+    g.dz = g.dz >= 0.0f ? 0x1p-24f * (256.0f + 32.0f * g.dz) : g.dz;
+    return g;
+}
+
+// how many of the 2 * half (8 or 16) positions are at most x
+__host__ __device__ __forceinline__ int sat_count_le(const float* pos, int half, float x)
+{
+    int i = 0;
+    for (int s = half; s; s >>= 1) i += pos[i + s - 1] <= x ? s : 0;
+    return i + (pos[i] <= x ? 1 : 0);
+}
+
+// sat_row_range for the row at height y
+__host__ __device__ __forceinline__ void sat_row_range_far(const float4* e, float y, const float* X, int half, bool keep,
+                                                           int& p, int& left)
+{
+    const float4 c6 = e[6], c7 = e[7], c8 = e[8];
+    const float u0 = c7.x * y + c8.x, u1 = c7.y * y + c8.y, u2 = c7.z * y + c8.z;
+    const float lim = 1.0f + c6.w;
+    float lo = -1e30f, hi = 1e30f;
+    sat_x_range(c6.x, u0, lim, lo, hi);
+    sat_x_range(c6.y, u1, lim, lo, hi);
+    sat_x_range(c6.z, u2, lim, lo, hi);
+    const int a = sat_count_le(X, half, lo - 0.01f), b = sat_count_le(X, half, hi + 0.01f);
+    const int p1 = a > p ? a : p, pe = b < p + left ? b : p + left;
+    left = keep ? left : pe - p1;
+    p = keep ? p : p1;
 }
 
 // truncation that takes anything below 0 to 0
@@ -319,6 +367,28 @@ __host__ __device__ __forceinline__ void sat_row_column(SatRow& s, uint32_t& in,
     // layers [trunc(lo), trunc(hi)) with hi at most 16
     const uint32_t m = ~(~0u << sat_trunc(him)) & (~0u << sat_trunc(fminf(lom, 16.0f)));
     const uint32_t n = ~(~0u << sat_trunc(hii)) & (~0u << sat_trunc(fminf(loi, 16.0f)));
+    may = !(u > s.um) ? m : 0u;
+    in = u < -s.um ? n : 0u;
+}
+
+// The same far from the origin, for the layers of `rows` (a bit each); the row was set up
+// with layers of any height, `step` is X[p + 1] - X[p].
+__host__ __device__ __forceinline__ void sat_row_column_far(SatRow& s, const float* Z, int half, uint32_t rows, float step,
+                                                            uint32_t& in, uint32_t& may)
+{
+    const float lom = fmaxf(fmaxf(s.w0 - s.m0, s.w1 - s.m1), fmaxf(fmaxf(s.w2 - s.m2, s.pw - s.pm), s.lom));
+    const float loi = fmaxf(fmaxf(s.w0 - s.n0, s.w1 - s.n1), fmaxf(fmaxf(s.w2 - s.n2, s.pw - s.pn), s.loi));
+    const float him = fminf(fminf(s.w0 + s.m0, s.w1 + s.m1), fminf(fminf(s.w2 + s.m2, s.pw + s.pm), s.him));
+    const float hii = fminf(fminf(s.w0 + s.n0, s.w1 + s.n1), fminf(fminf(s.w2 + s.n2, s.pw + s.pn), s.hii));
+    const float u = fmaxf(fmaxf(fabsf(s.u0), fabsf(s.u1)), fabsf(s.u2)) - 1.0f;
+    s.w0 += s.a0 * step; s.w1 += s.a1 * step; s.w2 += s.a2 * step; s.pw += s.pa * step;
+    s.u0 += s.e0 * step; s.u1 += s.e1 * step; s.u2 += s.e2 * step;
+    const int a = sat_count_le(Z, half, lom), b = sat_count_le(Z, half, him);
+    int c = a, d = b;
+    while (c < d && Z[c] <= loi) ++c;
+    while (d > c && Z[d - 1] > hii) --d;
+    const uint32_t m = ~(~0u << b) & (~0u << a) & rows;
+    const uint32_t n = ~(~0u << d) & (~0u << c) & rows;
     may = !(u > s.um) ? m : 0u;
     in = u < -s.um ? n : 0u;
 }

@@ -97,6 +97,58 @@ extern "C" void satrow_pieces(int64_t n, int n2, int piece, const float* tv, con
     }
 }
 
+// satrow_pieces with the positions taken from the tables (grids far from the origin).
+extern "C" void satrow_far(int64_t n, int n2, int piece, const float* tv, const float* cx, const float* cy, const float* cz,
+                           const float* lo, const float* hi, const float* g2, const float* h, int cuda_l2,
+                           uint32_t* in, uint32_t* may, uint8_t* is_loose)
+{
+    const int half = n2 > 8 ? 8 : 4;
+    for (int64_t i = 0; i < n; ++i) {
+        const float* t = tv + 9 * i;
+        const float* C[3] = {cx + n2 * i, cy + n2 * i, cz + n2 * i};
+        gpv::SatScale g;
+        gpv::sat_scale_axis(lo[3 * i], hi[3 * i], g2[3 * i], cuda_l2 != 0, g.sx, g.dx);
+        gpv::sat_scale_axis(lo[3 * i + 1], hi[3 * i + 1], g2[3 * i + 1], cuda_l2 != 0, g.sy, g.dy);
+        gpv::sat_scale_axis(lo[3 * i + 2], hi[3 * i + 2], g2[3 * i + 2], cuda_l2 != 0, g.sz, g.dz);
+        float pos[3][16];
+        const float s[3] = {g.sx, g.sy, g.sz};
+        int end[3][2];
+        for (int a = 0; a < 3; ++a) {
+            end[a][0] = n2;
+            end[a][1] = -1;
+            for (int p = 0; p < 16; ++p) {
+                pos[a][p] = p < n2 ? (C[a][p] - C[a][0]) * s[a] + (a == 2 ? 1.0f : 0.0f) : __builtin_inff();
+                if (p < n2 && axis_ok(t[a], t[3 + a], t[6 + a], C[a][p], h[3 * i + a])) {
+                    end[a][0] = p < end[a][0] ? p : end[a][0];
+                    end[a][1] = p;
+                }
+            }
+        }
+        const int pa = end[0][0], pb = end[0][1], ra = end[2][0], rb = end[2][1];
+        const gpv::SatScale f = gpv::sat_scale_far(g);
+        float4 e[gpv::kSatEntry4];
+        bool loose = gpv::sat_entry_part(0, t, C[0][0], C[1][0], C[2][0], f, e);
+        loose = gpv::sat_entry_part(1, t, C[0][0], C[1][0], C[2][0], f, e) || loose;
+        is_loose[i] = loose;
+        for (int q = 0; q < n2; ++q) {
+            uint32_t* oi = in + (int64_t)(i * n2 + q) * n2;
+            uint32_t* om = may + (int64_t)(i * n2 + q) * n2;
+            for (int p = 0; p < n2; ++p) oi[p] = om[p] = 0;
+            if (pb < 0 || rb < 0 || q < end[1][0] || q > end[1][1]) continue;
+            int p = pa, left = pb - pa + 1;
+            gpv::sat_row_range_far(e, pos[1][q], pos[0], half, loose, p, left);
+            for (; left > 0; p += piece, left -= piece) {
+                gpv::SatRow r = gpv::sat_row_xy(e, pos[1][q], -1e9f, 1e9f, pos[0][p]);
+                gpv::sat_row_loose(r, loose, -1, 1 << 30);
+                const int m = left < piece ? left : piece;
+                for (int k = 0; k < m; ++k)
+                    gpv::sat_row_column_far(r, pos[2], half, (2u << rb) - (1u << ra), k + 1 < m ? pos[0][p + k + 1] - pos[0][p + k] : 0.0f,
+                                            oi[p + k], om[p + k]);
+            }
+        }
+    }
+}
+
 // Level1: case i's index AABB (lo, dd: 3 ints each) on a grid with centers
 // cx/cy/cz, bounds lo3/hi3 and voxel g1; per column of it in (q, p) order from
 // off[i]: [am, ai, bi, bm).
