@@ -355,9 +355,9 @@ inline L2Heavy l2_heavy(uint64_t ncols, int64_t ncol, int64_t nwaves)
     const uint64_t above = 4 * mean > 128 ? 4 * mean : 128;
     return L2Heavy{nullptr, nullptr, (uint32_t)above, nwaves < 16384 ? 0 : (int64_t)(ncols / (above + 1))};
 }
-// n2max, nzmax: the largest Level2 resolution and layer count of the run; occ: the
+// B boundary voxels; n2max, nzmax: the largest Level2 resolution and layer count of the run; occ: the
 // columns that hold boundary voxels (or nullptr)
-void launch_l2_parity(const uint64_t* bnd, const uint32_t* wprefix, const uint64_t* occ, int64_t nwaves, bool many,
+void launch_l2_parity(const uint64_t* bnd, const uint32_t* wprefix, const uint64_t* occ, int64_t B, int64_t nwaves, bool many,
                       int n2max, int nzmax, const uint32_t* coff, const uint2* ent, const float* tris, int waves,
                       const GridDev& g0, const Meshes& M, const L2Heavy& H, bool far, uint64_t* par2, hipStream_t s);
 

@@ -2487,8 +2487,8 @@ void launch_l2_sat(const float* tris, const int32_t* bidx, int64_t B, int64_t ng
 //
 // A column of several windows looks up each window's voxels in the 64-layer words that hold
 // them (28,000 columns of 16,000 layers at n2 = 4 28.3 -> 6.5 ms with every word scanned once).
-// A wave per voxel is still the faster way in few columns of thousands of layers at n2 = 16 (by a
-// quarter).
+// A wave per voxel is still the faster way in a few hundred columns of thousands of layers at
+// n2 = 16 (by a quarter).
 //
 // What bounds it: the chain of dependent LDS and global reads of each wave
 // (VALU issue 0.39-0.47), hence one wave per block (an empty column's wave
@@ -2951,7 +2951,7 @@ static void launch_l2_parity_k(const uint64_t* bnd, const uint32_t* wprefix, con
     else launch_l2_parity_w<KB, 4>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, g0, M, H, par2, s);
 }
 
-void launch_l2_parity(const uint64_t* bnd, const uint32_t* wprefix, const uint64_t* occ, int64_t nwaves, bool many, int n2max, int nzmax,
+void launch_l2_parity(const uint64_t* bnd, const uint32_t* wprefix, const uint64_t* occ, int64_t B, int64_t nwaves, bool many, int n2max, int nzmax,
                       const uint32_t* coff, const uint2* ent, const float* tris, int waves, const GridDev& g0, const Meshes& M,
                       const L2Heavy& H, bool far, uint64_t* par2, hipStream_t s)
 {
@@ -2965,7 +2965,11 @@ void launch_l2_parity(const uint64_t* bnd, const uint32_t* wprefix, const uint64
         if (far) launch_l2_parity_w<16384, L2P_SHARE, L2P_SHARE, true>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, g0, M, list, par2, s);
         else launch_l2_parity_w<16384, L2P_SHARE, L2P_SHARE>(bnd, wprefix, occ, nwaves, many, nzmax, coff, ent, tris, g0, M, list, par2, s);
     };
-    if (nwaves <= 1024) {
+    // So they do where a column takes more than eight windows of a wave's own on average (rods of 1,200
+    // columns and 4,096 layers at n2 = 16 3.75 -> 1.82 ms, 1,100 and 8,192 at 8 3.38 -> 1.99; 7,488
+    // and 8,192 at 8, seven windows, 3.00 -> 3.35)
+    const int64_t slot = (int64_t)n2max * n2max * (n2max > 8 ? 2 : 1);   // bytes of a boundary voxel
+    if (nwaves <= 1024 || B * slot > 8 * (n2max <= 8 ? 2048 : 4096) * nwaves) {
         share(L2Heavy{});
         return;
     }

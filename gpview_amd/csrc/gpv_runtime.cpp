@@ -1113,7 +1113,7 @@ int l2_parity_kernels(Job* J, hipStream_t s)
     if (!J->heavy_cleared) launch_fill_u32(J->heavy.count, 0, 1, s);   // a parity made again
     J->heavy_cleared = false;
     if (J->B > 0)
-        launch_l2_parity(J->bnd, J->wprefix, J->col_occ, J->l2p_waves, J->ncol >= kL2ParityMany, J->n2max, J->nzmax, J->coff, J->cent,
+        launch_l2_parity(J->bnd, J->wprefix, J->col_occ, J->B, J->l2p_waves, J->ncol >= kL2ParityMany, J->n2max, J->nzmax, J->coff, J->cent,
                          J->tris, J->ctx->tune.l2_parity_waves, J->g[0], J->view(), J->heavy, J->far2, J->par2, s);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipEventRecord(J->ev[11], s));
